@@ -385,20 +385,45 @@ int wait_done(exh_context *c) {
   return e == hipSuccess ? 0 : hip_fail(c, e, "waiting for queued work");
 }
 
-// Constants and scratch of the split-precision path for nmod moduli.
-int oz_prepare(exh_context *c, int nmod, OzLayout &L, int &bits) {
-  L = oz_layout(c->ngkmax, c->Ktot, nmod);
-  bits = oz_bits(nmod, c->Ktot);
-  if (!c->oz_consts) {
-    hipError_t e = oz_upload_constants(nmod);
-    if (e != hipSuccess) return hip_fail(c, e, "split: constants");
-    c->oz_consts = true;
+// The modular contraction of a setup with these flags (EXH_SPLIT(n)).
+OzPlan oz_plan(const exh_context *c, int flags) {
+  (void)c;
+  const int n = (flags >> 8) & 0xff;
+  return n ? oz_split(n) : OzPlan();
+}
+
+bool oz_fits(const exh_context *c, const OzLayout &L) {
+  return c->ozq.bytes >= L.q_bytes * L.nops && c->ozr.bytes >= L.r_bytes &&
+         c->oze.bytes >= L.e_bytes * L.nops;
+}
+
+// Plan, layout and scratch of the modular contraction; P.nmod = 0 when the
+// setup runs on the FP64 MFMA kernels instead, which is also where an FP64
+// setup goes when the device has no room for the residues or the stream is
+// being captured before the first call (nothing may be allocated then).
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, OzPlan &P, OzLayout &L) {
+  P = oz_plan(c, flags);
+  if (P.nmod == 0) return 0;
+  const bool split = (flags & 0xff00) != 0;
+  L = oz_layout(c->ngkmax, c->Ktot, P, only_o, c->have_h1aa);
+  if (oz_fits(c, L)) return 0;
+  if (!split) {
+    size_t avail = 0, total = 0;
+    const size_t need = L.q_bytes * L.nops + L.r_bytes + L.e_bytes * L.nops;
+    if (capturing || hipMemGetInfo(&avail, &total) != hipSuccess ||
+        avail < need + (size_t(1) << 30)) {
+      P = OzPlan();
+      return 0;
+    }
   }
-  int rc = ensure(c, c->ozqx, L.qx_bytes);
-  if (!rc) rc = ensure(c, c->ozqb, L.qb_bytes);
+  int rc = ensure(c, c->ozq, L.q_bytes * L.nops);
   if (!rc) rc = ensure(c, c->ozr, L.r_bytes);
-  if (!rc) rc = ensure(c, c->ozex, L.e_bytes);
-  if (!rc) rc = ensure(c, c->ozeb, L.e_bytes);
+  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops);
+  if (rc && !split) {  // another allocation took the room meanwhile
+    (void)hipGetLastError();
+    P = OzPlan();
+    return 0;
+  }
   return rc;
 }
 
@@ -409,8 +434,7 @@ int oz_prepare(exh_context *c, int nmod, OzLayout &L, int &bits) {
 // passes `scratch` itself to a kernel (on the host the name is only a
 // stand-in for the symbol): exh_create looks up each device's address once,
 // with that device current, and the entry point uses that address.
-constexpr size_t kNoallocScratchBytes = size_t(64) << 20;
-static __device__ __align__(256) unsigned char scratch[kNoallocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[exh::kNoallocScratchBytes];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -487,7 +511,7 @@ void exh_destroy(exh_context *c) {
                     &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu, &c->mt_match.piv,
                     &c->aa, &c->loa, &c->lolo, &c->salo, &c->ololo_eff, &c->h1aa,
                     &c->ivg, &c->ivgig, &c->ist, &c->cf_stage, &c->vf_stage, &c->mf_stage,
-                    &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->ozqx, &c->ozqb, &c->ozr, &c->ozex, &c->ozeb, &c->s_apwalm, &c->s_igpig,
+                    &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->ozq, &c->ozr, &c->oze, &c->s_apwalm, &c->s_igpig,
                     &c->s_vgpc, &c->s_h, &c->s_o, &c->s_gpc, &c->s_tpgpc, &c->s_sfac,
                     &c->bbt, &c->bat, &c->ba2t, &c->bivgk, &c->ifz, &c->igeo, &c->i_in0,
                     &c->i_in1, &c->i_out0, &c->i_out1, &c->i_out2, &c->apwfr_d, &c->hml_fl,
@@ -788,6 +812,9 @@ int exh_match_device(exh_context *c, void *stream, int ngp, const double *gpc,
 struct SetupScratch {
   double2 *bt = nullptr, *a2t = nullptr, *at = nullptr;
   int4 *ivgk = nullptr;
+  // modular contraction (oz_prepare); plan.nmod = 0: the FP64 MFMA kernels
+  OzPlan plan;
+  OzLayout layout;
 };
 
 // The single-k setup.  o_only: overlapsetup.f90 alone -- O accumulated and
@@ -815,13 +842,12 @@ static int check_setup(exh_context *c, int ngp, int rank, const exh_z *apwalm, c
   return 0;
 }
 
-// Enqueue the FP64 kernels (and, with EXH_SPLIT, the split-precision stages,
-// whose scratch the caller has prepared with oz_prepare).  `record` brackets
-// each launch with the profiling events.
+// Enqueue the kernels of one setup on the scratch the caller has prepared.
+// `record` brackets each launch with the profiling events.
 static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const exh_z *apwalm,
                         const int *igpig, const double *vgpc, exh_z *h, exh_z *o, int flags,
                         bool o_only, const SetupScratch &w, bool record) {
-  const int nmod = (flags >> 8) & 0xff;
+  const int nmod = w.plan.nmod;
   const int ldb = (c->ngkmax + 63) / 64 * 64;
   exh_z *hw = o_only ? nullptr : h;  // H the kernels write
   auto run = [&](int k, auto &&launch) {
@@ -843,8 +869,6 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
                        vgpc, (double2 *)hw, (double2 *)o, rank, flags);
     });
   if (e == hipSuccess && nmod > 0) {
-    OzLayout L = oz_layout(c->ngkmax, c->Ktot, nmod);
-    const int bits = oz_bits(nmod, c->Ktot);
     long long ldx;
     const double2 *X = k_major_operand(c, A, w.at, &ldx);
     const int lo0 = c->intgv[0], lo1 = c->intgv[1], lo2 = c->intgv[2];
@@ -853,10 +877,9 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
     const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
     for (int st = 0; st < 3 && e == hipSuccess; st++)
       e = run(kid[st], [&] {
-        return launch_ozaki(s, c, ngp, X, ldx, w.bt, ldb, nmod, bits, L, (int8_t *)c->ozqx.p,
-                            (int8_t *)c->ozqb.p, (uint8_t *)c->ozr.p, (int *)c->ozex.p,
-                            (int *)c->ozeb.p, box, (double2 *)h, (double2 *)o, rank,
-                            flags & EXH_ACCUMULATE, 1 << st);
+        return launch_ozaki(s, c, ngp, w.plan, w.layout, oz_scratch(c), X, ldx, w.bt,
+                            c->have_h1aa ? w.a2t : nullptr, ldb, box, (double2 *)hw,
+                            (double2 *)o, rank, flags & EXH_ACCUMULATE, 1 << st);
       });
   }
   if (e == hipSuccess)
@@ -876,19 +899,17 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   int rc = check_setup(c, ngp, rank, apwalm, igpig, vgpc, h, o, flags, o_only);
   if (rc) return rc;
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-  const int nmod = (flags >> 8) & 0xff;
+  SetupScratch w;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) cap = hipStreamCaptureStatusNone;
   const size_t op = (size_t)std::max(c->Ktot, 1) * ((c->ngkmax + 63) / 64 * 64) * sizeof(double2);
   rc = o_only ? 0 : ensure(c, c->bt, op);
   if (!rc && c->have_h1aa) rc = ensure(c, c->a2t, op);
   if (!rc && !c->contig) rc = ensure(c, c->at, op);
   if (!rc) rc = ensure(c, c->ivgk, (size_t)std::max(c->ngkmax, 1) * sizeof(int4));
-  if (!rc && nmod > 0) {
-    OzLayout L;
-    int bits = 0;
-    rc = oz_prepare(c, nmod, L, bits);
-  }
+  if (!rc)
+    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, w.plan, w.layout);
   if (rc) return rc;
-  SetupScratch w;
   w.bt = (double2 *)c->bt.p;
   w.a2t = (double2 *)c->a2t.p;
   w.at = (double2 *)c->at.p;

@@ -59,16 +59,17 @@ void free_entry(exh_context::BatchEntry *E) {
   delete E;
 }
 
-// Upper tiles (I0 <= J0 + TMJ - 1) of the k-points [k0, k0 + nk), k-major
-// then J-major, k numbered from 0 within the group.  With xcd the list is
+// Upper tiles (I0 <= J0 + TMJ - 1) of those of the k-points [k0, k0 + nk)
+// that run on the H/O kernel (skip[i] = 0), k-major then J-major, k numbered
+// from 0 within the group.  With xcd the list is
 // split into 8 contiguous ranges and interleaved so that list position t
 // (which runs on XCD t % 8) walks range t % 8 in order; k < 0 pads.
-void build_tiles(const exh_kpoint *kp, int k0, int nk, int tmi, int tmj, bool xcd,
-                 std::vector<int4> &out) {
+void build_tiles(const exh_kpoint *kp, const std::vector<char> &skip, int k0, int nk, int tmi,
+                 int tmj, bool xcd, std::vector<int4> &out) {
   std::vector<int4> t;
   for (int kl = 0; kl < nk; kl++) {
     const int ngp = kp[k0 + kl].ngp;
-    if (ngp <= 0) continue;
+    if (ngp <= 0 || skip[k0 + kl]) continue;
     const int nI = (int)cdivl(ngp, tmi), nJ = (int)cdivl(ngp, tmj);
     for (int J = 0; J < nJ; J++)
       for (int I = 0; I < nI && I * tmi <= J * tmj + tmj - 1; I++)
@@ -102,8 +103,7 @@ uint64_t state_signature(const exh_context *c) {
                           &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu,
                           &c->mt_match.piv, &c->aa, &c->loa, &c->lolo, &c->salo,
                           &c->ololo_eff, &c->h1aa, &c->ivg, &c->ist, &c->bbt, &c->bat,
-                          &c->ba2t, &c->bivgk, &c->bmtab, &c->ozqx, &c->ozqb, &c->ozr, &c->ozex,
-                          &c->ozeb};
+                          &c->ba2t, &c->bivgk, &c->bmtab, &c->ozq, &c->ozr, &c->oze};
   for (const DevBuf *b : bufs) mix(&b->p, sizeof b->p);
   const int sc[] = {c->nspecies, c->natmtot, c->lmaxapw, c->lmaxmat, c->apwordmax, c->nlomax,
                     c->ngkmax, c->maxaa, c->maxnlo, c->nlotot, c->lmmax, c->Ktot,
@@ -214,9 +214,16 @@ CallContexts call_contexts(int nk, exh_context *const *kc) {
   return cc;
 }
 
+// Modular contraction of each context of a call (nmod = 0: FP64 MFMA tiles).
+struct OzParams {
+  std::vector<OzPlan> P;
+  std::vector<OzLayout> L;
+};
+
 exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
-                                     const exh_kpoint *kp, const CallContexts &cc, int plan,
-                                     int flags, std::vector<unsigned char> key, int *rc) {
+                                     const exh_kpoint *kp, const CallContexts &cc,
+                                     const OzParams &oz, int plan, int flags,
+                                     std::vector<unsigned char> key, int *rc) {
   *rc = 0;
   if (lead->bcache.size() >= kMaxEntries) {
     // the oldest entry may still be read by queued work on any stream
@@ -251,13 +258,15 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
   // k-points are grouped in order; a group closes when one of its contexts
   // has used all its scratch slots
   std::vector<int> cnt(nctx, 0), ingroup(nctx, 0);
+  std::vector<char> skip(nk);  // k-points on the modular contraction: no H/O tiles
+  for (int i = 0; i < nk; i++) skip[i] = oz.P[cc.kci[i]].nmod > 0;
   E->kd.resize(nk);
   exh_context::BatchEntry::Group g{};
   g.k0 = 0;
   auto close_group = [&](int kend) {
     g.dims.nk = kend - g.k0;
     g.t0 = (int)E->tiles.size();
-    build_tiles(kp, g.k0, g.dims.nk, S.tmi, S.tmj, P.xcd != 0, E->tiles);
+    build_tiles(kp, skip, g.k0, g.dims.nk, S.tmi, S.tmj, P.xcd != 0, E->tiles);
     g.nt = (int)E->tiles.size() - g.t0;
     long long nwg = g.nt;
     if (P.persistent) {
@@ -330,15 +339,9 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
   return E;
 }
 
-// Split-precision layout and bit count of each context of a call.
-struct OzParams {
-  std::vector<OzLayout> L;
-  std::vector<int> bits;
-};
-
 hipError_t enqueue(exh_context *lead, hipStream_t s, const exh_context::BatchEntry &E, int flags,
                    int plan, const OzParams &oz) {
-  const int nmod = (flags >> 8) & 0xff, acc = flags & EXH_ACCUMULATE;
+  const int acc = flags & EXH_ACCUMULATE;
   const PlanInfo P = plan_info(plan);
   const KDesc *kd0 = (const KDesc *)E.kd_d.p;
   const int4 *tiles = (const int4 *)E.tiles_d.p;
@@ -356,14 +359,16 @@ hipError_t enqueue(exh_context *lead, hipStream_t s, const exh_context::BatchEnt
       e = timed(lead, EXH_K_BT, s, [&] { return launch_bt_grouped(s, D, kd); });
     if (e == hipSuccess && D.any_a2t)
       e = timed(lead, EXH_K_A2T, s, [&] { return launch_a2t_grouped(s, D, kd); });
-    if (e == hipSuccess && nmod == 0)
+    if (e == hipSuccess && g.nt > 0)
       e = timed(lead, EXH_K_HOGRP, s, [&] {
         return launch_ho_grouped(s, P.shape, kd, tiles + g.t0, g.nt, g.nwg, acc);
       });
-    if (nmod > 0)
-      for (int i = g.k0; i < g.k0 + D.nk && e == hipSuccess; i++) {
+    // the k-points on the modular contraction, one after the other: they share
+    // their context's residue scratch
+    for (int i = g.k0; i < g.k0 + D.nk && e == hipSuccess; i++) {
         const KDesc &d = E.kd[i];
         const int j = E.kci[i];
+        if (oz.P[j].nmod == 0) continue;
         const exh_context *c = E.ctxs[j];
         const SDesc &S = E.sd[j];
         IstBox box{d.ivgk, d.vgpc, (const IstEntry *)c->ist.p, S.lo0, S.lo1, S.lo2,
@@ -371,12 +376,10 @@ hipError_t enqueue(exh_context *lead, hipStream_t s, const exh_context::BatchEnt
         const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
         for (int st = 0; st < 3 && e == hipSuccess; st++)
           e = timed(lead, kid[st], s, [&] {
-            return launch_ozaki(s, c, d.ngp, d.x, S.ldx, d.bt, S.ldb, nmod, oz.bits[j],
-                                oz.L[j], (int8_t *)c->ozqx.p, (int8_t *)c->ozqb.p,
-                                (uint8_t *)c->ozr.p, (int *)c->ozex.p, (int *)c->ozeb.p, box,
-                                d.h, d.o, d.ldh, acc, 1 << st);
+            return launch_ozaki(s, c, d.ngp, oz.P[j], oz.L[j], oz_scratch(c), d.x, S.ldx, d.bt,
+                                d.a2t, S.ldb, box, d.h, d.o, d.ldh, acc, 1 << st);
           });
-      }
+    }
     if (e == hipSuccess)
       e = timed(lead, EXH_K_LOBORDER, s,
                 [&] { return launch_lo_border_grouped(s, D, kd, acc); });
@@ -403,25 +406,21 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   const CallContexts cc = call_contexts(nk, kc);
   const size_t nctx = cc.ctxs.size();
   OzParams oz;
+  oz.P.resize(nctx);
   oz.L.resize(nctx);
-  oz.bits.assign(nctx, 0);
   for (size_t j = 0; j < nctx; j++) {
     exh_context *c = cc.ctxs[j];
     if (outer_capture) {
       // nothing may be allocated or uploaded inside a caller's capture
-      if (!scratch_fits(c, cc.nkg[j]) || (nmod && (!c->oz_consts || !c->ozr.p)))
+      oz.P[j] = oz_plan(c, flags);
+      if (oz.P[j].nmod) oz.L[j] = oz_layout(c->ngkmax, c->Ktot, oz.P[j], false, c->have_h1aa);
+      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, oz.L[j]);
+      if (!oz_ok && !nmod) oz.P[j] = OzPlan();  // as the call outside capture ran
+      if (!scratch_fits(c, cc.nkg[j]) || (nmod && !oz_ok))
         return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
-      if (nmod) {
-        oz.L[j] = oz_layout(c->ngkmax, c->Ktot, nmod);
-        oz.bits[j] = oz_bits(nmod, c->Ktot);
-        if (c->ozqx.bytes < oz.L[j].qx_bytes || c->ozqb.bytes < oz.L[j].qb_bytes ||
-            c->ozr.bytes < oz.L[j].r_bytes || c->ozex.bytes < oz.L[j].e_bytes ||
-            c->ozeb.bytes < oz.L[j].e_bytes)
-          return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
-      }
     } else {
       rc = ensure_scratch(c, cc.nkg[j]);
-      if (!rc && nmod) rc = oz_prepare(c, nmod, oz.L[j], oz.bits[j]);
+      if (!rc) rc = oz_prepare(c, flags, false, false, oz.P[j], oz.L[j]);
       if (rc) {
         if (c != lead) fail(lead, rc, c->err);
         return rc;
@@ -442,6 +441,7 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
     const uint64_t sig[3] = {(uint64_t)(uintptr_t)c, c->epoch, state_signature(c)};
     put(sig, sizeof sig);
     put(&cc.nkg[j], sizeof(int));
+    put(&oz.P[j].nmod, sizeof(int));
   }
   put(kp, nk * sizeof(exh_kpoint));
   put(cc.kci.data(), nk * sizeof(int));
@@ -449,7 +449,7 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   if (!E) {
     if (outer_capture)
       return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
-    E = build_entry(lead, s, nk, kp, cc, plan, flags, std::move(key), &rc);
+    E = build_entry(lead, s, nk, kp, cc, oz, plan, flags, std::move(key), &rc);
     if (!E) return rc;
   }
   E->use = ++lead->bclock;
@@ -563,6 +563,15 @@ int exh_tune_batch(exh_context *c, void *stream, int nk, const exh_kpoint *kp, i
   if (nk == 0) return fail(c, EXH_EINVAL, "tune: no k-points");
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, EXH_ESTATE, "hipSetDevice");
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  OzPlan P;
+  OzLayout L;
+  rc = oz_prepare(c, flags, false, false, P, L);
+  if (rc) return rc;
+  if (P.nmod) {  // no tiles to shape: every plan is the same call
+    rc = exh_setup_batch_device(c, s, nk, kp, flags);
+    if (!rc && plan) *plan = exh_get_batch_plan(c);
+    return rc;
+  }
   // tune on leading k-points worth about 4 TFLOP of contraction (1 to 8)
   int nt = 0;
   double fl = 0.0;

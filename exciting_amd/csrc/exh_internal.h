@@ -33,15 +33,30 @@ struct LoRow {
   int ias, ilo, mi, l;
 };
 
-// Split-precision (Ozaki scheme II) path.
-constexpr int kOzMaxMod = 12;
-extern const int kOzPrimes[kOzMaxMod];
+// Static device scratch of exh_setup_device_noalloc (api.hip).
+constexpr size_t kNoallocScratchBytes = size_t(64) << 20;
+
+// Modular (Ozaki scheme II) contraction: split precision, and FP64 for large
+// bases.
+constexpr int kOzMaxMod = 12;  // EXH_SPLIT(n), n <= 12
+constexpr int kOzModuli = 15;  // moduli available
+// largest K whose int32 sums of residue products (|r| <= 121) stay exact
+constexpr int kOzMaxK = 146000;
+struct OzPlan {
+  int nmod = 0;  // moduli (0: not on this path)
+  int bits = 0;  // c: the scaled columns' 2-norms are below 2^(c-1)
+};
 struct OzLayout {
-  int Gpad = 0, Kpad = 0;       // G rounded to the 128 tile, K to the 64 stage
-  size_t qstride = 0;           // bytes of one residue array (Kpad * Gpad)
-  long long max_pairs = 0;      // upper tile pairs at ngkmax
-  size_t qx_bytes = 0, qb_bytes = 0, r_bytes = 0;
+  int Gpad = 0, Kpad = 0;  // G rounded to the row panel, K to the 64 stage
+  size_t qstride = 0;      // bytes of one residue array (Kpad * Gpad)
+  int nops = 0;            // operands (X; B unless O alone; (1+h1)A for iora*)
+  size_t q_bytes = 0;      // residues of one operand
+  size_t r_bytes = 0;      // residues of the products
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
+};
+struct OzScratch {
+  int8_t *q = nullptr, *r = nullptr;
+  void *e = nullptr;
 };
 
 // APW-lo border tables (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133)
@@ -219,8 +234,7 @@ struct exh_context {
   exh::DevBuf bt, a2t, at, ivgk, mtab;
   // this device's copy of the static scratch of exh_setup_device_noalloc
   void *noalloc_scratch = nullptr;
-  exh::DevBuf ozqx, ozqb, ozr, ozex, ozeb;
-  bool oz_consts = false;
+  exh::DevBuf ozq, ozr, oze;  // modular contraction: residues, products, exponents
   bool contig = true;  // colA[k] == k * ngkmax
   // host-API staging
   exh::DevBuf s_apwalm, s_igpig, s_vgpc, s_h, s_o, s_gpc, s_tpgpc, s_sfac;
@@ -295,16 +309,22 @@ hipError_t launch_lolo(hipStream_t s, const exh_context *c, int ngp,
                        double2 *h, double2 *o, int ldh, int flags);
 const double2 *k_major_operand(const exh_context *c, const double2 *apwalm, const double2 *at,
                                long long *ld);
-int oz_bits(int nmod, int Ktot);
-hipError_t oz_upload_constants(int nmod);
-OzLayout oz_layout(int ngkmax, int Ktot, int nmod);
-int oz_prepare(exh_context *c, int nmod, OzLayout &L, int &bits);
 struct IstBox;
-hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const double2 *X,
-                        long long ldx, const double2 *B, long long ldb, int nmod, int bits,
-                        const OzLayout &L, int8_t *QX, int8_t *QB, uint8_t *R, int *ex,
-                        int *eb, const IstBox &box, double2 *h, double2 *o, int ldh,
-                        int accumulate, int stage_mask);
+OzPlan oz_split(int n);
+OzPlan oz_fp64();
+OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool third);
+OzPlan oz_plan(const exh_context *c, int flags);
+bool oz_fits(const exh_context *c, const OzLayout &L);
+inline OzScratch oz_scratch(const exh_context *c) {
+  return OzScratch{(int8_t *)c->ozq.p, (int8_t *)c->ozr.p, c->oze.p};
+}
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, OzPlan &P, OzLayout &L);
+// h = nullptr: O alone (B is not read).  Y = nullptr: the overlap's column
+// operand is X.  stage_mask: 1 residues, 2 products, 4 reconstruction.
+hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const OzPlan &P,
+                        const OzLayout &L, const OzScratch &w, const double2 *X, long long ldx,
+                        const double2 *B, const double2 *Y, long long ldb, const IstBox &box,
+                        double2 *h, double2 *o, int ldh, int accumulate, int stage_mask);
 // tab: match_table_bytes(c) of scratch for the k-point's radial factors and
 // spherical harmonics
 size_t match_table_bytes(const exh_context *c);

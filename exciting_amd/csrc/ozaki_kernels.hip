@@ -1,39 +1,49 @@
-// Split-precision muffin-tin contraction: Ozaki scheme II on int8 MFMA.
+// Modular muffin-tin contraction (Ozaki scheme II on int8 MFMA): exact
+// integer products of rounded operands through residues.
 //
-// The FP64 products H_MT = X^H B and O_MT = X^H X (X = A^T, B = (aa A)^T,
-// K = every atom's (l, m, io) stacked) are emulated with integer arithmetic:
+// The products H_MT = X^H B and O_MT = X^H Y (X = A^T, B = (aa A)^T, Y = X or,
+// for iora*, ((1+h1) A)^T; K = every atom's (l, m, io) stacked) are computed
+// as follows:
 //
-//  1. Each G column of X and of B gets a power-of-two scale 2^s so that its
-//     2-norm is at most 2^(c-1); the scaled values are rounded to integers,
-//     which keeps the norm below 2^c.  This rounding is the only
-//     approximation: the error is <= 1/2 of 2^-s per component, i.e. about
-//     2^-c of the column's norm.
-//  2. The integers are reduced modulo N primes p_m <= 251 into int8 residues
-//     in [-(p-1)/2, (p-1)/2], stored in 16-byte k blocks per G row: the
-//     operand format of v_mfma_i32_32x32x32_i8.
-//  3. For each modulus and each of six real products (Karatsuba for the
-//     conjugated complex product, exact in modular arithmetic):
-//        H: P1 = xr.br, P2 = xi.bi, P3 = (xr+xi).(br-bi)
-//        O: Q1 = xr.xr, Q2 = xi.xi, Q3 = (xr+xi).(xr-xi)
-//     an upper-triangular int8 GEMM accumulates exactly in int32 and stores
-//     the result modulo p_m as one byte per element (operands streamed
-//     global -> LDS by direct DMA loads).
-//  4. Re = P1+P2 and Im = P1-P2-P3 are formed modulo each p_m and turned
-//     back into exact integers by Garner's mixed-radix algorithm with
-//     symmetric digits (no cancellation for small results), evaluated in
-//     FP64 and rescaled by 2^-(s_i+s_j).  The interstitial terms and the
-//     conj mirror are added as in the FP64 path.
+//  1. Each G column of an operand gets a power-of-two scale 2^s so that its
+//     2-norm is at most 2^(c-1); the scaled values are rounded to integers.
+//     This rounding is the only approximation: at most 1/2 of 2^-s per
+//     component, i.e. about 2^-c of the column's norm.
+//  2. The moduli p_m are products of primes = 1 mod 4, where -1 has a square
+//     root I_m.  The Gaussian integer z = zr + i zi then has the two residues
+//     z+ = zr + I zi and z- = zr - I zi mod p, which multiply separately:
+//     (conj(x) y)+ = x- y+ and (conj(x) y)- = x+ y-.  A complex product costs
+//     two real products instead of the three of Karatsuba's scheme modulo
+//     arbitrary primes (28.0 -> 18.1 ms at K = 15488, G = 9340, 7 moduli), and
+//     two residue arrays per operand instead of three or four.  Residues are
+//     int8 in [-p/2, p/2], stored in 16-byte k blocks per G row: the operand
+//     format of v_mfma_i32_32x32x32_i8.
+//  3. Per modulus and sign, an upper-triangular int8 GEMM accumulates H and O
+//     exactly in int32 (K <= kOzMaxK) and stores them modulo p as one signed
+//     byte per element (operands streamed global -> LDS by direct DMA loads).
+//  4. Re = (P+ + P-)/2 and Im = (P+ - P-)/(2 I) modulo every p are turned
+//     back into the exact integers by the Chinese remainder theorem in two-
+//     word FP64 (the high words sum without rounding) and rescaled by
+//     2^-(s_i+s_j).  The interstitial terms and the conj mirror are added as
+//     in the FP64 path.
 //
-// The reconstructed integers are Re and Im of x_i^H b_j (the Karatsuba
-// products only meet modulo p), bounded by ||x_i|| ||b_j|| <= 2^(2c)
-// (Cauchy-Schwarz); c is the largest value with 2^(2c) < prod(p)/2, so every
-// element is recovered exactly from its residues.  Against scaling by the
-// largest entry and the worst case 6 K 2^(2b) this gains
-// (log2(6K) + 2 log2(max/norm ratio of the columns)) / 2 bits per operand.
+// The integers are Re and Im of x_i^H b_j, bounded by ||x_i|| ||b_j|| <=
+// 2^(2c-2) (Cauchy-Schwarz), so n moduli with prod p > 2^(2c-1) recover every
+// element exactly.
+//
+// EXH_SPLIT(n) fixes c as the caller asked (27 bits for n = 7).  Without that
+// flag, large bases run here with 15 moduli and c = 56 (oz_fp64): the
+// operands keep 55 bits relative to the column norm and nothing else is
+// rounded, so the products are closer to the exact ones than those of the
+// FP64 MFMA kernels (relative Frobenius error of the contraction alone at 16
+// atoms, K = 3872: 2e-16 against 2.4e-15; median element 6e-16 against
+// 2.7e-15), whose K-long FP64 accumulation rounds 4 K times per element.
+//
+// Columns whose norm is not finite give NaN rows and columns of H and O, as
+// any FP64 sum over them would; zero columns give zeros.
 #include <algorithm>
 #include <climits>
 #include <cmath>
-#include <mutex>
 
 #include "exh_device.h"
 
@@ -45,121 +55,301 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int OZ_T = 128;   // output tile edge
 constexpr int OZ_KS = 64;   // k per LDS stage (4 blocks of 16)
-
-__constant__ int c_p[kOzMaxMod];
-__constant__ float c_rp[kOzMaxMod];          // 1/p
-__constant__ int c_w[kOzMaxMod];             // (p_0..p_{k-1})^{-1} mod p_k
-__constant__ int c_c[kOzMaxMod][kOzMaxMod];  // (p_0..p_{j-1}) * w_k mod p_k, j < k
+constexpr int OZ_N = kOzModuli;
 
 // ---------------------------------------------------------------------------
-// Column scales from the 2-norms: part[chunk][g] = sum over the chunk's 256
-// k of |x|^2, then per column the chunks in order (a fixed summation order,
-// so the scale is the same in every run) and emax[g] = E + 1 with
-// ||x_g|| < 2^E: the scale 2^(c - emax) takes the norm below 2^(c-1).
+// Moduli: the largest pairwise coprime products of primes = 1 mod 4 below
+// 256 (221 = 13*17, 205 = 5*41), and a square root of -1 for each.
 // ---------------------------------------------------------------------------
-constexpr int OZ_NCH = 256;  // k per partial sum
+constexpr int kP[OZ_N] = {241, 233, 229, 221, 205, 197, 193, 181,
+                          173, 157, 149, 137, 113, 109, 101};
 
-__global__ void colnorm_part_kernel(int ngp, int Ktot, const double2 *__restrict__ X,
-                                    long long ldx, double *__restrict__ part, int ldp) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ngp) return;
-  const int k0 = blockIdx.y * OZ_NCH, k1 = min(Ktot, k0 + OZ_NCH);
-  double s = 0.0;
-  for (int k = k0; k < k1; k++) {
-    const double2 v = X[(size_t)k * ldx + g];
-    s = fma(v.x, v.x, s);
-    s = fma(v.y, v.y, s);
-  }
-  part[(size_t)blockIdx.y * ldp + g] = s;
+constexpr int sym(long long x, int p) {  // representative in [-p/2, p/2]
+  long long r = x % p;
+  if (r < 0) r += p;
+  return (int)(2 * r > p ? r - p : r);
+}
+constexpr int root(int p) {
+  for (int i = 2; i < p; i++)
+    if ((i * i + 1) % p == 0) return sym(i, p);
+  return 0;
+}
+constexpr int inverse(long long a, int p) {
+  long long r = ((a % p) + p) % p;
+  for (int x = 1; x < p; x++)
+    if (r * x % p == 1) return x;
+  return 0;
 }
 
-__global__ void colnorm_final_kernel(int ngp, int nchunk, const double *__restrict__ part,
-                                     int ldp, int *__restrict__ emax) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+// Residue constants of one modulus.  kMagic + r is exact for integers
+// |r| < 2^51 and holds r in its low 32 bits; nk cancels it in the quotient.
+constexpr double kMagic = 6755399441055744.0;  // 1.5 * 2^52
+constexpr int kSplit = 27;                     // y = h 2^27 + l
+struct OzMod {
+  double p, rp, nk;   // p, 1/p, -kMagic/p
+  double c1, c2, im;  // 2^27, 2^27 I, I mod p (symmetric)
+};
+struct OzMods {
+  OzMod m[OZ_N];
+};
+constexpr OzMods make_mods() {
+  OzMods t{};
+  for (int k = 0; k < OZ_N; k++) {
+    const int p = kP[k], i = root(p);
+    t.m[k].p = p;
+    t.m[k].rp = 1.0 / p;
+    t.m[k].nk = -(kMagic * (1.0 / p));
+    t.m[k].c1 = sym(1ll << kSplit, p);
+    t.m[k].c2 = sym((1ll << kSplit) * i, p);
+    t.m[k].im = i;
+  }
+  return t;
+}
+__constant__ const OzMods c_mod = make_mods();
+
+// CRT constants for the first n moduli, P = their product: with s = P+ + P-
+// and d = P+ - P- (signed bytes, |s|, |d| <= 2 * 121),
+//   Re = sum_m s_m re_m mod P,  Im = sum_m d_m im_m mod P,
+//   re_m = (P/p) [(P/p)^-1 / 2 mod p],  im_m = (P/p) [(P/p)^-1 / (2 I) mod p]
+// (symmetric), each split into a high word that is a multiple of 2^T and a
+// low word |.| < 2^T.  T is such that the sums of high words stay below
+// 2^(T+53) and are therefore exact; the low words contribute rounding errors
+// of at most 2^(T+13-53), 2^-81 P at n = 15.
+struct OzCrt {
+  double reh[OZ_N], rel[OZ_N], imh[OZ_N], iml[OZ_N];
+  double rP, Ph, Pl;
+};
+struct OzCrts {
+  OzCrt t[OZ_N + 1];
+};
+typedef __int128 i128;
+constexpr int bits_of(i128 x) {
+  int n = 0;
+  while (x > 0) {
+    x >>= 1;
+    n++;
+  }
+  return n;
+}
+constexpr double to_double(i128 x) {  // exact when x has at most 53 bits after its trailing zeros
+  return (double)x;
+}
+constexpr OzCrts make_crts() {
+  OzCrts all{};
+  for (int n = 1; n <= OZ_N; n++) {
+    OzCrt &c = all.t[n];
+    i128 P = 1;
+    for (int k = 0; k < n; k++) P *= kP[k];
+    // sum |s| |re| <= n * 242 * P/2 < 2^(bits(P) + 11)
+    const int T = bits_of(P) + 11 > 53 ? bits_of(P) + 11 - 53 : 0;
+    const i128 unit = (i128)1 << T;
+    c.rP = 1.0 / to_double(P);
+    c.Ph = to_double(P / unit * unit);
+    c.Pl = to_double(P % unit);
+    for (int k = 0; k < n; k++) {
+      const int p = kP[k];
+      const i128 Q = P / p;
+      const long long qi = inverse((long long)(Q % p), p);
+      const long long a = sym(qi * inverse(2, p), p);
+      const long long b = sym(qi * inverse(2ll * root(p), p), p);
+      const i128 re = Q * a, im = Q * b;
+      const i128 reh = re / unit * unit, imh = im / unit * unit;  // truncated toward 0
+      c.reh[k] = to_double(reh);
+      c.rel[k] = to_double(re - reh);
+      c.imh[k] = to_double(imh);
+      c.iml[k] = to_double(im - imh);
+    }
+  }
+  return all;
+}
+__constant__ const OzCrts c_crt = make_crts();
+
+// ---------------------------------------------------------------------------
+// Column norms.  part[chunk][g] = sum over the chunk's 256 k of |x|^2 in a
+// fixed order (four k groups per workgroup, added in order), scaled by
+// 2^(-2 pe[chunk][g]); pe is 0 unless the chunk holds magnitudes whose
+// squares would leave FP64's range.  The final kernel adds the chunks in
+// order and sets emax[g] = E + 1 with ||x_g|| < 2^E: the scale 2^(c - emax)
+// takes the norm below 2^(c-1).  emax = INT_MIN for a zero column, INT_MAX
+// for one that is not finite.  Bound by reading the operands once: 64
+// columns x 256 k per workgroup and one launch for all operands keep enough
+// loads in flight also at a thousand G+k (norms and residues of an 8-atom
+// k-point, K = 1936, G = 1166, 9 moduli: 294 -> 75 us).
+// ---------------------------------------------------------------------------
+constexpr int OZ_NCH = 256;      // k per partial sum
+constexpr int OZ_LO = -400, OZ_HI = 400;  // exponents whose squares are safe
+
+struct OzOperands {  // operands of one call: X, B and, for iora*, (1+h1)A
+  const double2 *x[3];
+  long long ld[3];
+  int *e[3];       // column exponents
+  double *part[3]; // partial sums, then their exponents
+  int8_t *q[3];    // residues
+};
+
+__device__ __forceinline__ int exponent_of(double a) {  // of a normal |a|; -1023 for 0
+  return (int)((__double_as_longlong(a) >> 52) & 0x7ff) - 1023;
+}
+
+__global__ __launch_bounds__(256) void colnorm_part_kernel(int ngp, int Ktot, OzOperands op,
+                                                           int ldp, int nch) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int g = blockIdx.x * 64 + lane, z = blockIdx.z;
+  const double2 *X = z == 0 ? op.x[0] : z == 1 ? op.x[1] : op.x[2];
+  const long long ldx = z == 0 ? op.ld[0] : z == 1 ? op.ld[1] : op.ld[2];
+  double *part = z == 0 ? op.part[0] : z == 1 ? op.part[1] : op.part[2];
+  __shared__ double ss[4][64];
+  __shared__ int sm[4][64];
+  const int k0 = blockIdx.y * OZ_NCH, k1 = min(Ktot, k0 + OZ_NCH);
+  const double2 *xp = X + min(g, ngp - 1);
+  double s = 0.0, amax = 0.0;
+#pragma unroll 8
+  for (int k = k0 + w; k < k1; k += 4) {
+    const double2 v = xp[(size_t)k * ldx];
+    s = fma(v.x, v.x, s);
+    s = fma(v.y, v.y, s);
+    amax = fmax(amax, fmax(fabs(v.x), fabs(v.y)));
+  }
+  ss[w][lane] = s;
+  sm[w][lane] = exponent_of(amax);
+  __syncthreads();
+  int e = max(max(sm[0][lane], sm[1][lane]), max(sm[2][lane], sm[3][lane]));
+  const bool rescale = e < OZ_LO || (e > OZ_HI && e < 1024);
+  if (__any(rescale)) {  // rare: squares out of range, sum the scaled values
+    e = rescale ? (e == -1023 ? -1022 : e) : 0;
+    s = 0.0;
+    for (int k = k0 + w; k < k1; k += 4) {
+      const double2 v = xp[(size_t)k * ldx];
+      const double a = ldexp(v.x, -e), b = ldexp(v.y, -e);
+      s = fma(a, a, s);
+      s = fma(b, b, s);
+    }
+    __syncthreads();
+    ss[w][lane] = s;
+  } else {
+    e = 0;
+  }
+  __syncthreads();
+  if (w == 0 && g < ngp) {
+    part[(size_t)blockIdx.y * ldp + g] = ((ss[0][lane] + ss[1][lane]) + ss[2][lane]) + ss[3][lane];
+    ((int *)(part + (size_t)nch * ldp))[(size_t)blockIdx.y * ldp + g] = e;
+  }
+}
+
+__global__ __launch_bounds__(64) void colnorm_final_kernel(int ngp, int nch, OzOperands op,
+                                                           int ldp) {
+  const int g = blockIdx.x * 64 + threadIdx.x, z = blockIdx.y;
   if (g >= ngp) return;
+  const double *part = z == 0 ? op.part[0] : z == 1 ? op.part[1] : op.part[2];
+  int *emax = z == 0 ? op.e[0] : z == 1 ? op.e[1] : op.e[2];
+  const int *pe = (const int *)(part + (size_t)nch * ldp);
+  int em = -5000;  // running exponent of the sum s 2^(2 em)
   double s = 0.0;
-  for (int c = 0; c < nchunk; c++) s += part[(size_t)c * ldp + g];
+#pragma unroll 8
+  for (int c = 0; c < nch; c++) {
+    const double v = part[(size_t)c * ldp + g];
+    const int ec = v == 0.0 ? em : pe[(size_t)c * ldp + g], m = max(em, ec);
+    s = ldexp(s, 2 * (em - m)) + ldexp(v, 2 * (ec - m));
+    em = m;
+  }
   int e = INT_MIN;
-  if (s > 0.0) {
+  if (!(s - s == 0.0)) {
+    e = INT_MAX;  // Inf or NaN in the column
+  } else if (s > 0.0) {
     (void)frexp(sqrt(s), &e);  // norm = f 2^e, f in [0.5, 1): norm < 2^e
-    e += 1;
+    e += 1 + em;
   }
   emax[g] = e;
 }
 
-__device__ __forceinline__ int smod(double x, int m) {
-  // symmetric residue of the integer-valued double x modulo the odd prime p_m
-  const double p = (double)c_p[m];
-  return (int)(x - p * rint(x * (1.0 / p)));
+// ---------------------------------------------------------------------------
+// Residues: one thread per (16-k block, G row), blockIdx.z the operand.
+// y = rint(x 2^s) = h 2^27 + l; then per modulus, all in exact FP64 integers,
+//   y+- = (hr c1 + lr) +- (hi c2 + li I),   r = y+- - p rint(y+- / p),
+// the low byte of kMagic + r being the residue.  |r| <= (1/2 + 2^-9) p.
+// Rows ngp..rows-1 and k >= Ktot are written as zeros (no masking
+// downstream).  Layout: Q[(2 m + t) * qstride + (kblk * Gpad + g) * 16 + byte], t = 0 for
+// y+, 1 for y-.  About 13 FP64 operations per (element, modulus) beside
+// 2 bytes written: bound by HBM and the vector unit alike.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int low_word(double x) { return (int)__double_as_longlong(x); }
+
+// low bytes of the low words of four doubles
+__device__ __forceinline__ int pack4(double a, double b, double c, double d) {
+  const unsigned x = __builtin_amdgcn_perm((unsigned)low_word(b), (unsigned)low_word(a), 0x0c0c0400);
+  const unsigned y = __builtin_amdgcn_perm((unsigned)low_word(d), (unsigned)low_word(c), 0x04000c0c);
+  return (int)(x | y);
 }
 
-// ---------------------------------------------------------------------------
-// Residues: one thread per (16-k block, G row).  X gives four arrays
-// (xr, xi, xr+xi, xr-xi), B gives three (br, bi, br-bi), per modulus.
-// Rows >= ngp and k >= Ktot are written as zeros (no masking downstream).
-// Layout: Q[(m * narr + t) * qstride + (kblk * Gpad + g) * 16 + byte].
-// ---------------------------------------------------------------------------
-template <int NARR>
-__global__ void residue_kernel(int ngp, int Ktot, int Gpad, const double2 *__restrict__ X,
-                               long long ldx, const int *__restrict__ emax, int bits, int nmod,
-                               size_t qstride, int8_t *__restrict__ Q) {
+__global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpad, int rows,
+                                                      OzOperands op, int bits, int nmod,
+                                                      size_t qstride) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kb = blockIdx.y;
-  if (g >= Gpad) return;
-  double re[16], im[16];
-  int s = 0;
-  if (g < ngp) {
-    const int e = emax[g];
-    s = (e == INT_MIN) ? 0 : bits - e;
-  }
+  const int kb = blockIdx.y, z = blockIdx.z;
+  if (g >= rows) return;
+  const double2 *X = z == 0 ? op.x[0] : z == 1 ? op.x[1] : op.x[2];
+  const long long ldx = z == 0 ? op.ld[0] : z == 1 ? op.ld[1] : op.ld[2];
+  const int *emax = z == 0 ? op.e[0] : z == 1 ? op.e[1] : op.e[2];
+  int8_t *Q = z == 0 ? op.q[0] : z == 1 ? op.q[1] : op.q[2];
+  double hr[16], lr[16], hi[16], li[16];
+  int e = INT_MIN;
+  if (g < ngp) e = emax[g];
+  const bool live = e != INT_MIN && e != INT_MAX;
+  const int s = live ? bits - e : 0;
 #pragma unroll
   for (int t = 0; t < 16; t++) {
     const int k = kb * 16 + t;
     double2 v = z2(0.0, 0.0);
-    if (g < ngp && k < Ktot) v = X[(size_t)k * ldx + g];
-    re[t] = rint(ldexp(v.x, s));
-    im[t] = rint(ldexp(v.y, s));
+    if (live && k < Ktot) v = X[(size_t)k * ldx + g];
+    const double yr = rint(ldexp(v.x, s)), yi = rint(ldexp(v.y, s));
+    constexpr double D = (double)(1ll << kSplit);
+    hr[t] = rint(yr * (1.0 / D));
+    lr[t] = fma(-D, hr[t], yr) + kMagic;
+    hi[t] = rint(yi * (1.0 / D));
+    li[t] = fma(-D, hi[t], yi);
   }
-  const size_t off = ((size_t)kb * Gpad + g) * 16;
+  int8_t *out = Q + ((size_t)kb * Gpad + g) * 16;
+#pragma unroll 1
   for (int m = 0; m < nmod; m++) {
+    const double p = c_mod.m[m].p, rp = c_mod.m[m].rp, nk = c_mod.m[m].nk;
+    const double c1 = c_mod.m[m].c1, c2 = c_mod.m[m].c2, im = c_mod.m[m].im;
+    int wp[4], wm[4];
 #pragma unroll
-    for (int a = 0; a < NARR; a++) {
-      int w[4];
+    for (int q = 0; q < 4; q++) {
+      double rpos[4], rneg[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        unsigned packed = 0;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int k = 4 * q + t;
-          double x;
-          if (a == 0) x = re[k];
-          else if (a == 1) x = im[k];
-          else if (a == 2) x = (NARR == 4) ? re[k] + im[k] : re[k] - im[k];
-          else x = re[k] - im[k];
-          packed |= (unsigned)(smod(x, m) & 0xff) << (8 * t);
-        }
-        w[q] = (int)packed;
+      for (int t = 0; t < 4; t++) {
+        const int k = 4 * q + t;
+        const double a = fma(hr[k], c1, lr[k]);
+        const double b = fma(hi[k], c2, li[k] * im);
+        const double u = a + b, v = a - b;
+        rpos[t] = fma(-p, rint(fma(u, rp, nk)), u);
+        rneg[t] = fma(-p, rint(fma(v, rp, nk)), v);
       }
-      *(v4i *)(Q + (size_t)(m * NARR + a) * qstride + off) = v4i{w[0], w[1], w[2], w[3]};
+      wp[q] = pack4(rpos[0], rpos[1], rpos[2], rpos[3]);
+      wm[q] = pack4(rneg[0], rneg[1], rneg[2], rneg[3]);
     }
+    *(v4i *)(out + (size_t)(2 * m) * qstride) = v4i{wp[0], wp[1], wp[2], wp[3]};
+    *(v4i *)(out + (size_t)(2 * m + 1) * qstride) = v4i{wm[0], wm[1], wm[2], wm[3]};
   }
 }
 
 // ---------------------------------------------------------------------------
 // Upper-triangular int8 GEMMs.  One workgroup computes the product pair
-// (H_q, O_q) of one modulus (q = 0, 1, 2) for a row panel of the row operand
-// (xr, xi or xr+xi) against one 128-column block J of the H and O column
-// operands:
+// (H, O) of one modulus and sign for a 384-row panel of the row operand
+// (x- for the sign +, x+ for -) against one 128-column block J of the H and O
+// column operands:
 //   C_H[i][j] = sum_k A[k][i] BH[k][j],  C_O[i][j] = sum_k A[k][i] BO[k][j]
-// (int32, exact), each stored mod p as bytes in the 128x128 tiles on or
-// above the diagonal.  The H and O products share the row operand, as the
-// FP64 kernel shares conj(A) between H and O.  Each wave owns 96 rows x 64
-// columns of both products (3 x 2 blocks of v_mfma_i32_32x32x32_i8 each, 192
-// accumulator registers) and reads 7 operand fragments from LDS per 12
-// MFMAs; NW waves form NW/2 row groups x 2 column groups, so the panel is
-// 48*NW rows.  NW = 8: 384-row panels, one workgroup per CU.  (NW = 4, two
-// 192-row workgroups per CU whose barriers fall at different times, gives
-// the same products and measured 1 % slower at the 64-atom shape.)
+// (int32, exact), each stored mod p as signed bytes in the 128x128 tiles on
+// or above the diagonal.  The H and O products share the row operand, as the
+// FP64 kernel shares conj(A) between H and O.  With ONLY_O (overlapsetup) the
+// second column operand is the next 128 columns of O instead.  Each wave owns
+// 96 rows x 64 columns of both products (3 x 2 blocks of
+// v_mfma_i32_32x32x32_i8 each, 192 accumulator registers) and reads 7 operand
+// fragments from LDS per 12 MFMAs; 8 waves form 4 row groups x 2 column
+// groups, one workgroup per CU.  (192-row panels, two 4-wave workgroups per
+// CU whose barriers fall at different times, gave the same products and
+// measured 1 % slower at the 64-atom shape.)
 // Operands stream global -> LDS directly (global_load_lds, 16 bytes per
 // lane, one 64-row chunk of one k block per instruction), two stages of 64 k
 // double-buffered.
@@ -173,78 +363,91 @@ constexpr int OZ_R = 48 * OZ_NWG;  // rows of the row panel per workgroup
 #define EXH_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 #define EXH_GLB(p) ((const __attribute__((address_space(1))) void *)(p))
 
-// Residues mod p of one 32 x 64 strip (block row a of a wave) per product,
-// four consecutive rows packed per 32-bit store, into the 128x128 tile it
-// lies in when that tile is on or above the diagonal.
-__device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], int p, float rp,
-                                               int rg, int wc, int lh, int l32, int IT, int J,
-                                               uint8_t *Rp) {
+// Residues mod p of the 96 x 64 strip of a wave, four consecutive rows packed
+// per 32-bit store, into the 128x128 tiles on or above the diagonal.  A tile
+// is stored as 16 sub-blocks of 32 x 32 (4 bj + bi) in accumulator order --
+// word 64 h + lane holds rows 8 h + 4 (lane/32) .. + 3 of column lane%32 --
+// so that each store instruction writes 256 contiguous bytes here and each
+// load instruction of the reconstruction reads them.
+__device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], const OzMod &M,
+                                               int rg, int wc, int lane, int IT, int J,
+                                               int8_t *Rp) {
+  const double p = M.p, rp = M.rp, nk = M.nk;
 #pragma unroll
   for (int a = 0; a < OZ_WR; a++) {
     const int row = IT * OZ_R + rg * 32 * OZ_WR + a * 32;
     const int I = row >> 7;
     if (I > J) continue;  // below the diagonal (uniform per wave)
-    uint8_t *out = Rp + ((long long)J * (J + 1) / 2 + I) * (OZ_T * OZ_T);
+    int8_t *out = Rp + ((long long)J * (J + 1) / 2 + I) * (OZ_T * OZ_T) + 4 * lane;
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int h = 0; h < 4; h++) {
-        unsigned packed = 0;
+        double r[4];
 #pragma unroll
-        for (int t4 = 0; t4 < 4; t4++) {
-          const int x = acc[a][b][4 * h + t4];
-          int q = (int)floorf((float)x * rp);
-          int r = x - q * p;
-          r += (r < 0) ? p : 0;
-          r -= (r >= p) ? p : 0;
-          packed |= (unsigned)r << (8 * t4);
+        for (int t = 0; t < 4; t++) {
+          const double x = (double)acc[a][b][4 * h + t] + kMagic;
+          r[t] = fma(-p, rint(fma(x, rp, nk)), x);
         }
-        const int il = (row & 127) + 8 * h + 4 * lh;
-        const int jl = wc * 64 + b * 32 + l32;
-        *(unsigned *)(out + il + OZ_T * jl) = packed;
+        const int sub = 4 * (2 * wc + b) + ((row & 127) >> 5);
+        *(int *)(out + sub * 1024 + h * 256) = pack4(r[0], r[1], r[2], r[3]);
       }
   }
 }
 
-// Row panels column block J needs: those starting at or above its last row.
+// Row panels that columns up to (and including) block j of 128 need.
 __host__ __device__ inline int oz_npan(int j) { return (j * OZ_T + OZ_T - 1) / OZ_R + 1; }
 
+// Column steps of one GEMM and the last 128-column block of step j: the
+// fused products step by one block, O alone by two (nt blocks in all).
+template <bool ONLY_O>
+__host__ __device__ inline int oz_steps(int nt) { return ONLY_O ? (nt + 1) / 2 : nt; }
+template <bool ONLY_O>
+__host__ __device__ inline int oz_last(int j, int nt) {
+  const int l = ONLY_O ? 2 * j + 1 : j;
+  return l < nt ? l : nt - 1;
+}
+
 // Panels per GEMM.
+template <bool ONLY_O>
 __host__ __device__ inline long long oz_panels(int nt) {
   long long n = 0;
-  for (int j = 0; j < nt; j++) n += oz_npan(j);
+  for (int j = 0; j < oz_steps<ONLY_O>(nt); j++) n += oz_npan(oz_last<ONLY_O>(j, nt));
   return n;
 }
 
-// Panel order: super-columns of OZ_SJ column blocks, each walked in chunks
+// Panel order: super-columns of OZ_SJ column steps, each walked in chunks
 // of OZ_SI row panels (4 x 384 rows), so that the workgroups an XCD runs at
 // once share a few row panels and column panels in its L2 (the column-major
 // order had 32 co-resident workgroups share about 1 column panel and 19 row
 // panels); 3.6 % faster at the 64-atom shape, bitwise the same products.
 constexpr int OZ_SJ = 8, OZ_SI = 4 * 384 / OZ_R;
 
-// Panel o of one GEMM -> (column block J, row panel IT), IT < oz_npan(J).
+// Panel o of one GEMM -> (column step J, row panel IT).
+template <bool ONLY_O>
 __device__ __forceinline__ void oz_panel_at(int o, int nt, int &J, int &IT) {
+  const int ns = oz_steps<ONLY_O>(nt);
+  auto npan = [&](int j) { return oz_npan(oz_last<ONLY_O>(j, nt)); };
   int rem = o, j0 = 0;
   for (;; j0 += OZ_SJ) {
-    const int j1 = min(nt, j0 + OZ_SJ);
+    const int j1 = min(ns, j0 + OZ_SJ);
     int cnt = 0;
-    for (int j = j0; j < j1; j++) cnt += oz_npan(j);
+    for (int j = j0; j < j1; j++) cnt += npan(j);
     if (rem < cnt) break;
     rem -= cnt;
   }
-  const int j1 = min(nt, j0 + OZ_SJ);
+  const int j1 = min(ns, j0 + OZ_SJ);
   int i0 = 0;
   for (;; i0 += OZ_SI) {
     int cnt = 0;
-    for (int j = j0; j < j1; j++) cnt += max(0, min(OZ_SI, oz_npan(j) - i0));
+    for (int j = j0; j < j1; j++) cnt += max(0, min(OZ_SI, npan(j) - i0));
     if (rem < cnt) break;
     rem -= cnt;
   }
   J = j0;
   IT = i0;
   for (int j = j0; j < j1; j++) {
-    const int cj = max(0, min(OZ_SI, oz_npan(j) - i0));
+    const int cj = max(0, min(OZ_SI, npan(j) - i0));
     if (rem < cj) {
       J = j;
       IT = i0 + rem;
@@ -255,25 +458,30 @@ __device__ __forceinline__ void oz_panel_at(int o, int nt, int &J, int &IT) {
 }
 
 // two waves per SIMD whatever the workgroup size: at most 256 VGPRs
+template <bool ONLY_O>
 __global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 ozgemm_kernel(
     int nt, int nslab, int Gpad, int nmod, const int8_t *__restrict__ QX,
-    const int8_t *__restrict__ QB, size_t qstride, uint8_t *__restrict__ R) {
-  // XCD-contiguous remap over the whole grid, then (pair*nmod+m, panel)
+    const int8_t *__restrict__ QB, const int8_t *__restrict__ QY, size_t qstride,
+    int8_t *__restrict__ R) {
+  // XCD-contiguous remap over the whole grid, then (sign * nmod + m, panel)
   const int bid = blockIdx.x, nb = gridDim.x;
   const int xcd = bid & 7, i8 = bid >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int t = xcd * q8 + (xcd < r8 ? xcd : r8) + i8;
-  const int per = (int)oz_panels(nt);
+  const int per = (int)oz_panels<ONLY_O>(nt);
   const int qm = t / per, o = t - qm * per;
-  const int q = qm / nmod, m = qm - q * nmod;
+  const int q = qm / nmod, m = qm - q * nmod;  // q = 0: sign +, 1: sign -
   int J, IT;
-  oz_panel_at(o, nt, J, IT);
+  oz_panel_at<ONLY_O>(o, nt, J, IT);
   const long long npairs = (long long)nt * (nt + 1) / 2;
-  const int I0 = IT * OZ_R, J0 = J * OZ_T;
+  const int JH = ONLY_O ? 2 * J : J, JO = ONLY_O ? 2 * J + 1 : J;
+  const int I0 = IT * OZ_R, H0 = JH * OZ_T;
+  // past the last block (odd nt): any valid columns, not stored
+  const int O0 = min(JO, nt - 1) * OZ_T;
 
-  const int8_t *Ab = QX + (size_t)(m * 4 + q) * qstride;
-  const int8_t *Hb = QB + (size_t)(m * 3 + q) * qstride;
-  const int8_t *Ob = QX + (size_t)(m * 4 + (q == 2 ? 3 : q)) * qstride;
+  const int8_t *Ab = QX + (size_t)(2 * m + 1 - q) * qstride;
+  const int8_t *Hb = (ONLY_O ? QY : QB) + (size_t)(2 * m + q) * qstride;
+  const int8_t *Ob = QY + (size_t)(2 * m + q) * qstride;
 
   // one LDS array per stage and operand: the compiler then sees the DMA into
   // one stage and the reads of the other as disjoint (no wait inserted)
@@ -309,9 +517,11 @@ ozgemm_kernel(
     for (int u = 0; u < NBC; u++) {
       const int ci = w * NBC + u;
       const int kk = ci >> 1, rc = ci & 1;
-      const size_t boff = (((size_t)s * 4 + kk) * Gpad + J0 + rc * 64) * 16;
-      __builtin_amdgcn_global_load_lds(EXH_GLB(Hb + boff + voff), EXH_LDS(&dH[kk][rc * 64]), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(EXH_GLB(Ob + boff + voff), EXH_LDS(&dO[kk][rc * 64]), 16, 0, 0);
+      const size_t row = ((size_t)s * 4 + kk) * Gpad + rc * 64;
+      __builtin_amdgcn_global_load_lds(EXH_GLB(Hb + (row + H0) * 16 + voff),
+                                       EXH_LDS(&dH[kk][rc * 64]), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(EXH_GLB(Ob + (row + O0) * 16 + voff),
+                                       EXH_LDS(&dO[kk][rc * 64]), 16, 0, 0);
     }
   };
   auto compute = [&](v4i (*sA)[OZ_R], v4i (*sH)[OZ_T], v4i (*sO)[OZ_T]) {
@@ -353,255 +563,264 @@ ozgemm_kernel(
     }
   }
 
-  const int p = c_p[m];
-  const float rp = c_rp[m];
-  store_residues(ah, p, rp, rg, wc, lh, l32, IT, J,
-                 R + (size_t)(q * nmod + m) * npairs * (OZ_T * OZ_T));
-  store_residues(ao, p, rp, rg, wc, lh, l32, IT, J,
-                 R + (size_t)((3 + q) * nmod + m) * npairs * (OZ_T * OZ_T));
-}
-
-// Garner with symmetric digits: the integer x in (-M/2, M/2) with residues r_k.
-template <int NM>
-__device__ __forceinline__ double garner(const int *r) {
-  int v[NM];
-  double x = 0.0;
-#pragma unroll
-  for (int k = 0; k < NM; k++) {
-    const int p = c_p[k];
-    int acc = r[k] * c_w[k];
-#pragma unroll
-    for (int j = 0; j < k; j++) acc -= v[j] * c_c[j][k];
-    int q = (int)floorf((float)acc * c_rp[k]);
-    int d = acc - q * p;
-    d += (d < 0) ? p : 0;
-    d -= (d >= p) ? p : 0;
-    if (d > (p >> 1)) d -= p;
-    v[k] = d;
+  // planes: (H+, H-, O+, O-) x modulus, or (O+, O-) x modulus
+  const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
+  int8_t *Rq = R + (size_t)(q * nmod + m) * plane;
+  store_residues(ah, c_mod.m[m], rg, wc, lane, IT, JH, Rq);
+  if (ONLY_O) {
+    if (JO < nt) store_residues(ao, c_mod.m[m], rg, wc, lane, IT, JO, Rq);
+  } else {
+    store_residues(ao, c_mod.m[m], rg, wc, lane, IT, JO, Rq + (size_t)2 * nmod * plane);
   }
-#pragma unroll
-  for (int k = NM - 1; k >= 0; k--) x = fma(x, (double)c_p[k], (double)v[k]);
-  return x;
-}
-
-
-__device__ __forceinline__ int modp(int x, int k) {
-  const int p = c_p[k];
-  int r = x % p;
-  return r < 0 ? r + p : r;
 }
 
 // ---------------------------------------------------------------------------
 // Residues -> FP64 H and O upper elements (+ interstitial, + mirror).
-// One workgroup per 128x128 tile, walked in 32x32 sub-blocks: each thread
-// reconstructs four elements of a sub-block and writes them to the upper
-// triangle (coalesced along i); the sub-block is staged in LDS and written
-// back transposed and conjugated to the lower triangle (coalesced along j).
+// One workgroup per 32x32 sub-block of a tile: each thread reconstructs four
+// consecutive rows of one column from one 32-bit word per plane, the
+// sub-block is staged in LDS and written to the upper triangle (coalesced
+// along i) and, transposed and conjugated, to the lower one (coalesced along
+// j).  Per value and modulus: one add, one conversion and two FMAs (Garner's
+// algorithm needs m multiply-adds and a reduction at step m).  Bound by HBM:
+// 4 n bytes read and 64 written per upper element; 2.6 -> 1.26 ms at G = 9340
+// with 7 moduli (4.0 GB, 3.2 TB/s), 375 -> 24 us at G = 1166 with 9, where one
+// workgroup per 128 x 128 tile left most of the chip idle.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ int byte_of(int w, int t) { return (int)((unsigned)w << (24 - 8 * t)) >> 24; }
+
 template <int NM>
+__device__ __forceinline__ double crt(double hi, double lo) {
+  const OzCrt &C = c_crt.t[NM];
+  const double q = rint(hi * C.rP);  // |x| < 0.48 P: the low words cannot change it
+  return fma(-q, C.Ph, hi) + fma(-q, C.Pl, lo);
+}
+
+template <int NM, bool ONLY_O>
 __global__ __launch_bounds__(256) void ozcombine_kernel(
-    int ngp, int npairs, const uint8_t *__restrict__ R, const int *__restrict__ ex,
-    const int *__restrict__ eb, int bits, IstBox box, double2 *__restrict__ H,
-    double2 *__restrict__ O, long long ldh, int accumulate) {
-  const int tile = blockIdx.x;
+    int ngp, int npairs, const int8_t *__restrict__ R, const int *__restrict__ ex,
+    const int *__restrict__ eb, const int *__restrict__ ey, int bits, IstBox box,
+    double2 *__restrict__ H, double2 *__restrict__ O, long long ldh, int accumulate) {
+  const int tile = blockIdx.x >> 4, sb = blockIdx.x & 15;
   int J = (int)((sqrt(8.0 * (double)tile + 1.0) - 1.0) * 0.5);
   while ((J + 1) * (J + 2) / 2 <= tile) J++;
   while (J * (J + 1) / 2 > tile) J--;
   const int I = tile - J * (J + 1) / 2;
-  const int I0 = I * OZ_T, J0 = J * OZ_T;
-  const size_t TT = (size_t)OZ_T * OZ_T;
-  __shared__ double2 sH[32][33], sO[32][33];
-  const int tid = threadIdx.x, lo = tid & 31, hi8 = tid >> 5;
-  for (int sb = 0; sb < 16; sb++) {
-    const int bi = sb & 3, bj = sb >> 2;
-    if (I == J && bi > bj) continue;  // wholly below the diagonal (uniform)
-#pragma unroll 1
-    for (int r = 0; r < 4; r++) {
-      const int il = bi * 32 + lo, jl = bj * 32 + hi8 + 8 * r;
-      const int i = I0 + il, j = J0 + jl;
-      if (i >= ngp || j >= ngp || i > j) continue;
-      const int e = il + OZ_T * jl;
-      int hre[NM], him[NM], ore[NM], oim[NM];
+  const int i0 = I * OZ_T + (sb & 3) * 32, j0 = J * OZ_T + (sb >> 2) * 32;
+  if (i0 > j0 || i0 >= ngp || j0 >= ngp) return;  // below the diagonal or outside
+  constexpr int NV = ONLY_O ? 1 : 2;              // matrices
+  __shared__ double2 sT[NV][32][33];
+  const int tid = threadIdx.x, lane = tid & 63, h = tid >> 6;
+  const int il = 8 * h + 4 * (lane >> 5), jl = lane & 31;
+  const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
+  const int8_t *r0 = R + (size_t)tile * (OZ_T * OZ_T) + sb * 1024 + tid * 4;
+
+  double rh[NV][4], rl[NV][4], mh[NV][4], ml[NV][4];
 #pragma unroll
-      for (int k = 0; k < NM; k++) {
-        int rr[6];
+  for (int v = 0; v < NV; v++)
 #pragma unroll
-        for (int pr = 0; pr < 6; pr++)
-          rr[pr] = R[((size_t)(pr * NM + k) * npairs + tile) * TT + e];
-        hre[k] = modp(rr[0] + rr[1], k);
-        him[k] = modp(rr[0] - rr[1] - rr[2], k);
-        ore[k] = modp(rr[3] + rr[4], k);
-        oim[k] = modp(rr[3] - rr[4] - rr[5], k);
+    for (int t = 0; t < 4; t++) rh[v][t] = rl[v][t] = mh[v][t] = ml[v][t] = 0.0;
+  const OzCrt &C = c_crt.t[NM];
+#pragma unroll
+  for (int k = 0; k < NM; k++)
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const int wp = *(const int *)(r0 + (size_t)((2 * v) * NM + k) * plane);
+      const int wm = *(const int *)(r0 + (size_t)((2 * v + 1) * NM + k) * plane);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int a = byte_of(wp, t), b = byte_of(wm, t);
+        const double s = (double)(a + b), d = (double)(a - b);
+        rh[v][t] = fma(s, C.reh[k], rh[v][t]);
+        rl[v][t] = fma(s, C.rel[k], rl[v][t]);
+        mh[v][t] = fma(d, C.imh[k], mh[v][t]);
+        ml[v][t] = fma(d, C.iml[k], ml[v][t]);
       }
-      const int si = ex[i] == INT_MIN ? 0 : bits - ex[i];
-      const int sjb = eb[j] == INT_MIN ? 0 : bits - eb[j];
-      const int sjx = ex[j] == INT_MIN ? 0 : bits - ex[j];
-      double hr = ldexp(garner<NM>(hre), -(si + sjb));
-      double hv = ldexp(garner<NM>(him), -(si + sjb));
-      double orr = ldexp(garner<NM>(ore), -(si + sjx));
-      double oi = ldexp(garner<NM>(oim), -(si + sjx));
-      const size_t up = (size_t)i + (size_t)j * ldh;
+    }
+
+  const int j = j0 + jl;
+  if (j < ngp) {
+    const int ebj = ONLY_O ? 0 : eb[j], eyj = ey[j];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int i = i0 + il + t;
+      if (i >= ngp || i > j) continue;
+      const int exi = ex[i];
+      auto value = [&](int v, int ej) {
+        // 2^-(s_i + s_j); a column that is not finite makes the element NaN
+        const bool bad = exi == INT_MAX || ej == INT_MAX;
+        const int si = exi == INT_MIN ? 0 : bits - exi, sj = ej == INT_MIN ? 0 : bits - ej;
+        const int sh = bad ? 0 : -(si + sj);
+        const double nan = __builtin_nan("");
+        const double re = ldexp(crt<NM>(rh[v][t], rl[v][t]), sh);
+        const double im = ldexp(crt<NM>(mh[v][t], ml[v][t]), sh);
+        return bad ? z2(nan, nan) : z2(re, im);
+      };
+      double2 hv = z2(0.0, 0.0), ov = value(NV - 1, eyj);
+      if (!ONLY_O) hv = value(0, ebj);
+      ist_add(box, i, j, hv.x, hv.y, ov.x, ov.y);
+      if (!ONLY_O) sT[0][jl][il + t] = hv;
+      sT[NV - 1][jl][il + t] = ov;
+    }
+  }
+  __syncthreads();
+  const int lo = tid & 31, hi8 = tid >> 5;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int c = hi8 + 8 * r, i = i0 + lo, jj = j0 + c;
+    if (i >= ngp || jj >= ngp || i > jj) continue;
+    const size_t up = (size_t)i + (size_t)jj * ldh;
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      double2 *M = (!ONLY_O && v == 0) ? H : O;
+      double2 x = sT[v][c][lo];
       if (accumulate) {
-        const double2 h0 = H[up], o0 = O[up];
-        hr += h0.x;
-        hv += h0.y;
-        orr += o0.x;
-        oi += o0.y;
+        const double2 old = M[up];
+        x.x += old.x;
+        x.y += old.y;
+        sT[v][c][lo] = x;
       }
-      ist_add(box, i, j, hr, hv, orr, oi);
-      H[up] = z2(hr, hv);
-      O[up] = z2(orr, oi);
-      sH[jl - bj * 32][lo] = z2(hr, -hv);
-      sO[jl - bj * 32][lo] = z2(orr, -oi);
+      M[up] = x;
     }
-    __syncthreads();
-    // lower triangle: element (j, i) = conj(upper (i, j)), i < j
-#pragma unroll 1
-    for (int r = 0; r < 4; r++) {
-      const int jl = bj * 32 + lo, il = bi * 32 + hi8 + 8 * r;
-      const int i = I0 + il, j = J0 + jl;
-      if (i >= ngp || j >= ngp || i >= j) continue;
-      const size_t lw = (size_t)j + (size_t)i * ldh;
-      H[lw] = sH[lo][hi8 + 8 * r];
-      O[lw] = sO[lo][hi8 + 8 * r];
+  }
+  if (accumulate) __syncthreads();
+  // lower triangle: element (j, i) = conj(upper (i, j)), i < j
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int c = hi8 + 8 * r, jj = j0 + lo, i = i0 + c;
+    if (i >= ngp || jj >= ngp || i >= jj) continue;
+    const size_t lw = (size_t)jj + (size_t)i * ldh;
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      double2 *M = (!ONLY_O && v == 0) ? H : O;
+      const double2 x = sT[v][lo][c];
+      M[lw] = z2(x.x, -x.y);
     }
-    __syncthreads();
   }
 }
-
 
 inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
+// EXH_SPLIT(n) rounds to the c bits that the product of the n largest primes
+// <= 251 would allow, whatever moduli recover the products.
+constexpr int kPrimes[kOzMaxMod] = {251, 241, 239, 233, 229, 227, 223, 211, 199, 197, 193, 191};
+
 }  // namespace
 
-const int kOzPrimes[kOzMaxMod] = {251, 241, 239, 233, 229, 227, 223, 211, 199, 197, 193, 191};
-
-int oz_bits(int nmod, int Ktot) {
-  (void)Ktot;
+OzPlan oz_split(int n) {
   double lm = 0.0;
-  for (int k = 0; k < nmod; k++) lm += std::log2((double)kOzPrimes[k]);
-  // |Re|, |Im| of x^H b <= ||x|| ||b|| <= 2^(2c) must stay below prod(p)/2
-  // (a hair below the exact bound guards the floating-point log2); the
-  // scaled entries stay well inside FP64's exact integers
-  const double c = std::floor((lm - 1.0) * 0.5 - 1e-9);
-  return (int)std::min(50.0, c);
+  for (int k = 0; k < n; k++) lm += std::log2((double)kPrimes[k]);
+  // the largest c with 2^(2c) < prod/2 (a hair below guards the log2)
+  OzPlan P;
+  P.bits = (int)std::min(50.0, std::floor((lm - 1.0) * 0.5 - 1e-9));
+  // the scaled columns' norms are below 2^(c-1) + sqrt(2K)/2, so the products
+  // need prod(p) > 2^(2c-1) (1 + 2^-13 at c = 23)
+  double need = 2.0 * P.bits - 1.0 + 1e-3;
+  for (P.nmod = 0; need > 0.0; P.nmod++) need -= std::log2((double)kP[P.nmod]);
+  return P;
 }
 
-// The tables cover all kOzMaxMod moduli whatever nmod a call uses, so they are
-// written once per device and process; the mutex keeps contexts on other host
-// threads from writing them while this one does.
-hipError_t oz_upload_constants(int nmod) {
-  constexpr int kMaxDevices = 64;
-  static std::mutex mu;
-  static bool done[kMaxDevices] = {};
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> guard(mu);
-  if (dev < kMaxDevices && done[dev]) return hipSuccess;
-  int p[kOzMaxMod], w[kOzMaxMod], cc[kOzMaxMod][kOzMaxMod];
-  float rp[kOzMaxMod];
-  auto inv = [](long long a, int m) {  // a^-1 mod m, m prime
-    long long r = 1, b = ((a % m) + m) % m, e = m - 2;
-    while (e) {
-      if (e & 1) r = r * b % m;
-      b = b * b % m;
-      e >>= 1;
-    }
-    return (int)r;
-  };
-  for (int k = 0; k < kOzMaxMod; k++) {
-    p[k] = kOzPrimes[k];
-    rp[k] = 1.0f / (float)p[k];
-    long long P = 1;  // p_0 ... p_{k-1} mod p_k
-    for (int j = 0; j < k; j++) P = P * kOzPrimes[j] % kOzPrimes[k];
-    w[k] = k == 0 ? 1 : inv(P, kOzPrimes[k]);
-    long long Pj = 1;  // p_0 ... p_{j-1} mod p_k
-    for (int j = 0; j < kOzMaxMod; j++) {
-      cc[j][k] = (j < k) ? (int)(Pj * w[k] % kOzPrimes[k]) : 0;
-      if (j < k) Pj = Pj * kOzPrimes[j] % kOzPrimes[k];
-    }
-  }
-  (void)nmod;
-  e = hipMemcpyToSymbol(HIP_SYMBOL(c_p), p, sizeof p);
-  if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(c_rp), rp, sizeof rp);
-  if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(c_w), w, sizeof w);
-  if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(c_c), cc, sizeof cc);
-  if (e == hipSuccess && dev < kMaxDevices) done[dev] = true;
-  return e;
+// c = 56: norms below 2^55, products below 2^110 < 0.47 prod(p) = 2^111.09.
+OzPlan oz_fp64() {
+  OzPlan P;
+  P.bits = 56;
+  P.nmod = OZ_N;
+  return P;
 }
 
-OzLayout oz_layout(int ngkmax, int Ktot, int nmod) {
+OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool third) {
   OzLayout L;
-  // rows padded to 384: a multiple of the row panel (384 or 192 rows) and of
-  // the 128-column blocks, so every panel and column block loads inside it
+  // rows padded to 384: a multiple of the row panel and of the 128-column
+  // blocks, so every panel and column block loads inside it
   constexpr int GA = 384;
   static_assert(GA % OZ_R == 0 && GA % OZ_T == 0, "row padding");
   L.Gpad = (ngkmax + GA - 1) / GA * GA;
   L.Kpad = (Ktot + OZ_KS - 1) / OZ_KS * OZ_KS;
   L.qstride = (size_t)L.Kpad * L.Gpad;
   const long long nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
-  L.max_pairs = nt * (nt + 1) / 2;
-  L.qx_bytes = (size_t)nmod * 4 * L.qstride;
-  L.qb_bytes = (size_t)nmod * 3 * L.qstride;
-  L.r_bytes = (size_t)6 * nmod * L.max_pairs * OZ_T * OZ_T;
-  // per operand: the column exponents, then the partial norms
-  L.e_part_off = ((size_t)std::max(ngkmax, 1) * sizeof(int) + 255) / 256 * 256;
-  L.e_bytes = L.e_part_off +
-              sizeof(double) * (size_t)((Ktot + OZ_NCH - 1) / OZ_NCH) * std::max(ngkmax, 1);
+  L.q_bytes = (size_t)P.nmod * 2 * L.qstride;
+  L.r_bytes = (size_t)(only_o ? 2 : 4) * P.nmod * (nt * (nt + 1) / 2) * OZ_T * OZ_T;
+  // per operand: the column exponents, then the partial norms and theirs
+  const size_t ng = std::max(ngkmax, 1), nch = (Ktot + OZ_NCH - 1) / OZ_NCH;
+  L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
+  L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * nch * ng + 255) / 256 * 256;
+  L.nops = 1 + (only_o ? 0 : 1) + (third ? 1 : 0);
   return L;
 }
 
-hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const double2 *X,
-                        long long ldx, const double2 *B, long long ldb, int nmod, int bits,
-                        const OzLayout &L, int8_t *QX, int8_t *QB, uint8_t *R, int *ex, int *eb,
-                        const IstBox &box, double2 *h, double2 *o, int ldh, int accumulate,
-                        int stage_mask) {
+hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const OzPlan &P,
+                        const OzLayout &L, const OzScratch &w, const double2 *X, long long ldx,
+                        const double2 *B, const double2 *Y, long long ldb, const IstBox &box,
+                        double2 *h, double2 *o, int ldh, int accumulate, int stage_mask) {
   if (ngp <= 0) return hipSuccess;
   const int K = c->Ktot;
   const long long nt = (ngp + OZ_T - 1) / OZ_T;
   const long long npairs = nt * (nt + 1) / 2;
   const int nslab = L.Kpad / OZ_KS;
+  // operands: X, then B (not for O alone), then Y where the overlap has its own
+  const bool only_o = h == nullptr;
+  OzOperands op{};
+  const double2 *src[3] = {X, B, Y};
+  int n = 0, iB = 0, iY = 0;
+  for (int z = 0; z < 3; z++) {
+    if ((z == 1 && only_o) || (z == 2 && !Y)) continue;
+    if (z == 1) iB = n;
+    if (z == 2) iY = n;
+    char *e = (char *)w.e + (size_t)n * L.e_bytes;
+    op.x[n] = src[z];
+    op.ld[n] = z == 0 ? ldx : ldb;
+    op.e[n] = (int *)e;
+    op.part[n] = (double *)(e + L.e_part_off);
+    op.q[n] = w.q + (size_t)n * L.q_bytes;
+    n++;
+  }
   if (stage_mask & 1) {
     const int nch = (K + OZ_NCH - 1) / OZ_NCH;
     const int ldp = std::max(c->ngkmax, 1);
-    double *px = (double *)((char *)ex + L.e_part_off);
-    double *pb = (double *)((char *)eb + L.e_part_off);
-    dim3 ge(cdiv(ngp, 256), nch);
-    hipLaunchKernelGGL(colnorm_part_kernel, ge, dim3(256), 0, s, ngp, K, X, ldx, px, ldp);
-    hipLaunchKernelGGL(colnorm_part_kernel, ge, dim3(256), 0, s, ngp, K, B, ldb, pb, ldp);
-    hipLaunchKernelGGL(colnorm_final_kernel, dim3(cdiv(ngp, 256)), dim3(256), 0, s, ngp, nch,
-                       px, ldp, ex);
-    hipLaunchKernelGGL(colnorm_final_kernel, dim3(cdiv(ngp, 256)), dim3(256), 0, s, ngp, nch,
-                       pb, ldp, eb);
-    dim3 gr(cdiv(L.Gpad, 256), L.Kpad / 16);
-    hipLaunchKernelGGL(residue_kernel<4>, gr, dim3(256), 0, s, ngp, K, L.Gpad, X, ldx, ex, bits,
-                       nmod, L.qstride, QX);
-    hipLaunchKernelGGL(residue_kernel<3>, gr, dim3(256), 0, s, ngp, K, L.Gpad, B, ldb, eb, bits,
-                       nmod, L.qstride, QB);
+    hipLaunchKernelGGL(colnorm_part_kernel, dim3(cdiv(ngp, 64), nch, n), dim3(256), 0, s, ngp, K,
+                       op, ldp, nch);
+    hipLaunchKernelGGL(colnorm_final_kernel, dim3(cdiv(ngp, 64), n), dim3(64), 0, s, ngp, nch, op,
+                       ldp);
+    // rows up to the last row panel this k-point uses
+    const int rows = (ngp + OZ_R - 1) / OZ_R * OZ_R;
+    hipLaunchKernelGGL(residue_kernel, dim3(cdiv(rows, 256), L.Kpad / 16, n), dim3(256), 0, s,
+                       ngp, K, L.Gpad, rows, op, P.bits, P.nmod, L.qstride);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (stage_mask & 2) {
-    const long long per = oz_panels((int)nt);
-    hipLaunchKernelGGL(ozgemm_kernel, dim3((unsigned)(per * 3 * nmod)), dim3(64 * OZ_NWG), 0, s,
-                       (int)nt,
-                       nslab, L.Gpad, nmod, QX, QB, L.qstride, R);
+    const long long per = only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt);
+    const dim3 grid((unsigned)(per * 2 * P.nmod));
+    if (only_o)
+      hipLaunchKernelGGL(ozgemm_kernel<true>, grid, dim3(64 * OZ_NWG), 0, s, (int)nt, nslab,
+                         L.Gpad, P.nmod, op.q[0], op.q[iY], op.q[iY], L.qstride, w.r);
+    else
+      hipLaunchKernelGGL(ozgemm_kernel<false>, grid, dim3(64 * OZ_NWG), 0, s, (int)nt, nslab,
+                         L.Gpad, P.nmod, op.q[0], op.q[iB], op.q[iY], L.qstride, w.r);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (stage_mask & 4) {
-    switch (nmod) {
-#define EXH_OZC(N)                                                                          \
-  case N:                                                                                   \
-    hipLaunchKernelGGL(ozcombine_kernel<N>, dim3((unsigned)npairs), dim3(256), 0, s, ngp,     \
-                       (int)npairs, R, ex, eb, bits, box, h, o, (long long)ldh, accumulate); \
-    break;
-      EXH_OZC(6) EXH_OZC(7) EXH_OZC(8) EXH_OZC(9) EXH_OZC(10) EXH_OZC(11) EXH_OZC(12)
-#undef EXH_OZC
-      default:
-        return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(npairs * 16));
+#define EXH_OZC(N, OO)                                                                         \
+  hipLaunchKernelGGL((ozcombine_kernel<N, OO>), grid, dim3(256), 0, s, ngp, (int)npairs, w.r,  \
+                     op.e[0], op.e[iB], op.e[iY], P.bits, box, h, o, (long long)ldh, accumulate)
+    if (only_o) {
+      if (P.nmod != OZ_N) return hipErrorInvalidValue;  // EXH_SPLIT is refused for O alone
+      EXH_OZC(OZ_N, true);
+    } else {
+      switch (P.nmod) {
+        case 6: EXH_OZC(6, false); break;
+        case 7: EXH_OZC(7, false); break;
+        case 8: EXH_OZC(8, false); break;
+        case 9: EXH_OZC(9, false); break;
+        case 10: EXH_OZC(10, false); break;
+        case 11: EXH_OZC(11, false); break;
+        case 13: EXH_OZC(13, false); break;  // EXH_SPLIT(12)
+        case OZ_N: EXH_OZC(OZ_N, false); break;
+        default: return hipErrorInvalidValue;
+      }
     }
+#undef EXH_OZC
   }
   return hipGetLastError();
 }

@@ -92,8 +92,9 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
         gpad = (sys_.ngkmax + 383) // 384 * 384     # rows padded to the GEMM's panel
         kpad = (K + 63) // 64 * 64
         nt = (sys_.ngkmax + 127) // 128
-        scratch += 7 * nmod_max * kpad * gpad    # int8 residues of A and aa.A
-        scratch += 6 * nmod_max * nt * (nt + 1) // 2 * 128 * 128   # product residues
+        moduli = nmod_max + 1                       # SPLIT(12) runs 13 moduli
+        scratch += 4 * moduli * kpad * gpad         # int8 residues of A and aa.A
+        scratch += 4 * moduli * nt * (nt + 1) // 2 * 128 * 128   # product residues
     perk = len(sys_.kpts) * sys_.ngkmax * (16 * sys_.natmtot + 8 * 7 + 4)
     # Cholesky factor, the two triangular solves' results, the reduced matrix
     # and its Hermitian average, and the eigensolver's copy and workspace

@@ -65,11 +65,12 @@ enum {
 };
 /* Split precision: EXH_SPLIT(n), 6 <= n <= 12, OR-ed into flags, computes the
  * muffin-tin APW-APW products with the Ozaki scheme II on int8 matrix cores:
- * A and aa.A are rounded per G column to b-bit integers (b is the largest
- * value for which n primes <= 251 recover every product exactly; b = 26 for
- * n = 9 at K = 15488) and multiplied exactly through n modular int8 GEMMs.
- * The rounding is the only approximation (relative 2^-b per column).  Match,
- * the lo blocks and the interstitial stay FP64.  Not combined with h1aa. */
+ * A and aa.A are rounded per G column to integers (the column's 2-norm scaled
+ * below 2^(c-1), c the largest value with 2^(2c) below half the product of
+ * the n largest primes <= 251: c = 27 for n = 7, 34 for n = 9) and multiplied
+ * exactly through modular int8 GEMMs.  The rounding is the only approximation
+ * (2^-c of the column's norm).  Match, the lo blocks and the interstitial
+ * stay FP64.  Not combined with h1aa. */
 #define EXH_SPLIT(n) ((n) << 8)
 
 /* ---- context ------------------------------------------------------------ */
