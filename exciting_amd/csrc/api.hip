@@ -385,11 +385,20 @@ int wait_done(exh_context *c) {
   return e == hipSuccess ? 0 : hip_fail(c, e, "waiting for queued work");
 }
 
-// The modular contraction of a setup with these flags (EXH_SPLIT(n)).
+// The modular contraction of a setup with these flags: EXH_SPLIT(n), or for
+// FP64 the 15-moduli plan when one K-major operand (16 Ktot ldb bytes) is
+// larger than the static array of exh_setup_device_noalloc, so that wherever
+// that entry point takes a basis it runs the kernels exh_setup_device runs.
+// At that line the modular path is already the faster one (whole match +
+// setup, FP64 MFMA kernels against modular): 79 MB operands, K = 2904,
+// G = 1780: 2.39 against 1.45 ms; 107 MB, K = 2646, G = 2657: 3.20 against
+// 1.43 ms, O alone 1.54 against 0.75 ms; 2.3 GB, K = 15488, G = 9340: 168
+// against 50.7 ms.
 OzPlan oz_plan(const exh_context *c, int flags) {
-  (void)c;
   const int n = (flags >> 8) & 0xff;
-  return n ? oz_split(n) : OzPlan();
+  if (n) return oz_split(n);
+  const size_t op = (size_t)c->Ktot * ((c->ngkmax + 63) / 64 * 64) * sizeof(double2);
+  return op > kNoallocScratchBytes && c->Ktot <= kOzMaxK ? oz_fp64() : OzPlan();
 }
 
 bool oz_fits(const exh_context *c, const OzLayout &L) {

@@ -88,11 +88,13 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     K = sys_.natmtot * sys_.maxaa
     ldb = (sys_.ngkmax + 63) // 64 * 64
     scratch = 16 * K * ldb                       # aa.A operand
-    if nmod_max:
+    fp64_modular = 16 * K * ldb > 64 << 20       # FP64 on the 15-moduli products
+    if nmod_max or fp64_modular:
         gpad = (sys_.ngkmax + 383) // 384 * 384     # rows padded to the GEMM's panel
         kpad = (K + 63) // 64 * 64
         nt = (sys_.ngkmax + 127) // 128
-        moduli = nmod_max + 1                       # SPLIT(12) runs 13 moduli
+        # SPLIT(12) runs 13 moduli
+        moduli = max(nmod_max + 1 if nmod_max else 0, 15 if fp64_modular else 0)
         scratch += 4 * moduli * kpad * gpad         # int8 residues of A and aa.A
         scratch += 4 * moduli * nt * (nt + 1) // 2 * 128 * 128   # product residues
     perk = len(sys_.kpts) * sys_.ngkmax * (16 * sys_.natmtot + 8 * 7 + 4)

@@ -70,7 +70,17 @@ enum {
  * the n largest primes <= 251: c = 27 for n = 7, 34 for n = 9) and multiplied
  * exactly through modular int8 GEMMs.  The rounding is the only approximation
  * (2^-c of the column's norm).  Match, the lo blocks and the interstitial
- * stay FP64.  Not combined with h1aa. */
+ * stay FP64.  Not combined with h1aa.
+ *
+ * Without EXH_SPLIT, setups of large bases (16 natmtot*maxaa * ngkmax rounded
+ * up > 64 MiB) use the same exact products with c = 56: each operand keeps 55
+ * bits relative to its column's 2-norm and nothing else is rounded before the
+ * result, which is nearer to the exact product than FP64 accumulation over
+ * K (H and O at 64 atoms: relative Frobenius error 1e-16 against 5e-15).
+ * They need 60 bytes of scratch per (K, G+k) pair and 60 per upper element
+ * of H; a device without that room, or a stream captured before a first call
+ * has allocated it, runs the FP64 MFMA kernels instead (results differ by
+ * rounding). */
 #define EXH_SPLIT(n) ((n) << 8)
 
 /* ---- context ------------------------------------------------------------ */
