@@ -47,7 +47,7 @@ struct OzPlan {
   int bits = 0;  // c: the scaled columns' 2-norms are below 2^(c-1)
 };
 struct OzLayout {
-  int Gpad = 0, Kpad = 0;  // G rounded to the row panel, K to the 64 stage
+  int Gpad = 0, Kpad = 0;  // G rounded to the row panel, K to two 64-k stages
   size_t qstride = 0;      // bytes of one residue array (Kpad * Gpad)
   int nops = 0;            // operands (X; B unless O alone; (1+h1)A for iora*)
   size_t q_bytes = 0;      // residues of one operand

@@ -350,15 +350,22 @@ __global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpa
 // groups, one workgroup per CU.  (192-row panels, two 4-wave workgroups per
 // CU whose barriers fall at different times, gave the same products and
 // measured 1 % slower at the 64-atom shape.)
-// Operands stream global -> LDS directly (global_load_lds, 16 bytes per
+// Operands stream global -> LDS directly (buffer loads to LDS, 16 bytes per
 // lane, one 64-row chunk of one k block per instruction), two stages of 64 k
 // double-buffered.
+// Bound by the power the matrix cores draw: at K = 15488, G = 9340, 14
+// products, 16.4 ms = 2.30 POP/s with the cores busy 72 % of the cycles at
+// 1.56 GHz; with all-zero operands (same instructions) 13.4 ms.  Reading the
+// fragments ahead took it there from 17.9 ms (60 % busy), where both waves of
+// a SIMD waited for LDS four times per stage.  A third stage in LDS (16.5 ms)
+// and raised wave priority around the MFMAs (16.3-16.4 ms) change nothing.
 // Operand lane layout: row/column = lane%32, 16 k bytes from k block
 // 2*ks + lane/32; result D[8*(r/4) + 4*(lane/32) + r%4][lane%32].
 // ---------------------------------------------------------------------------
 constexpr int OZ_WR = 3;           // 32-row blocks per wave (96 rows)
 constexpr int OZ_NWG = 8;          // waves per workgroup
 constexpr int OZ_R = 48 * OZ_NWG;  // rows of the row panel per workgroup
+constexpr int OZ_W = OZ_R + 2 * OZ_T;  // rows and columns of one LDS stage
 
 #define EXH_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 #define EXH_GLB(p) ((const __attribute__((address_space(1))) void *)(p))
@@ -469,10 +476,13 @@ ozgemm_kernel(
   const int xcd = bid & 7, i8 = bid >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int t = xcd * q8 + (xcd < r8 ? xcd : r8) + i8;
   const int per = (int)oz_panels<ONLY_O>(nt);
-  const int qm = t / per, o = t - qm * per;
-  const int q = qm / nmod, m = qm - q * nmod;  // q = 0: sign +, 1: sign -
+  const int qm = __builtin_amdgcn_readfirstlane(t / per), o = t - qm * per;
+  const int q = qm >= nmod ? 1 : 0, m = qm - q * nmod;  // q = 0: sign +, 1: sign -
   int J, IT;
   oz_panel_at<ONLY_O>(o, nt, J, IT);
+  // uniform by construction; scalar registers for the addresses that follow
+  J = __builtin_amdgcn_readfirstlane(J);
+  IT = __builtin_amdgcn_readfirstlane(IT);
   const long long npairs = (long long)nt * (nt + 1) / 2;
   const int JH = ONLY_O ? 2 * J : J, JO = ONLY_O ? 2 * J + 1 : J;
   const int I0 = IT * OZ_R, H0 = JH * OZ_T;
@@ -483,10 +493,10 @@ ozgemm_kernel(
   const int8_t *Hb = (ONLY_O ? QY : QB) + (size_t)(2 * m + q) * qstride;
   const int8_t *Ob = QY + (size_t)(2 * m + q) * qstride;
 
-  // one LDS array per stage and operand: the compiler then sees the DMA into
-  // one stage and the reads of the other as disjoint (no wait inserted)
-  __shared__ v4i sA0[4][OZ_R], sH0[4][OZ_T], sO0[4][OZ_T];
-  __shared__ v4i sA1[4][OZ_R], sH1[4][OZ_T], sO1[4][OZ_T];
+  // one LDS array per stage: the compiler then sees the DMA into one stage and
+  // the reads of the other as disjoint (no wait inserted).  Rows 0..383 hold
+  // the row operand, then 128 columns of H and of O.
+  __shared__ v4i sm0[4][OZ_W], sm1[4][OZ_W];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = w >> 1, wc = w & 1, l32 = lane & 31, lh = lane >> 5;
@@ -500,68 +510,98 @@ ozgemm_kernel(
     }
 
   // Chunks of 64 rows x 16 bytes per stage: 4 k blocks x OZ_R/64 row chunks
-  // of A (3 per wave), 4 k blocks x 2 of H and of O (8 / OZ_NWG each per
-  // wave); each lane moves its 16 bytes to chunk base + 16 lane
-  constexpr int RC = OZ_R / 64, NBC = 8 / OZ_NWG;
-  static_assert(4 * RC == OZ_WR * OZ_NWG && NBC * OZ_NWG == 8, "chunking");
+  // of A (3 per wave), 4 k blocks x 2 of H and of O (one each per wave); each
+  // lane moves its 16 bytes to chunk base + 16 lane.  Buffer loads keep the
+  // addresses in scalar registers, which leaves the vector registers to the
+  // second set of operand fragments below.
+  constexpr int RC = OZ_R / 64;
+  static_assert(4 * RC == OZ_WR * OZ_NWG && OZ_NWG == 8, "chunking");
   const int voff = lane * 16;
-  auto issue = [&](int s, v4i (*dA)[OZ_R], v4i (*dH)[OZ_T], v4i (*dO)[OZ_T]) {
+  auto issue = [&](int s, v4i (*d)[OZ_W]) {
+    const size_t so = (size_t)s * 4 * Gpad * 16;
+    const int span = 4 * Gpad * 16;  // bytes of the stage's four k blocks
+    constexpr int kRaw = 0x00020000;
+    const auto rA = __builtin_amdgcn_make_buffer_rsrc((void *)(Ab + so), 0, span, kRaw);
+    const auto rH = __builtin_amdgcn_make_buffer_rsrc((void *)(Hb + so), 0, span, kRaw);
+    const auto rO = __builtin_amdgcn_make_buffer_rsrc((void *)(Ob + so), 0, span, kRaw);
 #pragma unroll
     for (int u = 0; u < OZ_WR; u++) {
       const int ci = w * OZ_WR + u;
       const int kk = ci / RC, rc = ci - RC * kk;
-      const int8_t *src = Ab + (((size_t)s * 4 + kk) * Gpad + I0 + rc * 64) * 16;
-      __builtin_amdgcn_global_load_lds(EXH_GLB(src + voff), EXH_LDS(&dA[kk][rc * 64]), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, EXH_LDS(&d[kk][rc * 64]), 16, voff,
+                                               (kk * Gpad + I0 + rc * 64) * 16, 0, 0);
     }
-#pragma unroll
-    for (int u = 0; u < NBC; u++) {
-      const int ci = w * NBC + u;
-      const int kk = ci >> 1, rc = ci & 1;
-      const size_t row = ((size_t)s * 4 + kk) * Gpad + rc * 64;
-      __builtin_amdgcn_global_load_lds(EXH_GLB(Hb + (row + H0) * 16 + voff),
-                                       EXH_LDS(&dH[kk][rc * 64]), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(EXH_GLB(Ob + (row + O0) * 16 + voff),
-                                       EXH_LDS(&dO[kk][rc * 64]), 16, 0, 0);
-    }
+    const int kk = w >> 1, rc = w & 1;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rH, EXH_LDS(&d[kk][OZ_R + rc * 64]), 16, voff,
+                                             (kk * Gpad + H0 + rc * 64) * 16, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rO, EXH_LDS(&d[kk][OZ_R + OZ_T + rc * 64]), 16, voff,
+                                             (kk * Gpad + O0 + rc * 64) * 16, 0, 0);
   };
-  auto compute = [&](v4i (*sA)[OZ_R], v4i (*sH)[OZ_T], v4i (*sO)[OZ_T]) {
+  const int ra = rg * 32 * OZ_WR + l32, ca = OZ_R + wc * 64 + l32;
+  auto rdA = [&](v4i (*d)[OZ_W], int ks, int a) { return d[2 * ks + lh][ra + a * 32]; };
+  auto rdH = [&](v4i (*d)[OZ_W], int ks, int b) { return d[2 * ks + lh][ca + b * 32]; };
+  auto rdO = [&](v4i (*d)[OZ_W], int ks, int b) { return d[2 * ks + lh][ca + OZ_T + b * 32]; };
+  // four MFMAs of block row a, kept apart from the reads before and after
+  auto mm = [&](int a, v4i A, const v4i (&h)[2], const v4i (&o)[2]) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      const int kk = 2 * ks + lh;
-      v4i av[OZ_WR], hv[2], ov[2];
-#pragma unroll
-      for (int a = 0; a < OZ_WR; a++) av[a] = sA[kk][rg * 32 * OZ_WR + a * 32 + l32];
-#pragma unroll
-      for (int b = 0; b < 2; b++) {
-        hv[b] = sH[kk][wc * 64 + b * 32 + l32];
-        ov[b] = sO[kk][wc * 64 + b * 32 + l32];
-      }
-#pragma unroll
-      for (int a = 0; a < OZ_WR; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-          ah[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[a], hv[b], ah[a][b], 0, 0, 0);
-          ao[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[a], ov[b], ao[a][b], 0, 0, 0);
-        }
+    for (int b = 0; b < 2; b++) {
+      ah[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, h[b], ah[a][b], 0, 0, 0);
+      ao[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, o[b], ao[a][b], 0, 0, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // vmcnt(0): every DMA of this wave has landed in LDS; the barrier then
-  // makes all waves' chunks visible and frees the stage read last
-  issue(0, sA0, sH0, sO0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  __syncthreads();
+  // One stage of 64 k: six groups of four MFMAs.  The fragments of a group
+  // are read from LDS one or two groups ahead (h1, o1: the second 32 k; then
+  // h0, o0 of the next stage), so the two waves of a SIMD, which the barrier
+  // keeps in step, do not both wait for LDS.  At the barrier every read of
+  // `cur` has returned (lgkmcnt) and the next stage has landed (vmcnt): `cur`
+  // is refilled with stage s + 2, and eight MFMAs whose operands are in
+  // registers cover the first reads of `nxt`.  The last two refills repeat
+  // the last stage and are not read.
+  v4i h0[2], o0[2], h1[2], o1[2], x0, x1, x2;
+#define EXH_STAGE_BARRIER(N) \
+  asm volatile("s_waitcnt vmcnt(" #N ") lgkmcnt(0)\n\ts_barrier" ::: "memory")
+  auto stage = [&](int s, v4i (*cur)[OZ_W], v4i (*nxt)[OZ_W]) {
+    x1 = rdA(cur, 0, 1);
+    h1[0] = rdH(cur, 1, 0);
+    mm(0, x0, h0, o0);
+    x2 = rdA(cur, 0, 2);
+    h1[1] = rdH(cur, 1, 1);
+    o1[0] = rdO(cur, 1, 0);
+    mm(1, x1, h0, o0);
+    x0 = rdA(cur, 1, 0);
+    o1[1] = rdO(cur, 1, 1);
+    x1 = rdA(cur, 1, 1);
+    mm(2, x2, h0, o0);
+    x2 = rdA(cur, 1, 2);
+    mm(0, x0, h1, o1);
+    EXH_STAGE_BARRIER(0);
+    issue(min(s + 2, nslab - 1), cur);
+    __builtin_amdgcn_sched_barrier(0);
+    h0[0] = rdH(nxt, 0, 0);
+    o0[0] = rdO(nxt, 0, 0);
+    h0[1] = rdH(nxt, 0, 1);
+    mm(1, x1, h1, o1);
+    o0[1] = rdO(nxt, 0, 1);
+    x0 = rdA(nxt, 0, 0);
+    mm(2, x2, h1, o1);
+  };
+  issue(0, sm0);
+  issue(1, sm1);
+  EXH_STAGE_BARRIER(5);  // stage 0 has landed, stage 1 (5 loads) may be in flight
+  h0[0] = rdH(sm0, 0, 0);
+  o0[0] = rdO(sm0, 0, 0);
+  h0[1] = rdH(sm0, 0, 1);
+  o0[1] = rdO(sm0, 0, 1);
+  x0 = rdA(sm0, 0, 0);
   for (int s = 0; s < nslab; s += 2) {
-    if (s + 1 < nslab) issue(s + 1, sA1, sH1, sO1);
-    compute(sA0, sH0, sO0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (s + 1 < nslab) {
-      if (s + 2 < nslab) issue(s + 2, sA0, sH0, sO0);
-      compute(sA1, sH1, sO1);
-      __builtin_amdgcn_s_waitcnt(0x0F70);
-      __syncthreads();
-    }
+    stage(s, sm0, sm1);
+    stage(s + 1, sm1, sm0);
   }
+#undef EXH_STAGE_BARRIER
+  // the LDS must outlive the last refills
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 
   // planes: (H+, H-, O+, O-) x modulus, or (O+, O-) x modulus
   const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
@@ -734,7 +774,7 @@ OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool thir
   constexpr int GA = 384;
   static_assert(GA % OZ_R == 0 && GA % OZ_T == 0, "row padding");
   L.Gpad = (ngkmax + GA - 1) / GA * GA;
-  L.Kpad = (Ktot + OZ_KS - 1) / OZ_KS * OZ_KS;
+  L.Kpad = (Ktot + 2 * OZ_KS - 1) / (2 * OZ_KS) * (2 * OZ_KS);  // an even number of stages
   L.qstride = (size_t)L.Kpad * L.Gpad;
   const long long nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
   L.q_bytes = (size_t)P.nmod * 2 * L.qstride;

@@ -91,7 +91,7 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     fp64_modular = 16 * K * ldb > 64 << 20       # FP64 on the 15-moduli products
     if nmod_max or fp64_modular:
         gpad = (sys_.ngkmax + 383) // 384 * 384     # rows padded to the GEMM's panel
-        kpad = (K + 63) // 64 * 64
+        kpad = (K + 127) // 128 * 128
         nt = (sys_.ngkmax + 127) // 128
         # SPLIT(12) runs 13 moduli
         moduli = max(nmod_max + 1 if nmod_max else 0, 15 if fp64_modular else 0)
