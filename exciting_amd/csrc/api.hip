@@ -893,7 +893,7 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
   }
   if (e == hipSuccess)
     e = run(EXH_K_LOBORDER, [&] {
-      return launch_lo_border(s, c, ngp, A, (double2 *)hw, (double2 *)o, rank, flags);
+      return launch_lo_border(s, c, ngp, A, w.at, (double2 *)hw, (double2 *)o, rank, flags);
     });
   if (e == hipSuccess)
     e = run(EXH_K_LOLO, [&] { return launch_lolo(s, c, ngp, (double2 *)hw, (double2 *)o, rank, flags); });

@@ -62,11 +62,10 @@ struct OzScratch {
 // APW-lo border tables (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133)
 // of one structure, device pointers.
 struct LoTables {
-  const long long *colA;
   const int *Koff, *Ms, *atom_species, *losize, *lobase;
+  const LoRow *lorow;
   const double2 *loa;
   int maxnlo, maxaa;
-  const int *nlorb, *lorbl;
   int nlomax;
   const int *apword;
   int lmaxapw, pmax, lmmax, ngkmax;
@@ -302,7 +301,7 @@ hipError_t launch_ho(hipStream_t s, const exh_context *c, int ngp,
                      const double *vgpc, double2 *h, double2 *o, int ldh,
                      int flags);
 hipError_t launch_lo_border(hipStream_t s, const exh_context *c, int ngp,
-                            const double2 *apwalm, double2 *h, double2 *o,
+                            const double2 *apwalm, const double2 *at, double2 *h, double2 *o,
                             int ldh, int flags);
 hipError_t launch_mirror(hipStream_t s, int n, double2 *m, int ld);
 hipError_t launch_lolo(hipStream_t s, const exh_context *c, int ngp,

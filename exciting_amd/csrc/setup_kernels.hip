@@ -572,118 +572,159 @@ __global__ __launch_bounds__(64 * (TMI / 32) * (TMJ / 32)) void ho_grouped_kerne
 }
 
 // ---------------------------------------------------------------------------
-// APW-lo border (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133).
-// One thread per (G, atom):  H(lo rows, G) = loa . A   (+ mirror),
-//                            O(G, lo cols) = sum_io conj(A_io,lm s_io) (+ mirror)
-// with s = oalo + h1loa.
+// APW-lo border (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133):
+//   H(lo rows, G) = loa . A   (+ mirror),
+//   O(G, lo cols) = sum_io conj(A_io,lm s_io) (+ mirror),  s = oalo + h1loa.
+// One workgroup per (16 G+k, atom) and up to 16 NB local orbitals: the
+// product over f runs on FP64 MFMA (rows G, columns lo), its f range split
+// over the four waves and the four partial sums added in wave order through
+// LDS, from where both triangles are written in contiguous runs (lo rows:
+// 16 los bytes, columns: 256 bytes).  Bound by reading A once; the split over
+// f and the short tiles keep the chain short where a basis has few G+k (one
+// thread per (G+k, atom) looping over f took 105 us at 2 atoms, 349 us at 8,
+// 1.21 ms at 64; now 13 us, 21 us, 0.66 ms = 4.4 TB/s of A, H and O).  Tiles
+// of 64 G+k: 17 us, 29 us, 0.645 ms.
 // ---------------------------------------------------------------------------
-template <int MAXLO, typename PA, typename PH>
-__device__ __forceinline__ void lo_border_body(int g, int ias, int ngp, PA __restrict__ apwalm,
+constexpr int LOB_TH = 256;
+
+template <int NB, typename PA, typename PH>
+__device__ __forceinline__ void lo_border_body(int tile, int ias, int ngp, PA __restrict__ X,
+                                               long long ldx, PA __restrict__ apwalm,
                                                const LoTables &t, PH __restrict__ H,
                                                PH __restrict__ O, long long ldh,
                                                int accumulate) {
-  // every table index below is uniform across the wave: scalar loads
-  const EXH_C long long *__restrict__ colA = cptr(t.colA);
-  const EXH_C int *__restrict__ nlorb = cptr(t.nlorb);
-  const EXH_C int *__restrict__ lorbl = cptr(t.lorbl);
-  const EXH_C int *__restrict__ apword = cptr(t.apword);
-  const EXH_C double *__restrict__ salo = cptr(t.salo);
-  const int maxnlo = t.maxnlo, nlomax = t.nlomax, lmaxapw = t.lmaxapw, pmax = t.pmax,
-            lmmax = t.lmmax, ngkmax = t.ngkmax;
-  const EXH_C int *__restrict__ Koff = cptr(t.Koff);
-  const EXH_C int *__restrict__ Ms = cptr(t.Ms);
-  const EXH_C int *__restrict__ lobase = cptr(t.lobase);
-  const EXH_C double2 *__restrict__ loa = cptr(t.loa);
-  const int maxaa = t.maxaa;
+  constexpr int NG = 16, NL = 16 * NB;
+  __shared__ double2 sH[NL][NG + 1], sO[NL][NG + 1];
   const int is = cptr(t.atom_species)[ias];
   const int los = cptr(t.losize)[is];
-  if (los == 0 || g >= ngp) return;
-  const int r0 = ngp + lobase[ias];
-  const EXH_C long long *col = colA + Koff[ias];
-  const int M = Ms[ias];
-  const EXH_C double2 *L = loa + (size_t)ias * maxnlo * maxaa;
+  const int g0 = tile * NG;
+  if (los == 0 || g0 >= ngp) return;  // uniform per workgroup
+  const int lob = cptr(t.lobase)[ias], r0 = ngp + lob;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ng = min(NG, ngp - g0);
+
+  // O: one element per thread and pass, along G
+  for (int i = tid; i < NG * los; i += LOB_TH) {
+    const int r = i / NG, g = i - r * NG;
+    if (g >= ng) continue;
+    const LoRow q = t.lorow[lob + r];
+    const int lm = q.l * q.l + q.mi, p = t.apword[q.l + (t.lmaxapw + 1) * is];
+    const size_t e = (size_t)(g0 + g) + (size_t)(r0 + r) * ldh;
+    double2 v = accumulate ? ld(O + e) : z2(0, 0);
+    for (int io = 0; io < p; io++) {
+      const double2 a = ld(apwalm + (g0 + g) +
+                           (size_t)t.ngkmax * (io + (size_t)t.pmax * (lm + (size_t)t.lmmax * ias)));
+      const double sv = t.salo[io + t.pmax * (q.ilo + (size_t)t.nlomax * ias)];
+      v.x += a.x * sv;
+      v.y += -(a.y * sv);
+    }
+    st(O + e, v);
+    sO[r][g] = v;
+  }
 
   if (H) {  // null for overlapsetup alone
-  double2 acc[MAXLO];
+    const int M = cptr(t.Ms)[ias], koff = cptr(t.Koff)[ias];
+    const double2 *L = t.loa + (size_t)ias * t.maxnlo * t.maxaa;
+    const int steps = (M + 3) / 4, per = (steps + 3) / 4;
+    const int k0 = 4 * per * w, k1 = min(M, 4 * per * (w + 1));
+    dx4 re[NB], im[NB];
 #pragma unroll
-  for (int r = 0; r < MAXLO; r++) acc[r] = z2(0, 0);
-  for (int f = 0; f < M; f++) {
-    const double2 a = ld(apwalm + col[f] + g);
-    const EXH_C double2 *Lf = L + (size_t)maxnlo * f;
+    for (int b = 0; b < NB; b++) re[b] = im[b] = dx4{0, 0, 0, 0};
+    // rows past ngp and columns past los feed outputs that are not stored;
+    // the f tail is zeroed in the lo operand
+    const PA xp = X + (size_t)koff * ldx + min(g0 + lr, ngp - 1);
+    const double2 *lp[NB];
 #pragma unroll
-    for (int r = 0; r < MAXLO; r++)
-      if (r < los) {
-        const double2 lv = ld(Lf + r);
-        acc[r].x += a.x * lv.x - a.y * lv.y;
-        acc[r].y += a.x * lv.y + a.y * lv.x;
+    for (int b = 0; b < NB; b++) lp[b] = L + min(16 * b + lr, los - 1);
+#pragma unroll 4
+    for (int k = k0; k < k1; k += 4) {
+      const int kc = min(k + lk, k1 - 1);
+      const double f = k + lk < k1 ? 1.0 : 0.0;
+      const double2 x = ld(xp + (size_t)kc * ldx);
+      double2 y[NB];
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        y[b] = lp[b][(size_t)t.maxnlo * kc];
+        y[b].x *= f;
+        y[b].y *= f;
       }
-  }
 #pragma unroll
-  for (int r = 0; r < MAXLO; r++)
-    if (r < los) {
-      const size_t e = (size_t)(r0 + r) + (size_t)g * ldh;
-      double2 v = acc[r];
+      for (int b = 0; b < NB; b++) {
+        re[b] = mfma(x.x, y[b].x, re[b]);
+        im[b] = mfma(x.x, y[b].y, im[b]);
+        re[b] = mfma(-x.y, y[b].y, re[b]);
+        im[b] = mfma(x.y, y[b].x, im[b]);
+      }
+    }
+#pragma unroll 1
+    for (int v = 0; v < 4; v++) {
+      if (v == w) {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            double2 &d = sH[16 * b + lr][lk + 4 * r];
+            const double2 o = v ? d : z2(0, 0);
+            d = z2(o.x + re[b][r], o.y + im[b][r]);
+          }
+      }
+      __syncthreads();
+    }
+    for (int i = tid; i < ng * los; i += LOB_TH) {
+      const int g = i / los, r = i - g * los;
+      const size_t e = (size_t)(r0 + r) + (size_t)(g0 + g) * ldh;
+      double2 v = sH[r][g];
       if (accumulate) {
-        double2 h0 = ld(H + e);
+        const double2 h0 = ld(H + e);
         v.x += h0.x;
         v.y += h0.y;
+        sH[r][g] = v;
       }
       st(H + e, v);
-      st(H + (size_t)g + (size_t)(r0 + r) * ldh, z2(v.x, -v.y));
     }
   }
-
-  int c = r0;
-  for (int ilo = 0; ilo < nlorb[is]; ilo++) {
-    const int l = lorbl[ilo + nlomax * is];
-    const int p = apword[l + (lmaxapw + 1) * is];
-    for (int mi = 0; mi <= 2 * l; mi++, c++) {
-      const int lm = l * l + mi;
-      const size_t e = (size_t)g + (size_t)c * ldh;
-      double2 v = accumulate ? ld(O + e) : z2(0, 0);
-      for (int io = 0; io < p; io++) {
-        const double2 a =
-            ld(apwalm + g + (size_t)ngkmax * (io + (size_t)pmax * (lm + (size_t)lmmax * ias)));
-        const double s = salo[io + pmax * (ilo + (size_t)nlomax * ias)];
-        v.x += a.x * s;
-        v.y += -(a.y * s);
-      }
-      st(O + e, v);
-      st(O + (size_t)c + (size_t)g * ldh, z2(v.x, -v.y));
-    }
+  __syncthreads();
+  for (int i = tid; i < ng * los; i += LOB_TH) {
+    const int g = i / los, r = i - g * los;
+    const double2 v = sO[r][g];
+    st(O + (size_t)(r0 + r) + (size_t)(g0 + g) * ldh, z2(v.x, -v.y));
   }
+  if (H)
+    for (int i = tid; i < NG * los; i += LOB_TH) {
+      const int r = i / NG, g = i - r * NG;
+      if (g >= ng) continue;
+      const double2 v = sH[r][g];
+      st(H + (size_t)(g0 + g) + (size_t)(r0 + r) * ldh, z2(v.x, -v.y));
+    }
 }
 
-template <int MAXLO>
-__global__ __launch_bounds__(64) void lo_border_kernel(int ngp, const double2 *__restrict__ apwalm,
-                                                       LoTables t, double2 *__restrict__ H,
-                                                       double2 *__restrict__ O, long long ldh,
-                                                       int accumulate) {
-  lo_border_body<MAXLO>(blockIdx.x * 64 + threadIdx.x, blockIdx.y, ngp, apwalm, t, H, O, ldh,
-                        accumulate);
+template <int NB>
+__global__ __launch_bounds__(LOB_TH) void lo_border_kernel(
+    int ngp, const double2 *__restrict__ X, long long ldx, const double2 *__restrict__ apwalm,
+    LoTables t, double2 *__restrict__ H, double2 *__restrict__ O, long long ldh, int accumulate) {
+  lo_border_body<NB>(blockIdx.x, blockIdx.y, ngp, X, ldx, apwalm, t, H, O, ldh, accumulate);
 }
 
 // Grouped: blockIdx.z selects the k-point, blockIdx.y the atom.
-template <int MAXLO>
-__global__ __launch_bounds__(64) void lo_border_grouped_kernel(const KDesc *__restrict__ kd,
-                                                               int accumulate) {
+template <int NB>
+__global__ __launch_bounds__(LOB_TH) void lo_border_grouped_kernel(const KDesc *__restrict__ kd,
+                                                                   int accumulate) {
   const KDesc &d = kd[blockIdx.z];
   const EXH_C SDesc &S = *cptr(d.sd);
   if ((int)blockIdx.y >= S.natmtot || S.nlotot == 0) return;
   // field by field: scalar loads from the descriptor
   const EXH_C LoTables &L = S.lo;
   LoTables t;
-  t.colA = L.colA;
   t.Koff = L.Koff;
   t.Ms = L.Ms;
   t.atom_species = L.atom_species;
   t.losize = L.losize;
   t.lobase = L.lobase;
+  t.lorow = L.lorow;
   t.loa = L.loa;
   t.maxnlo = L.maxnlo;
   t.maxaa = L.maxaa;
-  t.nlorb = L.nlorb;
-  t.lorbl = L.lorbl;
   t.nlomax = L.nlomax;
   t.apword = L.apword;
   t.lmaxapw = L.lmaxapw;
@@ -691,9 +732,9 @@ __global__ __launch_bounds__(64) void lo_border_grouped_kernel(const KDesc *__re
   t.lmmax = L.lmmax;
   t.ngkmax = L.ngkmax;
   t.salo = L.salo;
-  lo_border_body<MAXLO>(blockIdx.x * 64 + threadIdx.x, blockIdx.y, d.ngp,
-                        gptr((const double2 *)d.apwalm), t, gptr(d.h), gptr(d.o), d.ldh,
-                        accumulate);
+  lo_border_body<NB>(blockIdx.x, blockIdx.y, d.ngp, gptr(d.x), S.ldx,
+                         gptr((const double2 *)d.apwalm), t, gptr(d.h), gptr(d.o), d.ldh,
+                         accumulate);
 }
 
 // ---------------------------------------------------------------------------
@@ -880,14 +921,12 @@ static LoTables lo_tables(const exh_context *c) {
   const int *ki = (const int *)c->katom.p;
   const int *lo = (const int *)c->lobase_d.p;  // [lobase(natmtot), losize(nspecies), nlorb, lorbl]
   LoTables t;
-  t.colA = (const long long *)c->colA.p;
   t.Koff = ki;
   t.Ms = ki + c->natmtot;
   t.atom_species = (const int *)c->atom_species_d.p;
   t.lobase = lo;
   t.losize = lo + c->natmtot;
-  t.nlorb = t.losize + c->nspecies;
-  t.lorbl = t.nlorb + c->nspecies;
+  t.lorow = (const LoRow *)c->lorow.p;
   t.loa = (const double2 *)c->loa.p;
   t.maxnlo = c->maxnlo;
   t.maxaa = c->maxaa;
@@ -902,17 +941,19 @@ static LoTables lo_tables(const exh_context *c) {
 }
 
 hipError_t launch_lo_border(hipStream_t s, const exh_context *c, int ngp,
-                            const double2 *apwalm, double2 *h, double2 *o,
+                            const double2 *apwalm, const double2 *at, double2 *h, double2 *o,
                             int ldh, int flags) {
   if (ngp <= 0 || c->nlotot == 0) return hipSuccess;
-  dim3 grid(cdiv(ngp, 64), c->natmtot);
+  long long ldx;
+  const double2 *X = k_major_view(c, apwalm, at, &ldx);
   const LoTables t = lo_tables(c);
-#define EXH_LOB(N)                                                                     \
-  hipLaunchKernelGGL(lo_border_kernel<N>, grid, dim3(64), 0, s, ngp, apwalm, t, h, o,  \
-                     (long long)ldh, flags & EXH_ACCUMULATE)
-  if (c->maxnlo <= 16) EXH_LOB(16);
-  else if (c->maxnlo <= 32) EXH_LOB(32);
-  else EXH_LOB(64);
+  const dim3 grid(cdiv(ngp, 16), c->natmtot);
+#define EXH_LOB(N)                                                                           \
+  hipLaunchKernelGGL(lo_border_kernel<N>, grid, dim3(LOB_TH), 0, s, ngp, X, ldx, apwalm, t, h, \
+                     o, (long long)ldh, flags & EXH_ACCUMULATE)
+  if (c->maxnlo <= 16) EXH_LOB(1);
+  else if (c->maxnlo <= 32) EXH_LOB(2);
+  else EXH_LOB(4);
 #undef EXH_LOB
   return hipGetLastError();
 }
@@ -1071,13 +1112,13 @@ int ho_grouped_occupancy(int shape) {
 hipError_t launch_lo_border_grouped(hipStream_t s, const GroupDims &g, const KDesc *kd,
                                     int accumulate) {
   if (g.nk <= 0 || g.ngpmax <= 0 || g.nlotot == 0 || g.natmax <= 0) return hipSuccess;
-  dim3 grid(cdiv(g.ngpmax, 64), g.natmax, g.nk);
-  if (g.maxnlo <= 16)
-    hipLaunchKernelGGL(lo_border_grouped_kernel<16>, grid, dim3(64), 0, s, kd, accumulate);
-  else if (g.maxnlo <= 32)
-    hipLaunchKernelGGL(lo_border_grouped_kernel<32>, grid, dim3(64), 0, s, kd, accumulate);
-  else
-    hipLaunchKernelGGL(lo_border_grouped_kernel<64>, grid, dim3(64), 0, s, kd, accumulate);
+  const dim3 grid(cdiv(g.ngpmax, 16), g.natmax, g.nk);
+#define EXH_LOB(N) \
+  hipLaunchKernelGGL(lo_border_grouped_kernel<N>, grid, dim3(LOB_TH), 0, s, kd, accumulate)
+  if (g.maxnlo <= 16) EXH_LOB(1);
+  else if (g.maxnlo <= 32) EXH_LOB(2);
+  else EXH_LOB(4);
+#undef EXH_LOB
   return hipGetLastError();
 }
 
