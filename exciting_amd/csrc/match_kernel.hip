@@ -183,19 +183,22 @@ __device__ __forceinline__ void d_sbesseldm(int m, double x,
 
 // ---------------------------------------------------------------------------
 // One workgroup: MG = 256 consecutive G+k vectors (one per lane) x MA
-// consecutive atoms, after match_prep has tabulated, per G+k,
+// consecutive atoms and one l, after match_prep has tabulated, per G+k,
 // conj(Y_lm) * 4 pi i^l / sqrt(Omega) and, per (G+k, species),
-// |G+k|^io j_l^(io)(|G+k| R).  For each l the workgroup solves the boundary
-// system D v = (j_l^(io)) per (G+k, atom) with the LU factors of (l, atom)
-// (zgetrs order on the real radial vector; the complex factor
-// S_a(G+k) conj(Y_lm) fpso i^l multiplies the solution), then for each m
-// reads the harmonics once and writes apwalm(G, io, lm, a) = v_io S_a yt_lm
-// for every atom of the tile.  All four waves walk the same column sequence,
+// |G+k|^io j_l^(io)(|G+k| R).  The workgroup solves the boundary system
+// D v = (j_l^(io)) per (G+k, atom) with the LU factors of (l, atom) (zgetrs
+// order on the real radial vector; the complex factor S_a(G+k) conj(Y_lm)
+// fpso i^l multiplies the solution), then for each m reads the harmonics once
+// and writes apwalm(G, io, lm, a) = v_io S_a yt_lm for every atom of the
+// tile.  All four waves walk the same column sequence,
 // so every column receives 4 KB contiguous per workgroup step: the widest
 // row segments apwalm's leading dimension (the caller's ngkmax, not aligned
 // to cache lines) allows.  The tables (a few MB per k-point) stay in cache;
 // the loop holds few registers and no LDS, so many waves keep stores in
-// flight.
+// flight: 2.33 GB in 0.474 ms (4.9 TB/s) at 64 atoms.  One l per workgroup:
+// with every l in one workgroup a cell of 8 atoms filled 10 CUs (tables and
+// tiles together 90 -> 28 us at 2 atoms, 193 -> 43 us at 8, 0.58 -> 0.50 ms at
+// 64).
 // ---------------------------------------------------------------------------
 constexpr int MG = 256;   // G+k vectors per workgroup
 constexpr int MA = 4;     // atoms per workgroup
@@ -265,54 +268,49 @@ __device__ __forceinline__ void ylm_row(double sn, double cs, double phi, double
   }
 }
 
+// the harmonics of the one l that is asked for
 template <int LM, int L = 0, typename PO>
-__device__ __forceinline__ void ylm_all(double sn, double cs, double phi, double fpso, PO yt,
-                                        size_t stride) {
+__device__ __forceinline__ void ylm_of(int l, double sn, double cs, double phi, double fpso,
+                                       PO yt, size_t stride) {
   if constexpr (L <= LM) {
-    ylm_row<L>(sn, cs, phi, fpso, yt + (size_t)L * L * stride, stride);
-    ylm_all<LM, L + 1>(sn, cs, phi, fpso, yt, stride);
+    if (l == L) ylm_row<L>(sn, cs, phi, fpso, yt + (size_t)L * L * stride, stride);
+    else ylm_of<LM, L + 1>(l, sn, cs, phi, fpso, yt, stride);
   }
 }
 
-// |G+k|^io j_l^(io)(|G+k| R), io < omax (match.f90:114-131)
+// |G+k|^io j_l^(io)(|G+k| R) for one io (match.f90:114-131)
 template <int LM>
-__device__ __forceinline__ void radial_row(double q, double rmt, int omax, double (&djl)[PCAP][LM + 1]) {
+__device__ __forceinline__ void radial_row(double q, double rmt, int io, double (&djl)[LM + 1]) {
   const double x = q * rmt;
-  {
-    double jl[LM + 1];
-    d_sbessel<LM>(x, jl);
-#pragma unroll
-    for (int l = 0; l <= LM; l++) djl[0][l] = jl[l];
+  if (io == 0) {
+    d_sbessel<LM>(x, djl);
+    return;
   }
+  double jp1[LM + 2];
 #pragma unroll
-  for (int io = 1; io < PCAP; io++)
+  for (int l = 0; l <= LM + 1; l++) jp1[l] = 0.0;
+  if (x > 1.0) d_sbessel<LM + 1>(x, jp1);
+  double t1 = q;
 #pragma unroll
-    for (int l = 0; l <= LM; l++) djl[io][l] = 0.0;
-  if (omax > 1) {
-    double jp1[LM + 2];
+  for (int j = 1; j < PCAP; j++)
+    if (j == io) {
+      d_sbesseldm<LM>(j, x, jp1, djl);
 #pragma unroll
-    for (int l = 0; l <= LM + 1; l++) jp1[l] = 0.0;
-    if (x > 1.0) d_sbessel<LM + 1>(x, jp1);
-    double t1 = 1.0;
-#pragma unroll
-    for (int io = 1; io < PCAP; io++) {
-      if (io < omax) {
-        double d[LM + 1];
-        d_sbesseldm<LM>(io, x, jp1, d);
-        t1 = t1 * q;
-#pragma unroll
-        for (int l = 0; l <= LM; l++) djl[io][l] = t1 * d[l];
-      }
+      for (int l = 0; l <= LM; l++) djl[l] = t1 * djl[l];
+    } else {
+      t1 = t1 * q;
     }
-  }
 }
 
 // Tables of one k-point, in its match scratch (ld = ngkmax):
 //   rad[((is * PCAP + io) * (LM + 1) + l) * ld + g] = |G+k|^io j_l^(io)(|G+k| R_is),
-//     zero for io >= omax(is);
+//     io < omax(is);
 //   yt[lm * ld + g] = conj(Y_lm(G+k)) * 4 pi i^l / sqrt(Omega).
-// One thread per (G+k, role): role < nspecies the radial factors of that
-// species, role == nspecies the spherical harmonics.
+// One thread per (G+k, role): roles 0..LM the spherical harmonics of that l,
+// then the radial factors of one (species, io).  The recursions are serial
+// chains that leave most of the chip idle at a few hundred G+k, so each chain
+// (one l, one order) gets its own thread (13 us at 194 G+k, 17 us at 1166,
+// 29 us at 9340).
 __host__ __device__ inline size_t match_rad_doubles(int nspecies, int lmaxapw, int ld) {
   // rounded so that the harmonics that follow are 256-byte aligned
   return ((size_t)nspecies * PCAP * (lmaxapw + 1) * ld + 31) / 32 * 32;
@@ -325,19 +323,22 @@ __device__ __forceinline__ void prep_body(int g, int role, int ngp, int nspecies
                                           const int *__restrict__ omaxs, double fpso,
                                           PR __restrict__ rad, PY __restrict__ yt) {
   if (g >= ngp) return;
-  if (role < nspecies) {
-    double djl[PCAP][LM + 1];
-    radial_row<LM>(gpc[g], rmt[role], omaxs[role], djl);
-#pragma unroll
-    for (int io = 0; io < PCAP; io++)
-#pragma unroll
-      for (int l = 0; l <= LM; l++)
-        rad[((size_t)(role * PCAP + io) * (LM + 1) + l) * ld + g] = djl[io][l];
-  } else {
+  if (role <= LM) {
     const double th = tpgpc[2 * g], phi = tpgpc[2 * g + 1];
-    ylm_all<LM>(sin(th), cos(th), phi, fpso, yt + g, (size_t)ld);
+    ylm_of<LM>(role, sin(th), cos(th), phi, fpso, yt + g, (size_t)ld);
+    return;
   }
+  const int is = (role - LM - 1) / PCAP, io = (role - LM - 1) % PCAP;
+  if (is >= nspecies || io >= omaxs[is]) return;
+  double djl[LM + 1];
+  radial_row<LM>(gpc[g], rmt[is], io, djl);
+#pragma unroll
+  for (int l = 0; l <= LM; l++)
+    rad[((size_t)(is * PCAP + io) * (LM + 1) + l) * ld + g] = djl[l];
 }
+
+// Roles of the prep kernel, by how many species it has to cover.
+constexpr int prep_roles(int lmaxapw, int nspecies) { return lmaxapw + 1 + PCAP * nspecies; }
 
 template <int LM>
 __global__ __launch_bounds__(64) void match_prep_kernel(int ngp, int nspecies, int ld,
@@ -355,7 +356,7 @@ template <int LM>
 __global__ __launch_bounds__(64) void match_prep_grouped_kernel(const KDesc *__restrict__ kd) {
   const KDesc &d = kd[blockIdx.z];
   const SDesc &S = *d.sd;
-  if (S.lmaxapw != LM || (int)blockIdx.y > S.nspecies) return;
+  if (S.lmaxapw != LM) return;
   double *tab = d.mtab;
   prep_body<LM>(blockIdx.x * 64 + threadIdx.x, blockIdx.y, d.ngp, S.nspecies, S.ngkmax,
                 gptr(d.gpc), gptr(d.tpgpc), S.rmt, S.omax, S.fpso, gptr(tab),
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(64) void match_prep_grouped_kernel(const KDesc *__r
 
 template <int LM, typename PS, typename PA, typename PR, typename PY>
 __device__ __forceinline__ void match_tile(
-    int g0, int a0, int ngp, int natmtot, int ld, int pmax, PS __restrict__ sfacgp,
+    int g0, int a0, int l, int ngp, int natmtot, int ld, int pmax, PS __restrict__ sfacgp,
     PA __restrict__ apwalm, const int *__restrict__ atom_species, PR __restrict__ rad,
     PY __restrict__ yt, const int *__restrict__ apword, const double *__restrict__ lu,
     const int *__restrict__ piv) {
@@ -383,70 +384,67 @@ __device__ __forceinline__ void match_tile(
     is[u] = u < na ? ASt[a0 + u] : 0;
     S[u] = u < na ? exh::ld(sfacgp + g + (size_t)ld * (a0 + u)) : z2(0.0, 0.0);
   }
+  // boundary solutions of every atom of the tile for this l
+  double v[MA][PCAP];
+  int p[MA];
+#pragma unroll
+  for (int u = 0; u < MA; u++) {
+    p[u] = 0;
+    if (u >= na) continue;
+    const int pu = APt[l + (LM + 1) * is[u]];
+    p[u] = pu;
+    const EXH_C double *LU = LUt + (size_t)PCAP * PCAP * (l + (LM + 1) * (a0 + u));
+    const EXH_C int *PV = PVt + PCAP * (l + (LM + 1) * (a0 + u));
+    double x[PCAP];
+#pragma unroll
+    for (int io = 0; io < PCAP; io++)
+      x[io] = io < pu ? exh::ld(rad + ((size_t)(is[u] * PCAP + io) * (LM + 1) + l) * ld + g)
+                      : 0.0;
+    // zgetrs: row interchanges, unit-lower then upper solve
+#pragma unroll
+    for (int i = 0; i < PCAP; i++)
+      if (i < pu) {
+        const int ip = PV[i] - 1;
+        if (ip != i) {
+          double tt = x[i];
+#pragma unroll
+          for (int j = 0; j < PCAP; j++)
+            if (j == ip) {
+              x[i] = x[j];
+              x[j] = tt;
+            }
+        }
+      }
+#pragma unroll
+    for (int k = 0; k < PCAP; k++)
+#pragma unroll
+      for (int i = k + 1; i < PCAP; i++)
+        if (i < pu) x[i] = fma(-x[k], LU[i + PCAP * k], x[i]);
+#pragma unroll
+    for (int k = PCAP - 1; k >= 0; k--)
+      if (k < pu) {
+        x[k] = x[k] / LU[k + PCAP * k];
+#pragma unroll
+        for (int i = 0; i < k; i++) x[i] = fma(-x[k], LU[i + PCAP * k], x[i]);
+      }
+#pragma unroll
+    for (int io = 0; io < PCAP; io++) v[u][io] = x[io];
+  }
 #pragma unroll 1
-  for (int l = 0; l <= LM; l++) {
-    // boundary solutions of every atom of the tile for this l
-    double v[MA][PCAP];
-    int p[MA];
+  for (int lm = l * l; lm < (l + 1) * (l + 1); lm++) {
+    const double2 y = exh::ld(yt + (size_t)lm * ld + g);
 #pragma unroll
     for (int u = 0; u < MA; u++) {
-      p[u] = 0;
-      if (u >= na) continue;
-      const int pu = APt[l + (LM + 1) * is[u]];
-      p[u] = pu;
-      const EXH_C double *LU = LUt + (size_t)PCAP * PCAP * (l + (LM + 1) * (a0 + u));
-      const EXH_C int *PV = PVt + PCAP * (l + (LM + 1) * (a0 + u));
-      double x[PCAP];
+      if (u >= na) break;
+      // explicit fma: the same rounding in every instantiation of the tile
+      // (the compiler would otherwise fuse either product)
+      const double wr = fma(S[u].x, y.x, -(S[u].y * y.y));
+      const double wi = fma(S[u].x, y.y, S[u].y * y.x);
+      const PA out = apwalm + g + (size_t)ld * pmax * ((LM + 1) * (LM + 1)) * (a0 + u);
 #pragma unroll
       for (int io = 0; io < PCAP; io++)
-        x[io] = io < pu ? exh::ld(rad + ((size_t)(is[u] * PCAP + io) * (LM + 1) + l) * ld + g)
-                        : 0.0;
-      // zgetrs: row interchanges, unit-lower then upper solve
-#pragma unroll
-      for (int i = 0; i < PCAP; i++)
-        if (i < pu) {
-          const int ip = PV[i] - 1;
-          if (ip != i) {
-            double tt = x[i];
-#pragma unroll
-            for (int j = 0; j < PCAP; j++)
-              if (j == ip) {
-                x[i] = x[j];
-                x[j] = tt;
-              }
-          }
-        }
-#pragma unroll
-      for (int k = 0; k < PCAP; k++)
-#pragma unroll
-        for (int i = k + 1; i < PCAP; i++)
-          if (i < pu) x[i] = fma(-x[k], LU[i + PCAP * k], x[i]);
-#pragma unroll
-      for (int k = PCAP - 1; k >= 0; k--)
-        if (k < pu) {
-          x[k] = x[k] / LU[k + PCAP * k];
-#pragma unroll
-          for (int i = 0; i < k; i++) x[i] = fma(-x[k], LU[i + PCAP * k], x[i]);
-        }
-#pragma unroll
-      for (int io = 0; io < PCAP; io++) v[u][io] = x[io];
-    }
-#pragma unroll 1
-    for (int lm = l * l; lm < (l + 1) * (l + 1); lm++) {
-      const double2 y = exh::ld(yt + (size_t)lm * ld + g);
-#pragma unroll
-      for (int u = 0; u < MA; u++) {
-        if (u >= na) break;
-        // explicit fma: the same rounding in every instantiation of the tile
-        // (the compiler would otherwise fuse either product)
-        const double wr = fma(S[u].x, y.x, -(S[u].y * y.y));
-        const double wi = fma(S[u].x, y.y, S[u].y * y.x);
-        const PA out = apwalm + g + (size_t)ld * pmax * ((LM + 1) * (LM + 1)) * (a0 + u);
-#pragma unroll
-        for (int io = 0; io < PCAP; io++)
-          if (io < p[u])
-            st_nt(out + (size_t)ld * (io + (size_t)pmax * lm), z2(v[u][io] * wr, v[u][io] * wi));
-      }
+        if (io < p[u])
+          st_nt(out + (size_t)ld * (io + (size_t)pmax * lm), z2(v[u][io] * wr, v[u][io] * wi));
     }
   }
 }
@@ -457,7 +455,7 @@ __global__ __launch_bounds__(MTH) void match_kernel(
     double2 *__restrict__ apwalm, const int *__restrict__ atom_species,
     const double *__restrict__ tab, const int *__restrict__ apword,
     const double *__restrict__ lu, const int *__restrict__ piv) {
-  match_tile<LM>(blockIdx.x * MG, blockIdx.y * MA, ngp, natmtot, ld, pmax, sfacgp, apwalm,
+  match_tile<LM>(blockIdx.x * MG, blockIdx.y / (LM + 1) * MA, LM - blockIdx.y % (LM + 1), ngp, natmtot, ld, pmax, sfacgp, apwalm,
                  atom_species, tab,
                  (const double2 *)(tab + match_rad_doubles(nspecies, LM, ld)), apword, lu, piv);
 }
@@ -471,7 +469,7 @@ __global__ __launch_bounds__(MTH) void match_grouped_kernel(const KDesc *__restr
   const EXH_C SDesc &S = *cptr(d.sd);
   if (S.lmaxapw != LM) return;
   const double *tab = d.mtab;
-  match_tile<LM>(blockIdx.x * MG, blockIdx.y * MA, d.ngp, S.natmtot, S.ngkmax, S.pmax,
+  match_tile<LM>(blockIdx.x * MG, blockIdx.y / (LM + 1) * MA, LM - blockIdx.y % (LM + 1), d.ngp, S.natmtot, S.ngkmax, S.pmax,
                  gptr(d.sfac), gptr(d.apwalm), S.atom_species, gptr(tab),
                  gptr((const double2 *)(tab + match_rad_doubles(S.nspecies, LM, S.ngkmax))),
                  S.apword, S.lu, S.piv);
@@ -495,8 +493,8 @@ hipError_t launch_match(hipStream_t s, const exh_context *c, int ngp,
                         const double2 *sfacgp, double2 *apwalm, double *tab) {
   if (ngp <= 0 || c->natmtot <= 0) return hipSuccess;
   const double fpso = 12.566370614359172954 / sqrt(c->omega);
-  dim3 gridp(cdiv(ngp, 64), c->nspecies + 1);
-  dim3 grid(cdiv(ngp, MG), cdiv(c->natmtot, MA));
+  const dim3 gridp(cdiv(ngp, 64), prep_roles(c->lmaxapw, c->nspecies));
+  const dim3 grid(cdiv(ngp, MG), cdiv(c->natmtot, MA) * (c->lmaxapw + 1));
   const int *as = (const int *)c->atom_species_d.p;
   const int *apw = (const int *)c->apword_d.p;
   const int *om = (const int *)c->omax_d.p;
@@ -523,11 +521,11 @@ hipError_t launch_match(hipStream_t s, const exh_context *c, int ngp,
 
 hipError_t launch_match_grouped(hipStream_t s, const GroupDims &g, const KDesc *kd) {
   if (g.nk <= 0 || g.ngpmax <= 0 || g.natmax <= 0) return hipSuccess;
-  dim3 gridp(cdiv(g.ngpmax, 64), g.nspmax + 1, g.nk);
-  dim3 grid(cdiv(g.ngpmax, MG), cdiv(g.natmax, MA), g.nk);
   if (g.lmax_mask >> (kMatchLmaxCap + 1)) return hipErrorInvalidValue;
 #define EXH_M(L)                                                                  \
   if (g.lmax_mask & (1u << L)) {                                                  \
+    const dim3 gridp(cdiv(g.ngpmax, 64), prep_roles(L, g.nspmax), g.nk);          \
+    const dim3 grid(cdiv(g.ngpmax, MG), cdiv(g.natmax, MA) * (L + 1), g.nk);   \
     hipLaunchKernelGGL(match_prep_grouped_kernel<L>, gridp, dim3(64), 0, s, kd);  \
     hipLaunchKernelGGL(match_grouped_kernel<L>, grid, dim3(MTH), 0, s, kd);       \
     hipError_t e = hipGetLastError();                                             \
