@@ -385,49 +385,63 @@ int wait_done(exh_context *c) {
   return e == hipSuccess ? 0 : hip_fail(c, e, "waiting for queued work");
 }
 
+// Moduli that exh_setup_device_noalloc can hold residues of at a time beside
+// the products of all of them; 0 when the products alone do not fit.
+int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L) {
+  const size_t fixed = align256(L.r_bytes) + align256(L.e_bytes * L.nops);
+  if (fixed >= kNoallocModularBytes) return 0;
+  return (int)std::min<size_t>(P.nmod, (kNoallocModularBytes - fixed) / (2 * L.qstride * L.nops));
+}
+
 // The modular contraction of a setup with these flags: EXH_SPLIT(n), or for
-// FP64 the 15-moduli plan when one K-major operand (16 Ktot ldb bytes) is
-// larger than the static array of exh_setup_device_noalloc, so that wherever
-// that entry point takes a basis it runs the kernels exh_setup_device runs.
-// At that line the modular path is already the faster one (whole match +
-// setup, FP64 MFMA kernels against modular): 79 MB operands, K = 2904,
-// G = 1780: 2.39 against 1.45 ms; 107 MB, K = 2646, G = 2657: 3.20 against
-// 1.43 ms, O alone 1.54 against 0.75 ms; 2.3 GB, K = 15488, G = 9340: 168
-// against 50.7 ms.
+// FP64 the 15-moduli plan.  The rule looks at the context only, so that single,
+// grouped, overlap-only and allocation-free setups of one basis agree: bases
+// of fewer than 2^15 (K, G+k) pairs stay on the FP64 MFMA tiles, where one
+// launch beats five, and so do the few bases that exh_setup_device_noalloc
+// accepts but whose products its static array cannot hold.  Contraction of
+// one k-point on FP64 MFMA against modular: K = 242, G = 146: 88 against 53 us;
+// 968, 587: 290 against 80; 1936, 1175: 557 against 235 (O alone 993 against
+// 149); 15488, 9340: 162 against 41 ms.  Below the line, 98, 143: 49 against
+// 48, and 47 against 66 for eight of them in one grouped launch.
 OzPlan oz_plan(const exh_context *c, int flags) {
   const int n = (flags >> 8) & 0xff;
   if (n) return oz_split(n);
-  const size_t op = (size_t)c->Ktot * ((c->ngkmax + 63) / 64 * 64) * sizeof(double2);
-  return op > kNoallocScratchBytes && c->Ktot <= kOzMaxK ? oz_fp64() : OzPlan();
+  const size_t pairs = (size_t)c->Ktot * ((c->ngkmax + 63) / 64 * 64);
+  if (pairs < (size_t(1) << 15) || c->Ktot > kOzMaxK) return OzPlan();
+  const OzPlan P = oz_fp64();
+  if (pairs * sizeof(double2) > kNoallocScratchBytes) return P;  // refused there
+  const OzLayout L = oz_layout(c->ngkmax, c->Ktot, P, false, c->have_h1aa);
+  return oz_noalloc_chunk(P, L) > 0 ? P : OzPlan();
 }
 
-bool oz_fits(const exh_context *c, const OzLayout &L) {
-  return c->ozq.bytes >= L.q_bytes * L.nops && c->ozr.bytes >= L.r_bytes &&
-         c->oze.bytes >= L.e_bytes * L.nops;
+bool oz_fits(const exh_context *c, const OzLayout &L, int slots) {
+  return c->ozq.bytes >= L.q_bytes * L.nops * slots && c->ozr.bytes >= L.r_bytes * slots &&
+         c->oze.bytes >= L.e_bytes * L.nops * slots;
 }
 
-// Plan, layout and scratch of the modular contraction; P.nmod = 0 when the
-// setup runs on the FP64 MFMA kernels instead, which is also where an FP64
-// setup goes when the device has no room for the residues or the stream is
-// being captured before the first call (nothing may be allocated then).
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, OzPlan &P, OzLayout &L) {
+// Plan, layout and scratch of the modular contraction for `slots` k-points;
+// P.nmod = 0 when the setup runs on the FP64 MFMA kernels instead, which is
+// also where an FP64 setup goes when the device has no room for the residues
+// or the stream is being captured before the first call (nothing may be
+// allocated then).
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, OzPlan &P,
+               OzLayout &L) {
   P = oz_plan(c, flags);
   if (P.nmod == 0) return 0;
   const bool split = (flags & 0xff00) != 0;
   L = oz_layout(c->ngkmax, c->Ktot, P, only_o, c->have_h1aa);
-  if (oz_fits(c, L)) return 0;
+  if (oz_fits(c, L, slots)) return 0;
   if (!split) {
     size_t avail = 0, total = 0;
-    const size_t need = L.q_bytes * L.nops + L.r_bytes + L.e_bytes * L.nops;
     if (capturing || hipMemGetInfo(&avail, &total) != hipSuccess ||
-        avail < need + (size_t(1) << 30)) {
+        avail < L.bytes() * slots + (size_t(1) << 30)) {
       P = OzPlan();
       return 0;
     }
   }
-  int rc = ensure(c, c->ozq, L.q_bytes * L.nops);
-  if (!rc) rc = ensure(c, c->ozr, L.r_bytes);
-  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops);
+  int rc = ensure(c, c->ozq, L.q_bytes * L.nops * slots);
+  if (!rc) rc = ensure(c, c->ozr, L.r_bytes * slots);
+  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops * slots);
   if (rc && !split) {  // another allocation took the room meanwhile
     (void)hipGetLastError();
     P = OzPlan();
@@ -443,7 +457,7 @@ int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, OzPlan &P
 // passes `scratch` itself to a kernel (on the host the name is only a
 // stand-in for the symbol): exh_create looks up each device's address once,
 // with that device current, and the entry point uses that address.
-static __device__ __align__(256) unsigned char scratch[exh::kNoallocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[exh::kNoallocScratchBytes + exh::kNoallocModularBytes];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -464,8 +478,6 @@ int scratch_address(int device, void **out) {
   *out = g_scratch_addr[device];
   return 0;
 }
-
-inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 }  // namespace
 
 using namespace exh;
@@ -824,6 +836,7 @@ struct SetupScratch {
   // modular contraction (oz_prepare); plan.nmod = 0: the FP64 MFMA kernels
   OzPlan plan;
   OzLayout layout;
+  OzScratch oz;
 };
 
 // The single-k setup.  o_only: overlapsetup.f90 alone -- O accumulated and
@@ -883,13 +896,17 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
     const int lo0 = c->intgv[0], lo1 = c->intgv[1], lo2 = c->intgv[2];
     IstBox box{w.ivgk, vgpc, (const IstEntry *)c->ist.p, lo0, lo1, lo2,
                c->intgv[3] - lo0 + 1, c->intgv[4] - lo1 + 1, c->intgv[5] - lo2 + 1};
-    const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
-    for (int st = 0; st < 3 && e == hipSuccess; st++)
-      e = run(kid[st], [&] {
-        return launch_ozaki(s, c, ngp, w.plan, w.layout, oz_scratch(c), X, ldx, w.bt,
-                            c->have_h1aa ? w.a2t : nullptr, ldb, box, (double2 *)hw,
-                            (double2 *)o, rank, flags & EXH_ACCUMULATE, 1 << st);
-      });
+    const OzK d = make_ozk(c, ngp, w.plan, w.layout, w.oz, X, ldx, w.bt,
+                           c->have_h1aa ? w.a2t : nullptr, ldb, box, (double2 *)hw, (double2 *)o,
+                           rank);
+    const int acc = flags & EXH_ACCUMULATE;
+    if (w.oz.chunk < nmod) {
+      e = launch_ozaki(s, d, w.oz.chunk, acc, 7);
+    } else {
+      const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
+      for (int st = 0; st < 3 && e == hipSuccess; st++)
+        e = run(kid[st], [&] { return launch_ozaki(s, d, nmod, acc, 1 << st); });
+    }
   }
   if (e == hipSuccess)
     e = run(EXH_K_LOBORDER, [&] {
@@ -917,8 +934,9 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   if (!rc && !c->contig) rc = ensure(c, c->at, op);
   if (!rc) rc = ensure(c, c->ivgk, (size_t)std::max(c->ngkmax, 1) * sizeof(int4));
   if (!rc)
-    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, w.plan, w.layout);
+    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, 1, w.plan, w.layout);
   if (rc) return rc;
+  if (w.plan.nmod) w.oz = oz_scratch(c, w.plan, w.layout, 0);
   w.bt = (double2 *)c->bt.p;
   w.a2t = (double2 *)c->a2t.p;
   w.at = (double2 *)c->at.p;
@@ -971,6 +989,16 @@ int exh_setup_device_noalloc(exh_context *c, void *stream, int ngp, int rank,
     off += op;
   }
   if (!c->contig) w.at = (double2 *)(base + off);
+  w.plan = oz_plan(c, flags);
+  if (w.plan.nmod) {
+    // [product residues | exponents and norms | residues of `chunk` moduli]
+    w.layout = oz_layout(c->ngkmax, c->Ktot, w.plan, false, c->have_h1aa);
+    w.oz.chunk = oz_noalloc_chunk(w.plan, w.layout);
+    unsigned char *mod = base + kNoallocScratchBytes;
+    w.oz.r = (int8_t *)mod;
+    w.oz.e = mod + align256(w.layout.r_bytes);
+    w.oz.q = (int8_t *)w.oz.e + align256(w.layout.e_bytes * w.layout.nops);
+  }
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   return setup_launch(c, s, ngp, rank, apwalm, igpig, vgpc, h, o, flags, false, w, false);
 }

@@ -141,4 +141,22 @@ __device__ __forceinline__ void store_upper_o(PH O, long long ldh, int i, int j,
   if (i != j) st(O + (size_t)j + (size_t)i * ldh, z2(orr, -oi));
 }
 
+// One k-point of the modular contraction: operands (X; B unless O alone;
+// (1+h1)A for iora*), scratch and outputs, by value for a single launch or in
+// device memory for a grouped one.
+struct OzK {
+  int ngp, Ktot, nt, nslab, Gpad, nmod, bits;
+  int nops, iB, iY;       // operands; which one is B, and the overlap's columns
+  int ldp, nch;           // partial norms: leading dimension, chunks
+  size_t qstride, q_bytes;  // one residue array; one operand's arrays
+  const double2 *x[3];
+  long long ld[3];
+  int *e[3];        // column exponents
+  double *part[3];  // partial norms, then their exponents
+  int8_t *q, *r;    // residues of the operands and of the products
+  IstBox box;
+  double2 *h, *o;   // h null: O alone
+  long long ldh;
+};
+
 }  // namespace exh

@@ -33,8 +33,11 @@ struct LoRow {
   int ias, ilo, mi, l;
 };
 
-// Static device scratch of exh_setup_device_noalloc (api.hip).
+// Static device scratch of exh_setup_device_noalloc (api.hip): the K-major
+// operands and the G+k map, then the modular contraction's part.
 constexpr size_t kNoallocScratchBytes = size_t(64) << 20;
+constexpr size_t kNoallocModularBytes = size_t(128) << 20;
+inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Modular (Ozaki scheme II) contraction: split precision, and FP64 for large
 // bases.
@@ -53,10 +56,13 @@ struct OzLayout {
   size_t q_bytes = 0;      // residues of one operand
   size_t r_bytes = 0;      // residues of the products
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
+  long long panels = 0;    // workgroups of the products at ngkmax
+  size_t bytes() const { return q_bytes * nops + r_bytes + e_bytes * nops; }
 };
 struct OzScratch {
   int8_t *q = nullptr, *r = nullptr;
   void *e = nullptr;
+  int chunk = 0;  // moduli whose residues q holds
 };
 
 // APW-lo border tables (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133)
@@ -313,17 +319,29 @@ OzPlan oz_split(int n);
 OzPlan oz_fp64();
 OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool third);
 OzPlan oz_plan(const exh_context *c, int flags);
-bool oz_fits(const exh_context *c, const OzLayout &L);
-inline OzScratch oz_scratch(const exh_context *c) {
-  return OzScratch{(int8_t *)c->ozq.p, (int8_t *)c->ozr.p, c->oze.p};
+int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L);
+bool oz_fits(const exh_context *c, const OzLayout &L, int slots);
+// Slot `slot` of the context's modular scratch.
+inline OzScratch oz_scratch(const exh_context *c, const OzPlan &P, const OzLayout &L, int slot) {
+  OzScratch w;
+  w.q = (int8_t *)c->ozq.p + (size_t)slot * L.q_bytes * L.nops;
+  w.r = (int8_t *)c->ozr.p + (size_t)slot * L.r_bytes;
+  w.e = (char *)c->oze.p + (size_t)slot * L.e_bytes * L.nops;
+  w.chunk = P.nmod;
+  return w;
 }
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, OzPlan &P, OzLayout &L);
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, OzPlan &P,
+               OzLayout &L);
+struct OzK;
 // h = nullptr: O alone (B is not read).  Y = nullptr: the overlap's column
-// operand is X.  stage_mask: 1 residues, 2 products, 4 reconstruction.
-hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const OzPlan &P,
-                        const OzLayout &L, const OzScratch &w, const double2 *X, long long ldx,
-                        const double2 *B, const double2 *Y, long long ldb, const IstBox &box,
-                        double2 *h, double2 *o, int ldh, int accumulate, int stage_mask);
+// operand is X.
+OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
+             const OzScratch &w, const double2 *X, long long ldx, const double2 *B,
+             const double2 *Y, long long ldb, const IstBox &box, double2 *h, double2 *o, int ldh);
+// stage_mask: 1 norms and residues, 2 products, 4 reconstruction.
+hipError_t launch_ozaki(hipStream_t s, const OzK &d, int chunk, int accumulate, int stage_mask);
+hipError_t launch_ozaki_grouped(hipStream_t s, const OzK *d, const OzK *kd, int n, int accumulate,
+                                int stage_mask);
 // tab: match_table_bytes(c) of scratch for the k-point's radial factors and
 // spherical harmonics
 size_t match_table_bytes(const exh_context *c);

@@ -56,6 +56,10 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int OZ_T = 128;   // output tile edge
 constexpr int OZ_KS = 64;   // k per LDS stage (4 blocks of 16)
 constexpr int OZ_N = kOzModuli;
+constexpr int OZ_WR = 3;           // 32-row blocks per wave (96 rows)
+constexpr int OZ_NWG = 8;          // waves per workgroup
+constexpr int OZ_R = 48 * OZ_NWG;  // rows of the row panel per workgroup
+constexpr int OZ_W = OZ_R + 2 * OZ_T;  // rows and columns of one LDS stage
 
 // ---------------------------------------------------------------------------
 // Moduli: the largest pairwise coprime products of primes = 1 mod 4 below
@@ -179,33 +183,24 @@ __constant__ const OzCrts c_crt = make_crts();
 constexpr int OZ_NCH = 256;      // k per partial sum
 constexpr int OZ_LO = -400, OZ_HI = 400;  // exponents whose squares are safe
 
-struct OzOperands {  // operands of one call: X, B and, for iora*, (1+h1)A
-  const double2 *x[3];
-  long long ld[3];
-  int *e[3];       // column exponents
-  double *part[3]; // partial sums, then their exponents
-  int8_t *q[3];    // residues
-};
-
 __device__ __forceinline__ int exponent_of(double a) {  // of a normal |a|; -1023 for 0
   return (int)((__double_as_longlong(a) >> 52) & 0x7ff) - 1023;
 }
 
-__global__ __launch_bounds__(256) void colnorm_part_kernel(int ngp, int Ktot, OzOperands op,
-                                                           int ldp, int nch) {
+__device__ __forceinline__ void colnorm_part_body(const OzK &d, int z) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int g = blockIdx.x * 64 + lane, z = blockIdx.z;
-  const double2 *X = z == 0 ? op.x[0] : z == 1 ? op.x[1] : op.x[2];
-  const long long ldx = z == 0 ? op.ld[0] : z == 1 ? op.ld[1] : op.ld[2];
-  double *part = z == 0 ? op.part[0] : z == 1 ? op.part[1] : op.part[2];
+  const int g = blockIdx.x * 64 + lane;
+  const int k0 = blockIdx.y * OZ_NCH, k1 = min(d.Ktot, k0 + OZ_NCH);
+  if (z >= d.nops || (int)blockIdx.x * 64 >= d.ngp || k0 >= k1) return;  // uniform
+  const EXH_G double2 *xp = gptr(d.x[z]) + min(g, d.ngp - 1);
+  const long long ldx = d.ld[z];
+  EXH_G double *part = gptr(d.part[z]);
   __shared__ double ss[4][64];
   __shared__ int sm[4][64];
-  const int k0 = blockIdx.y * OZ_NCH, k1 = min(Ktot, k0 + OZ_NCH);
-  const double2 *xp = X + min(g, ngp - 1);
   double s = 0.0, amax = 0.0;
 #pragma unroll 8
   for (int k = k0 + w; k < k1; k += 4) {
-    const double2 v = xp[(size_t)k * ldx];
+    const double2 v = ld(xp + (size_t)k * ldx);
     s = fma(v.x, v.x, s);
     s = fma(v.y, v.y, s);
     amax = fmax(amax, fmax(fabs(v.x), fabs(v.y)));
@@ -219,7 +214,7 @@ __global__ __launch_bounds__(256) void colnorm_part_kernel(int ngp, int Ktot, Oz
     e = rescale ? (e == -1023 ? -1022 : e) : 0;
     s = 0.0;
     for (int k = k0 + w; k < k1; k += 4) {
-      const double2 v = xp[(size_t)k * ldx];
+      const double2 v = ld(xp + (size_t)k * ldx);
       const double a = ldexp(v.x, -e), b = ldexp(v.y, -e);
       s = fma(a, a, s);
       s = fma(b, b, s);
@@ -230,19 +225,19 @@ __global__ __launch_bounds__(256) void colnorm_part_kernel(int ngp, int Ktot, Oz
     e = 0;
   }
   __syncthreads();
-  if (w == 0 && g < ngp) {
-    part[(size_t)blockIdx.y * ldp + g] = ((ss[0][lane] + ss[1][lane]) + ss[2][lane]) + ss[3][lane];
-    ((int *)(part + (size_t)nch * ldp))[(size_t)blockIdx.y * ldp + g] = e;
+  if (w == 0 && g < d.ngp) {
+    part[(size_t)blockIdx.y * d.ldp + g] =
+        ((ss[0][lane] + ss[1][lane]) + ss[2][lane]) + ss[3][lane];
+    ((EXH_G int *)(part + (size_t)d.nch * d.ldp))[(size_t)blockIdx.y * d.ldp + g] = e;
   }
 }
 
-__global__ __launch_bounds__(64) void colnorm_final_kernel(int ngp, int nch, OzOperands op,
-                                                           int ldp) {
-  const int g = blockIdx.x * 64 + threadIdx.x, z = blockIdx.y;
-  if (g >= ngp) return;
-  const double *part = z == 0 ? op.part[0] : z == 1 ? op.part[1] : op.part[2];
-  int *emax = z == 0 ? op.e[0] : z == 1 ? op.e[1] : op.e[2];
-  const int *pe = (const int *)(part + (size_t)nch * ldp);
+__device__ __forceinline__ void colnorm_final_body(const OzK &d, int z) {
+  const int g = blockIdx.x * 64 + threadIdx.x;
+  if (z >= d.nops || g >= d.ngp) return;
+  const int nch = d.nch, ldp = d.ldp;
+  const EXH_G double *part = gptr((const double *)d.part[z]);
+  const EXH_G int *pe = (const EXH_G int *)(part + (size_t)nch * ldp);
   int em = -5000;  // running exponent of the sum s 2^(2 em)
   double s = 0.0;
 #pragma unroll 8
@@ -259,7 +254,7 @@ __global__ __launch_bounds__(64) void colnorm_final_kernel(int ngp, int nch, OzO
     (void)frexp(sqrt(s), &e);  // norm = f 2^e, f in [0.5, 1): norm < 2^e
     e += 1 + em;
   }
-  emax[g] = e;
+  gptr(d.e[z])[g] = e;
 }
 
 // ---------------------------------------------------------------------------
@@ -268,7 +263,7 @@ __global__ __launch_bounds__(64) void colnorm_final_kernel(int ngp, int nch, OzO
 //   y+- = (hr c1 + lr) +- (hi c2 + li I),   r = y+- - p rint(y+- / p),
 // the low byte of kMagic + r being the residue.  |r| <= (1/2 + 2^-9) p.
 // Rows ngp..rows-1 and k >= Ktot are written as zeros (no masking
-// downstream).  Layout: Q[(2 m + t) * qstride + (kblk * Gpad + g) * 16 + byte], t = 0 for
+// downstream).  Layout, m counted from m0: Q[(2 m + t) * qstride + (kblk * Gpad + g) * 16 + byte], t = 0 for
 // y+, 1 for y-.  About 13 FP64 operations per (element, modulus) beside
 // 2 bytes written: bound by HBM and the vector unit alike.
 // ---------------------------------------------------------------------------
@@ -281,26 +276,25 @@ __device__ __forceinline__ int pack4(double a, double b, double c, double d) {
   return (int)(x | y);
 }
 
-__global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpad, int rows,
-                                                      OzOperands op, int bits, int nmod,
-                                                      size_t qstride) {
+__device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kb = blockIdx.y, z = blockIdx.z;
-  if (g >= rows) return;
-  const double2 *X = z == 0 ? op.x[0] : z == 1 ? op.x[1] : op.x[2];
-  const long long ldx = z == 0 ? op.ld[0] : z == 1 ? op.ld[1] : op.ld[2];
-  const int *emax = z == 0 ? op.e[0] : z == 1 ? op.e[1] : op.e[2];
-  int8_t *Q = z == 0 ? op.q[0] : z == 1 ? op.q[1] : op.q[2];
+  const int kb = blockIdx.y;
+  const int ngp = d.ngp, Ktot = d.Ktot;
+  // rows up to the last row panel this k-point uses
+  const int rows = (ngp + OZ_R - 1) / OZ_R * OZ_R;
+  if (z >= d.nops || g >= rows || kb >= d.nslab * (OZ_KS / 16)) return;
+  const EXH_G double2 *X = gptr(d.x[z]);
+  const long long ldx = d.ld[z];
   double hr[16], lr[16], hi[16], li[16];
   int e = INT_MIN;
-  if (g < ngp) e = emax[g];
+  if (g < ngp) e = gptr((const int *)d.e[z])[g];
   const bool live = e != INT_MIN && e != INT_MAX;
-  const int s = live ? bits - e : 0;
+  const int s = live ? d.bits - e : 0;
 #pragma unroll
   for (int t = 0; t < 16; t++) {
     const int k = kb * 16 + t;
     double2 v = z2(0.0, 0.0);
-    if (live && k < Ktot) v = X[(size_t)k * ldx + g];
+    if (live && k < Ktot) v = exh::ld(X + (size_t)k * ldx + g);
     const double yr = rint(ldexp(v.x, s)), yi = rint(ldexp(v.y, s));
     constexpr double D = (double)(1ll << kSplit);
     hr[t] = rint(yr * (1.0 / D));
@@ -308,9 +302,10 @@ __global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpa
     hi[t] = rint(yi * (1.0 / D));
     li[t] = fma(-D, hi[t], yi);
   }
-  int8_t *out = Q + ((size_t)kb * Gpad + g) * 16;
+  const size_t qstride = d.qstride;
+  EXH_G int8_t *out = gptr(d.q) + z * d.q_bytes + ((size_t)kb * d.Gpad + g) * 16;
 #pragma unroll 1
-  for (int m = 0; m < nmod; m++) {
+  for (int m = m0; m < m1; m++) {
     const double p = c_mod.m[m].p, rp = c_mod.m[m].rp, nk = c_mod.m[m].nk;
     const double c1 = c_mod.m[m].c1, c2 = c_mod.m[m].c2, im = c_mod.m[m].im;
     int wp[4], wm[4];
@@ -329,8 +324,8 @@ __global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpa
       wp[q] = pack4(rpos[0], rpos[1], rpos[2], rpos[3]);
       wm[q] = pack4(rneg[0], rneg[1], rneg[2], rneg[3]);
     }
-    *(v4i *)(out + (size_t)(2 * m) * qstride) = v4i{wp[0], wp[1], wp[2], wp[3]};
-    *(v4i *)(out + (size_t)(2 * m + 1) * qstride) = v4i{wm[0], wm[1], wm[2], wm[3]};
+    *(EXH_G v4i *)(out + (size_t)(2 * (m - m0)) * qstride) = v4i{wp[0], wp[1], wp[2], wp[3]};
+    *(EXH_G v4i *)(out + (size_t)(2 * (m - m0) + 1) * qstride) = v4i{wm[0], wm[1], wm[2], wm[3]};
   }
 }
 
@@ -362,10 +357,6 @@ __global__ __launch_bounds__(256) void residue_kernel(int ngp, int Ktot, int Gpa
 // Operand lane layout: row/column = lane%32, 16 k bytes from k block
 // 2*ks + lane/32; result D[8*(r/4) + 4*(lane/32) + r%4][lane%32].
 // ---------------------------------------------------------------------------
-constexpr int OZ_WR = 3;           // 32-row blocks per wave (96 rows)
-constexpr int OZ_NWG = 8;          // waves per workgroup
-constexpr int OZ_R = 48 * OZ_NWG;  // rows of the row panel per workgroup
-constexpr int OZ_W = OZ_R + 2 * OZ_T;  // rows and columns of one LDS stage
 
 #define EXH_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 #define EXH_GLB(p) ((const __attribute__((address_space(1))) void *)(p))
@@ -378,14 +369,14 @@ constexpr int OZ_W = OZ_R + 2 * OZ_T;  // rows and columns of one LDS stage
 // load instruction of the reconstruction reads them.
 __device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], const OzMod &M,
                                                int rg, int wc, int lane, int IT, int J,
-                                               int8_t *Rp) {
+                                               EXH_G int8_t *Rp) {
   const double p = M.p, rp = M.rp, nk = M.nk;
 #pragma unroll
   for (int a = 0; a < OZ_WR; a++) {
     const int row = IT * OZ_R + rg * 32 * OZ_WR + a * 32;
     const int I = row >> 7;
     if (I > J) continue;  // below the diagonal (uniform per wave)
-    int8_t *out = Rp + ((long long)J * (J + 1) / 2 + I) * (OZ_T * OZ_T) + 4 * lane;
+    EXH_G int8_t *out = Rp + ((long long)J * (J + 1) / 2 + I) * (OZ_T * OZ_T) + 4 * lane;
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -397,7 +388,7 @@ __device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], cons
           r[t] = fma(-p, rint(fma(x, rp, nk)), x);
         }
         const int sub = 4 * (2 * wc + b) + ((row & 127) >> 5);
-        *(int *)(out + sub * 1024 + h * 256) = pack4(r[0], r[1], r[2], r[3]);
+        *(EXH_G int *)(out + sub * 1024 + h * 256) = pack4(r[0], r[1], r[2], r[3]);
       }
   }
 }
@@ -464,20 +455,20 @@ __device__ __forceinline__ void oz_panel_at(int o, int nt, int &J, int &IT) {
   }
 }
 
-// two waves per SIMD whatever the workgroup size: at most 256 VGPRs
+// Residues of the moduli m0 .. m0 + mc - 1 are in d.q, counted from m0.
 template <bool ONLY_O>
-__global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-ozgemm_kernel(
-    int nt, int nslab, int Gpad, int nmod, const int8_t *__restrict__ QX,
-    const int8_t *__restrict__ QB, const int8_t *__restrict__ QY, size_t qstride,
-    int8_t *__restrict__ R) {
-  // XCD-contiguous remap over the whole grid, then (sign * nmod + m, panel)
-  const int bid = blockIdx.x, nb = gridDim.x;
+__device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc) {
+  const int nt = d.nt, nslab = d.nslab, Gpad = d.Gpad;
+  const size_t qstride = d.qstride;
+  // XCD-contiguous remap over the k-point's panels (its first block runs on
+  // XCD 0: the grid's x extent is a multiple of 8), then (sign * mc + m, panel)
+  const int per = (int)oz_panels<ONLY_O>(nt);
+  const int bid = blockIdx.x, nb = per * 2 * mc;
+  if (bid >= nb) return;
   const int xcd = bid & 7, i8 = bid >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int t = xcd * q8 + (xcd < r8 ? xcd : r8) + i8;
-  const int per = (int)oz_panels<ONLY_O>(nt);
   const int qm = __builtin_amdgcn_readfirstlane(t / per), o = t - qm * per;
-  const int q = qm >= nmod ? 1 : 0, m = qm - q * nmod;  // q = 0: sign +, 1: sign -
+  const int q = qm >= mc ? 1 : 0, m = qm - q * mc;  // q = 0: sign +, 1: sign -
   int J, IT;
   oz_panel_at<ONLY_O>(o, nt, J, IT);
   // uniform by construction; scalar registers for the addresses that follow
@@ -489,9 +480,9 @@ ozgemm_kernel(
   // past the last block (odd nt): any valid columns, not stored
   const int O0 = min(JO, nt - 1) * OZ_T;
 
-  const int8_t *Ab = QX + (size_t)(2 * m + 1 - q) * qstride;
-  const int8_t *Hb = (ONLY_O ? QY : QB) + (size_t)(2 * m + q) * qstride;
-  const int8_t *Ob = QY + (size_t)(2 * m + q) * qstride;
+  const int8_t *Ab = d.q + (size_t)(2 * m + 1 - q) * qstride;
+  const int8_t *Ob = d.q + d.iY * d.q_bytes + (size_t)(2 * m + q) * qstride;
+  const int8_t *Hb = ONLY_O ? Ob : d.q + d.iB * d.q_bytes + (size_t)(2 * m + q) * qstride;
 
   // one LDS array per stage: the compiler then sees the DMA into one stage and
   // the reads of the other as disjoint (no wait inserted).  Rows 0..383 hold
@@ -517,7 +508,7 @@ ozgemm_kernel(
   constexpr int RC = OZ_R / 64;
   static_assert(4 * RC == OZ_WR * OZ_NWG && OZ_NWG == 8, "chunking");
   const int voff = lane * 16;
-  auto issue = [&](int s, v4i (*d)[OZ_W]) {
+  auto issue = [&](int s, v4i (*st)[OZ_W]) {
     const size_t so = (size_t)s * 4 * Gpad * 16;
     const int span = 4 * Gpad * 16;  // bytes of the stage's four k blocks
     constexpr int kRaw = 0x00020000;
@@ -528,19 +519,19 @@ ozgemm_kernel(
     for (int u = 0; u < OZ_WR; u++) {
       const int ci = w * OZ_WR + u;
       const int kk = ci / RC, rc = ci - RC * kk;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, EXH_LDS(&d[kk][rc * 64]), 16, voff,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, EXH_LDS(&st[kk][rc * 64]), 16, voff,
                                                (kk * Gpad + I0 + rc * 64) * 16, 0, 0);
     }
     const int kk = w >> 1, rc = w & 1;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rH, EXH_LDS(&d[kk][OZ_R + rc * 64]), 16, voff,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rH, EXH_LDS(&st[kk][OZ_R + rc * 64]), 16, voff,
                                              (kk * Gpad + H0 + rc * 64) * 16, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rO, EXH_LDS(&d[kk][OZ_R + OZ_T + rc * 64]), 16, voff,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rO, EXH_LDS(&st[kk][OZ_R + OZ_T + rc * 64]), 16, voff,
                                              (kk * Gpad + O0 + rc * 64) * 16, 0, 0);
   };
   const int ra = rg * 32 * OZ_WR + l32, ca = OZ_R + wc * 64 + l32;
-  auto rdA = [&](v4i (*d)[OZ_W], int ks, int a) { return d[2 * ks + lh][ra + a * 32]; };
-  auto rdH = [&](v4i (*d)[OZ_W], int ks, int b) { return d[2 * ks + lh][ca + b * 32]; };
-  auto rdO = [&](v4i (*d)[OZ_W], int ks, int b) { return d[2 * ks + lh][ca + OZ_T + b * 32]; };
+  auto rdA = [&](v4i (*st)[OZ_W], int ks, int a) { return st[2 * ks + lh][ra + a * 32]; };
+  auto rdH = [&](v4i (*st)[OZ_W], int ks, int b) { return st[2 * ks + lh][ca + b * 32]; };
+  auto rdO = [&](v4i (*st)[OZ_W], int ks, int b) { return st[2 * ks + lh][ca + OZ_T + b * 32]; };
   // four MFMAs of block row a, kept apart from the reads before and after
   auto mm = [&](int a, v4i A, const v4i (&h)[2], const v4i (&o)[2]) {
     __builtin_amdgcn_sched_barrier(0);
@@ -605,12 +596,13 @@ ozgemm_kernel(
 
   // planes: (H+, H-, O+, O-) x modulus, or (O+, O-) x modulus
   const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
-  int8_t *Rq = R + (size_t)(q * nmod + m) * plane;
-  store_residues(ah, c_mod.m[m], rg, wc, lane, IT, JH, Rq);
+  EXH_G int8_t *Rq = gptr(d.r) + (size_t)(q * d.nmod + m0 + m) * plane;
+  const OzMod &M = c_mod.m[m0 + m];
+  store_residues(ah, M, rg, wc, lane, IT, JH, Rq);
   if (ONLY_O) {
-    if (JO < nt) store_residues(ao, c_mod.m[m], rg, wc, lane, IT, JO, Rq);
+    if (JO < nt) store_residues(ao, M, rg, wc, lane, IT, JO, Rq);
   } else {
-    store_residues(ao, c_mod.m[m], rg, wc, lane, IT, JO, Rq + (size_t)2 * nmod * plane);
+    store_residues(ao, M, rg, wc, lane, IT, JO, Rq + (size_t)2 * d.nmod * plane);
   }
 }
 
@@ -636,11 +628,17 @@ __device__ __forceinline__ double crt(double hi, double lo) {
 }
 
 template <int NM, bool ONLY_O>
-__global__ __launch_bounds__(256) void ozcombine_kernel(
-    int ngp, int npairs, const int8_t *__restrict__ R, const int *__restrict__ ex,
-    const int *__restrict__ eb, const int *__restrict__ ey, int bits, IstBox box,
-    double2 *__restrict__ H, double2 *__restrict__ O, long long ldh, int accumulate) {
+__device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate) {
   const int tile = blockIdx.x >> 4, sb = blockIdx.x & 15;
+  const int npairs = d.nt * (d.nt + 1) / 2, ngp = d.ngp, bits = d.bits;
+  if (tile >= npairs) return;
+  const EXH_G int *ex = gptr((const int *)d.e[0]);
+  const EXH_G int *eb = gptr((const int *)d.e[d.iB]), *ey = gptr((const int *)d.e[d.iY]);
+  EXH_G double2 *H = gptr(d.h), *O = gptr(d.o);
+  const long long ldh = d.ldh;
+  const IstBoxT<const EXH_G int4 *, const EXH_G double *> box{
+      gptr(d.box.ivgk), gptr(d.box.vgpc), d.box.T, d.box.lo0, d.box.lo1, d.box.lo2,
+      d.box.n0, d.box.n1, d.box.n2};
   int J = (int)((sqrt(8.0 * (double)tile + 1.0) - 1.0) * 0.5);
   while ((J + 1) * (J + 2) / 2 <= tile) J++;
   while (J * (J + 1) / 2 > tile) J--;
@@ -652,7 +650,7 @@ __global__ __launch_bounds__(256) void ozcombine_kernel(
   const int tid = threadIdx.x, lane = tid & 63, h = tid >> 6;
   const int il = 8 * h + 4 * (lane >> 5), jl = lane & 31;
   const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
-  const int8_t *r0 = R + (size_t)tile * (OZ_T * OZ_T) + sb * 1024 + tid * 4;
+  const EXH_G int8_t *r0 = gptr((const int8_t *)d.r) + (size_t)tile * (OZ_T * OZ_T) + sb * 1024 + tid * 4;
 
   double rh[NV][4], rl[NV][4], mh[NV][4], ml[NV][4];
 #pragma unroll
@@ -664,16 +662,16 @@ __global__ __launch_bounds__(256) void ozcombine_kernel(
   for (int k = 0; k < NM; k++)
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      const int wp = *(const int *)(r0 + (size_t)((2 * v) * NM + k) * plane);
-      const int wm = *(const int *)(r0 + (size_t)((2 * v + 1) * NM + k) * plane);
+      const int wp = *(const EXH_G int *)(r0 + (size_t)((2 * v) * NM + k) * plane);
+      const int wm = *(const EXH_G int *)(r0 + (size_t)((2 * v + 1) * NM + k) * plane);
 #pragma unroll
       for (int t = 0; t < 4; t++) {
         const int a = byte_of(wp, t), b = byte_of(wm, t);
-        const double s = (double)(a + b), d = (double)(a - b);
+        const double s = (double)(a + b), f = (double)(a - b);
         rh[v][t] = fma(s, C.reh[k], rh[v][t]);
         rl[v][t] = fma(s, C.rel[k], rl[v][t]);
-        mh[v][t] = fma(d, C.imh[k], mh[v][t]);
-        ml[v][t] = fma(d, C.iml[k], ml[v][t]);
+        mh[v][t] = fma(f, C.imh[k], mh[v][t]);
+        ml[v][t] = fma(f, C.iml[k], ml[v][t]);
       }
     }
 
@@ -711,15 +709,15 @@ __global__ __launch_bounds__(256) void ozcombine_kernel(
     const size_t up = (size_t)i + (size_t)jj * ldh;
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      double2 *M = (!ONLY_O && v == 0) ? H : O;
+      EXH_G double2 *M = (!ONLY_O && v == 0) ? H : O;
       double2 x = sT[v][c][lo];
       if (accumulate) {
-        const double2 old = M[up];
+        const double2 old = ld(M + up);
         x.x += old.x;
         x.y += old.y;
         sT[v][c][lo] = x;
       }
-      M[up] = x;
+      st(M + up, x);
     }
   }
   if (accumulate) __syncthreads();
@@ -731,11 +729,54 @@ __global__ __launch_bounds__(256) void ozcombine_kernel(
     const size_t lw = (size_t)jj + (size_t)i * ldh;
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      double2 *M = (!ONLY_O && v == 0) ? H : O;
+      EXH_G double2 *M = (!ONLY_O && v == 0) ? H : O;
       const double2 x = sT[v][lo][c];
-      M[lw] = z2(x.x, -x.y);
+      st(M + lw, z2(x.x, -x.y));
     }
   }
+}
+
+// Single launches take the k-point by value, grouped ones an array of them;
+// blockIdx.z (with the operand) or blockIdx.y selects it.
+__global__ __launch_bounds__(256) void colnorm_part_kernel(OzK d) {
+  colnorm_part_body(d, blockIdx.z);
+}
+__global__ __launch_bounds__(256) void colnorm_part_grouped_kernel(const OzK *__restrict__ kd,
+                                                                   int nops) {
+  colnorm_part_body(kd[blockIdx.z / nops], blockIdx.z % nops);
+}
+__global__ __launch_bounds__(64) void colnorm_final_kernel(OzK d) {
+  colnorm_final_body(d, blockIdx.z);
+}
+__global__ __launch_bounds__(64) void colnorm_final_grouped_kernel(const OzK *__restrict__ kd,
+                                                                   int nops) {
+  colnorm_final_body(kd[blockIdx.z / nops], blockIdx.z % nops);
+}
+__global__ __launch_bounds__(256) void residue_kernel(OzK d, int m0, int m1) {
+  residue_body(d, blockIdx.z, m0, m1);
+}
+__global__ __launch_bounds__(256) void residue_grouped_kernel(const OzK *__restrict__ kd, int nops,
+                                                              int m1) {
+  residue_body(kd[blockIdx.z / nops], blockIdx.z % nops, 0, m1);
+}
+// two waves per SIMD whatever the workgroup size: at most 256 VGPRs
+template <bool ONLY_O>
+__global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+ozgemm_kernel(OzK d, int m0, int mc) {
+  ozgemm_body<ONLY_O>(d, m0, mc);
+}
+__global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+ozgemm_grouped_kernel(const OzK *__restrict__ kd, int mc) {
+  ozgemm_body<false>(kd[blockIdx.y], 0, mc);
+}
+template <int NM, bool ONLY_O>
+__global__ __launch_bounds__(256) void ozcombine_kernel(OzK d, int accumulate) {
+  ozcombine_body<NM, ONLY_O>(d, accumulate);
+}
+template <int NM>
+__global__ __launch_bounds__(256) void ozcombine_grouped_kernel(const OzK *__restrict__ kd,
+                                                                int accumulate) {
+  ozcombine_body<NM, false>(kd[blockIdx.y], accumulate);
 }
 
 inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
@@ -784,85 +825,136 @@ OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool thir
   L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
   L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * nch * ng + 255) / 256 * 256;
   L.nops = 1 + (only_o ? 0 : 1) + (third ? 1 : 0);
+  L.panels = 2 * P.nmod * (only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt));
   return L;
 }
 
-hipError_t launch_ozaki(hipStream_t s, const exh_context *c, int ngp, const OzPlan &P,
-                        const OzLayout &L, const OzScratch &w, const double2 *X, long long ldx,
-                        const double2 *B, const double2 *Y, long long ldb, const IstBox &box,
-                        double2 *h, double2 *o, int ldh, int accumulate, int stage_mask) {
-  if (ngp <= 0) return hipSuccess;
-  const int K = c->Ktot;
-  const long long nt = (ngp + OZ_T - 1) / OZ_T;
-  const long long npairs = nt * (nt + 1) / 2;
-  const int nslab = L.Kpad / OZ_KS;
-  // operands: X, then B (not for O alone), then Y where the overlap has its own
-  const bool only_o = h == nullptr;
-  OzOperands op{};
+OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
+             const OzScratch &w, const double2 *X, long long ldx, const double2 *B,
+             const double2 *Y, long long ldb, const IstBox &box, double2 *h, double2 *o,
+             int ldh) {
+  OzK d{};
+  d.ngp = ngp;
+  d.Ktot = c->Ktot;
+  d.nt = (ngp + OZ_T - 1) / OZ_T;
+  d.nslab = L.Kpad / OZ_KS;
+  d.Gpad = L.Gpad;
+  d.nmod = P.nmod;
+  d.bits = P.bits;
+  d.ldp = std::max(c->ngkmax, 1);
+  d.nch = (c->Ktot + OZ_NCH - 1) / OZ_NCH;
+  d.qstride = L.qstride;
+  d.q_bytes = w.chunk * 2 * L.qstride;
+  d.q = w.q;
+  d.r = w.r;
+  d.box = box;
+  d.h = h;
+  d.o = o;
+  d.ldh = ldh;
   const double2 *src[3] = {X, B, Y};
-  int n = 0, iB = 0, iY = 0;
   for (int z = 0; z < 3; z++) {
-    if ((z == 1 && only_o) || (z == 2 && !Y)) continue;
-    if (z == 1) iB = n;
-    if (z == 2) iY = n;
+    if ((z == 1 && !h) || (z == 2 && !Y)) continue;
+    const int n = d.nops++;
+    if (z == 1) d.iB = n;
+    if (z == 2) d.iY = n;
     char *e = (char *)w.e + (size_t)n * L.e_bytes;
-    op.x[n] = src[z];
-    op.ld[n] = z == 0 ? ldx : ldb;
-    op.e[n] = (int *)e;
-    op.part[n] = (double *)(e + L.e_part_off);
-    op.q[n] = w.q + (size_t)n * L.q_bytes;
-    n++;
+    d.x[n] = src[z];
+    d.ld[n] = z == 0 ? ldx : ldb;
+    d.e[n] = (int *)e;
+    d.part[n] = (double *)(e + L.e_part_off);
   }
+  return d;
+}
+
+// One k-point (kd null: by value from d) or the n k-points d[0..n) that kd
+// holds in device memory.  chunk: moduli whose residues the scratch holds; a
+// chunk below nmod runs residues and products in turn (all stages in one
+// call).
+static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, int chunk,
+                            int accumulate, int stage_mask) {
+  const bool only_o = d[0].h == nullptr;
+  const int nmod = d[0].nmod;
+  int ngp = 0, nch = 0, nops = 0, kb = 0, nt = 0;
+  for (int i = 0; i < n; i++) {
+    ngp = std::max(ngp, d[i].ngp);
+    nch = std::max(nch, d[i].nch);
+    nops = std::max(nops, d[i].nops);
+    kb = std::max(kb, d[i].nslab * (OZ_KS / 16));
+    nt = std::max(nt, d[i].nt);
+  }
+  if (ngp <= 0) return hipSuccess;
+  const unsigned nz = (unsigned)(nops * n);
   if (stage_mask & 1) {
-    const int nch = (K + OZ_NCH - 1) / OZ_NCH;
-    const int ldp = std::max(c->ngkmax, 1);
-    hipLaunchKernelGGL(colnorm_part_kernel, dim3(cdiv(ngp, 64), nch, n), dim3(256), 0, s, ngp, K,
-                       op, ldp, nch);
-    hipLaunchKernelGGL(colnorm_final_kernel, dim3(cdiv(ngp, 64), n), dim3(64), 0, s, ngp, nch, op,
-                       ldp);
-    // rows up to the last row panel this k-point uses
-    const int rows = (ngp + OZ_R - 1) / OZ_R * OZ_R;
-    hipLaunchKernelGGL(residue_kernel, dim3(cdiv(rows, 256), L.Kpad / 16, n), dim3(256), 0, s,
-                       ngp, K, L.Gpad, rows, op, P.bits, P.nmod, L.qstride);
+    const dim3 gp(cdiv(ngp, 64), nch, nz), gf(cdiv(ngp, 64), 1, nz);
+    if (kd) {
+      hipLaunchKernelGGL(colnorm_part_grouped_kernel, gp, dim3(256), 0, s, kd, nops);
+      hipLaunchKernelGGL(colnorm_final_grouped_kernel, gf, dim3(64), 0, s, kd, nops);
+    } else {
+      hipLaunchKernelGGL(colnorm_part_kernel, gp, dim3(256), 0, s, d[0]);
+      hipLaunchKernelGGL(colnorm_final_kernel, gf, dim3(64), 0, s, d[0]);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (stage_mask & 2) {
-    const long long per = only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt);
-    const dim3 grid((unsigned)(per * 2 * P.nmod));
-    if (only_o)
-      hipLaunchKernelGGL(ozgemm_kernel<true>, grid, dim3(64 * OZ_NWG), 0, s, (int)nt, nslab,
-                         L.Gpad, P.nmod, op.q[0], op.q[iY], op.q[iY], L.qstride, w.r);
-    else
-      hipLaunchKernelGGL(ozgemm_kernel<false>, grid, dim3(64 * OZ_NWG), 0, s, (int)nt, nslab,
-                         L.Gpad, P.nmod, op.q[0], op.q[iB], op.q[iY], L.qstride, w.r);
+  const dim3 gr(cdiv((long long)cdiv(ngp, OZ_R) * OZ_R, 256), kb, nz);
+  const long long per = only_o ? oz_panels<true>(nt) : oz_panels<false>(nt);
+  for (int m0 = 0; m0 < nmod; m0 += chunk) {
+    const int m1 = std::min(nmod, m0 + chunk);
+    if (stage_mask & 1) {
+      if (kd) hipLaunchKernelGGL(residue_grouped_kernel, gr, dim3(256), 0, s, kd, nops, m1);
+      else hipLaunchKernelGGL(residue_kernel, gr, dim3(256), 0, s, d[0], m0, m1);
+    }
+    if (stage_mask & 2) {
+      const long long nb = per * 2 * (m1 - m0);
+      const dim3 gg((unsigned)((nb + 7) / 8 * 8), n);
+      if (kd)
+        hipLaunchKernelGGL(ozgemm_grouped_kernel, gg, dim3(64 * OZ_NWG), 0, s, kd, m1 - m0);
+      else if (only_o)
+        hipLaunchKernelGGL(ozgemm_kernel<true>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0);
+      else
+        hipLaunchKernelGGL(ozgemm_kernel<false>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (stage_mask & 4) {
-    const dim3 grid((unsigned)(npairs * 16));
-#define EXH_OZC(N, OO)                                                                         \
-  hipLaunchKernelGGL((ozcombine_kernel<N, OO>), grid, dim3(256), 0, s, ngp, (int)npairs, w.r,  \
-                     op.e[0], op.e[iB], op.e[iY], P.bits, box, h, o, (long long)ldh, accumulate)
+    const dim3 grid((unsigned)(nt * (nt + 1) / 2 * 16), n);
     if (only_o) {
-      if (P.nmod != OZ_N) return hipErrorInvalidValue;  // EXH_SPLIT is refused for O alone
-      EXH_OZC(OZ_N, true);
-    } else {
-      switch (P.nmod) {
-        case 6: EXH_OZC(6, false); break;
-        case 7: EXH_OZC(7, false); break;
-        case 8: EXH_OZC(8, false); break;
-        case 9: EXH_OZC(9, false); break;
-        case 10: EXH_OZC(10, false); break;
-        case 11: EXH_OZC(11, false); break;
-        case 13: EXH_OZC(13, false); break;  // EXH_SPLIT(12)
-        case OZ_N: EXH_OZC(OZ_N, false); break;
-        default: return hipErrorInvalidValue;
-      }
+      if (nmod != OZ_N) return hipErrorInvalidValue;  // EXH_SPLIT is refused for O alone
+      hipLaunchKernelGGL((ozcombine_kernel<OZ_N, true>), grid, dim3(256), 0, s, d[0], accumulate);
+      return hipGetLastError();
+    }
+#define EXH_OZC(N)                                                                              \
+  case N:                                                                                       \
+    if (kd)                                                                                     \
+      hipLaunchKernelGGL(ozcombine_grouped_kernel<N>, grid, dim3(256), 0, s, kd, accumulate);   \
+    else                                                                                        \
+      hipLaunchKernelGGL((ozcombine_kernel<N, false>), grid, dim3(256), 0, s, d[0], accumulate); \
+    break;
+    switch (nmod) {
+      EXH_OZC(6)
+      EXH_OZC(7)
+      EXH_OZC(8)
+      EXH_OZC(9)
+      EXH_OZC(10)
+      EXH_OZC(11)
+      EXH_OZC(13)  // EXH_SPLIT(12)
+      EXH_OZC(OZ_N)
+      default:
+        return hipErrorInvalidValue;
     }
 #undef EXH_OZC
   }
   return hipGetLastError();
+}
+
+hipError_t launch_ozaki(hipStream_t s, const OzK &d, int chunk, int accumulate, int stage_mask) {
+  return launch_oz(s, &d, nullptr, 1, chunk, accumulate, stage_mask);
+}
+
+hipError_t launch_ozaki_grouped(hipStream_t s, const OzK *d, const OzK *kd, int n, int accumulate,
+                                int stage_mask) {
+  return launch_oz(s, d, kd, n, d[0].nmod, accumulate, stage_mask);
 }
 
 }  // namespace exh

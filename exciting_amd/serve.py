@@ -88,15 +88,17 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     K = sys_.natmtot * sys_.maxaa
     ldb = (sys_.ngkmax + 63) // 64 * 64
     scratch = 16 * K * ldb                       # aa.A operand
-    fp64_modular = 16 * K * ldb > 64 << 20       # FP64 on the 15-moduli products
+    fp64_modular = K * ldb >= 1 << 15            # FP64 on the 15-moduli products
     if nmod_max or fp64_modular:
         gpad = (sys_.ngkmax + 383) // 384 * 384     # rows padded to the GEMM's panel
         kpad = (K + 127) // 128 * 128
         nt = (sys_.ngkmax + 127) // 128
-        # SPLIT(12) runs 13 moduli
-        moduli = max(nmod_max + 1 if nmod_max else 0, 15 if fp64_modular else 0)
-        scratch += 4 * moduli * kpad * gpad         # int8 residues of A and aa.A
-        scratch += 4 * moduli * nt * (nt + 1) // 2 * 128 * 128   # product residues
+        # SPLIT(12) runs 13 moduli; one more for the rounding of the buffers
+        # that serve both precisions
+        moduli = max(nmod_max + 1 if nmod_max else 0, 15 if fp64_modular else 0) + bool(nmod_max)
+        # int8 residues of A and aa.A, and of the products; a launch may hold
+        # every slot's
+        scratch += slots * 4 * moduli * (kpad * gpad + nt * (nt + 1) // 2 * 128 * 128)
     perk = len(sys_.kpts) * sys_.ngkmax * (16 * sys_.natmtot + 8 * 7 + 4)
     # Cholesky factor, the two triangular solves' results, the reduced matrix
     # and its Hermitian average, and the eigensolver's copy and workspace

@@ -72,15 +72,15 @@ enum {
  * (2^-c of the column's norm).  Match, the lo blocks and the interstitial
  * stay FP64.  Not combined with h1aa.
  *
- * Without EXH_SPLIT, setups of large bases (16 natmtot*maxaa * ngkmax rounded
- * up > 64 MiB) use the same exact products with c = 56: each operand keeps 55
- * bits relative to its column's 2-norm and nothing else is rounded before the
- * result, which is nearer to the exact product than FP64 accumulation over
- * K (H and O at 64 atoms: relative Frobenius error 1e-16 against 5e-15).
- * They need 60 bytes of scratch per (K, G+k) pair and 60 per upper element
- * of H; a device without that room, or a stream captured before a first call
- * has allocated it, runs the FP64 MFMA kernels instead (results differ by
- * rounding). */
+ * Without EXH_SPLIT, all but the smallest bases (fewer than 2^15 pairs of
+ * K = natmtot*maxaa and ngkmax rounded up to 64) use the same exact products
+ * with c = 56: each operand keeps 55 bits relative to its column's 2-norm and
+ * nothing else is rounded before the result, which is nearer to the exact
+ * product than FP64 accumulation over K (H and O at 64 atoms: relative
+ * Frobenius error 1e-16 against 5e-15).  They need 60 bytes of scratch per
+ * (K, G+k) pair and 60 per upper element of H; a device without that room, or
+ * a stream captured before a first call has allocated it, runs the FP64 MFMA
+ * kernels instead (results differ by rounding). */
 #define EXH_SPLIT(n) ((n) << 8)
 
 /* ---- context ------------------------------------------------------------ */
@@ -298,8 +298,8 @@ int exh_setup_device(exh_context *ctx, void *stream, int ngp, int rank,
  * forbid hipMalloc).  The same setup as exh_setup_device (FP64; flags
  * EXH_ACCUMULATE or 0), with bitwise the same result, but its scratch
  * (G+k index map, aa.A operand, and for iora* or non-uniform layouts one
- * more operand) lives in a static 64 MiB device array instead of the
- * context's buffers: it calls no hipMalloc, hipFree or allocating library
+ * more operand) lives in a static 64 MiB device array, and the residues of
+ * the modular products in another 128 MiB, instead of the context's buffers: it calls no hipMalloc, hipFree or allocating library
  * routine.  Bases needing more than 64 MiB (16 * natmtot*maxaa * ngkmax
  * rounded up, per operand) are refused with EXH_ERANGE, split precision
  * with EXH_ENOTSUP.  Every context on a GPU shares that GPU's array, so

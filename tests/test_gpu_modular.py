@@ -1,5 +1,5 @@
-"""The modular (int8) contraction: FP64 setups of bases whose K-major operand
-exceeds 64 MiB, and every EXH_SPLIT modulus count.
+"""The modular (int8) contraction: FP64 setups of all but the smallest bases,
+and every EXH_SPLIT modulus count.
 
 A 12-atom cell (lmaxapw 10, K = 2904, 1766 G+k) runs on it.  Truncated to
 small and ragged G+k counts (edges of the 32, 128 and 384 tiles) H and O are
@@ -203,11 +203,33 @@ def test_split_modulus_counts(nmod):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name,path", [("tiny_multi", "ho_grouped"), ("fcc2", "oz_gemm"),
+                                       ("sc8_4k", "oz_gemm")])
+def test_route_by_basis_size(name, path):
+    """Bases below 2^15 (K, G+k) pairs stay on the FP64 MFMA tiles."""
+    import torch
+    s = _cases.system(name)
+    ctx = lapw.Context(0).load(s)
+    try:
+        dk = [lapw.DeviceKPoint(s, i) for i in range(len(s.kpts))]
+        ys = [lapw.newsystem(d.rank, device="cuda") for d in dk]
+        kp = [lapw.kpoint_struct(d, y.hamilton.za, y.overlap.za) for d, y in zip(dk, ys)]
+        ctx.profile(True)
+        ctx.profile_reset()
+        ctx.setup_batch(kp, flags=lapw.MATCH)
+        torch.cuda.synchronize()
+        ran = {n for n, v in ctx.profile_read().items() if v[1]}
+        assert path in ran and len(ran & {"ho_grouped", "oz_gemm"}) == 1
+    finally:
+        ctx.close()
+
+
+@pytest.mark.gpu
 def test_grouped_call_mixes_both_contractions(ctxs):
     """One grouped call over a modular and an FP64-MFMA structure, eager and
     replayed from a graph: bitwise the single path."""
     import torch
-    small = _cases.system("sc8_k0")
+    small = _cases.system("tiny_multi")
     s, ctx = ctxs()
     s = truncated(s, 257)
     c2 = lapw.Context(0).load(small)
