@@ -410,38 +410,38 @@ OzPlan oz_plan(const exh_context *c, int flags) {
   if (pairs < (size_t(1) << 15) || c->Ktot > kOzMaxK) return OzPlan();
   const OzPlan P = oz_fp64();
   if (pairs * sizeof(double2) > kNoallocScratchBytes) return P;  // refused there
-  const OzLayout L = oz_layout(c->ngkmax, c->Ktot, P, false, c->have_h1aa);
+  const OzLayout L = oz_layout(c, P, false);
   return oz_noalloc_chunk(P, L) > 0 ? P : OzPlan();
 }
 
-bool oz_fits(const exh_context *c, const OzLayout &L, int slots) {
+bool oz_fits(const exh_context *c, const OzLayout &L, int slots, int nk) {
   return c->ozq.bytes >= L.q_bytes * L.nops * slots && c->ozr.bytes >= L.r_bytes * slots &&
-         c->oze.bytes >= L.e_bytes * L.nops * slots;
+         c->oze.bytes >= L.e_bytes * L.nops * nk;
 }
 
-// Plan, layout and scratch of the modular contraction for `slots` k-points;
-// P.nmod = 0 when the setup runs on the FP64 MFMA kernels instead, which is
-// also where an FP64 setup goes when the device has no room for the residues
-// or the stream is being captured before the first call (nothing may be
-// allocated then).
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, OzPlan &P,
-               OzLayout &L) {
+// Plan, layout and scratch of the modular contraction for nk k-points, the
+// residues of `slots` of them at a time; P.nmod = 0 when the setup runs on the
+// FP64 MFMA kernels instead, which is also where an FP64 setup goes when the
+// device has no room for the residues or the stream is being captured before
+// the first call (nothing may be allocated then).
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, int nk,
+               OzPlan &P, OzLayout &L) {
   P = oz_plan(c, flags);
   if (P.nmod == 0) return 0;
   const bool split = (flags & 0xff00) != 0;
-  L = oz_layout(c->ngkmax, c->Ktot, P, only_o, c->have_h1aa);
-  if (oz_fits(c, L, slots)) return 0;
+  L = oz_layout(c, P, only_o);
+  if (oz_fits(c, L, slots, nk)) return 0;
   if (!split) {
     size_t avail = 0, total = 0;
     if (capturing || hipMemGetInfo(&avail, &total) != hipSuccess ||
-        avail < L.bytes() * slots + (size_t(1) << 30)) {
+        avail < L.bytes() * slots + L.e_bytes * L.nops * nk + (size_t(1) << 30)) {
       P = OzPlan();
       return 0;
     }
   }
   int rc = ensure(c, c->ozq, L.q_bytes * L.nops * slots);
   if (!rc) rc = ensure(c, c->ozr, L.r_bytes * slots);
-  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops * slots);
+  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops * nk);
   if (rc && !split) {  // another allocation took the room meanwhile
     (void)hipGetLastError();
     P = OzPlan();
@@ -876,13 +876,25 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
     return record ? timed(c, k, s, launch) : launch();
   };
   const double2 *A = (const double2 *)apwalm;
+  OzK d{};
+  NormOut norms;
+  if (nmod > 0) {
+    long long ldx;
+    const double2 *X = k_major_operand(c, A, w.at, &ldx);
+    const int lo0 = c->intgv[0], lo1 = c->intgv[1], lo2 = c->intgv[2];
+    IstBox box{w.ivgk, vgpc, (const IstEntry *)c->ist.p, lo0, lo1, lo2,
+               c->intgv[3] - lo0 + 1, c->intgv[4] - lo1 + 1, c->intgv[5] - lo2 + 1};
+    d = make_ozk(c, ngp, w.plan, w.layout, w.oz, X, ldx, w.bt, c->have_h1aa ? w.a2t : nullptr,
+                 ldb, box, (double2 *)hw, (double2 *)o, rank);
+    if (!o_only) norms = norm_out(d);
+  }
   hipError_t e = run(EXH_K_IVGK, [&] {
     return launch_ivgk(s, ngp, igpig, (const int *)c->ivg.p, c->ngrtot, w.ivgk);
   });
   if (e == hipSuccess && !c->contig)
     e = run(EXH_K_PACK, [&] { return launch_pack(s, c, ngp, A, w.at); });
   if (e == hipSuccess && !o_only)
-    e = run(EXH_K_BT, [&] { return launch_bt(s, c, ngp, A, w.at, w.bt, ldb); });
+    e = run(EXH_K_BT, [&] { return launch_bt(s, c, ngp, A, w.at, w.bt, ldb, norms); });
   if (e == hipSuccess && c->have_h1aa)
     e = run(EXH_K_A2T, [&] { return launch_a2t(s, c, ngp, A, w.a2t, ldb); });
   if (e == hipSuccess && nmod == 0)
@@ -891,14 +903,6 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
                        vgpc, (double2 *)hw, (double2 *)o, rank, flags);
     });
   if (e == hipSuccess && nmod > 0) {
-    long long ldx;
-    const double2 *X = k_major_operand(c, A, w.at, &ldx);
-    const int lo0 = c->intgv[0], lo1 = c->intgv[1], lo2 = c->intgv[2];
-    IstBox box{w.ivgk, vgpc, (const IstEntry *)c->ist.p, lo0, lo1, lo2,
-               c->intgv[3] - lo0 + 1, c->intgv[4] - lo1 + 1, c->intgv[5] - lo2 + 1};
-    const OzK d = make_ozk(c, ngp, w.plan, w.layout, w.oz, X, ldx, w.bt,
-                           c->have_h1aa ? w.a2t : nullptr, ldb, box, (double2 *)hw, (double2 *)o,
-                           rank);
     const int acc = flags & EXH_ACCUMULATE;
     if (w.oz.chunk < nmod) {
       e = launch_ozaki(s, d, w.oz.chunk, acc, 7);
@@ -934,9 +938,10 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   if (!rc && !c->contig) rc = ensure(c, c->at, op);
   if (!rc) rc = ensure(c, c->ivgk, (size_t)std::max(c->ngkmax, 1) * sizeof(int4));
   if (!rc)
-    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, 1, w.plan, w.layout);
+    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, 1, 1, w.plan,
+                    w.layout);
   if (rc) return rc;
-  if (w.plan.nmod) w.oz = oz_scratch(c, w.plan, w.layout, 0);
+  if (w.plan.nmod) w.oz = oz_scratch(c, w.plan, w.layout, 0, 0);
   w.bt = (double2 *)c->bt.p;
   w.a2t = (double2 *)c->a2t.p;
   w.at = (double2 *)c->at.p;
@@ -992,7 +997,7 @@ int exh_setup_device_noalloc(exh_context *c, void *stream, int ngp, int rank,
   w.plan = oz_plan(c, flags);
   if (w.plan.nmod) {
     // [product residues | exponents and norms | residues of `chunk` moduli]
-    w.layout = oz_layout(c->ngkmax, c->Ktot, w.plan, false, c->have_h1aa);
+    w.layout = oz_layout(c, w.plan, false);
     w.oz.chunk = oz_noalloc_chunk(w.plan, w.layout);
     unsigned char *mod = base + kNoallocScratchBytes;
     w.oz.r = (int8_t *)mod;

@@ -300,7 +300,7 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
     }
     g.nwg = (int)std::max<long long>(nwg, 0);
     g.w0 = (int)E->waves.size();
-    std::vector<int> used(nctx, 0);
+    std::vector<int> used(nctx, 0), nth(nctx, 0);
     exh_context::BatchEntry::Wave wv{(int)E->oz.size(), 0};
     auto close_wave = [&]() {
       if (wv.count) E->waves.push_back(wv);
@@ -312,13 +312,14 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
       if (!skip[i] || kp[i].ngp <= 0) continue;
       if (used[j] == oz.slots[j]) close_wave();
       const exh_context *c = cc.ctxs[j];
-      const KDesc &d = E->kd[i];
+      KDesc &d = E->kd[i];
       const SDesc &S = E->sd[j];
       IstBox box{d.ivgk, d.vgpc, (const IstEntry *)c->ist.p, S.lo0, S.lo1, S.lo2,
                  S.n0, S.n1, S.n2};
       E->oz.push_back(make_ozk(c, d.ngp, oz.P[j], oz.L[j],
-                               oz_scratch(c, oz.P[j], oz.L[j], used[j]), d.x, S.ldx, d.bt,
+                               oz_scratch(c, oz.P[j], oz.L[j], used[j], nth[j]++), d.x, S.ldx, d.bt,
                                d.a2t, S.ldb, box, d.h, d.o, d.ldh));
+      d.norms = norm_out(E->oz.back());
       used[j]++;
       wv.count++;
     }
@@ -339,6 +340,7 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
     const int ldb = ldb_of(c);
     const size_t op = (size_t)std::max(c->Ktot, 1) * ldb;
     KDesc &d = E->kd[i];
+    d.norms = NormOut();
     d.ngp = k.ngp;
     d.ldh = k.rank;
     d.gpc = k.gpc;
@@ -462,26 +464,26 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
     exh_context *c = cc.ctxs[j];
     oz.P[j] = oz_plan(c, flags);
     if (oz.P[j].nmod) {
-      oz.L[j] = oz_layout(c->ngkmax, c->Ktot, oz.P[j], false, c->have_h1aa);
+      oz.L[j] = oz_layout(c, oz.P[j], false);
       oz.slots[j] = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j]);
     }
     if (outer_capture) {
       // nothing may be allocated or uploaded inside a caller's capture
-      if (oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j])) oz.slots[j] = 1;
-      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, oz.L[j], 1);
+      if (oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j], cc.nkg[j])) oz.slots[j] = 1;
+      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, oz.L[j], 1, cc.nkg[j]);
       if (!oz_ok && !nmod) oz.P[j] = OzPlan();  // as the call outside capture ran
       if (!scratch_fits(c, cc.nkg[j]) || (nmod && !oz_ok))
         return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
     } else {
       rc = ensure_scratch(c, cc.nkg[j]);
-      if (!rc && oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j])) {
+      if (!rc && oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j], cc.nkg[j])) {
         // several slots only where the device has room for them
         size_t avail = 0, total = 0;
         if (oz.slots[j] > 1 &&
             (hipMemGetInfo(&avail, &total) != hipSuccess ||
              avail < oz.L[j].bytes() * oz.slots[j] + (size_t(2) << 30)))
           oz.slots[j] = 1;
-        rc = oz_prepare(c, flags, false, false, oz.slots[j], oz.P[j], oz.L[j]);
+        rc = oz_prepare(c, flags, false, false, oz.slots[j], cc.nkg[j], oz.P[j], oz.L[j]);
       }
       if (rc) {
         if (c != lead) fail(lead, rc, c->err);
@@ -628,7 +630,7 @@ int exh_tune_batch(exh_context *c, void *stream, int nk, const exh_kpoint *kp, i
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   OzPlan P;
   OzLayout L;
-  rc = oz_prepare(c, flags, false, false, 1, P, L);
+  rc = oz_prepare(c, flags, false, false, 1, 1, P, L);
   if (rc) return rc;
   if (P.nmod) {  // no tiles to shape: every plan is the same call
     rc = exh_setup_batch_device(c, s, nk, kp, flags);

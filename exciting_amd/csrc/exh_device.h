@@ -141,13 +141,24 @@ __device__ __forceinline__ void store_upper_o(PH O, long long ldh, int i, int j,
   if (i != j) st(O + (size_t)j + (size_t)i * ldh, z2(orr, -oi));
 }
 
+// Exponent of |a| (-1023 for 0 and denormals), and the mark of a partial column
+// norm with largest entry amax: beyond 2^+-400 FP64 squares may leave the range.
+__device__ __forceinline__ int exponent_of(double a) {
+  return (int)((__double_as_longlong(a) >> 52) & 0x7ff) - 1023;
+}
+__device__ __forceinline__ int norm_mark(double amax) {
+  const bool out = amax > 0.0 && (amax < 0x1p-400 || (amax > 0x1p400 && amax <= 0x1.fp1023));
+  return out ? kNormRecompute : 0;
+}
+
 // One k-point of the modular contraction: operands (X; B unless O alone;
 // (1+h1)A for iora*), scratch and outputs, by value for a single launch or in
 // device memory for a grouped one.
 struct OzK {
   int ngp, Ktot, nt, nslab, Gpad, nmod, bits;
   int nops, iB, iY;       // operands; which one is B, and the overlap's columns
-  int ldp, nch;           // partial norms: leading dimension, chunks
+  int ldp, nch[3];        // partial norms: leading dimension, chunks per operand
+  unsigned fused;         // operands whose partial norms bt has written
   size_t qstride, q_bytes;  // one residue array; one operand's arrays
   const double2 *x[3];
   long long ld[3];

@@ -36,7 +36,7 @@ struct LoRow {
 // Static device scratch of exh_setup_device_noalloc (api.hip): the K-major
 // operands and the G+k map, then the modular contraction's part.
 constexpr size_t kNoallocScratchBytes = size_t(64) << 20;
-constexpr size_t kNoallocModularBytes = size_t(128) << 20;
+constexpr size_t kNoallocModularBytes = size_t(256) << 20;
 inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Modular (Ozaki scheme II) contraction: split precision, and FP64 for large
@@ -50,12 +50,13 @@ struct OzPlan {
   int bits = 0;  // c: the scaled columns' 2-norms are below 2^(c-1)
 };
 struct OzLayout {
-  int Gpad = 0, Kpad = 0;  // G rounded to the row panel, K to two 64-k stages
+  int Gpad = 0, Kpad = 0;  // G rounded to the 128 tile, K to two 64-k stages
   size_t qstride = 0;      // bytes of one residue array (Kpad * Gpad)
   int nops = 0;            // operands (X; B unless O alone; (1+h1)A for iora*)
   size_t q_bytes = 0;      // residues of one operand
   size_t r_bytes = 0;      // residues of the products
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
+  int nch = 0;             // partial norms of an operand, at most
   long long panels = 0;    // workgroups of the products at ngkmax
   size_t bytes() const { return q_bytes * nops + r_bytes + e_bytes * nops; }
 };
@@ -64,6 +65,17 @@ struct OzScratch {
   void *e = nullptr;
   int chunk = 0;  // moduli whose residues q holds
 };
+
+// Partial squared column norms of the modular contraction's operands, as bt
+// writes them: per atom for X, per atom and 64 rows of aa for B, [chunk][G+k]
+// with leading dimension ld, each followed by as many int exponents (0, or
+// kNormRecompute where squares leave FP64's range).  x null: not wanted.
+struct NormOut {
+  double *x = nullptr, *b = nullptr;
+  int ld = 0, nx = 0, nb = 0;
+};
+constexpr int kNormRecompute = 1 << 20;
+constexpr int kNormRows = 64;  // rows of aa per partial norm of B
 
 // APW-lo border tables (hamiltonsetup.f90:124-151, overlapsetup.f90:116-133)
 // of one structure, device pointers.
@@ -124,6 +136,7 @@ struct KDesc {
   double2 *at, *bt, *a2t;
   int4 *ivgk;
   double *mtab;  // match: radial and harmonics tables of this k-point (batch scratch)
+  NormOut norms; // where bt leaves the partial column norms (modular contraction)
   const SDesc *sd;
 };
 
@@ -298,7 +311,8 @@ hipError_t launch_ist_table(hipStream_t s, const exh_context *c,
 hipError_t launch_pack(hipStream_t s, const exh_context *c, int ngp,
                        const double2 *apwalm, double2 *at);
 hipError_t launch_bt(hipStream_t s, const exh_context *c, int ngp,
-                     const double2 *apwalm, const double2 *at, double2 *bt, int ldb);
+                     const double2 *apwalm, const double2 *at, double2 *bt, int ldb,
+                     const NormOut &norms);
 hipError_t launch_a2t(hipStream_t s, const exh_context *c, int ngp,
                       const double2 *apwalm, double2 *a2t, int ldb);
 hipError_t launch_ho(hipStream_t s, const exh_context *c, int ngp,
@@ -315,24 +329,27 @@ hipError_t launch_lolo(hipStream_t s, const exh_context *c, int ngp,
 const double2 *k_major_operand(const exh_context *c, const double2 *apwalm, const double2 *at,
                                long long *ld);
 struct IstBox;
+struct OzK;
 OzPlan oz_split(int n);
 OzPlan oz_fp64();
-OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool third);
+OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o);
+NormOut norm_out(const OzK &d);
 OzPlan oz_plan(const exh_context *c, int flags);
 int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L);
-bool oz_fits(const exh_context *c, const OzLayout &L, int slots);
-// Slot `slot` of the context's modular scratch.
-inline OzScratch oz_scratch(const exh_context *c, const OzPlan &P, const OzLayout &L, int slot) {
+bool oz_fits(const exh_context *c, const OzLayout &L, int slots, int nk);
+// Residue slot `slot` of the context's modular scratch, norms of k-point `k` of
+// the group.
+inline OzScratch oz_scratch(const exh_context *c, const OzPlan &P, const OzLayout &L, int slot,
+                            int k) {
   OzScratch w;
   w.q = (int8_t *)c->ozq.p + (size_t)slot * L.q_bytes * L.nops;
   w.r = (int8_t *)c->ozr.p + (size_t)slot * L.r_bytes;
-  w.e = (char *)c->oze.p + (size_t)slot * L.e_bytes * L.nops;
+  w.e = (char *)c->oze.p + (size_t)k * L.e_bytes * L.nops;
   w.chunk = P.nmod;
   return w;
 }
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, OzPlan &P,
-               OzLayout &L);
-struct OzK;
+int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, int nk,
+               OzPlan &P, OzLayout &L);
 // h = nullptr: O alone (B is not read).  Y = nullptr: the overlap's column
 // operand is X.
 OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,

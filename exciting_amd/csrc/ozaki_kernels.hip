@@ -169,34 +169,29 @@ constexpr OzCrts make_crts() {
 __constant__ const OzCrts c_crt = make_crts();
 
 // ---------------------------------------------------------------------------
-// Column norms.  part[chunk][g] = sum over the chunk's 256 k of |x|^2 in a
-// fixed order (four k groups per workgroup, added in order), scaled by
-// 2^(-2 pe[chunk][g]); pe is 0 unless the chunk holds magnitudes whose
-// squares would leave FP64's range.  The final kernel adds the chunks in
-// order and sets emax[g] = E + 1 with ||x_g|| < 2^E: the scale 2^(c - emax)
-// takes the norm below 2^(c-1).  emax = INT_MIN for a zero column, INT_MAX
-// for one that is not finite.  Bound by reading the operands once: 64
-// columns x 256 k per workgroup and one launch for all operands keep enough
-// loads in flight also at a thousand G+k (norms and residues of an 8-atom
-// k-point, K = 1936, G = 1166, 9 moduli: 294 -> 75 us).
+// Column norms: partial sums of |x|^2, then per column their sum and
+// emax[g] = E + 1 with ||x_g|| < 2^E: the scale 2^(c - emax) takes the norm
+// below 2^(c-1).  emax = INT_MIN for a zero column, INT_MAX for one that is
+// not finite.  bt writes the partial sums of X and B from the values it holds
+// (a pass of their own read both operands again: 0.79 of 26 ms at 64 atoms, 7
+// moduli); the kernel below does it for operands that bt has not seen (O
+// alone, (1+h1)A): part[chunk][g] over 256 k in a fixed order (four k groups
+// per workgroup, added in order).  A partial sum whose squares would leave
+// FP64's range is marked kNormRecompute, and the final kernel then sums that
+// column again from scaled values.
 // ---------------------------------------------------------------------------
 constexpr int OZ_NCH = 256;      // k per partial sum
-constexpr int OZ_LO = -400, OZ_HI = 400;  // exponents whose squares are safe
-
-__device__ __forceinline__ int exponent_of(double a) {  // of a normal |a|; -1023 for 0
-  return (int)((__double_as_longlong(a) >> 52) & 0x7ff) - 1023;
-}
 
 __device__ __forceinline__ void colnorm_part_body(const OzK &d, int z) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = blockIdx.x * 64 + lane;
   const int k0 = blockIdx.y * OZ_NCH, k1 = min(d.Ktot, k0 + OZ_NCH);
-  if (z >= d.nops || (int)blockIdx.x * 64 >= d.ngp || k0 >= k1) return;  // uniform
+  if (z >= d.nops || (d.fused >> z & 1) || (int)blockIdx.x * 64 >= d.ngp || k0 >= k1)
+    return;  // uniform
   const EXH_G double2 *xp = gptr(d.x[z]) + min(g, d.ngp - 1);
   const long long ldx = d.ld[z];
   EXH_G double *part = gptr(d.part[z]);
-  __shared__ double ss[4][64];
-  __shared__ int sm[4][64];
+  __shared__ double ss[4][64], sm[4][64];
   double s = 0.0, amax = 0.0;
 #pragma unroll 8
   for (int k = k0 + w; k < k1; k += 4) {
@@ -206,48 +201,58 @@ __device__ __forceinline__ void colnorm_part_body(const OzK &d, int z) {
     amax = fmax(amax, fmax(fabs(v.x), fabs(v.y)));
   }
   ss[w][lane] = s;
-  sm[w][lane] = exponent_of(amax);
-  __syncthreads();
-  int e = max(max(sm[0][lane], sm[1][lane]), max(sm[2][lane], sm[3][lane]));
-  const bool rescale = e < OZ_LO || (e > OZ_HI && e < 1024);
-  if (__any(rescale)) {  // rare: squares out of range, sum the scaled values
-    e = rescale ? (e == -1023 ? -1022 : e) : 0;
-    s = 0.0;
-    for (int k = k0 + w; k < k1; k += 4) {
-      const double2 v = ld(xp + (size_t)k * ldx);
-      const double a = ldexp(v.x, -e), b = ldexp(v.y, -e);
-      s = fma(a, a, s);
-      s = fma(b, b, s);
-    }
-    __syncthreads();
-    ss[w][lane] = s;
-  } else {
-    e = 0;
-  }
+  sm[w][lane] = amax;
   __syncthreads();
   if (w == 0 && g < d.ngp) {
+    amax = fmax(fmax(sm[0][lane], sm[1][lane]), fmax(sm[2][lane], sm[3][lane]));
     part[(size_t)blockIdx.y * d.ldp + g] =
         ((ss[0][lane] + ss[1][lane]) + ss[2][lane]) + ss[3][lane];
-    ((EXH_G int *)(part + (size_t)d.nch * d.ldp))[(size_t)blockIdx.y * d.ldp + g] = e;
+    ((EXH_G int *)(part + (size_t)d.nch[z] * d.ldp))[(size_t)blockIdx.y * d.ldp + g] =
+        norm_mark(amax);
   }
 }
 
+// 64 columns per workgroup, the chunks split over four waves.
 __device__ __forceinline__ void colnorm_final_body(const OzK &d, int z) {
-  const int g = blockIdx.x * 64 + threadIdx.x;
-  if (z >= d.nops || g >= d.ngp) return;
-  const int nch = d.nch, ldp = d.ldp;
-  const EXH_G double *part = gptr((const double *)d.part[z]);
-  const EXH_G int *pe = (const EXH_G int *)(part + (size_t)nch * ldp);
-  int em = -5000;  // running exponent of the sum s 2^(2 em)
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int g = blockIdx.x * 64 + lane;
+  if (z >= d.nops || (int)blockIdx.x * 64 >= d.ngp) return;  // uniform
+  const int nch = d.nch[z], ldp = d.ldp, gc = min(g, d.ngp - 1);
+  const EXH_G double *part = gptr((const double *)d.part[z]) + gc;
+  const EXH_G int *pe = (const EXH_G int *)(gptr((const double *)d.part[z]) + (size_t)nch * ldp) + gc;
+  __shared__ double ss[4][64];
+  __shared__ int sm[4][64];
+  const int per = (nch + 3) / 4, c0 = w * per, c1 = min(nch, c0 + per);
   double s = 0.0;
+  int mark = 0;
 #pragma unroll 8
-  for (int c = 0; c < nch; c++) {
-    const double v = part[(size_t)c * ldp + g];
-    const int ec = v == 0.0 ? em : pe[(size_t)c * ldp + g], m = max(em, ec);
-    s = ldexp(s, 2 * (em - m)) + ldexp(v, 2 * (ec - m));
-    em = m;
+  for (int c = c0; c < c1; c++) {
+    s += part[(size_t)c * ldp];
+    mark |= pe[(size_t)c * ldp];
   }
-  int e = INT_MIN;
+  ss[w][lane] = s;
+  sm[w][lane] = mark;
+  __syncthreads();
+  if (w != 0 || g >= d.ngp) return;
+  s = ((ss[0][lane] + ss[1][lane]) + ss[2][lane]) + ss[3][lane];
+  int em = 0, e = INT_MIN;
+  if (sm[0][lane] | sm[1][lane] | sm[2][lane] | sm[3][lane]) {
+    // rare: squares out of range; the column again, scaled by its largest entry
+    const EXH_G double2 *xp = gptr(d.x[z]) + g;
+    double amax = 0.0;
+    for (int k = 0; k < d.Ktot; k++) {
+      const double2 v = ld(xp + (size_t)k * d.ld[z]);
+      amax = fmax(amax, fmax(fabs(v.x), fabs(v.y)));
+    }
+    em = min(max(exponent_of(amax), -1022), 1023);
+    s = 0.0;
+    for (int k = 0; k < d.Ktot; k++) {
+      const double2 v = ld(xp + (size_t)k * d.ld[z]);
+      const double a = ldexp(v.x, -em), b = ldexp(v.y, -em);
+      s = fma(a, a, s);
+      s = fma(b, b, s);
+    }
+  }
   if (!(s - s == 0.0)) {
     e = INT_MAX;  // Inf or NaN in the column
   } else if (s > 0.0) {
@@ -280,8 +285,7 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int kb = blockIdx.y;
   const int ngp = d.ngp, Ktot = d.Ktot;
-  // rows up to the last row panel this k-point uses
-  const int rows = (ngp + OZ_R - 1) / OZ_R * OZ_R;
+  const int rows = d.nt * OZ_T;  // whole tiles
   if (z >= d.nops || g >= rows || kb >= d.nslab * (OZ_KS / 16)) return;
   const EXH_G double2 *X = gptr(d.x[z]);
   const long long ldx = d.ld[z];
@@ -519,8 +523,10 @@ __device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc) {
     for (int u = 0; u < OZ_WR; u++) {
       const int ci = w * OZ_WR + u;
       const int kk = ci / RC, rc = ci - RC * kk;
+      // the last panel may reach past the padded rows: any rows, not stored
+      const int row = min(I0 + rc * 64, Gpad - 64);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, EXH_LDS(&st[kk][rc * 64]), 16, voff,
-                                               (kk * Gpad + I0 + rc * 64) * 16, 0, 0);
+                                               (kk * Gpad + row) * 16, 0, 0);
     }
     const int kk = w >> 1, rc = w & 1;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rH, EXH_LDS(&st[kk][OZ_R + rc * 64]), 16, voff,
@@ -745,10 +751,10 @@ __global__ __launch_bounds__(256) void colnorm_part_grouped_kernel(const OzK *__
                                                                    int nops) {
   colnorm_part_body(kd[blockIdx.z / nops], blockIdx.z % nops);
 }
-__global__ __launch_bounds__(64) void colnorm_final_kernel(OzK d) {
+__global__ __launch_bounds__(256) void colnorm_final_kernel(OzK d) {
   colnorm_final_body(d, blockIdx.z);
 }
-__global__ __launch_bounds__(64) void colnorm_final_grouped_kernel(const OzK *__restrict__ kd,
+__global__ __launch_bounds__(256) void colnorm_final_grouped_kernel(const OzK *__restrict__ kd,
                                                                    int nops) {
   colnorm_final_body(kd[blockIdx.z / nops], blockIdx.z % nops);
 }
@@ -808,25 +814,34 @@ OzPlan oz_fp64() {
   return P;
 }
 
-OzLayout oz_layout(int ngkmax, int Ktot, const OzPlan &P, bool only_o, bool third) {
+OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o) {
   OzLayout L;
-  // rows padded to 384: a multiple of the row panel and of the 128-column
-  // blocks, so every panel and column block loads inside it
-  constexpr int GA = 384;
-  static_assert(GA % OZ_R == 0 && GA % OZ_T == 0, "row padding");
-  L.Gpad = (ngkmax + GA - 1) / GA * GA;
+  const int ngkmax = c->ngkmax, Ktot = c->Ktot;
+  L.Gpad = (ngkmax + OZ_T - 1) / OZ_T * OZ_T;
   L.Kpad = (Ktot + 2 * OZ_KS - 1) / (2 * OZ_KS) * (2 * OZ_KS);  // an even number of stages
   L.qstride = (size_t)L.Kpad * L.Gpad;
   const long long nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
   L.q_bytes = (size_t)P.nmod * 2 * L.qstride;
   L.r_bytes = (size_t)(only_o ? 2 : 4) * P.nmod * (nt * (nt + 1) / 2) * OZ_T * OZ_T;
-  // per operand: the column exponents, then the partial norms and theirs
-  const size_t ng = std::max(ngkmax, 1), nch = (Ktot + OZ_NCH - 1) / OZ_NCH;
+  // per operand: the column exponents, then the partial norms and their marks
+  const size_t ng = std::max(ngkmax, 1);
+  const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
+  L.nch = std::max((Ktot + OZ_NCH - 1) / OZ_NCH, c->natmtot * rows);
   L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
-  L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * nch * ng + 255) / 256 * 256;
-  L.nops = 1 + (only_o ? 0 : 1) + (third ? 1 : 0);
+  L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * L.nch * ng + 255) / 256 * 256;
+  L.nops = 1 + (only_o ? 0 : 1) + (c->have_h1aa ? 1 : 0);
   L.panels = 2 * P.nmod * (only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt));
   return L;
+}
+
+NormOut norm_out(const OzK &d) {
+  NormOut n;
+  n.x = d.part[0];
+  n.b = d.part[d.iB];
+  n.ld = d.ldp;
+  n.nx = d.nch[0];
+  n.nb = d.nch[d.iB];
+  return n;
 }
 
 OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
@@ -842,7 +857,6 @@ OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
   d.nmod = P.nmod;
   d.bits = P.bits;
   d.ldp = std::max(c->ngkmax, 1);
-  d.nch = (c->Ktot + OZ_NCH - 1) / OZ_NCH;
   d.qstride = L.qstride;
   d.q_bytes = w.chunk * 2 * L.qstride;
   d.q = w.q;
@@ -858,6 +872,11 @@ OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
     if (z == 1) d.iB = n;
     if (z == 2) d.iY = n;
     char *e = (char *)w.e + (size_t)n * L.e_bytes;
+    // X and B: left by bt, per atom and per atom and 64 rows (norm_out)
+    const bool fused = h && z < 2;
+    const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
+    d.fused |= fused ? 1u << n : 0u;
+    d.nch[n] = !fused ? (c->Ktot + OZ_NCH - 1) / OZ_NCH : c->natmtot * (z == 1 ? rows : 1);
     d.x[n] = src[z];
     d.ld[n] = z == 0 ? ldx : ldb;
     d.e[n] = (int *)e;
@@ -877,8 +896,9 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
   int ngp = 0, nch = 0, nops = 0, kb = 0, nt = 0;
   for (int i = 0; i < n; i++) {
     ngp = std::max(ngp, d[i].ngp);
-    nch = std::max(nch, d[i].nch);
     nops = std::max(nops, d[i].nops);
+    for (int z = 0; z < d[i].nops; z++)  // chunks of operands bt has not summed
+      if (!(d[i].fused >> z & 1)) nch = std::max(nch, d[i].nch[z]);
     kb = std::max(kb, d[i].nslab * (OZ_KS / 16));
     nt = std::max(nt, d[i].nt);
   }
@@ -887,16 +907,16 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
   if (stage_mask & 1) {
     const dim3 gp(cdiv(ngp, 64), nch, nz), gf(cdiv(ngp, 64), 1, nz);
     if (kd) {
-      hipLaunchKernelGGL(colnorm_part_grouped_kernel, gp, dim3(256), 0, s, kd, nops);
-      hipLaunchKernelGGL(colnorm_final_grouped_kernel, gf, dim3(64), 0, s, kd, nops);
+      if (nch) hipLaunchKernelGGL(colnorm_part_grouped_kernel, gp, dim3(256), 0, s, kd, nops);
+      hipLaunchKernelGGL(colnorm_final_grouped_kernel, gf, dim3(256), 0, s, kd, nops);
     } else {
-      hipLaunchKernelGGL(colnorm_part_kernel, gp, dim3(256), 0, s, d[0]);
-      hipLaunchKernelGGL(colnorm_final_kernel, gf, dim3(64), 0, s, d[0]);
+      if (nch) hipLaunchKernelGGL(colnorm_part_kernel, gp, dim3(256), 0, s, d[0]);
+      hipLaunchKernelGGL(colnorm_final_kernel, gf, dim3(256), 0, s, d[0]);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const dim3 gr(cdiv((long long)cdiv(ngp, OZ_R) * OZ_R, 256), kb, nz);
+  const dim3 gr(cdiv(nt * OZ_T, 256), kb, nz);
   const long long per = only_o ? oz_panels<true>(nt) : oz_panels<false>(nt);
   for (int m0 = 0; m0 < nmod; m0 += chunk) {
     const int m1 = std::min(nmod, m0 + chunk);

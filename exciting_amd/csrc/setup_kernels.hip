@@ -36,6 +36,7 @@ constexpr int TK = 8;
 // same order
 constexpr int TKH = 8;
 constexpr int NTH = 256;  // 4 waves; wave w owns a 32x32 quadrant
+static_assert(kNormRows == TM, "one partial norm of B per bt tile");
 
 // ---------------------------------------------------------------------------
 // ivg(:, igpig(i)) for the G+k set; w = 0 flags an igpig outside 1..ngrtot.
@@ -126,29 +127,62 @@ __global__ void pack_grouped_kernel(const KDesc *__restrict__ kd) {
 // ---------------------------------------------------------------------------
 // Bt = (aa . A)^T per atom:  Bt[Koff+f][G] = sum_f' A^T[G][f'] aa(f, f')
 // (hamiltonsetup.f90:75-88, zm = aa * apwi).  X holds A^T K-major with
-// leading dimension ldx.  Grid (G tiles, f tiles, atoms).
+// leading dimension ldx.  Grid (G tiles of TG, f tiles of 64, atoms).  Bound
+// by FP64 MFMA at large bases (5.2 ms at 64 atoms: 57 of 78.6 TFLOP/s, f padded
+// from 242 to 256), by the chain of slabs at small ones.  For the modular
+// contraction it also leaves the partial column norms of both operands
+// (`norms`): X from the first f tile's slabs, B from the accumulators, so
+// neither is read again for them; the order of the sums does not depend on TG.
+// bt + residues with and without: 2 atoms 62 -> 48 us, 8 atoms x 8 k-points 1.28
+// -> 1.12 ms, 16 x 8 6.5 -> 6.0 ms, 64 atoms (7 moduli) 7.2 -> 7.0 ms.
 // ---------------------------------------------------------------------------
-template <typename PX, typename PB, typename PAA = const double2 *>
+// x of the lane N below, within each row of 16 lanes: a register move (through
+// LDS the reductions below cost 1 % of the kernel)
+template <int N>
+__device__ __forceinline__ double row_ror(double x) {
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)v, 0x120 + N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), 0x120 + N, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int TG, typename PX, typename PB, typename PAA = const double2 *>
 __device__ __forceinline__ void bt_body(
     int ias, int I0, int F0, int ngp, PX __restrict__ X, long long ldx,
     const int *__restrict__ Koff, const int *__restrict__ Ms,
-    PAA __restrict__ aa, int maxaa, PB __restrict__ bt, int ldb) {
+    PAA __restrict__ aa, int maxaa, PB __restrict__ bt, int ldb, const NormOut &norms) {
+  constexpr int NA = TG / 32;     // 16-row MFMA blocks per wave
+  constexpr int RX = NTH / TG;    // slab rows loaded per pass
+  constexpr int QX = TK / RX, QY = TK / 4;
   const int M = Ms[ias];
-  if (F0 >= M || I0 >= ngp) return;
+  if (I0 >= ngp) return;
+  const bool want = norms.x != nullptr;
+  const int chunk = F0 / TM, nF = (maxaa + TM - 1) / TM;
+  if (F0 >= M) {  // a chunk this atom does not have
+    const int i = I0 + (int)threadIdx.x;
+    if (want && (int)threadIdx.x < TG && i < ngp) {
+      const size_t e = (size_t)(ias * nF + chunk) * norms.ld + i;
+      gptr(norms.b)[e] = 0.0;
+      ((EXH_G int *)(gptr(norms.b) + (size_t)norms.nb * norms.ld))[e] = 0;
+    }
+    return;
+  }
   const int koff = Koff[ias];
   const PAA aat = aa + (size_t)ias * maxaa * maxaa;
 
-  __shared__ double sXr[TK][TM + 16], sXi[TK][TM + 16], sYr[TK][TM + 16], sYi[TK][TM + 16];
+  // [buffer][re, im][k][row]
+  __shared__ double sX[2][2][TK][TG + 16], sY[2][2][TK][TM + 16];
+  __shared__ double sN[4][2][TG];  // norms: {sum, largest} per wave
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wr = w >> 1, wc = w & 1, lr = lane & 15, lk = lane >> 4;
-  const int ii = tid & 63, kq = tid >> 6;
-  const bool vi = I0 + ii < ngp, vf = F0 + ii < M;
-  const PX xp = X + (size_t)koff * ldx + (vi ? I0 + ii : ngp - 1);
-  const PAA yp = aat + (vf ? F0 + ii : M - 1);
+  const int ix = tid % TG, kx = tid / TG, iy = tid & 63, ky = tid >> 6;
+  const bool vi = I0 + ix < ngp, vf = F0 + iy < M;
+  const PX xp = X + (size_t)koff * ldx + (vi ? I0 + ix : ngp - 1);
+  const PAA yp = aat + (vf ? F0 + iy : M - 1);
 
-  dx4 cre[2][2], cim[2][2];
+  dx4 cre[NA][2], cim[NA][2];
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int a = 0; a < NA; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++) {
       cre[a][b] = dx4{0, 0, 0, 0};
@@ -157,50 +191,67 @@ __device__ __forceinline__ void bt_body(
 
   // the validity factors are applied at the LDS store, after the slab's
   // MFMAs, so the prefetch loads stay in flight meanwhile
-  constexpr int QB = TK / 4;  // slab rows per thread (4 row groups of 64 threads)
-  double2 px[QB], py[QB];
-  double fxv[QB], fyv[QB];
+  double2 px[QX], py[QY];
+  double fxv[QX], fyv[QY];
   auto load = [&](int kb) {
 #pragma unroll
-    for (int q = 0; q < QB; q++) {
-      const int k = kb + kq + 4 * q;
-      const bool kv = k < M;
-      const int kc = kv ? k : M - 1;
-      px[q] = ld(xp + (size_t)kc * ldx);
-      py[q] = ld(yp + (size_t)maxaa * kc);
-      fxv[q] = (kv && vi) ? 1.0 : 0.0;
-      fyv[q] = (kv && vf) ? 1.0 : 0.0;
+    for (int q = 0; q < QX; q++) {
+      const int k = kb + kx + RX * q;
+      px[q] = ld(xp + (size_t)min(k, M - 1) * ldx);
+      fxv[q] = (k < M && vi) ? 1.0 : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < QY; q++) {
+      const int k = kb + ky + 4 * q;
+      py[q] = ld(yp + (size_t)maxaa * min(k, M - 1));
+      fyv[q] = (k < M && vf) ? 1.0 : 0.0;
     }
   };
-  load(0);
-  for (int kb = 0; kb < M; kb += TK) {
+  auto store = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < QB; q++) {
-      const int kk = kq + 4 * q;
-      sXr[kk][ii] = fxv[q] * px[q].x;
-      sXi[kk][ii] = fxv[q] * px[q].y;
-      sYr[kk][ii] = fyv[q] * py[q].x;
-      sYi[kk][ii] = fyv[q] * py[q].y;
+    for (int q = 0; q < QX; q++) {
+      const int kk = kx + RX * q;
+      sX[buf][0][kk][ix] = fxv[q] * px[q].x;
+      sX[buf][1][kk][ix] = fxv[q] * px[q].y;
     }
-    __syncthreads();
-    if (kb + TK < M) load(kb + TK);
+#pragma unroll
+    for (int q = 0; q < QY; q++) {
+      const int kk = ky + 4 * q;
+      sY[buf][0][kk][iy] = fyv[q] * py[q].x;
+      sY[buf][1][kk][iy] = fyv[q] * py[q].y;
+    }
+  };
+  // wave w sums rows 2w and 2w + 1 of every slab
+  const bool sumx = want && F0 == 0 && lane < TG;
+  double nx = 0.0, mx = 0.0;
+  auto compute = [&](int buf) {
+    if (sumx) {
+#pragma unroll
+      for (int u = 0; u < TK / 4; u++) {
+        const int kk = TK / 4 * w + u;
+        const double r = sX[buf][0][kk][lane], i = sX[buf][1][kk][lane];
+        nx = fma(r, r, nx);
+        nx = fma(i, i, nx);
+        mx = fmax(mx, fmax(fabs(r), fabs(i)));
+      }
+    }
 #pragma unroll
     for (int k4 = 0; k4 < TK / 4; k4++) {
       const int kk = 4 * k4 + lk;
-      double xr[2], xi[2], nxi[2], yr[2], yi[2];
+      double xr[NA], xi[NA], nxi[NA], yr[2], yi[2];
 #pragma unroll
-      for (int a = 0; a < 2; a++) {
-        xr[a] = sXr[kk][wr * 32 + a * 16 + lr];
-        xi[a] = sXi[kk][wr * 32 + a * 16 + lr];
+      for (int a = 0; a < NA; a++) {
+        xr[a] = sX[buf][0][kk][wr * (TG / 2) + a * 16 + lr];
+        xi[a] = sX[buf][1][kk][wr * (TG / 2) + a * 16 + lr];
         nxi[a] = -xi[a];
       }
 #pragma unroll
       for (int b = 0; b < 2; b++) {
-        yr[b] = sYr[kk][wc * 32 + b * 16 + lr];
-        yi[b] = sYi[kk][wc * 32 + b * 16 + lr];
+        yr[b] = sY[buf][0][kk][wc * 32 + b * 16 + lr];
+        yi[b] = sY[buf][1][kk][wc * 32 + b * 16 + lr];
       }
 #pragma unroll
-      for (int a = 0; a < 2; a++)
+      for (int a = 0; a < NA; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++) {
           cre[a][b] = mfma(xr[a], yr[b], cre[a][b]);
@@ -209,39 +260,104 @@ __device__ __forceinline__ void bt_body(
           cim[a][b] = mfma(xi[a], yr[b], cim[a][b]);
         }
     }
+  };
+  // double-buffered slabs, one barrier each, as in ho_tile; loads past the
+  // last slab are clamped and zero-weighted
+  const int nslab = (M + TK - 1) / TK;
+  load(0);
+  store(0);
+  __syncthreads();
+  load(TK);
+  for (int sl = 0; sl < nslab; sl++) {
+    compute(sl & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    store((sl + 1) & 1);
+    load((sl + 2) * TK);
     __syncthreads();
   }
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int a = 0; a < NA; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        int i = I0 + wr * 32 + a * 16 + lk + 4 * r;
+        int i = I0 + wr * (TG / 2) + a * 16 + lk + 4 * r;
         int f = F0 + wc * 32 + b * 16 + lr;
         if (i < ngp && f < M)
           st(bt + (size_t)(koff + f) * ldb + i, z2(cre[a][b][r], cim[a][b][r]));
       }
+  if (!want) return;
+  if (F0 == 0) {
+    if (sumx) {
+      sN[w][0][lane] = nx;
+      sN[w][1][lane] = mx;
+    }
+    __syncthreads();
+    if (tid < TG && I0 + tid < ngp) {
+      const size_t e = (size_t)ias * norms.ld + I0 + tid;
+      gptr(norms.x)[e] = ((sN[0][0][tid] + sN[1][0][tid]) + sN[2][0][tid]) + sN[3][0][tid];
+      ((EXH_G int *)(gptr(norms.x) + (size_t)norms.nx * norms.ld))[e] =
+          norm_mark(fmax(fmax(sN[0][1][tid], sN[1][1][tid]), fmax(sN[2][1][tid], sN[3][1][tid])));
+    }
+    __syncthreads();
+  }
+  // |B|^2 over this tile's rows: the lane's two blocks, the 16 lanes of a row
+  // block, then the two wave columns (f >= M holds zeros)
+#pragma unroll
+  for (int a = 0; a < NA; a++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      double s = 0.0, m = 0.0;
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        s = fma(cre[a][b][r], cre[a][b][r], s);
+        s = fma(cim[a][b][r], cim[a][b][r], s);
+        m = fmax(m, fmax(fabs(cre[a][b][r]), fabs(cim[a][b][r])));
+      }
+      s += row_ror<8>(s);
+      s += row_ror<4>(s);
+      s += row_ror<2>(s);
+      s += row_ror<1>(s);
+      m = fmax(m, row_ror<8>(m));
+      m = fmax(m, row_ror<4>(m));
+      m = fmax(m, row_ror<2>(m));
+      m = fmax(m, row_ror<1>(m));
+      if (lr == 0) {
+        const int i = wr * (TG / 2) + a * 16 + lk + 4 * r;
+        sN[wc][0][i] = s;
+        sN[wc][1][i] = m;
+      }
+    }
+  __syncthreads();
+  if (tid < TG && I0 + tid < ngp) {
+    const size_t e = (size_t)(ias * nF + chunk) * norms.ld + I0 + tid;
+    gptr(norms.b)[e] = sN[0][0][tid] + sN[1][0][tid];
+    ((EXH_G int *)(gptr(norms.b) + (size_t)norms.nb * norms.ld))[e] =
+        norm_mark(fmax(sN[0][1][tid], sN[1][1][tid]));
+  }
 }
 
+template <int TG>
 __global__ __launch_bounds__(NTH) void bt_kernel(
     int ngp, const double2 *__restrict__ X, long long ldx,
     const int *__restrict__ Koff, const int *__restrict__ Ms,
-    const double2 *__restrict__ aa, int maxaa, double2 *__restrict__ bt, int ldb) {
-  bt_body(blockIdx.z, blockIdx.x * TM, blockIdx.y * TM, ngp, X, ldx, Koff, Ms, aa, maxaa, bt,
-          ldb);
+    const double2 *__restrict__ aa, int maxaa, double2 *__restrict__ bt, int ldb,
+    NormOut norms) {
+  bt_body<TG>(blockIdx.z, blockIdx.x * TG, blockIdx.y * TM, ngp, X, ldx, Koff, Ms, aa, maxaa, bt,
+              ldb, norms);
 }
 
 // Grouped: blockIdx.z = ias + natmax * (k-point), natmax the largest atom
 // count of the group's structures.
+template <int TG>
 __global__ __launch_bounds__(NTH) void bt_grouped_kernel(const KDesc *__restrict__ kd,
                                                          int natmax) {
   const int k = blockIdx.z / natmax, ias = blockIdx.z - k * natmax;
   const KDesc &d = kd[k];
   const SDesc &S = *d.sd;
-  if (ias >= S.natmtot) return;
-  bt_body(ias, blockIdx.x * TM, blockIdx.y * TM, d.ngp, gptr(d.x), S.ldx, S.Koff, S.Ms,
-          gptr(S.aa), S.maxaa, gptr(d.bt), S.ldb);
+  if (ias >= S.natmtot || (int)blockIdx.y * TM >= (S.maxaa + TM - 1) / TM * TM) return;
+  bt_body<TG>(ias, blockIdx.x * TG, blockIdx.y * TM, d.ngp, gptr(d.x), S.ldx, S.Koff, S.Ms,
+              gptr(S.aa), S.maxaa, gptr(d.bt), S.ldb, d.norms);
 }
 
 // ---------------------------------------------------------------------------
@@ -863,15 +979,25 @@ const double2 *k_major_operand(const exh_context *c, const double2 *apwalm, cons
   return k_major_view(c, apwalm, at, ld);
 }
 
+// 32-row tiles while 64-row ones are too few to even out over 256 CUs: K = 242,
+// G = 146 (12 tiles of 64) 55 -> 34 us, K = 1452, G = 874 (336) 84 -> 74, K = 1936,
+// G = 1175 (608) 113-120 -> 112; from 640 on (4 k-points of G = 579) no gain.
+static bool bt_small(long long tiles64) { return tiles64 < 640; }
+
 hipError_t launch_bt(hipStream_t s, const exh_context *c, int ngp,
-                     const double2 *apwalm, const double2 *at, double2 *bt, int ldb) {
+                     const double2 *apwalm, const double2 *at, double2 *bt, int ldb,
+                     const NormOut &norms) {
   if (ngp <= 0 || c->natmtot <= 0) return hipSuccess;
   long long ldx;
   const double2 *X = k_major_view(c, apwalm, at, &ldx);
-  dim3 grid(cdiv(ngp, TM), cdiv(c->maxaa, TM), c->natmtot);
-  hipLaunchKernelGGL(bt_kernel, grid, dim3(NTH), 0, s, ngp, X, ldx,
-                     (const int *)c->katom.p, (const int *)c->katom.p + c->natmtot,
-                     (const double2 *)c->aa.p, c->maxaa, bt, ldb);
+  const int nf = (int)cdiv(c->maxaa, TM);
+  const int *Koff = (const int *)c->katom.p, *Ms = Koff + c->natmtot;
+#define EXH_BT(TG)                                                                           \
+  hipLaunchKernelGGL(bt_kernel<TG>, dim3(cdiv(ngp, TG), nf, c->natmtot), dim3(NTH), 0, s, ngp, \
+                     X, ldx, Koff, Ms, (const double2 *)c->aa.p, c->maxaa, bt, ldb, norms)
+  if (bt_small((long long)cdiv(ngp, 64) * nf * c->natmtot)) EXH_BT(32);
+  else EXH_BT(64);
+#undef EXH_BT
   return hipGetLastError();
 }
 
@@ -1056,8 +1182,13 @@ hipError_t launch_pack_grouped(hipStream_t s, const GroupDims &g, const KDesc *k
 
 hipError_t launch_bt_grouped(hipStream_t s, const GroupDims &g, const KDesc *kd) {
   if (g.nk <= 0 || g.ngpmax <= 0 || g.natmax <= 0) return hipSuccess;
-  dim3 grid(cdiv(g.ngpmax, TM), cdiv(g.maxaa, TM), g.natmax * g.nk);
-  hipLaunchKernelGGL(bt_grouped_kernel, grid, dim3(NTH), 0, s, kd, g.natmax);
+  const int nf = (int)cdiv(g.maxaa, TM);
+#define EXH_BT(TG)                                                                            \
+  hipLaunchKernelGGL(bt_grouped_kernel<TG>, dim3(cdiv(g.ngpmax, TG), nf, g.natmax * g.nk),    \
+                     dim3(NTH), 0, s, kd, g.natmax)
+  if (bt_small((long long)cdiv(g.ngpmax, 64) * nf * g.natmax * g.nk)) EXH_BT(32);
+  else EXH_BT(64);
+#undef EXH_BT
   return hipGetLastError();
 }
 
