@@ -214,9 +214,9 @@ struct exh_context {
   bool gvec_full = false;  // G set = the whole FFT box, ivgig inverse of ivg
   // muffin-tin table producer (hmlint): apwfr on the device, species and
   // Gaunt tables, spline weights, radial integrals, host-API staging
-  exh::DevBuf apwfr_d, hml_fl, hml_arow, hml_lrow, hml_count, hml_gstart, hml_glm2, hml_gval;
+  exh::DevBuf apwfr_d, hml_fl, hml_arow, hml_lrow, hml_count, hml_gcount, hml_chunk, hml_glm2, hml_gval;
   exh::DevBuf hml_w, hml_spr, hml_ipot, hml_ikin, hml_vin, hml_loin, hml_aa, hml_loa, hml_lolo;
-  int hml_lmaxvr = -1;
+  int hml_lmaxvr = -1, hml_nchunk = 0;
   exh::DevBuf so_dt, so_rowb, so_pairs, so_pstart, so_host;   // mt_so
   long long so_radial_epoch = -1, so_basis_epoch = -1;
   long long radial_epoch = 0, basis_epoch = 0, hml_radial_epoch = -1, hml_basis_epoch = -1;

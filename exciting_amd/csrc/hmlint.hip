@@ -14,11 +14,12 @@
 //             integral of fderiv.f90 (m = -1) with spline.f90 is linear in
 //             the integrand, so it is a weighted sum with per-species
 //             weights computed once on the host by applying that rule to unit
-//             vectors.  Radial functions and a slab of potential channels are
-//             staged in LDS per chunk of grid points.
-//   contract  one table element per thread: the sum over the Gaunt list of
-//             (lm1, lm3) of coefficient x radial integral, plus the kinetic
-//             integral when lm1 = lm3, in the reference's order.
+//             vectors.  The potential's integrals are then one product per
+//             atom, (pairs x points) (points x lm), on FP64 MFMA.
+//   contract  one element of the tables per thread and kChunkAtoms atoms: the
+//             sum over the Gaunt list of (lm1, lm3) of coefficient x radial
+//             integral, plus the kinetic integral when lm1 = lm3, in the
+//             reference's order.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -28,27 +29,35 @@
 namespace exh {
 namespace {
 
-constexpr int kRC = 32;        // grid points per LDS chunk
-constexpr int kCH = 8;         // potential channels (lm) per workgroup
-constexpr int kNfMax = 63;     // radial functions per atom (APW + LO)
-constexpr int kThreads = 256;    // contraction kernel
-constexpr int kRadThreads = 384; // radial kernel: one pair per thread up to 27 functions
+constexpr int kRC = 32;         // grid points per LDS chunk
+constexpr int kNfMax = 63;      // radial functions per atom (APW + LO)
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / 64;
+constexpr int kKinBlocks = 4;   // workgroups per atom of the kinetic integrals
+constexpr int kLF = kRC + 2;    // LDS row of one function: 2 mod 32 doubles, so
+                                // that 16 functions x 2 points hit 32 banks
+constexpr int kChunkAtoms = 4;  // atoms of one species per contraction thread
+
+typedef double dx4 __attribute__((ext_vector_type(4)));
 
 struct HmlArgs {
-  int nf, nfa, p, lmaxapw, nrmtmax, nlomax, lmmaxvr, nchunk;
+  int nf, nfa, p, lmaxapw, nrmtmax, nlomax, lmmaxvr;
+  int nkin, npg;  // kinetic blocks per atom; groups of kWaves pair tiles per atom
   double zora;   // alpha^2/2 when a mass factor is applied (mt_kin.f90:55-59)
   int kmass;     // kinetic mass factor on APW-APW pairs (1) / pairs with an LO (2)
 };
 
-__device__ __forceinline__ double radial_value(const HmlArgs &a, const double *__restrict__ apwfr,
-                                               const double *__restrict__ lofr, int ias, int f,
-                                               int ir, int k) {
+// radial function f of atom ias: u (k = 0) or its derivative term (k = 1)
+__device__ __forceinline__ const double *radial_ptr(const HmlArgs &a,
+                                                    const double *__restrict__ apwfr,
+                                                    const double *__restrict__ lofr, int ias,
+                                                    int f, int k) {
   if (f < a.nfa) {
     const int l = f / a.p, io = f - l * a.p;
-    return apwfr[ir + (size_t)a.nrmtmax *
-                          (k + 2 * (io + (size_t)a.p * (l + (size_t)(a.lmaxapw + 1) * ias)))];
+    return apwfr + (size_t)a.nrmtmax *
+                       (k + 2 * (io + (size_t)a.p * (l + (size_t)(a.lmaxapw + 1) * ias)));
   }
-  return lofr[ir + (size_t)a.nrmtmax * (k + 2 * ((f - a.nfa) + (size_t)a.nlomax * ias))];
+  return lofr + (size_t)a.nrmtmax * (k + 2 * ((f - a.nfa) + (size_t)a.nlomax * ias));
 }
 
 // pair t of the upper triangle (f1 <= f2) of nf functions
@@ -60,129 +69,157 @@ __device__ __forceinline__ void pair_of(int t, int &f1, int &f2) {
   f1 = t - b * (b + 1) / 2;
 }
 
-// blockIdx.x = atom, blockIdx.y = potential slab (lm0 = y * kCH) or, for
-// y == nchunk, the kinetic integrals.  ipot[ias][f1][f2][lm], ikin[ias][f1][f2],
-// both written for (f1,f2) and (f2,f1).
-template <int PPT>
-__global__ __launch_bounds__(kRadThreads) void hml_radial_kernel(
+// Kinetic integrals ikin[ias][f1][f2] of mt_kin.f90, both orders: one wave per
+// pair of equal l, its lanes over the grid points; zero for the other pairs.
+__device__ __forceinline__ void kinetic_body(const HmlArgs &a, int ias, int is, int nr, int block,
+                                             int nblocks, const double *__restrict__ wts,
+                                             const double *__restrict__ spr,
+                                             const int *__restrict__ fl,
+                                             const double *__restrict__ apwfr,
+                                             const double *__restrict__ lofr,
+                                             const double *__restrict__ veffmt,
+                                             double *__restrict__ ikin) {
+  const int lane = threadIdx.x & 63, npair = a.nf * (a.nf + 1) / 2;
+  const double y00 = 0.28209479177387814347;
+  for (int t = block * kWaves + (threadIdx.x >> 6); t < npair; t += nblocks * kWaves) {
+    int f1, f2;
+    pair_of(t, f1, f2);
+    const int l = fl[is * kNfMax + f1];
+    double v = 0.0;
+    if (l == fl[is * kNfMax + f2]) {
+      const double lfac = (double)(l * (l + 1));
+      const bool mass = a.kmass & (f2 >= a.nfa ? 2 : 1);   // f1 <= f2
+      const double *u1 = radial_ptr(a, apwfr, lofr, ias, f1, 0), *d1 = u1 + a.nrmtmax;
+      const double *u2 = radial_ptr(a, apwfr, lofr, ias, f2, 0), *d2 = u2 + a.nrmtmax;
+#pragma unroll 4
+      for (int ir = lane; ir < nr; ir += 64) {
+        const double x = spr[ir + (size_t)a.nrmtmax * is];
+        const double w = 0.5 * wts[ir + (size_t)a.nrmtmax * is];
+        double k = w * (d1[ir] * d2[ir] * (x * x) + lfac * (u1[ir] * u2[ir]));
+        if (mass) {
+          const double v00 = veffmt[(size_t)a.lmmaxvr * (ir + (size_t)a.nrmtmax * ias)];
+          k *= 1.0 / (1.0 - a.zora * v00 * y00);
+        }
+        v += k;
+      }
+      for (int m = 32; m; m >>= 1) v += __shfl_xor(v, m);
+    }
+    if (lane == 0) {
+      ikin[((size_t)ias * a.nf + f1) * a.nf + f2] = v;
+      ikin[((size_t)ias * a.nf + f2) * a.nf + f1] = v;
+    }
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void hml_kinetic_kernel(
+    HmlArgs a, const int *__restrict__ atom_species, const int *__restrict__ nrmt,
+    const double *__restrict__ wts, const double *__restrict__ spr,
+    const int *__restrict__ fl, const double *__restrict__ apwfr,
+    const double *__restrict__ lofr, const double *__restrict__ veffmt,
+    double *__restrict__ ikin) {
+  const int ias = blockIdx.x, is = atom_species[ias];
+  kinetic_body(a, ias, is, nrmt[is], blockIdx.y, gridDim.y, wts, spr, fl, apwfr, lofr, veffmt,
+               ikin);
+}
+
+// blockIdx.x = atom; blockIdx.y < nkin: kinetic integrals; then lm group (LT
+// tiles of 16 channels) x pair group (kWaves tiles of 16 pairs, one per wave).
+// ipot[ias][pair][lm], pairs f1 <= f2 as pair_of numbers them.
+//
+// With a pair per thread this was bound by LDS (5 words for 8 FMA) and by
+// uncoalesced staging; as a product P(pair, r) V(r, lm) with P = f1 f2 w r^2 formed in registers
+// from three LDS words, an MFMA of 1024 FMA needs one word of V per lane.  The next chunk's global reads are in flight while a chunk is
+// multiplied; the two LDS buffers leave one barrier per chunk.  64 atoms, 22
+// functions, 250 points, 81 channels: 113 -> 48 us, 10 of them the kinetic
+// workgroups (a wave per pair instead of a thread: the products of a wave's 64
+// points need no LDS); 16 us at the FP64 matrix rate, the rest latency of eight
+// short chunks at two workgroups per CU.
+template <int LT>
+__global__ __launch_bounds__(kThreads) void hml_radial_kernel(
     HmlArgs a, const int *__restrict__ atom_species, const int *__restrict__ nrmt,
     const double *__restrict__ wts, const double *__restrict__ spr,
     const int *__restrict__ fl, const double *__restrict__ apwfr,
     const double *__restrict__ lofr, const double *__restrict__ veffmt,
     double *__restrict__ ipot, double *__restrict__ ikin) {
-  __shared__ double sF[kRC][kNfMax + 1];
-  __shared__ double sD[kRC][kNfMax + 1];
-  __shared__ double sV[kRC][kCH];
-  __shared__ double sW[kRC], sR2[kRC], sRM[kRC];
+  constexpr int NL = 16 * LT;                       // channels: 16 mod 32 doubles
+  constexpr int NFI = (kNfMax * kRC + kThreads - 1) / kThreads;
+  constexpr int NVI = kRC * NL / kThreads;
+  extern __shared__ double hml_lds[];
   const int ias = blockIdx.x, is = atom_species[ias], nr = nrmt[is];
-  const bool kin = (int)blockIdx.y == a.nchunk;
-  const int lm0 = blockIdx.y * kCH;
+  if ((int)blockIdx.y < a.nkin) {
+    kinetic_body(a, ias, is, nr, blockIdx.y, a.nkin, wts, spr, fl, apwfr, lofr, veffmt, ikin);
+    return;
+  }
+  const int y = blockIdx.y - a.nkin, lm0 = y / a.npg * NL;
   const int nf = a.nf, npair = nf * (nf + 1) / 2, tid = threadIdx.x;
-  const double y00 = 0.28209479177387814347;
-  double acc[PPT][kCH];
+  const int lane = tid & 63, row = lane & 15, kq = lane >> 4;
+  const int t0 = (y % a.npg * kWaves + (tid >> 6)) * 16;
+  const int bufsz = nf * kLF + kRC * NL + kRC;
+  int f1 = 0, f2 = 0;
+  if (t0 + row < npair) pair_of(t0 + row, f1, f2);
+
+  // staging: thread tid brings point tid % kRC of functions tid / kRC + 8 i,
+  // and channels lm of points r, r * NL + lm = tid + kThreads * i
+  const int fr = tid % kRC, ff = tid / kRC;
+  const double *fp[NFI];
 #pragma unroll
-  for (int q = 0; q < PPT; q++)
+  for (int i = 0; i < NFI; i++)
+    fp[i] = radial_ptr(a, apwfr, lofr, ias, min(ff + i * (kThreads / kRC), nf - 1), 0);
+  const double *vp = veffmt + (size_t)a.lmmaxvr * a.nrmtmax * ias;
+  const double *wp = wts + (size_t)a.nrmtmax * is, *xp = spr + (size_t)a.nrmtmax * is;
+  double gf[NFI], gv[NVI], gw = 0.0, gx = 0.0;
+  auto load = [&](int r0) {
 #pragma unroll
-    for (int k = 0; k < kCH; k++) acc[q][k] = 0.0;
-  int pf1[PPT], pf2[PPT];
-  double lfac[PPT];
+    for (int i = 0; i < NFI; i++)
+      if (i * (kThreads / kRC) < nf) gf[i] = r0 + fr < nr ? fp[i][r0 + fr] : 0.0;
 #pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    const int t = tid + q * kRadThreads;
-    pf1[q] = pf2[q] = 0;
-    lfac[q] = 0.0;
-    if (t < npair) {
-      pair_of(t, pf1[q], pf2[q]);
-      const int l = fl[is * kNfMax + pf1[q]];
-      lfac[q] = (double)(l * (l + 1));
+    for (int i = 0; i < NVI; i++) {
+      const int e = tid + kThreads * i, ir = r0 + e / NL, lm = lm0 + e % NL;
+      gv[i] = ir < nr && lm < a.lmmaxvr ? vp[(size_t)a.lmmaxvr * ir + lm] : 0.0;
     }
-  }
-  for (int r0 = 0; r0 < nr; r0 += kRC) {
-    for (int i = tid; i < kRC * nf; i += kRadThreads) {
-      const int r = i / nf, f = i - r * nf, ir = r0 + r;
-      sF[r][f] = ir < nr ? radial_value(a, apwfr, lofr, ias, f, ir, 0) : 0.0;
-      if (kin) sD[r][f] = ir < nr ? radial_value(a, apwfr, lofr, ias, f, ir, 1) : 0.0;
+    if (tid < kRC) {
+      gw = r0 + tid < nr ? wp[r0 + tid] : 0.0;
+      gx = r0 + tid < nr ? xp[r0 + tid] : 0.0;
     }
-    if (kin) {
-      for (int r = tid; r < kRC; r += kRadThreads) {
-        const int ir = r0 + r;
-        double w = 0.0, r2 = 0.0, rm = 1.0;
-        if (ir < nr) {
-          const double x = spr[ir + (size_t)a.nrmtmax * is];
-          r2 = x * x;
-          w = 0.5 * wts[ir + (size_t)a.nrmtmax * is];
-          if (a.kmass) {
-            const double v00 = veffmt[(size_t)a.lmmaxvr * (ir + (size_t)a.nrmtmax * ias)];
-            rm = 1.0 / (1.0 - a.zora * v00 * y00);
-          }
-        }
-        sW[r] = w;
-        sR2[r] = r2;
-        sRM[r] = rm;
-      }
-    } else {
-      for (int i = tid; i < kRC * kCH; i += kRadThreads) {
-        const int r = i / kCH, k = i - r * kCH, ir = r0 + r, lm = lm0 + k;
-        sV[r][k] = (ir < nr && lm < a.lmmaxvr)
-                       ? veffmt[lm + (size_t)a.lmmaxvr * (ir + (size_t)a.nrmtmax * ias)]
-                       : 0.0;
-      }
-      for (int r = tid; r < kRC; r += kRadThreads) {
-        const int ir = r0 + r;
-        double w = 0.0;
-        if (ir < nr) {
-          const double x = spr[ir + (size_t)a.nrmtmax * is];
-          w = wts[ir + (size_t)a.nrmtmax * is] * (x * x);
-        }
-        sW[r] = w;
-      }
+  };
+  auto store = [&](double *buf) {
+#pragma unroll
+    for (int i = 0; i < NFI; i++) {
+      const int f = ff + i * (kThreads / kRC);
+      if (f < nf) buf[f * kLF + fr] = gf[i];
     }
+#pragma unroll
+    for (int i = 0; i < NVI; i++) buf[nf * kLF + tid + kThreads * i] = gv[i];
+    if (tid < kRC) buf[nf * kLF + kRC * NL + tid] = gw * (gx * gx);
+  };
+  dx4 acc[LT];
+#pragma unroll
+  for (int j = 0; j < LT; j++) acc[j] = {0.0, 0.0, 0.0, 0.0};
+  load(0);
+  int b = 0;
+  for (int r0 = 0; r0 < nr; r0 += kRC, b ^= 1) {
+    double *buf = hml_lds + b * bufsz;
+    store(buf);       // last read two chunks ago, before the barrier in between
     __syncthreads();
+    if (r0 + kRC < nr) load(r0 + kRC);
+    const double *s1 = buf + f1 * kLF + kq, *s2 = buf + f2 * kLF + kq;
+    const double *sv = buf + nf * kLF + kq * NL + row, *sw = buf + nf * kLF + kRC * NL + kq;
 #pragma unroll
-    for (int q = 0; q < PPT; q++) {
-      if (tid + q * kRadThreads >= npair) continue;
-      const int f1 = pf1[q], f2 = pf2[q];
-      if (kin) {  // acc[q][0]: plain, acc[q][1]: with the mass factor
-        double s0 = acc[q][0], s1 = acc[q][1];
-        for (int r = 0; r < kRC; r++) {
-          const double t =
-              sW[r] * (sD[r][f1] * sD[r][f2] * sR2[r] + lfac[q] * (sF[r][f1] * sF[r][f2]));
-          s0 += t;
-          s1 += t * sRM[r];
-        }
-        acc[q][0] = s0;
-        acc[q][1] = s1;
-      } else {
-        for (int r = 0; r < kRC; r++) {
-          const double pr = sF[r][f1] * sF[r][f2] * sW[r];
+    for (int r = 0; r < kRC; r += 4) {
+      const double p = s1[r] * s2[r] * sw[r];
 #pragma unroll
-          for (int k = 0; k < kCH; k++) acc[q][k] += pr * sV[r][k];
-        }
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    if (tid + q * kRadThreads >= npair) continue;
-    const int f1 = pf1[q], f2 = pf2[q];
-    if (kin) {
-      const bool same = fl[is * kNfMax + f1] == fl[is * kNfMax + f2];
-      const bool lo = f1 >= a.nfa || f2 >= a.nfa;
-      const bool mass = a.kmass & (lo ? 2 : 1);
-      const double v = same ? (mass ? acc[q][1] : acc[q][0]) : 0.0;
-      ikin[((size_t)ias * nf + f1) * nf + f2] = v;
-      ikin[((size_t)ias * nf + f2) * nf + f1] = v;
-    } else {
-#pragma unroll
-      for (int k = 0; k < kCH; k++) {
-        const int lm = lm0 + k;
-        if (lm >= a.lmmaxvr) break;
-        ipot[(((size_t)ias * nf + f1) * nf + f2) * a.lmmaxvr + lm] = acc[q][k];
-        ipot[(((size_t)ias * nf + f2) * nf + f1) * a.lmmaxvr + lm] = acc[q][k];
-      }
+      for (int j = 0; j < LT; j++)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(p, sv[r * NL + 16 * j], acc[j], 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int j = 0; j < LT; j++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int t = t0 + kq + 4 * q, lm = lm0 + 16 * j + row;
+      if (t < npair && lm < a.lmmaxvr)
+        ipot[((size_t)ias * npair + t) * a.lmmaxvr + lm] = acc[j][q];
+    }
 }
 
 // Rows of one table kind per species: int2 {lm (0-based), radial function}.
@@ -192,42 +229,94 @@ struct RowTable {
   int ld;
 };
 
+// One of aa (APW x APW), loa (LO x APW), lolo (LO x LO); its blocks are
+// blockIdx.x = block0 .. up to the next part's.
+struct ConPart {
+  RowTable r, c;
+  int ldo, nco, block0;
+  double2 *out;
+};
+struct ConArgs {
+  ConPart part[3];
+  int nparts;
+};
+
 // out(i, j, ias) (+)= [lm_i == lm_j] kin(f_i, f_j) + sum_t g_t ipot(f_i, f_j, lm2_t)
-// over the Gaunt list of (lm_i, lm_j): aa (APW x APW), loa (LO x APW) and
-// lolo (LO x LO) of mt_kin.f90:173-226 and mt_pot.f90:227-311.
+// over the Gaunt list of (lm_i, lm_j) (mt_kin.f90:173-226, mt_pot.f90:227-311),
+// for the atoms of chunk blockIdx.y: {first, count, species}.  Entry t of the
+// lists lies at [t][lm_j][lm_i], so that the lanes (consecutive i) read
+// consecutive entries; each entry read serves all atoms of the chunk.  64 atoms,
+// aa of order 162: 112 us with the lists one after the other, a thread per
+// element and atom and a launch per table, 48 us now; 31 MB are written (8 us),
+// the gathers of the integrals (about 30 lines each) bound it.
 __global__ __launch_bounds__(kThreads) void hml_contract_kernel(
-    int nf, int lmmaxvr, int lmmaxmat, const int *__restrict__ atom_species, RowTable R,
-    RowTable C, int ldo, int nco, const int *__restrict__ gstart, const int *__restrict__ glm2,
+    int nf, int lmmaxvr, int lmmaxmat, const int4 *__restrict__ chunks, ConArgs P,
+    const int *__restrict__ gcount, const int *__restrict__ glm2,
     const double2 *__restrict__ gval, const double *__restrict__ ipot,
-    const double *__restrict__ ikin, double2 *__restrict__ out, int accumulate, int with_kin) {
-  const int ias = blockIdx.y;
-  const long long e = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (e >= (long long)ldo * nco) return;
-  const int i = (int)(e % ldo), j = (int)(e / ldo);
-  const int is = atom_species[ias];
-  double2 *o = out + (size_t)i + (size_t)ldo * (j + (size_t)nco * ias);
-  double re = 0.0, im = 0.0;
-  if (accumulate) {
-    re = o->x;
-    im = o->y;
+    const double *__restrict__ ikin, int accumulate, int with_kin) {
+  int k = 0;
+  while (k + 1 < P.nparts && (int)blockIdx.x >= P.part[k + 1].block0) k++;
+  const RowTable R = P.part[k].r, C = P.part[k].c;
+  const int ldo = P.part[k].ldo, nco = P.part[k].nco;
+  const unsigned e = (blockIdx.x - P.part[k].block0) * kThreads + threadIdx.x;
+  if (e >= (unsigned)(ldo * nco)) return;
+  const int4 ch = chunks[blockIdx.y];
+  const int ias = ch.x, na = ch.y, is = ch.z;
+  const int j = e / (unsigned)ldo, i = e - j * ldo;
+  const size_t so = (size_t)ldo * nco;
+  double2 *o = P.part[k].out + (size_t)i + (size_t)ldo * j + so * ias;
+  double re[kChunkAtoms], im[kChunkAtoms];
+#pragma unroll
+  for (int q = 0; q < kChunkAtoms; q++) {
+    re[q] = im[q] = 0.0;
+    if (accumulate && q < na) {
+      const double2 z = o[so * q];
+      re[q] = z.x;
+      im[q] = z.y;
+    }
   }
   if (i < R.count[is] && j < C.count[is]) {
     const int2 ri = R.rows[is * R.ld + i], cj = C.rows[is * C.ld + j];
-    const size_t base = ((size_t)ias * nf + ri.y) * nf + cj.y;
-    if (with_kin && ri.x == cj.x) re += ikin[base];
-    double zr = 0.0, zi = 0.0;
-    const int q = ri.x * lmmaxmat + cj.x;
-    const double *ip = ipot + base * lmmaxvr;
-    for (int t = gstart[q]; t < gstart[q + 1]; t++) {
-      const double v = ip[glm2[t]];
-      const double2 g = gval[t];
-      zr += g.x * v;
-      zi += g.y * v;
+    if (with_kin && ri.x == cj.x) {
+#pragma unroll
+      for (int q = 0; q < kChunkAtoms; q++)
+        if (q < na) re[q] += ikin[((size_t)(ias + q) * nf + ri.y) * nf + cj.y];
     }
-    re += zr;
-    im += zi;
+    const int f1 = min(ri.y, cj.y), f2 = max(ri.y, cj.y), npair = nf * (nf + 1) / 2;
+    const size_t sa = (size_t)npair * lmmaxvr, nq = (size_t)lmmaxmat * lmmaxmat;
+    const double *ip[kChunkAtoms];   // atoms beyond the chunk repeat its last
+#pragma unroll
+    for (int q = 0; q < kChunkAtoms; q++)
+      ip[q] = ipot + sa * (ias + min(q, na - 1)) + (size_t)(f2 * (f2 + 1) / 2 + f1) * lmmaxvr;
+    const size_t g0 = (size_t)cj.x * lmmaxmat + ri.x;
+    const int n = gcount[g0];
+    double zr[kChunkAtoms] = {}, zi[kChunkAtoms] = {};
+    // the next entry is read while this one's integrals are on their way
+    int lm = n ? glm2[g0] : 0;
+    double2 g = n ? gval[g0] : make_double2(0.0, 0.0);
+    for (int t = 0; t < n; t++) {
+      double v[kChunkAtoms];
+#pragma unroll
+      for (int q = 0; q < kChunkAtoms; q++) v[q] = ip[q][lm];
+      const size_t e = min(t + 1, n - 1) * nq + g0;
+      const double2 gt = g;
+      lm = glm2[e];
+      g = gval[e];
+#pragma unroll
+      for (int q = 0; q < kChunkAtoms; q++) {
+        zr[q] += gt.x * v[q];
+        zi[q] += gt.y * v[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kChunkAtoms; q++) {
+      re[q] += zr[q];
+      im[q] += zi[q];
+    }
   }
-  *o = make_double2(re, im);
+#pragma unroll
+  for (int q = 0; q < kChunkAtoms; q++)
+    if (q < na) o[so * q] = make_double2(re[q], im[q]);
 }
 
 // ---- host-side tables --------------------------------------------------
@@ -402,26 +491,41 @@ int prepare(exh_context *c, int lmaxvr) {
     }
     lcount[is] = nl;
   }
-  // Gaunt list: for lm1, then lm3 (both <= lmmaxmat), the lm2 <= lmmaxvr with a
-  // nonzero coefficient, in increasing lm2 (the order of init1.f90:592-609)
-  std::vector<int> gstart((size_t)lmmaxmat * lmmaxmat + 1), glm2;
+  // Gaunt lists: for (lm1, lm3), both <= lmmaxmat, the lm2 <= lmmaxvr with a
+  // nonzero coefficient, in increasing lm2 (the order of init1.f90:592-609);
+  // entry t of every list at [t][lm3][lm1]
+  const size_t nq = (size_t)lmmaxmat * lmmaxmat;
+  std::vector<int> gcount(nq, 0), glm2;
   std::vector<double2> gval;
   for (int l1 = 0; l1 <= lmaxmat; l1++)
     for (int m1 = -l1; m1 <= l1; m1++)
       for (int l3 = 0; l3 <= lmaxmat; l3++)
         for (int m3 = -l3; m3 <= l3; m3++) {
-          gstart[(size_t)(l1 * (l1 + 1) + m1) * lmmaxmat + l3 * (l3 + 1) + m3] = (int)glm2.size();
+          const size_t q = (size_t)(l3 * (l3 + 1) + m3) * lmmaxmat + l1 * (l1 + 1) + m1;
           for (int l2 = 0; l2 <= lmaxvr; l2++)
             for (int m2 = -l2; m2 <= l2; m2++) {
               double re, im;
               gaunt_real_middle(l1, l2, l3, m1, m2, m3, &re, &im);
               if (std::sqrt(re * re + im * im) > 1e-20) {
-                glm2.push_back(l2 * (l2 + 1) + m2);
-                gval.push_back(make_double2(re, im));
+                const size_t e = nq * gcount[q]++ + q;
+                if (e >= glm2.size()) {
+                  glm2.resize(nq * gcount[q]);
+                  gval.resize(nq * gcount[q]);
+                }
+                glm2[e] = l2 * (l2 + 1) + m2;
+                gval[e] = make_double2(re, im);
               }
             }
         }
-  gstart.back() = (int)glm2.size();
+  // chunks of atoms of one species: {first atom, atoms, species}
+  std::vector<int4> chunks;
+  for (int is = 0, ias = 0; is < ns; is++)
+    for (int left = c->natoms[is]; left > 0;) {
+      const int n = std::min(left, kChunkAtoms);
+      chunks.push_back(make_int4(ias, n, is, 0));
+      ias += n;
+      left -= n;
+    }
   // spline weights per species
   std::vector<double> w((size_t)c->nrmtmax * ns, 0.0);
   for (int is = 0; is < ns; is++) {
@@ -443,13 +547,15 @@ int prepare(exh_context *c, int lmaxvr) {
   counts.insert(counts.end(), lcount.begin(), lcount.end());
   counts.insert(counts.end(), sp_int.begin(), sp_int.end());
   if (!rc) rc = put(c->hml_count, counts.data(), counts.size() * sizeof(int));
-  if (!rc) rc = put(c->hml_gstart, gstart.data(), gstart.size() * sizeof(int));
+  if (!rc) rc = put(c->hml_gcount, gcount.data(), gcount.size() * sizeof(int));
+  if (!rc) rc = put(c->hml_chunk, chunks.data(), chunks.size() * sizeof(int4));
   if (!rc) rc = put(c->hml_glm2, glm2.data(), std::max<size_t>(glm2.size(), 1) * sizeof(int));
   if (!rc) rc = put(c->hml_gval, gval.data(), std::max<size_t>(gval.size(), 1) * sizeof(double2));
   if (!rc) rc = put(c->hml_w, w.data(), w.size() * sizeof(double));
   std::vector<double> spr(c->spr_h);
   if (!rc) rc = put(c->hml_spr, spr.data(), spr.size() * sizeof(double));
   if (rc) return rc;
+  c->hml_nchunk = (int)chunks.size();
   c->hml_lmaxvr = lmaxvr;
   c->hml_radial_epoch = c->radial_epoch;
   c->hml_basis_epoch = c->basis_epoch;
@@ -660,29 +766,29 @@ static int hmlint_impl(exh_context *c, void *stream, int lmaxvr, const double *v
   if (int rc = prepare(c, lmaxvr)) return rc;
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   const int p = c->apwordmax, nfa = (c->lmaxmat + 1) * p, nf = nfa + c->nlomax;
-  const int lmmaxvr = (lmaxvr + 1) * (lmaxvr + 1), nchunk = (lmmaxvr + kCH - 1) / kCH;
+  const int lmmaxvr = (lmaxvr + 1) * (lmaxvr + 1), npair = nf * (nf + 1) / 2;
   const int natm = c->natmtot, mnlo = std::max(c->maxnlo, 1);
-  int rc = ensure(c, c->hml_ipot, (size_t)natm * nf * nf * lmmaxvr * sizeof(double));
+  int rc = ensure(c, c->hml_ipot, (size_t)natm * npair * lmmaxvr * sizeof(double));
   if (!rc) rc = ensure(c, c->hml_ikin, (size_t)natm * nf * nf * sizeof(double));
   if (rc) return rc;
   const double alpha = 1.0 / 137.03599911;
-  HmlArgs a{nf, nfa, p, c->lmaxapw, c->nrmtmax, std::max(c->nlomax, 1), lmmaxvr, nchunk,
-            0.5 * alpha * alpha, valence_rel_none ? 0 : 3};
+  const int npg = cdiv_ll(npair, 16 * kWaves), ntile = cdiv_ll(lmmaxvr, 16);
+  HmlArgs a{nf, nfa, p, c->lmaxapw, c->nrmtmax, std::max(c->nlomax, 1), lmmaxvr,
+            with_kin ? kKinBlocks : 0, npg, 0.5 * alpha * alpha, valence_rel_none ? 0 : 3};
   const int *counts = (const int *)c->hml_count.p;
-  const int npair = nf * (nf + 1) / 2;
   const double *lf = lofr ? lofr : (const double *)c->hml_w.p;  // never read when nlomax = 0
   hipError_t e = timed(c, EXH_K_HMLRAD, s, [&] {
-    dim3 grid(natm, nchunk + (with_kin ? 1 : 0));
-#define LAUNCH(P)                                                                               \
-  hipLaunchKernelGGL(hml_radial_kernel<P>, grid, dim3(kRadThreads), 0, s, a,                       \
+#define LAUNCH(LT)                                                                              \
+  hipLaunchKernelGGL(hml_radial_kernel<LT>, dim3(natm, a.nkin + npg * cdiv_ll(ntile, LT)),      \
+                     dim3(kThreads), 2 * (nf * kLF + kRC * 16 * LT + kRC) * sizeof(double), s, a,     \
                      (const int *)c->atom_species_d.p, counts + 2 * c->nspecies,                \
                      (const double *)c->hml_w.p, (const double *)c->hml_spr.p,                  \
                      (const int *)c->hml_fl.p, (const double *)c->apwfr_d.p, lf, veffmt,        \
                      (double *)c->hml_ipot.p, (double *)c->hml_ikin.p)
-    if (npair <= kRadThreads) LAUNCH(1);
-    else if (npair <= 2 * kRadThreads) LAUNCH(2);
-    else if (npair <= 4 * kRadThreads) LAUNCH(4);
-    else LAUNCH(8);
+    // three channel tiles per wave share one P; single tiles while those would
+    // leave some of the 256 CUs without a workgroup
+    if (natm * npg * cdiv_ll(ntile, 3) >= 256) LAUNCH(3);
+    else LAUNCH(1);
 #undef LAUNCH
     return hipGetLastError();
   });
@@ -690,26 +796,23 @@ static int hmlint_impl(exh_context *c, void *stream, int lmaxvr, const double *v
   const int lmmaxmat = (c->lmaxmat + 1) * (c->lmaxmat + 1);
   RowTable A{(const int2 *)c->hml_arow.p, counts, c->maxaa};
   RowTable L{(const int2 *)c->hml_lrow.p, counts + c->nspecies, mnlo};
-  struct Part {
-    RowTable r, col;
-    int ldo, nco;
-    exh_z *out;
-  } parts[3] = {{A, A, c->maxaa, c->maxaa, aa}, {L, A, mnlo, c->maxaa, loa}, {L, L, mnlo, mnlo, lolo}};
-  const int nparts = c->nlomax > 0 ? 3 : 1;
+  ConArgs P{{{A, A, c->maxaa, c->maxaa, 0, (double2 *)aa},
+             {L, A, mnlo, c->maxaa, 0, (double2 *)loa},
+             {L, L, mnlo, mnlo, 0, (double2 *)lolo}},
+            c->nlomax > 0 ? 3 : 1};
+  int blocks = 0;
+  for (int k = 0; k < P.nparts; k++) {
+    P.part[k].block0 = blocks;
+    blocks += cdiv_ll((long long)P.part[k].ldo * P.part[k].nco, kThreads);
+  }
   e = timed(c, EXH_K_HMLCON, s, [&] {
-    hipError_t le = hipSuccess;
-    for (int k = 0; k < nparts && le == hipSuccess; k++) {
-      const Part &P = parts[k];
-      dim3 grid(cdiv_ll((long long)P.ldo * P.nco, kThreads), natm);
-      hipLaunchKernelGGL(hml_contract_kernel, grid, dim3(kThreads), 0, s, nf, lmmaxvr, lmmaxmat,
-                         (const int *)c->atom_species_d.p, P.r, P.col, P.ldo, P.nco,
-                         (const int *)c->hml_gstart.p, (const int *)c->hml_glm2.p,
-                         (const double2 *)c->hml_gval.p, (const double *)c->hml_ipot.p,
-                         (const double *)c->hml_ikin.p, (double2 *)P.out,
-                         (flags & EXH_ACCUMULATE) ? 1 : 0, with_kin ? 1 : 0);
-      le = hipGetLastError();
-    }
-    return le;
+    hipLaunchKernelGGL(hml_contract_kernel, dim3(blocks, c->hml_nchunk), dim3(kThreads), 0, s, nf,
+                       lmmaxvr, lmmaxmat, (const int4 *)c->hml_chunk.p, P,
+                       (const int *)c->hml_gcount.p, (const int *)c->hml_glm2.p,
+                       (const double2 *)c->hml_gval.p, (const double *)c->hml_ipot.p,
+                       (const double *)c->hml_ikin.p, (flags & EXH_ACCUMULATE) ? 1 : 0,
+                       with_kin ? 1 : 0);
+    return hipGetLastError();
   });
   if (e == hipSuccess) e = mark_done(c, s);
   return e == hipSuccess ? 0 : hip_fail(c, e, "hmlint contract");
@@ -744,25 +847,16 @@ int exh_mt_kinetic_device(exh_context *c, void *stream, int lmaxvr, const double
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   const int p = c->apwordmax, nfa = (c->lmaxmat + 1) * p, nf = nfa + c->nlomax;
   const double alpha = 1.0 / 137.03599911;
-  HmlArgs a{nf, nfa, p, c->lmaxapw, c->nrmtmax, std::max(c->nlomax, 1), (lmv + 1) * (lmv + 1), 0,
-            0.5 * alpha * alpha, mass_flags};
+  HmlArgs a{nf, nfa, p, c->lmaxapw, c->nrmtmax, std::max(c->nlomax, 1), (lmv + 1) * (lmv + 1),
+            kKinBlocks, 0, 0.5 * alpha * alpha, mass_flags};
   const int *counts = (const int *)c->hml_count.p;
-  const int npair = nf * (nf + 1) / 2;
   const double *lf = lofr ? lofr : (const double *)c->hml_w.p;  // never read when nlomax = 0
   const double *vm = veffmt ? veffmt : (const double *)c->hml_w.p;  // read only with a mass flag
   hipError_t e = timed(c, EXH_K_HMLRAD, s, [&] {
-    dim3 grid(c->natmtot, 1);
-#define LAUNCH(P)                                                                               \
-  hipLaunchKernelGGL(hml_radial_kernel<P>, grid, dim3(kRadThreads), 0, s, a,                    \
-                     (const int *)c->atom_species_d.p, counts + 2 * c->nspecies,                \
-                     (const double *)c->hml_w.p, (const double *)c->hml_spr.p,                  \
-                     (const int *)c->hml_fl.p, (const double *)c->apwfr_d.p, lf, vm,            \
-                     (double *)nullptr, tkin)
-    if (npair <= kRadThreads) LAUNCH(1);
-    else if (npair <= 2 * kRadThreads) LAUNCH(2);
-    else if (npair <= 4 * kRadThreads) LAUNCH(4);
-    else LAUNCH(8);
-#undef LAUNCH
+    hipLaunchKernelGGL(hml_kinetic_kernel, dim3(c->natmtot, kKinBlocks), dim3(kThreads), 0, s, a,
+                       (const int *)c->atom_species_d.p, counts + 2 * c->nspecies,
+                       (const double *)c->hml_w.p, (const double *)c->hml_spr.p,
+                       (const int *)c->hml_fl.p, (const double *)c->apwfr_d.p, lf, vm, tkin);
     return hipGetLastError();
   });
   if (e == hipSuccess) e = mark_done(c, s);
