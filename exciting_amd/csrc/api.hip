@@ -541,7 +541,7 @@ void exh_destroy(exh_context *c) {
                     &c->ivg, &c->ivgig, &c->ist, &c->cf_stage, &c->vf_stage, &c->mf_stage,
                     &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->ozq, &c->ozr, &c->oze, &c->s_apwalm, &c->s_igpig,
                     &c->s_vgpc, &c->s_h, &c->s_o, &c->s_gpc, &c->s_tpgpc, &c->s_sfac,
-                    &c->bbt, &c->bat, &c->ba2t, &c->bivgk, &c->ifz, &c->igeo, &c->i_in0,
+                    &c->bbt, &c->bat, &c->ba2t, &c->bivgk, &c->ifz, &c->igeo, &c->iphase, &c->i_in0,
                     &c->i_in1, &c->i_out0, &c->i_out1, &c->i_out2, &c->apwfr_d, &c->hml_fl,
                     &c->hml_arow, &c->hml_lrow, &c->hml_count, &c->hml_gcount, &c->hml_chunk, &c->hml_glm2,
                     &c->hml_gval, &c->hml_w, &c->hml_spr, &c->hml_ipot, &c->hml_ikin,

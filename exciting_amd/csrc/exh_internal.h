@@ -207,8 +207,9 @@ struct exh_context {
   exh::DevBuf ivg, ivgig, ist;  // ist: IstEntry per box point
   exh::DevBuf cf_stage, vf_stage, mf_stage, m2_stage;
   // interstitial producers: FFT work arrays (up to 3 grids), geometry,
-  // host-API staging, and hipFFT plans per batch count 1..3 (opaque here)
-  exh::DevBuf ifz, igeo, i_in0, i_in1, i_out0, i_out1, i_out2;
+  // and phase tables, host-API staging, and hipFFT plans (opaque here): complex
+  // for one grid, real-to-complex for 1..3 grids
+  exh::DevBuf ifz, igeo, iphase, i_in0, i_in1, i_out0, i_out1, i_out2;
   void *fft_plan[4] = {nullptr, nullptr, nullptr, nullptr};
   int fft_grid[3] = {0, 0, 0};
   bool gvec_full = false;  // G set = the whole FFT box, ivgig inverse of ivg

@@ -31,63 +31,123 @@ struct CfunArgs {
   double epslat;
   double damp;   // cfdamp / gmaxvr, 0 = no damping
   int n1, n2, n3;
+  int lo[3];    // the box holds i_d = lo_d .. lo_d + n_d - 1
+  int off[3];   // -lo_d mod n_d
   int nspecies;
 };
 
-__device__ __forceinline__ int fft_index(int i1, int i2, int i3, int n1, int n2, int n3) {
-  const int j1 = i1 >= 0 ? i1 : n1 + i1;
-  const int j2 = i2 >= 0 ? i2 : n2 + i2;
-  const int j3 = i3 >= 0 ? i3 : n3 + i3;
-  return (j3 * n2 + j2) * n1 + j1;
+// position in the box of FFT index j along one axis
+__device__ __forceinline__ int box_index(int j, int off, int n) {
+  return j + off < n ? j + off : j + off - n;
 }
 
-// gencfun.f90:120-157 for one G vector per thread, then :70 (scatter of the
-// undamped value to its grid point) and :76-82 (damping of cfunig).  geo
-// holds per species {rmt, first atom, end atom} followed by atposc(3,natmtot)
-// in species-major order; its reads are uniform across the wave.
-__global__ __launch_bounds__(256) void cfunig_kernel(int ng, const int *__restrict__ ivg,
-                                                     CfunArgs a,
+// Phase tables of gencfun.f90:150-155: exp(-i G.tau) is the product over the
+// three axes of exp(-i i_d b_d.tau), so the sine and cosine are taken for
+// natm (n1 + n2 + n3) arguments instead of natm n1 n2 n3.  tab[atom][j], j the
+// FFT index along axis 1, then 2, then 3.  The argument is held in two words
+// (b_d.tau to twice the working precision, then the integer multiple), so that
+// an entry is good to an ulp however large the phase is.
+__global__ __launch_bounds__(256) void phase_table_kernel(CfunArgs a, int natm,
+                                                          const double *__restrict__ geo,
+                                                          double2 *__restrict__ tab) {
+  const int nt = a.n1 + a.n2 + a.n3, e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= natm * nt) return;
+  const int ia = e / nt, j = e - ia * nt;
+  const int d = j < a.n1 ? 0 : j < a.n1 + a.n2 ? 1 : 2;
+  const int n = d == 0 ? a.n1 : d == 1 ? a.n2 : a.n3;
+  const int jd = j - (d == 0 ? 0 : d == 1 ? a.n1 : a.n1 + a.n2);
+  const double i = a.lo[d] + box_index(jd, a.off[d], n);
+  const double *tau = geo + 3 * a.nspecies + 3 * ia;
+  double hi = 0.0, low = 0.0;   // b_d . tau
+  for (int k = 0; k < 3; k++) {
+    const double p = a.b[3 * d + k] * tau[k], ep = fma(a.b[3 * d + k], tau[k], -p);
+    const double s = hi + p, v = s - hi;
+    low += (hi - (s - v)) + (p - v) + ep;
+    hi = s;
+  }
+  const double ph = i * hi, dl = fma(i, hi, -ph) + i * low;
+  double s, c;
+  sincos(ph, &s, &c);
+  tab[e] = make_double2(c - s * dl, -(s + c * dl));
+}
+
+// gencfun.f90:120-157, then :70 (the undamped value at its grid point) and
+// :76-82 (damping of cfunig).  One thread per (j1, j2) of the grid and kRows
+// consecutive j3: per atom the phase of (j1, j2) is formed once, and each row
+// costs one complex multiply-add with a factor that the whole wave shares.
+// geo holds per species {rmt, first atom, end atom}, then the positions.
+// Per grid point and atom 4 FMA and 4/kRows (10 us for 64 atoms on 80^3), bound
+// by the latency of the tables' loads at two waves per SIMD: 93 us with a sincos
+// per G vector and atom, 34 now with 2 to 4 rows, 44 with 8; error of cfunig
+// against extended precision 4.7e-15 -> 3e-17 (relative norm).
+constexpr int kRows = 4;
+__global__ __launch_bounds__(256) void cfunig_kernel(CfunArgs a, const int *__restrict__ ivgig,
                                                      const double *__restrict__ geo,
+                                                     const double2 *__restrict__ tab,
                                                      double2 *__restrict__ cfunig,
                                                      double2 *__restrict__ zfft) {
-  const int ig = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ig >= ng) return;
-  const int i1 = ivg[3 * ig], i2 = ivg[3 * ig + 1], i3 = ivg[3 * ig + 2];
-  const double d1 = i1, d2 = i2, d3 = i3;
-  double v[3];
+  const int plane = a.n1 * a.n2, q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j30 = blockIdx.y * kRows, nt = a.n1 + a.n2 + a.n3;
+  if (q >= plane) return;
+  const int j2 = q / a.n1, j1 = q - j2 * a.n1;
+  const int b1 = box_index(j1, a.off[0], a.n1), b2 = box_index(j2, a.off[1], a.n2);
+  const int i1 = a.lo[0] + b1, i2 = a.lo[1] + b2;
+  double gc[kRows], re[kRows], im[kRows];
 #pragma unroll
-  for (int d = 0; d < 3; d++) v[d] = d1 * a.b[d] + d2 * a.b[3 + d] + d3 * a.b[6 + d];
-  const double gc = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-  const bool finite = gc > a.epslat;
-  double re = finite ? 0.0 : 1.0, im = 0.0;
-  const double *tau = geo + 3 * a.nspecies;
+  for (int r = 0; r < kRows; r++) {
+    const int i3 = a.lo[2] + box_index(min(j30 + r, a.n3 - 1), a.off[2], a.n3);
+    double v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+      v[d] = (double)i1 * a.b[d] + (double)i2 * a.b[3 + d] + (double)i3 * a.b[6 + d];
+    gc[r] = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    re[r] = gc[r] > a.epslat ? 0.0 : 1.0;
+    im[r] = 0.0;
+  }
   for (int is = 0; is < a.nspecies; is++) {
     const double rmt = geo[3 * is];
     const int ia0 = (int)geo[3 * is + 1], ia1 = (int)geo[3 * is + 2];
-    double ff;
-    if (finite) {
-      const double t2 = gc * rmt;
-      double s, c;
-      sincos(t2, &s, &c);
-      ff = a.t1 * (s - t2 * c) / (gc * gc * gc);
-    } else {
-      ff = a.t1 / 3.0 * rmt * rmt * rmt;
-    }
+    if (ia0 == ia1) continue;
+    double sr[kRows] = {}, si[kRows] = {};
     for (int ia = ia0; ia < ia1; ia++) {
-      const double t2 = -(v[0] * tau[3 * ia] + v[1] * tau[3 * ia + 1] + v[2] * tau[3 * ia + 2]);
-      double s, c;
-      sincos(t2, &s, &c);
-      re -= ff * c;
-      im -= ff * s;
+      const double2 *t = tab + (size_t)ia * nt;
+      const double2 x = t[j1], y = t[a.n1 + j2];
+      const double px = x.x * y.x - x.y * y.y, py = x.x * y.y + x.y * y.x;
+#pragma unroll
+      for (int r = 0; r < kRows; r++) {
+        const double2 z = t[a.n1 + a.n2 + min(j30 + r, a.n3 - 1)];
+        sr[r] += px * z.x - py * z.y;
+        si[r] += px * z.y + py * z.x;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+      double ff;
+      if (gc[r] > a.epslat) {
+        const double t2 = gc[r] * rmt;
+        double s, c;
+        sincos(t2, &s, &c);
+        ff = a.t1 * (s - t2 * c) / (gc[r] * gc[r] * gc[r]);
+      } else {
+        ff = a.t1 / 3.0 * rmt * rmt * rmt;
+      }
+      re[r] -= ff * sr[r];
+      im[r] -= ff * si[r];
     }
   }
-  zfft[fft_index(i1, i2, i3, a.n1, a.n2, a.n3)] = make_double2(re, im);
-  if (a.damp > 0.0) {
-    const double t = a.damp * gc, f = exp(-t * t);
-    re *= f;
-    im *= f;
+#pragma unroll
+  for (int r = 0; r < kRows; r++) {
+    const int j3 = j30 + r;
+    if (j3 >= a.n3) break;
+    zfft[(size_t)j3 * plane + q] = make_double2(re[r], im[r]);
+    if (a.damp > 0.0) {
+      const double t = a.damp * gc[r], f = exp(-t * t);
+      re[r] *= f;
+      im[r] *= f;
+    }
+    const int b3 = box_index(j3, a.off[2], a.n3);
+    cfunig[ivgig[b1 + (size_t)a.n1 * (b2 + (size_t)a.n2 * b3)] - 1] = make_double2(re[r], im[r]);
   }
-  cfunig[ig] = make_double2(re, im);
 }
 
 // gencfun.f90:74: cfunir = Re(zfft).
@@ -98,43 +158,55 @@ __global__ __launch_bounds__(256) void real_part_kernel(int n, const double2 *__
 }
 
 // genveffig.f90:33 and genmeffig.f90:38,50: the selected products, stored as
-// consecutive grids of n complex values in the order veff, meff, m2eff.
+// consecutive real grids of n values in the order veff, meff, m2eff.
 __global__ __launch_bounds__(256) void products_kernel(int n, const double *__restrict__ veffir,
                                                        const double *__restrict__ cfunir,
                                                        int which, double a2,
-                                                       double2 *__restrict__ z) {
+                                                       double *__restrict__ z) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double v = veffir[i], c = cfunir[i];
-  double2 *p = z + i;
+  double *p = z + i;
   if (which & EXH_VEFFIG) {
-    *p = make_double2(v * c, 0.0);
+    *p = v * c;
     p += n;
   }
   if (which & (EXH_MEFFIG | EXH_M2EFFIG)) {
     const double d = 1.0 - v * a2;
     if (which & EXH_MEFFIG) {
-      *p = make_double2(c / d, 0.0);
+      *p = c / d;
       p += n;
     }
-    if (which & EXH_M2EFFIG) *p = make_double2(c / (d * d), 0.0);
+    if (which & EXH_M2EFFIG) *p = c / (d * d);
   }
 }
 
 // genveffig.f90:36-39 (and genmeffig.f90:41-44, :53-56): out_b(ig) = the
 // forward transform at G's grid point, times the 1/N of zfftifc.f90:70-77.
+// The grids are real, so only j1 <= n1 / 2 is transformed: the other half is
+// the conjugate at -j (mod n).  Two products of 80^3: 42 us as complex
+// transforms, 32 so, at the same error (2e-16, relative norm).
 __global__ __launch_bounds__(256) void gather_kernel(int ngvec, const int *__restrict__ ivg,
                                                      int n1, int n2, int n3, int nb,
                                                      const double2 *__restrict__ z, double scale,
                                                      double2 *o0, double2 *o1, double2 *o2) {
   const int ig = blockIdx.x * blockDim.x + threadIdx.x;
   if (ig >= ngvec) return;
-  const size_t n = (size_t)n1 * n2 * n3;
-  const size_t j = fft_index(ivg[3 * ig], ivg[3 * ig + 1], ivg[3 * ig + 2], n1, n2, n3);
+  const int i1 = ivg[3 * ig], i2 = ivg[3 * ig + 1], i3 = ivg[3 * ig + 2];
+  int j1 = i1 >= 0 ? i1 : n1 + i1, j2 = i2 >= 0 ? i2 : n2 + i2, j3 = i3 >= 0 ? i3 : n3 + i3;
+  const int h1 = n1 / 2 + 1;
+  double sy = scale;
+  if (j1 >= h1) {
+    j1 = n1 - j1;
+    j2 = j2 ? n2 - j2 : 0;
+    j3 = j3 ? n3 - j3 : 0;
+    sy = -scale;
+  }
+  const size_t n = (size_t)h1 * n2 * n3, j = ((size_t)j3 * n2 + j2) * h1 + j1;
   double2 *outs[3] = {o0, o1, o2};
   for (int b = 0; b < nb; b++) {
     const double2 x = z[b * n + j];
-    outs[b][ig] = make_double2(x.x * scale, x.y * scale);
+    outs[b][ig] = make_double2(x.x * scale, x.y * sy);
   }
 }
 
@@ -167,7 +239,8 @@ const char *fft_error(hipfftResult r) {
   }
 }
 
-// In-place double-complex plan over the context's grid for nb grids.
+// Plan over the context's grid: nb = 0 the in-place double-complex transform of
+// one grid, nb > 0 the forward transform of nb real grids.
 int fft_plan(exh_context *c, int nb, hipfftHandle *out) {
   int n[3];
   grid_of(c, n);
@@ -178,9 +251,9 @@ int fft_plan(exh_context *c, int nb, hipfftHandle *out) {
   if (!c->fft_plan[nb]) {
     hipfftHandle h = nullptr;
     int dims[3] = {n[2], n[1], n[0]};
-    const int dist = c->ngrtot;
-    hipfftResult r = hipfftPlanMany(&h, 3, dims, nullptr, 1, dist, nullptr, 1, dist,
-                                    HIPFFT_Z2Z, nb);
+    const int dist = c->ngrtot, odist = nb ? (n[0] / 2 + 1) * n[1] * n[2] : dist;
+    hipfftResult r = hipfftPlanMany(&h, 3, dims, nullptr, 1, dist, nullptr, 1, odist,
+                                    nb ? HIPFFT_D2Z : HIPFFT_Z2Z, std::max(nb, 1));
     if (r != HIPFFT_SUCCESS)
       return fail(c, EXH_ESTATE, std::string("hipfftPlanMany: ") + fft_error(r));
     c->fft_plan[nb] = (void *)h;
@@ -189,17 +262,31 @@ int fft_plan(exh_context *c, int nb, hipfftHandle *out) {
   return 0;
 }
 
-int run_fft(exh_context *c, hipStream_t s, int nb, double2 *z, int direction) {
+// nb = 0: z in place, to the grid; nb > 0: the real grids x into z
+int run_fft(exh_context *c, hipStream_t s, int nb, double *x, double2 *z) {
   hipfftHandle h;
   if (int rc = fft_plan(c, nb, &h)) return rc;
   hipfftResult r = hipfftSetStream(h, s);
   hipError_t e = timed(c, EXH_K_IFFT, s, [&] {
     if (r == HIPFFT_SUCCESS)
-      r = hipfftExecZ2Z(h, (hipfftDoubleComplex *)z, (hipfftDoubleComplex *)z, direction);
+      r = nb ? hipfftExecD2Z(h, x, (hipfftDoubleComplex *)z)
+             : hipfftExecZ2Z(h, (hipfftDoubleComplex *)z, (hipfftDoubleComplex *)z,
+                             HIPFFT_BACKWARD);
     return hipSuccess;
   });
-  if (r != HIPFFT_SUCCESS) return fail(c, EXH_ESTATE, std::string("hipfftExecZ2Z: ") + fft_error(r));
+  if (r != HIPFFT_SUCCESS) return fail(c, EXH_ESTATE, std::string("hipfftExec: ") + fft_error(r));
   return e == hipSuccess ? 0 : hip_fail(c, e, "fft");
+}
+
+// The geometry goes to the device as kernel arguments, kGeoWords at a time: a
+// copy from the caller's memory would have to be waited for.
+constexpr int kGeoWords = 384;
+struct GeoWords {
+  double v[kGeoWords];
+};
+__global__ __launch_bounds__(kGeoWords) void put_words_kernel(GeoWords g, int n,
+                                                              double *__restrict__ out) {
+  if ((int)threadIdx.x < n) out[threadIdx.x] = g.v[threadIdx.x];
 }
 
 template <typename T>
@@ -262,8 +349,12 @@ int exh_gencfun_device(exh_context *c, void *stream, const double *bvec, const d
       for (int d = 0; d < 3; d++) geo[k++] = atposc[d + 3 * ((size_t)ia + (size_t)maxatoms * is)];
     geo[3 * is + 2] = ias;
   }
-  int rc = copy_in(c, c->igeo, geo.data(), geo.size());
+  int rc = ensure(c, c->igeo, geo.size() * sizeof(double));
   if (!rc) rc = ensure(c, c->ifz, (size_t)c->ngrtot * sizeof(double2));
+  int n[3];
+  grid_of(c, n);
+  const size_t ntab = (size_t)c->natmtot * (n[0] + n[1] + n[2]);
+  if (!rc) rc = ensure(c, c->iphase, std::max<size_t>(ntab, 1) * sizeof(double2));
   if (rc) return rc;
 
   CfunArgs a;
@@ -272,17 +363,33 @@ int exh_gencfun_device(exh_context *c, void *stream, const double *bvec, const d
   a.epslat = epslat;
   a.damp = cfdamp > 0.0 ? cfdamp / gmaxvr : 0.0;
   grid_of(c, &a.n1);
+  for (int d = 0; d < 3; d++) {
+    a.lo[d] = c->intgv[d];
+    a.off[d] = (int)(((-(long long)a.lo[d]) % n[d] + n[d]) % n[d]);
+  }
   a.nspecies = c->nspecies;
   const int ng = c->ngrtot;
   double2 *z = (double2 *)c->ifz.p;
   hipError_t e = timed(c, EXH_K_CFUNIG, s, [&] {
-    hipLaunchKernelGGL(cfunig_kernel, dim3(cdiv_i(ng, 256)), dim3(256), 0, s, ng,
-                       (const int *)c->ivg.p, a, (const double *)c->igeo.p,
+    for (size_t w0 = 0; w0 < geo.size(); w0 += kGeoWords) {
+      GeoWords g;
+      const int nw = (int)std::min<size_t>(kGeoWords, geo.size() - w0);
+      std::memcpy(g.v, geo.data() + w0, nw * sizeof(double));
+      hipLaunchKernelGGL(put_words_kernel, dim3(1), dim3(kGeoWords), 0, s, g, nw,
+                         (double *)c->igeo.p + w0);
+    }
+    if (ntab)
+      hipLaunchKernelGGL(phase_table_kernel, dim3(cdiv_i(ntab, 256)), dim3(256), 0, s, a,
+                         c->natmtot, (const double *)c->igeo.p,
+                         (double2 *)c->iphase.p);
+    hipLaunchKernelGGL(cfunig_kernel, dim3(cdiv_i((long long)n[0] * n[1], 256), cdiv_i(n[2], kRows)),
+                       dim3(256), 0, s, a, (const int *)c->ivgig.p,
+                       (const double *)c->igeo.p, (const double2 *)c->iphase.p,
                        (double2 *)cfunig, z);
     return hipGetLastError();
   });
   if (e != hipSuccess) return hip_fail(c, e, "gencfun");
-  if ((rc = run_fft(c, s, 1, z, HIPFFT_BACKWARD))) return rc;
+  if ((rc = run_fft(c, s, 0, nullptr, z))) return rc;
   e = timed(c, EXH_K_IGATHER, s, [&] {
     hipLaunchKernelGGL(real_part_kernel, dim3(cdiv_i(ng, 256)), dim3(256), 0, s, ng,
                        (const double2 *)z, cfunir);
@@ -311,18 +418,22 @@ int exh_genveffig_device(exh_context *c, void *stream, const double *veffir,
   if (which & EXH_MEFFIG) outs[nb++] = (double2 *)meffig;
   if (which & EXH_M2EFFIG) outs[nb++] = (double2 *)m2effig;
   const int n = c->ngrtot;
-  if (int rc = ensure(c, c->ifz, (size_t)nb * n * sizeof(double2))) return rc;
+  int g[3];
+  grid_of(c, g);
+  // [nb half grids, complex | nb grids, real]
+  const size_t half = (size_t)nb * (g[0] / 2 + 1) * g[1] * g[2];
+  if (int rc = ensure(c, c->ifz, half * sizeof(double2) + (size_t)nb * n * sizeof(double)))
+    return rc;
   double2 *z = (double2 *)c->ifz.p;
+  double *x = (double *)(z + half);
   const double a2 = 0.5 * kAlpha * kAlpha;
   hipError_t e = timed(c, EXH_K_IPROD, s, [&] {
     hipLaunchKernelGGL(products_kernel, dim3(cdiv_i(n, 256)), dim3(256), 0, s, n, veffir,
-                       cfunir, which, a2, z);
+                       cfunir, which, a2, x);
     return hipGetLastError();
   });
   if (e != hipSuccess) return hip_fail(c, e, "genveffig");
-  if (int rc = run_fft(c, s, nb, z, HIPFFT_FORWARD)) return rc;
-  int g[3];
-  grid_of(c, g);
+  if (int rc = run_fft(c, s, nb, x, z)) return rc;
   const double scale = 1.0 / (double)n;
   e = timed(c, EXH_K_IGATHER, s, [&] {
     hipLaunchKernelGGL(gather_kernel, dim3(cdiv_i(c->ngvec, 256)), dim3(256), 0, s, c->ngvec,
