@@ -16,107 +16,104 @@ __device__ __forceinline__ dx4 mfma16(double a, double b, dx4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-constexpr int CT = 64;    // output tile edge (rows i and columns j)
-constexpr int CK = 8;     // K slab staged in LDS per step (16: 2 %, 32: 6 % slower)
-constexpr int CNT = 256;  // 4 waves, each a 32 x 32 quadrant of 2 x 2 MFMA blocks
+// the value of the neighbouring lane (lane ^ 1), its sign flipped by mask; on
+// the integer units, since FP64 multiplies share the matrix cores' pipe
+__device__ __forceinline__ double swap_pair(double v, int mask) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return __hiloint2double(hi ^ mask, lo);
+}
+
+constexpr int CT = 64;    // output rows of a workgroup: 16 per wave
+constexpr int CK = 8;     // K slab of X staged in LDS per step
+constexpr int CNT = 256;  // 4 waves
+constexpr int CNTILE = 8; // column tiles of a workgroup at most
 
 // part[s][i][j] = sum over k in chunk s of conj(A[k][i]) X[k][j] (asign = -1)
-// or A[k][i] X[k][j] (asign = 1), for a 64 x 64 tile (i, j) of the output;
-// chunk s is [s * kchunk, min(K, (s+1) * kchunk)).
+// or A[k][i] X[k][j] (asign = 1); chunk s is [s * kchunk, min(K, (s+1) * kchunk)).
 // A(k, i) at A[k * lda + i], X(k, j) at X[k * ldx + j], part[s] row-major with
-// leading dimension m.  Loads are clamped to valid addresses and zero-weighted
-// outside the tile, so every thread runs the same slab loop.
+// leading dimension m.
+//
+// Bound by A's bytes (16 nout K) up to about 16 columns, by the FP64 matrix
+// cores beyond.  The columns are taken as the 2m real columns re, im, re, ..
+// that X and part hold in memory: out[c] = Re A X[c] +- Im A X[c ^ 1], so m is
+// padded to a multiple of 8 and not of 64, and the workgroups' column tiles fit
+// m.  The 16 rows of a wave are nobody else's: its A fragments come from memory
+// in the MFMA's own lane order (16 lanes read 256 consecutive bytes), without
+// LDS, one slab ahead.  X is shared by the waves through two LDS buffers (one
+// barrier per slab; row length 16 mod 32 doubles, so that two rows fill the
+// banks), its neighbouring column comes from the neighbouring lane.  Rows and
+// columns out of range are clamped and not stored, k out of range is zero.
+// n = 10364, 64 x 64 tiles of zero-padded columns before, this now (us, with the
+// reduction, chunks of K as below): 8 columns 870 -> 333, 24: 870 -> 474, 40:
+// 870 -> 681, 56: 886 -> 903 (5.4 TB/s of A at 8, 57 TFLOP/s at 56), 80: 1740 ->
+// 1290.  Slabs of 16 K need 171 registers at seven tiles (926 us at 56), 32 rows
+// per wave 206 (943).
+template <int NT>
 __global__ __launch_bounds__(CNT) void cx_part_kernel(int nout, int m, int K, int kchunk,
                                                       const double2 *__restrict__ A,
                                                       long long lda, double asign,
                                                       const double2 *__restrict__ X,
                                                       long long ldx,
                                                       double2 *__restrict__ part) {
-  const int I0 = blockIdx.x * CT, J0 = blockIdx.y * CT, s = blockIdx.z;
-  const int k0 = s * kchunk, k1 = min(K, k0 + kchunk);
-  __shared__ double sAr[CK][CT + 16], sAi[CK][CT + 16], sXr[CK][CT + 16], sXi[CK][CT + 16];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wr = w >> 1, wc = w & 1, lr = lane & 15, lk = lane >> 4;
-  const int ii = tid & 63, kq = tid >> 6;  // loads: tile column ii, slab rows kq + 4q
-  const bool vi = I0 + ii < nout, vj = J0 + ii < m;
-  const double2 *ap = A + (vi ? I0 + ii : nout - 1);
-  const double2 *xp = X + (vj ? J0 + ii : m - 1);
+  constexpr int W = 16 * NT, LX = W + (W % 32 ? 0 : 16);
+  __shared__ double sx[2][CK][LX];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int I0 = blockIdx.x * CT + (tid >> 6) * 16, C0 = blockIdx.y * W, s = blockIdx.z;
+  const int k0 = s * kchunk, k1 = min(K, k0 + kchunk), m2 = 2 * m;
+  const double2 *ap = A + min(I0 + lr, nout - 1);
+  const double *xp = (const double *)X + C0;
+  const int flip = (lr & 1 ? asign : -asign) < 0.0 ? (int)0x80000000 : 0;
+  constexpr int NX = (CK * W + CNT - 1) / CNT;
 
-  dx4 cre[2][2], cim[2][2];
+  dx4 acc[NT];
 #pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++) {
-      cre[a][b] = dx4{0, 0, 0, 0};
-      cim[a][b] = dx4{0, 0, 0, 0};
-    }
-
-  constexpr int QB = CK / 4;
-  double2 pa[QB], px[QB];
-  double fa[QB], fx[QB];
+  for (int t = 0; t < NT; t++) acc[t] = dx4{0, 0, 0, 0};
+  double2 an[CK / 4];
+  double xn[NX];
   auto load = [&](int kb) {
 #pragma unroll
-    for (int q = 0; q < QB; q++) {
-      const int k = kb + kq + 4 * q;
-      const bool kv = k < k1;
-      const int kc = kv ? k : k1 - 1;
-      pa[q] = ap[(size_t)kc * lda];
-      px[q] = xp[(size_t)kc * ldx];
-      fa[q] = (kv && vi) ? 1.0 : 0.0;
-      fx[q] = (kv && vj) ? 1.0 : 0.0;
+    for (int q = 0; q < CK / 4; q++) an[q] = ap[(size_t)min(kb + 4 * q + lk, k1 - 1) * lda];
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int e = tid + CNT * i;
+      xn[i] = xp[(size_t)min(kb + e / W, k1 - 1) * (2 * ldx) + min(e % W, m2 - 1 - C0)];
     }
   };
   load(k0);
-  for (int kb = k0; kb < k1; kb += CK) {
-    // conj(A): the imaginary part is stored negated (asign = -1)
+  int b = 0;
+  for (int kb = k0; kb < k1; kb += CK, b ^= 1) {
+    double2 a[CK / 4];
 #pragma unroll
-    for (int q = 0; q < QB; q++) {
-      const int kk = kq + 4 * q;
-      sAr[kk][ii] = fa[q] * pa[q].x;
-      sAi[kk][ii] = asign * (fa[q] * pa[q].y);
-      sXr[kk][ii] = fx[q] * px[q].x;
-      sXi[kk][ii] = fx[q] * px[q].y;
+    for (int q = 0; q < CK / 4; q++) a[q] = kb + 4 * q + lk < k1 ? an[q] : z2(0.0, 0.0);
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int e = tid + CNT * i;
+      if (CK * W % CNT == 0 || e < CK * W) sx[b][e / W][e % W] = kb + e / W < k1 ? xn[i] : 0.0;
     }
     __syncthreads();
     if (kb + CK < k1) load(kb + CK);
 #pragma unroll
-    for (int k4 = 0; k4 < CK / 4; k4++) {
-      const int kk = 4 * k4 + lk;
-      double ar[2], ai[2], nai[2], xr[2], xi[2];
+    for (int q = 0; q < CK / 4; q++) {
+      double x[NT], y[NT];
 #pragma unroll
-      for (int a = 0; a < 2; a++) {
-        ar[a] = sAr[kk][wr * 32 + a * 16 + lr];
-        ai[a] = sAi[kk][wr * 32 + a * 16 + lr];
-        nai[a] = -ai[a];
-      }
+      for (int t = 0; t < NT; t++) x[t] = sx[b][4 * q + lk][16 * t + lr];
 #pragma unroll
-      for (int b = 0; b < 2; b++) {
-        xr[b] = sXr[kk][wc * 32 + b * 16 + lr];
-        xi[b] = sXi[kk][wc * 32 + b * 16 + lr];
-      }
+      for (int t = 0; t < NT; t++) y[t] = swap_pair(x[t], flip);
 #pragma unroll
-      for (int a = 0; a < 2; a++)
+      for (int t = 0; t < NT; t++) acc[t] = mfma16(a[q].x, x[t], acc[t]);
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-          cre[a][b] = mfma16(ar[a], xr[b], cre[a][b]);
-          cre[a][b] = mfma16(nai[a], xi[b], cre[a][b]);
-          cim[a][b] = mfma16(ar[a], xi[b], cim[a][b]);
-          cim[a][b] = mfma16(ai[a], xr[b], cim[a][b]);
-        }
+      for (int t = 0; t < NT; t++) acc[t] = mfma16(a[q].y, y[t], acc[t]);
     }
-    __syncthreads();
   }
-  double2 *ps = part + (size_t)s * nout * m;
+  double *ps = (double *)(part + (size_t)s * nout * m);
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = I0 + wr * 32 + a * 16 + lk + 4 * r;
-        const int j = J0 + wc * 32 + b * 16 + lr;
-        if (i < nout && j < m) ps[(size_t)i * m + j] = z2(cre[a][b][r], cim[a][b][r]);
-      }
+    for (int r = 0; r < 4; r++) {
+      const int i = I0 + lk + 4 * r, c = C0 + 16 * t + lr;
+      if (i < nout && c < m2) ps[(size_t)i * m2 + c] = acc[t][r];
+    }
 }
 
 // One column (m = 1: the matrix-vector products of the Lanczos bound): the
@@ -208,11 +205,19 @@ extern "C" int exh_zgemm_cn_device(void *stream, int conj_a, int nout, int m, in
                        (const double2 *)a, lda, conj_a ? -1.0 : 1.0, (const double2 *)x, ldx,
                        (double2 *)work);
   } else {
-    const dim3 grid((unsigned)((nout + CT - 1) / CT), (unsigned)((m + CT - 1) / CT),
-                    (unsigned)S);
-    hipLaunchKernelGGL(cx_part_kernel, grid, dim3(CNT), 0, s, nout, m, k, kchunk,
-                       (const double2 *)a, lda, conj_a ? -1.0 : 1.0, (const double2 *)x, ldx,
-                       (double2 *)work);
+    // column tiles of 8, spread evenly over the workgroups that share A
+    const int tiles = (m + 7) / 8, jb = (tiles + CNTILE - 1) / CNTILE, nt = (tiles + jb - 1) / jb;
+    const dim3 grid((unsigned)((nout + CT - 1) / CT), (unsigned)jb, (unsigned)S);
+#define LAUNCH(NT)                                                                          \
+  case NT:                                                                                  \
+    hipLaunchKernelGGL(cx_part_kernel<NT>, grid, dim3(CNT), 0, s, nout, m, k, kchunk,       \
+                       (const double2 *)a, lda, conj_a ? -1.0 : 1.0, (const double2 *)x,    \
+                       ldx, (double2 *)work);                                               \
+    break;
+    switch (nt) {
+      LAUNCH(1) LAUNCH(2) LAUNCH(3) LAUNCH(4) LAUNCH(5) LAUNCH(6) LAUNCH(7) LAUNCH(8)
+    }
+#undef LAUNCH
   }
   const size_t total = (size_t)nout * m;
   hipLaunchKernelGGL(cx_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
