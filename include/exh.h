@@ -299,8 +299,8 @@ int exh_setup_device(exh_context *ctx, void *stream, int ngp, int rank,
  * EXH_ACCUMULATE or 0), with bitwise the same result, but its scratch
  * (G+k index map, aa.A operand, and for iora* or non-uniform layouts one
  * more operand) lives in a static 64 MiB device array, and the residues of
- * the modular products in another 128 MiB, instead of the context's buffers: it calls no hipMalloc, hipFree or allocating library
- * routine.  Bases needing more than 64 MiB (16 * natmtot*maxaa * ngkmax
+ * the modular products in another 256 MiB, instead of the context's buffers:
+ * it calls no hipMalloc, hipFree or allocating library routine.  Bases needing more than 64 MiB (16 * natmtot*maxaa * ngkmax
  * rounded up, per operand) are refused with EXH_ERANGE, split precision
  * with EXH_ENOTSUP.  Every context on a GPU shares that GPU's array, so
  * calls that overlap on one GPU (two streams, two host threads) race; the
