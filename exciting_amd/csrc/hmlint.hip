@@ -129,11 +129,11 @@ __global__ __launch_bounds__(kThreads) void hml_kinetic_kernel(
 // With a pair per thread this was bound by LDS (5 words for 8 FMA) and by
 // uncoalesced staging; as a product P(pair, r) V(r, lm) with P = f1 f2 w r^2 formed in registers
 // from three LDS words, an MFMA of 1024 FMA needs one word of V per lane.  The next chunk's global reads are in flight while a chunk is
-// multiplied; the two LDS buffers leave one barrier per chunk.  64 atoms, 22
+// multiplied; the two LDS buffers leave one barrier per chunk.  64 atoms, 26
 // functions, 250 points, 81 channels: 113 -> 48 us, 10 of them the kinetic
 // workgroups (a wave per pair instead of a thread: the products of a wave's 64
 // points need no LDS); 16 us at the FP64 matrix rate, the rest latency of eight
-// short chunks at two workgroups per CU.
+// short chunks at three workgroups per CU.
 template <int LT>
 __global__ __launch_bounds__(kThreads) void hml_radial_kernel(
     HmlArgs a, const int *__restrict__ atom_species, const int *__restrict__ nrmt,
@@ -246,8 +246,8 @@ struct ConArgs {
 // for the atoms of chunk blockIdx.y: {first, count, species}.  Entry t of the
 // lists lies at [t][lm_j][lm_i], so that the lanes (consecutive i) read
 // consecutive entries; each entry read serves all atoms of the chunk.  64 atoms,
-// aa of order 162: 112 us with the lists one after the other, a thread per
-// element and atom and a launch per table, 48 us now; 31 MB are written (8 us),
+// aa of order 242: 112 us with the lists one after the other, a thread per
+// element and atom and a launch per table, 48 us now; 64 MB are written (14 us),
 // the gathers of the integrals (about 30 lines each) bound it.
 __global__ __launch_bounds__(kThreads) void hml_contract_kernel(
     int nf, int lmmaxvr, int lmmaxmat, const int4 *__restrict__ chunks, ConArgs P,
@@ -502,8 +502,9 @@ int prepare(exh_context *c, int lmaxvr) {
       for (int l3 = 0; l3 <= lmaxmat; l3++)
         for (int m3 = -l3; m3 <= l3; m3++) {
           const size_t q = (size_t)(l3 * (l3 + 1) + m3) * lmmaxmat + l1 * (l1 + 1) + m1;
-          for (int l2 = 0; l2 <= lmaxvr; l2++)
-            for (int m2 = -l2; m2 <= l2; m2++) {
+          const int d = std::abs(m1 - m3);   // zero unless m1 = m3 +- m2
+          for (int l2 = d; l2 <= lmaxvr; l2++)
+            for (int m2 = -d; m2 <= d; m2 += std::max(2 * d, 1)) {
               double re, im;
               gaunt_real_middle(l1, l2, l3, m1, m2, m3, &re, &im);
               if (std::sqrt(re * re + im * im) > 1e-20) {
