@@ -486,7 +486,7 @@ def interstitial_sample(ctx, s, reps=20):
     t = k["cfunig"] * 1e-3
     res["gencfun"] = {
         "ms": w, "kernels_ms": k,
-        "cfunig_kernel": {"bound": "fp64 sincos throughput",
+        "cfunig_kernel": {"bound": "latency of the phase tables' loads",
                           "pairs_per_s": n * s.natmtot / t,
                           "hbm_GBps": 44.0 * n / t / 1e9,
                           "bytes_per_G": 44},
