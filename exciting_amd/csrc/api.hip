@@ -421,9 +421,9 @@ OzPlan oz_plan(const exh_context *c, int flags) {
   return oz_noalloc_chunk(P, L) > 0 ? P : OzPlan();
 }
 
-bool oz_fits(const exh_context *c, const OzLayout &L, int slots, int nk) {
-  return c->ozq.bytes >= L.q_bytes * L.nops * slots && c->ozr.bytes >= L.r_bytes * slots &&
-         c->oze.bytes >= L.e_bytes * L.nops * nk;
+bool oz_fits(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots,
+             int nk) {
+  return c->oz[use][P.split].bytes >= L.bytes(slots, nk);
 }
 
 // Plan, layout and scratch of the modular contraction for nk k-points, the
@@ -431,25 +431,30 @@ bool oz_fits(const exh_context *c, const OzLayout &L, int slots, int nk) {
 // FP64 MFMA kernels instead, which is also where an FP64 setup goes when the
 // device has no room for the residues or the stream is being captured before
 // the first call (nothing may be allocated then).
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, int nk,
-               OzPlan &P, OzLayout &L) {
+//
+// The buffer of a single FP64 setup has the size of the basis alone, as the
+// other scratch of that call: O alone and the full setup, with or without h1aa,
+// all get the room that the largest of them needs, so only a larger basis
+// (which moves aa.A too) moves it.
+int oz_prepare(exh_context *c, OzUse use, int flags, bool only_o, bool capturing, int slots,
+               int nk, OzPlan &P, OzLayout &L) {
   P = oz_plan(c, flags);
   if (P.nmod == 0) return 0;
-  const bool split = (flags & 0xff00) != 0;
   L = oz_layout(c, P, only_o);
-  if (oz_fits(c, L, slots, nk)) return 0;
-  if (!split) {
+  if (oz_fits(c, use, P, L, slots, nk)) return 0;
+  const size_t need = use == kOzSingle && !P.split
+                          ? oz_layout_ops(c, P, false, 3).bytes(1, 1)
+                          : L.bytes(slots, nk);
+  if (!P.split) {
     size_t avail = 0, total = 0;
     if (capturing || hipMemGetInfo(&avail, &total) != hipSuccess ||
-        avail < L.bytes() * slots + L.e_bytes * L.nops * nk + (size_t(1) << 30)) {
+        avail < need + (size_t(1) << 30)) {
       P = OzPlan();
       return 0;
     }
   }
-  int rc = ensure(c, c->ozq, L.q_bytes * L.nops * slots);
-  if (!rc) rc = ensure(c, c->ozr, L.r_bytes * slots);
-  if (!rc) rc = ensure(c, c->oze, L.e_bytes * L.nops * nk);
-  if (rc && !split) {  // another allocation took the room meanwhile
+  const int rc = ensure(c, c->oz[use][P.split], need);
+  if (rc && !P.split) {  // another allocation took the room meanwhile
     (void)hipGetLastError();
     P = OzPlan();
     return 0;
@@ -539,7 +544,7 @@ void exh_destroy(exh_context *c) {
                     &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu, &c->mt_match.piv,
                     &c->aa, &c->loa, &c->lolo, &c->salo, &c->ololo_eff, &c->h1aa,
                     &c->ivg, &c->ivgig, &c->ist, &c->cf_stage, &c->vf_stage, &c->mf_stage,
-                    &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->ozq, &c->ozr, &c->oze, &c->s_apwalm, &c->s_igpig,
+                    &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->oz[0][0], &c->oz[0][1], &c->oz[1][0], &c->oz[1][1], &c->s_apwalm, &c->s_igpig,
                     &c->s_vgpc, &c->s_h, &c->s_o, &c->s_gpc, &c->s_tpgpc, &c->s_sfac,
                     &c->bbt, &c->bat, &c->ba2t, &c->bivgk, &c->ifz, &c->igeo, &c->iphase, &c->i_in0,
                     &c->i_in1, &c->i_out0, &c->i_out1, &c->i_out2, &c->apwfr_d, &c->hml_fl,
@@ -945,10 +950,10 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   if (!rc && !c->contig) rc = ensure(c, c->at, op);
   if (!rc) rc = ensure(c, c->ivgk, (size_t)std::max(c->ngkmax, 1) * sizeof(int4));
   if (!rc)
-    rc = oz_prepare(c, flags, o_only, cap == hipStreamCaptureStatusActive, 1, 1, w.plan,
-                    w.layout);
+    rc = oz_prepare(c, kOzSingle, flags, o_only, cap == hipStreamCaptureStatusActive, 1, 1,
+                    w.plan, w.layout);
   if (rc) return rc;
-  if (w.plan.nmod) w.oz = oz_scratch(c, w.plan, w.layout, 0, 0);
+  if (w.plan.nmod) w.oz = oz_scratch(c, kOzSingle, w.plan, w.layout, 1, 0, 0);
   w.bt = (double2 *)c->bt.p;
   w.a2t = (double2 *)c->a2t.p;
   w.at = (double2 *)c->at.p;

@@ -112,7 +112,7 @@ uint64_t state_signature(const exh_context *c) {
                           &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu,
                           &c->mt_match.piv, &c->aa, &c->loa, &c->lolo, &c->salo,
                           &c->ololo_eff, &c->h1aa, &c->ivg, &c->ist, &c->bbt, &c->bat,
-                          &c->ba2t, &c->bivgk, &c->bmtab, &c->ozq, &c->ozr, &c->oze};
+                          &c->ba2t, &c->bivgk, &c->bmtab, &c->oz[kOzGroup][0], &c->oz[kOzGroup][1]};
   for (const DevBuf *b : bufs) mix(&b->p, sizeof b->p);
   const int sc[] = {c->nspecies, c->natmtot, c->lmaxapw, c->lmaxmat, c->apwordmax, c->nlomax,
                     c->ngkmax, c->maxaa, c->maxnlo, c->nlotot, c->lmmax, c->Ktot,
@@ -236,11 +236,15 @@ struct OzParams {
 // workspace limit.  8 k-points of K = 1936, G = 1172 in one wave against one by
 // one: norms and residues 0.73 -> 0.51 ms, products 1.05 -> 0.88, reconstruction
 // 0.23 -> 0.18.
-int oz_slots(const exh_context *c, const OzPlan &P, const OzLayout &L, int nk) {
+// `most` is the room to allocate: unlike the equal waves it never shrinks when
+// nk grows, so only a longer list (which moves the other scratch too) moves it.
+int oz_slots(const exh_context *c, const OzPlan &P, const OzLayout &L, int nk, int *most) {
+  *most = 1;
   if (P.nmod == 0 || nk <= 1) return 1;
   constexpr long long kTarget = 8192;
   long long n = std::min<long long>(nk, cdivl(kTarget, std::max<long long>(L.panels, 1)));
-  n = std::min<long long>(n, std::max<long long>(1, c->batch_ws_limit / std::max<size_t>(L.bytes(), 1)));
+  n = std::min<long long>(n, std::max<long long>(1, c->batch_ws_limit / std::max<size_t>(L.bytes(1, 1), 1)));
+  *most = (int)n;
   const long long waves = cdivl(nk, n);
   return (int)cdivl(nk, waves);
 }
@@ -317,8 +321,9 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
       IstBox box{d.ivgk, d.vgpc, (const IstEntry *)c->ist.p, S.lo0, S.lo1, S.lo2,
                  S.n0, S.n1, S.n2};
       E->oz.push_back(make_ozk(c, d.ngp, oz.P[j], oz.L[j],
-                               oz_scratch(c, oz.P[j], oz.L[j], used[j], nth[j]++), d.x, S.ldx, d.bt,
-                               d.a2t, S.ldb, box, d.h, d.o, d.ldh));
+                               oz_scratch(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], used[j],
+                                          nth[j]++),
+                               d.x, S.ldx, d.bt, d.a2t, S.ldb, box, d.h, d.o, d.ldh));
       d.norms = norm_out(E->oz.back());
       used[j]++;
       wv.count++;
@@ -463,27 +468,28 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   for (size_t j = 0; j < nctx; j++) {
     exh_context *c = cc.ctxs[j];
     oz.P[j] = oz_plan(c, flags);
+    int most = 1;
     if (oz.P[j].nmod) {
       oz.L[j] = oz_layout(c, oz.P[j], false);
-      oz.slots[j] = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j]);
+      oz.slots[j] = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j], &most);
     }
     if (outer_capture) {
       // nothing may be allocated or uploaded inside a caller's capture
-      if (oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j], cc.nkg[j])) oz.slots[j] = 1;
-      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, oz.L[j], 1, cc.nkg[j]);
+      if (oz.P[j].nmod && !oz_fits(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], cc.nkg[j])) oz.slots[j] = 1;
+      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, kOzGroup, oz.P[j], oz.L[j], 1, cc.nkg[j]);
       if (!oz_ok && !nmod) oz.P[j] = OzPlan();  // as the call outside capture ran
       if (!scratch_fits(c, cc.nkg[j]) || (nmod && !oz_ok))
         return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
     } else {
       rc = ensure_scratch(c, cc.nkg[j]);
-      if (!rc && oz.P[j].nmod && !oz_fits(c, oz.L[j], oz.slots[j], cc.nkg[j])) {
+      if (!rc && oz.P[j].nmod && !oz_fits(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], cc.nkg[j])) {
         // several slots only where the device has room for them
         size_t avail = 0, total = 0;
         if (oz.slots[j] > 1 &&
             (hipMemGetInfo(&avail, &total) != hipSuccess ||
-             avail < oz.L[j].bytes() * oz.slots[j] + (size_t(2) << 30)))
-          oz.slots[j] = 1;
-        rc = oz_prepare(c, flags, false, false, oz.slots[j], cc.nkg[j], oz.P[j], oz.L[j]);
+             avail < oz.L[j].bytes(most, cc.nkg[j]) + (size_t(2) << 30)))
+          oz.slots[j] = most = 1;
+        rc = oz_prepare(c, kOzGroup, flags, false, false, most, cc.nkg[j], oz.P[j], oz.L[j]);
       }
       if (rc) {
         if (c != lead) fail(lead, rc, c->err);
@@ -630,7 +636,7 @@ int exh_tune_batch(exh_context *c, void *stream, int nk, const exh_kpoint *kp, i
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   OzPlan P;
   OzLayout L;
-  rc = oz_prepare(c, flags, false, false, 1, 1, P, L);
+  rc = oz_prepare(c, kOzGroup, flags, false, false, 1, 1, P, L);
   if (rc) return rc;
   if (P.nmod) {  // no tiles to shape: every plan is the same call
     rc = exh_setup_batch_device(c, s, nk, kp, flags);

@@ -48,6 +48,7 @@ constexpr int kOzMaxK = 146000;
 struct OzPlan {
   int nmod = 0;  // moduli (0: not on this path)
   int bits = 0;  // c: the scaled columns' 2-norms are below 2^(c-1)
+  bool split = false;  // EXH_SPLIT(n)
 };
 struct OzLayout {
   int Gpad = 0, Kpad = 0;  // G rounded to the 128 tile, K to two 64-k stages
@@ -58,7 +59,10 @@ struct OzLayout {
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
   int nch = 0;             // partial norms of an operand, at most
   long long panels = 0;    // workgroups of the products at ngkmax
-  size_t bytes() const { return q_bytes * nops + r_bytes + e_bytes * nops; }
+  // residues of one k-point's operands and products; its exponents and norms
+  size_t slot_bytes() const { return align256(q_bytes * nops) + align256(r_bytes); }
+  size_t exp_bytes() const { return e_bytes * nops; }
+  size_t bytes(int slots, int nk) const { return slot_bytes() * slots + exp_bytes() * nk; }
 };
 struct OzScratch {
   int8_t *q = nullptr, *r = nullptr;
@@ -253,7 +257,11 @@ struct exh_context {
   exh::DevBuf bt, a2t, at, ivgk, mtab;
   // this device's copy of the static scratch of exh_setup_device_noalloc
   void *noalloc_scratch = nullptr;
-  exh::DevBuf ozq, ozr, oze;  // modular contraction: residues, products, exponents
+  // Modular contraction, [single or grouped call][FP64 or EXH_SPLIT]: residues
+  // of `slots` k-points, then exponents of nk.  Each kind of call has its own,
+  // so that a single setup may run beside a grouped call on another stream, and
+  // no other kind of call frees what a caller's captured graph of one reads.
+  exh::DevBuf oz[2][2];
   bool contig = true;  // colA[k] == k * ngkmax
   // host-API staging
   exh::DevBuf s_apwalm, s_igpig, s_vgpc, s_h, s_o, s_gpc, s_tpgpc, s_sfac;
@@ -334,23 +342,26 @@ struct OzK;
 OzPlan oz_split(int n);
 OzPlan oz_fp64();
 OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o);
+OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int nops);
 NormOut norm_out(const OzK &d);
 OzPlan oz_plan(const exh_context *c, int flags);
 int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L);
-bool oz_fits(const exh_context *c, const OzLayout &L, int slots, int nk);
-// Residue slot `slot` of the context's modular scratch, norms of k-point `k` of
-// the group.
-inline OzScratch oz_scratch(const exh_context *c, const OzPlan &P, const OzLayout &L, int slot,
-                            int k) {
+enum OzUse { kOzSingle, kOzGroup };
+bool oz_fits(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots,
+             int nk);
+int oz_prepare(exh_context *c, OzUse use, int flags, bool only_o, bool capturing, int slots,
+               int nk, OzPlan &P, OzLayout &L);
+// Residue slot `slot` of `slots`, norms of k-point `k` of the group.
+inline OzScratch oz_scratch(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L,
+                            int slots, int slot, int k) {
+  char *p = (char *)c->oz[use][P.split].p;
   OzScratch w;
-  w.q = (int8_t *)c->ozq.p + (size_t)slot * L.q_bytes * L.nops;
-  w.r = (int8_t *)c->ozr.p + (size_t)slot * L.r_bytes;
-  w.e = (char *)c->oze.p + (size_t)k * L.e_bytes * L.nops;
+  w.q = (int8_t *)p + slot * L.slot_bytes();
+  w.r = w.q + align256(L.q_bytes * L.nops);
+  w.e = p + slots * L.slot_bytes() + k * L.exp_bytes();
   w.chunk = P.nmod;
   return w;
 }
-int oz_prepare(exh_context *c, int flags, bool only_o, bool capturing, int slots, int nk,
-               OzPlan &P, OzLayout &L);
 // h = nullptr: O alone (B is not read).  Y = nullptr: the overlap's column
 // operand is X.
 OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,

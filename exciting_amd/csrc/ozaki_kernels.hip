@@ -798,6 +798,7 @@ OzPlan oz_split(int n) {
   for (int k = 0; k < n; k++) lm += std::log2((double)kPrimes[k]);
   // the largest c with 2^(2c) < prod/2 (a hair below guards the log2)
   OzPlan P;
+  P.split = true;
   P.bits = (int)std::min(50.0, std::floor((lm - 1.0) * 0.5 - 1e-9));
   // the scaled columns' norms are below 2^(c-1) + sqrt(2K)/2, so the products
   // need prod(p) > 2^(2c-1) (1 + 2^-13 at c = 23)
@@ -815,6 +816,10 @@ OzPlan oz_fp64() {
 }
 
 OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o) {
+  return oz_layout_ops(c, P, only_o, 1 + (only_o ? 0 : 1) + (c->have_h1aa ? 1 : 0));
+}
+
+OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int nops) {
   OzLayout L;
   const int ngkmax = c->ngkmax, Ktot = c->Ktot;
   L.Gpad = (ngkmax + OZ_T - 1) / OZ_T * OZ_T;
@@ -829,7 +834,7 @@ OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o) {
   L.nch = std::max((Ktot + OZ_NCH - 1) / OZ_NCH, c->natmtot * rows);
   L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
   L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * L.nch * ng + 255) / 256 * 256;
-  L.nops = 1 + (only_o ? 0 : 1) + (c->have_h1aa ? 1 : 0);
+  L.nops = nops;
   L.panels = 2 * P.nmod * (only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt));
   return L;
 }

@@ -27,6 +27,15 @@
  *     _device entry points may run on any stream; an exh_set_* call first
  *     waits for the context's last queued work, so tables are never rewritten
  *     under a running kernel.
+ *   - Scratch.  Each kind of call -- match, a single setup (with or without H,
+ *     FP64 or split), a grouped call -- has its own scratch in the context, so
+ *     calls of different kinds may run on different streams at once; two calls
+ *     of one kind have to follow each other.  A single FP64 call's scratch is
+ *     sized by the basis at the first such call (either of exh_setup_device and
+ *     exh_overlapsetup_device) and moves only after an exh_set_basis with a
+ *     larger one, a grouped call's when its list of k-points is longer than
+ *     any before: a HIP graph that the caller has captured from either stays
+ *     valid until then.
  */
 #ifndef EXH_H
 #define EXH_H
