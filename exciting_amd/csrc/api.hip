@@ -392,12 +392,10 @@ int wait_done(exh_context *c) {
   return e == hipSuccess ? 0 : hip_fail(c, e, "waiting for queued work");
 }
 
-// Moduli that exh_setup_device_noalloc can hold residues of at a time beside
-// the products of all of them; 0 when the products alone do not fit.
-int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L) {
-  const size_t fixed = align256(L.r_bytes) + align256(L.e_bytes * L.nops);
-  if (fixed >= kNoallocModularBytes) return 0;
-  return (int)std::min<size_t>(P.nmod, (kNoallocModularBytes - fixed) / (2 * L.qstride * L.nops));
+// Part of the products that exh_setup_device_noalloc's static array holds.
+OzFit oz_noalloc_fit(const OzLayout &L) {
+  const size_t e = align256(L.exp_bytes());
+  return e < kNoallocModularBytes ? oz_fit(L, kNoallocModularBytes - e) : OzFit();
 }
 
 // The modular contraction of a setup with these flags: EXH_SPLIT(n), or for
@@ -418,48 +416,77 @@ OzPlan oz_plan(const exh_context *c, int flags) {
   const OzPlan P = oz_fp64();
   if (pairs * sizeof(double2) > kNoallocScratchBytes) return P;  // refused there
   const OzLayout L = oz_layout(c, P, false);
-  return oz_noalloc_chunk(P, L) > 0 ? P : OzPlan();
+  const OzFit f = oz_noalloc_fit(L);
+  return f.chunk > 0 && f.steps == L.full.steps ? P : OzPlan();
 }
 
-bool oz_fits(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots,
-             int nk) {
-  return c->oz[use][P.split].bytes >= L.bytes(slots, nk);
+// Allocate `want` bytes of modular scratch, or what the device can spare beside
+// 1 GiB for the caller, down to `least`.
+static int oz_allocate(exh_context *c, OzUse use, const OzPlan &P, size_t want, size_t least) {
+  DevBuf &b = c->oz[use][P.split];
+  c->oz_asked[use][P.split] = want;
+  if (c->oz_pinned[use][P.split] && b.p) {
+    c->oz_retired.push_back(b);
+    b = DevBuf();
+    c->oz_pinned[use][P.split] = false;
+    c->epoch++;
+  }
+  size_t avail = 0, total = 0, n = want;
+  if (hipMemGetInfo(&avail, &total) == hipSuccess) {
+    const size_t spare = avail + b.bytes > (size_t(1) << 30) ? avail + b.bytes - (size_t(1) << 30) : 0;
+    n = std::max(least, std::min(want, spare));
+  }
+  for (;;) {
+    const int rc = ensure(c, b, n);
+    if (rc == 0 || n == least) return rc;
+    (void)hipGetLastError();
+    n = std::max(least, n / 2);
+  }
 }
 
-// Plan, layout and scratch of the modular contraction for nk k-points, the
-// residues of `slots` of them at a time; P.nmod = 0 when the setup runs on the
-// FP64 MFMA kernels instead, which is also where an FP64 setup goes when the
-// device has no room for the residues or the stream is being captured before
-// the first call (nothing may be allocated then).
+// Scratch of the modular contraction for nk k-points, the residues of `slots`
+// of them at a time (`most`: of as many as any call with this list's length
+// may take).  Neither free memory nor capture decides where a setup runs:
+// where there is no room for everything at once, the products run in parts
+// (oz_fit), with the same results; only a device without room for one modulus
+// and one column step fails.
 //
 // The buffer of a single FP64 setup has the size of the basis alone, as the
 // other scratch of that call: O alone and the full setup, with or without h1aa,
 // all get the room that the largest of them needs, so only a larger basis
-// (which moves aa.A too) moves it.
-int oz_prepare(exh_context *c, OzUse use, int flags, bool only_o, bool capturing, int slots,
-               int nk, OzPlan &P, OzLayout &L) {
-  P = oz_plan(c, flags);
-  if (P.nmod == 0) return 0;
-  L = oz_layout(c, P, only_o);
-  if (oz_fits(c, use, P, L, slots, nk)) return 0;
-  const size_t need = use == kOzSingle && !P.split
-                          ? oz_layout_ops(c, P, false, 3).bytes(1, 1)
-                          : L.bytes(slots, nk);
-  if (!P.split) {
-    size_t avail = 0, total = 0;
-    if (capturing || hipMemGetInfo(&avail, &total) != hipSuccess ||
-        avail < need + (size_t(1) << 30)) {
-      P = OzPlan();
-      return 0;
+// (which moves aa.A too) moves it.  A buffer that a captured graph reads is
+// kept until the context ends when a larger one replaces it.
+int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int most,
+               int nk, bool capturing, OzRoom &room) {
+  size_t want = L.bytes(most, nk), least = L.least(nk);
+  if (use == kOzSingle && !P.split) {
+    const OzLayout all = oz_layout_ops(c, P, false, 3), o = oz_layout_ops(c, P, true, 2);
+    want = all.bytes(1, 1);
+    least = std::max(all.least(1), o.least(1));
+  }
+  DevBuf *b = &c->oz[use][P.split];
+  bool *pinned = &c->oz_pinned[use][P.split];
+  if (b->bytes < least || (b->bytes < want && c->oz_asked[use][P.split] < want && !capturing)) {
+    // under capture nothing should be allocated: the other precision's buffer
+    // serves where there is one
+    if (capturing && c->oz[use][!P.split].bytes >= least) {
+      b = &c->oz[use][!P.split];
+      pinned = &c->oz_pinned[use][!P.split];
+    } else {
+      const int rc = oz_allocate(c, use, P, want, least);
+      if (rc) return rc;
     }
   }
-  const int rc = ensure(c, c->oz[use][P.split], need);
-  if (rc && !P.split) {  // another allocation took the room meanwhile
-    (void)hipGetLastError();
-    P = OzPlan();
-    return 0;
+  if (capturing) *pinned = true;
+  const size_t have = b->bytes - L.exp_bytes() * nk;
+  room.p = (char *)b->p;
+  room.fit = L.full;
+  room.slots = (int)std::min<size_t>(slots, have / L.slot_bytes(L.full));
+  if (room.slots == 0) {
+    room.slots = 1;
+    room.fit = oz_fit(L, have);
   }
-  return rc;
+  return 0;
 }
 
 }  // namespace exh
@@ -539,6 +566,7 @@ void exh_destroy(exh_context *c) {
   batch_release_all(c);
   interstitial_release(c);
   pin_release(c);
+  for (DevBuf &b : c->oz_retired) release(b);
   if (c->done_ev) (void)hipEventDestroy(c->done_ev);
   DevBuf *bufs[] = {&c->colA, &c->katom, &c->atom_species_d, &c->apword_d, &c->omax_d,
                     &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu, &c->mt_match.piv,
@@ -884,7 +912,7 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
   const int nmod = w.plan.nmod;
   const int ldb = (c->ngkmax + 63) / 64 * 64;
   exh_z *hw = o_only ? nullptr : h;  // H the kernels write
-  auto run = [&](int k, auto &&launch) {
+  auto run = [&](int k, const std::function<hipError_t()> &launch) {
     return record ? timed(c, k, s, launch) : launch();
   };
   const double2 *A = (const double2 *)apwalm;
@@ -916,13 +944,7 @@ static int setup_launch(exh_context *c, hipStream_t s, int ngp, int rank, const 
     });
   if (e == hipSuccess && nmod > 0) {
     const int acc = flags & EXH_ACCUMULATE;
-    if (w.oz.chunk < nmod) {
-      e = launch_ozaki(s, d, w.oz.chunk, acc, 7);
-    } else {
-      const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
-      for (int st = 0; st < 3 && e == hipSuccess; st++)
-        e = run(kid[st], [&] { return launch_ozaki(s, d, nmod, acc, 1 << st); });
-    }
+    e = launch_ozaki(s, d, w.oz.fit, acc, run);
   }
   if (e == hipSuccess)
     e = run(EXH_K_LOBORDER, [&] {
@@ -949,11 +971,15 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   if (!rc && c->have_h1aa) rc = ensure(c, c->a2t, op);
   if (!rc && !c->contig) rc = ensure(c, c->at, op);
   if (!rc) rc = ensure(c, c->ivgk, (size_t)std::max(c->ngkmax, 1) * sizeof(int4));
-  if (!rc)
-    rc = oz_prepare(c, kOzSingle, flags, o_only, cap == hipStreamCaptureStatusActive, 1, 1,
-                    w.plan, w.layout);
+  w.plan = oz_plan(c, flags);
+  if (!rc && w.plan.nmod) {
+    OzRoom room;
+    w.layout = oz_layout(c, w.plan, o_only);
+    rc = oz_prepare(c, kOzSingle, w.plan, w.layout, 1, 1, 1, cap == hipStreamCaptureStatusActive,
+                    room);
+    if (!rc) w.oz = oz_scratch(w.layout, room, 0, 0);
+  }
   if (rc) return rc;
-  if (w.plan.nmod) w.oz = oz_scratch(c, kOzSingle, w.plan, w.layout, 1, 0, 0);
   w.bt = (double2 *)c->bt.p;
   w.a2t = (double2 *)c->a2t.p;
   w.at = (double2 *)c->at.p;
@@ -1008,13 +1034,11 @@ int exh_setup_device_noalloc(exh_context *c, void *stream, int ngp, int rank,
   if (!c->contig) w.at = (double2 *)(base + off);
   w.plan = oz_plan(c, flags);
   if (w.plan.nmod) {
-    // [product residues | exponents and norms | residues of `chunk` moduli]
     w.layout = oz_layout(c, w.plan, false);
-    w.oz.chunk = oz_noalloc_chunk(w.plan, w.layout);
-    unsigned char *mod = base + kNoallocScratchBytes;
-    w.oz.r = (int8_t *)mod;
-    w.oz.e = mod + align256(w.layout.r_bytes);
-    w.oz.q = (int8_t *)w.oz.e + align256(w.layout.e_bytes * w.layout.nops);
+    OzRoom room;
+    room.p = (char *)base + kNoallocScratchBytes;
+    room.fit = oz_noalloc_fit(w.layout);
+    w.oz = oz_scratch(w.layout, room, 0, 0);
   }
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   return setup_launch(c, s, ngp, rank, apwalm, igpig, vgpc, h, o, flags, false, w, false);

@@ -33,6 +33,7 @@ struct exh_context::BatchEntry {
   // together (each on its own slot of its context's residue scratch)
   struct Wave {
     int first, count;
+    exh::OzFit fit;
   };
   std::vector<exh::OzK> oz;
   std::vector<Wave> waves;
@@ -227,7 +228,7 @@ CallContexts call_contexts(int nk, exh_context *const *kc) {
 struct OzParams {
   std::vector<OzPlan> P;
   std::vector<OzLayout> L;
-  std::vector<int> slots;  // k-points whose residues the context's scratch holds
+  std::vector<OzRoom> room;  // the context's scratch: k-points at a time, or part of one
 };
 
 // K-points of one context that share a launch of each modular stage: enough
@@ -305,28 +306,32 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
     g.nwg = (int)std::max<long long>(nwg, 0);
     g.w0 = (int)E->waves.size();
     std::vector<int> used(nctx, 0), nth(nctx, 0);
-    exh_context::BatchEntry::Wave wv{(int)E->oz.size(), 0};
+    exh_context::BatchEntry::Wave wv{(int)E->oz.size(), 0, {}};
     auto close_wave = [&]() {
       if (wv.count) E->waves.push_back(wv);
-      wv = exh_context::BatchEntry::Wave{(int)E->oz.size(), 0};
+      wv = exh_context::BatchEntry::Wave{(int)E->oz.size(), 0, {}};
       std::fill(used.begin(), used.end(), 0);
     };
     for (int i = g.k0; i < kend; i++) {
       const int j = cc.kci[i];
       if (!skip[i] || kp[i].ngp <= 0) continue;
-      if (used[j] == oz.slots[j]) close_wave();
+      const bool part = oz.room[j].fit.chunk < oz.L[j].full.chunk ||
+                        oz.room[j].fit.steps < oz.L[j].full.steps;
+      if (used[j] == oz.room[j].slots || part) close_wave();
       const exh_context *c = cc.ctxs[j];
       KDesc &d = E->kd[i];
       const SDesc &S = E->sd[j];
       IstBox box{d.ivgk, d.vgpc, (const IstEntry *)c->ist.p, S.lo0, S.lo1, S.lo2,
                  S.n0, S.n1, S.n2};
       E->oz.push_back(make_ozk(c, d.ngp, oz.P[j], oz.L[j],
-                               oz_scratch(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], used[j],
-                                          nth[j]++),
-                               d.x, S.ldx, d.bt, d.a2t, S.ldb, box, d.h, d.o, d.ldh));
+                               oz_scratch(oz.L[j], oz.room[j], used[j], nth[j]++), d.x, S.ldx,
+                               d.bt, d.a2t, S.ldb, box, d.h, d.o, d.ldh));
       d.norms = norm_out(E->oz.back());
       used[j]++;
       wv.count++;
+      wv.fit = oz.room[j].fit;
+      // products in parts: a launch of its own
+      if (part) close_wave();
     }
     close_wave();
     g.nw = (int)E->waves.size() - g.w0;
@@ -429,12 +434,11 @@ hipError_t enqueue(exh_context *lead, hipStream_t s, const exh_context::BatchEnt
     for (int v = g.w0; v < g.w0 + g.nw && e == hipSuccess; v++) {
       const auto &wv = E.waves[v];
       const OzK *d = E.oz.data() + wv.first, *dd = (const OzK *)E.oz_d.p + wv.first;
-      const int kid[3] = {EXH_K_OZRES, EXH_K_OZGEMM, EXH_K_OZCOMB};
-      for (int st = 0; st < 3 && e == hipSuccess; st++)
-        e = timed(lead, kid[st], s, [&] {
-          return wv.count == 1 ? launch_ozaki(s, *d, d->nmod, acc, 1 << st)
-                               : launch_ozaki_grouped(s, d, dd, wv.count, acc, 1 << st);
-        });
+      const OzRun run = [&](int k, const std::function<hipError_t()> &launch) {
+        return timed(lead, k, s, launch);
+      };
+      e = wv.count == 1 ? launch_ozaki(s, *d, wv.fit, acc, run)
+                        : launch_ozaki_grouped(s, d, dd, wv.count, acc, run);
     }
     if (e == hipSuccess)
       e = timed(lead, EXH_K_LOBORDER, s,
@@ -464,37 +468,29 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   OzParams oz;
   oz.P.resize(nctx);
   oz.L.resize(nctx);
-  oz.slots.assign(nctx, 1);
+  oz.room.resize(nctx);
   for (size_t j = 0; j < nctx; j++) {
     exh_context *c = cc.ctxs[j];
     oz.P[j] = oz_plan(c, flags);
-    int most = 1;
-    if (oz.P[j].nmod) {
-      oz.L[j] = oz_layout(c, oz.P[j], false);
-      oz.slots[j] = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j], &most);
-    }
+    // nothing may be allocated or uploaded inside a caller's capture
     if (outer_capture) {
-      // nothing may be allocated or uploaded inside a caller's capture
-      if (oz.P[j].nmod && !oz_fits(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], cc.nkg[j])) oz.slots[j] = 1;
-      const bool oz_ok = oz.P[j].nmod == 0 || oz_fits(c, kOzGroup, oz.P[j], oz.L[j], 1, cc.nkg[j]);
-      if (!oz_ok && !nmod) oz.P[j] = OzPlan();  // as the call outside capture ran
-      if (!scratch_fits(c, cc.nkg[j]) || (nmod && !oz_ok))
+      if (!scratch_fits(c, cc.nkg[j]))
         return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
     } else {
       rc = ensure_scratch(c, cc.nkg[j]);
-      if (!rc && oz.P[j].nmod && !oz_fits(c, kOzGroup, oz.P[j], oz.L[j], oz.slots[j], cc.nkg[j])) {
-        // several slots only where the device has room for them
-        size_t avail = 0, total = 0;
-        if (oz.slots[j] > 1 &&
-            (hipMemGetInfo(&avail, &total) != hipSuccess ||
-             avail < oz.L[j].bytes(most, cc.nkg[j]) + (size_t(2) << 30)))
-          oz.slots[j] = most = 1;
-        rc = oz_prepare(c, kOzGroup, flags, false, false, most, cc.nkg[j], oz.P[j], oz.L[j]);
-      }
-      if (rc) {
-        if (c != lead) fail(lead, rc, c->err);
-        return rc;
-      }
+    }
+    if (!rc && oz.P[j].nmod) {
+      int most = 1;
+      oz.L[j] = oz_layout(c, oz.P[j], false);
+      const int slots = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j], &most);
+      if (outer_capture && c->oz[kOzGroup][oz.P[j].split].bytes < oz.L[j].least(cc.nkg[j]))
+        return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
+      rc = oz_prepare(c, kOzGroup, oz.P[j], oz.L[j], slots, most, cc.nkg[j], outer_capture,
+                      oz.room[j]);
+    }
+    if (rc) {
+      if (c != lead) fail(lead, rc, c->err);
+      return rc;
     }
   }
   // key: arguments, plan, and per context its address, group size,
@@ -511,7 +507,7 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
     const uint64_t sig[3] = {(uint64_t)(uintptr_t)c, c->epoch, state_signature(c)};
     put(sig, sizeof sig);
     put(&cc.nkg[j], sizeof(int));
-    const int route[2] = {oz.P[j].nmod, oz.slots[j]};
+    const int route[4] = {oz.P[j].nmod, oz.room[j].slots, oz.room[j].fit.chunk, oz.room[j].fit.steps};
     put(route, sizeof route);
   }
   put(kp, nk * sizeof(exh_kpoint));
@@ -634,11 +630,7 @@ int exh_tune_batch(exh_context *c, void *stream, int nk, const exh_kpoint *kp, i
   if (nk == 0) return fail(c, EXH_EINVAL, "tune: no k-points");
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, EXH_ESTATE, "hipSetDevice");
   hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-  OzPlan P;
-  OzLayout L;
-  rc = oz_prepare(c, kOzGroup, flags, false, false, 1, 1, P, L);
-  if (rc) return rc;
-  if (P.nmod) {  // no tiles to shape: every plan is the same call
+  if (oz_plan(c, flags).nmod) {  // no tiles to shape: every plan is the same call
     rc = exh_setup_batch_device(c, s, nk, kp, flags);
     if (!rc && plan) *plan = exh_get_batch_plan(c);
     return rc;

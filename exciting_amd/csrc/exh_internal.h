@@ -3,7 +3,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -50,24 +52,37 @@ struct OzPlan {
   int bits = 0;  // c: the scaled columns' 2-norms are below 2^(c-1)
   bool split = false;  // EXH_SPLIT(n)
 };
+// What of a setup's modular products is in flight at a time: the residues of
+// `chunk` moduli, and the products of `steps` column steps of the matrices.
+// The products are exact, so H and O do not depend on it.
+struct OzFit {
+  int chunk = 0, steps = 0;
+};
 struct OzLayout {
   int Gpad = 0, Kpad = 0;  // G rounded to the 128 tile, K to two 64-k stages
   size_t qstride = 0;      // bytes of one residue array (Kpad * Gpad)
   int nops = 0;            // operands (X; B unless O alone; (1+h1)A for iora*)
-  size_t q_bytes = 0;      // residues of one operand
-  size_t r_bytes = 0;      // residues of the products
+  int nt = 0, width = 1;   // 128-column blocks at ngkmax, and those of a column step
+  int planes = 0;          // residue planes of the products: matrices x signs x moduli
+  OzFit full;              // everything at once
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
   int nch = 0;             // partial norms of an operand, at most
   long long panels = 0;    // workgroups of the products at ngkmax
+  size_t q_bytes(int chunk) const { return align256(2 * qstride * nops * chunk); }
+  size_t r_bytes(int steps) const {  // of the last `steps` column steps, the largest
+    const size_t j0 = (size_t)std::max(0, full.steps - steps) * width;
+    return (size_t)planes * (((size_t)nt * (nt + 1) - j0 * (j0 + 1)) / 2) * 128 * 128;
+  }
   // residues of one k-point's operands and products; its exponents and norms
-  size_t slot_bytes() const { return align256(q_bytes * nops) + align256(r_bytes); }
+  size_t slot_bytes(const OzFit &f) const { return q_bytes(f.chunk) + r_bytes(f.steps); }
   size_t exp_bytes() const { return e_bytes * nops; }
-  size_t bytes(int slots, int nk) const { return slot_bytes() * slots + exp_bytes() * nk; }
+  size_t bytes(int slots, int nk) const { return slot_bytes(full) * slots + exp_bytes() * nk; }
+  size_t least(int nk) const { return slot_bytes({1, 1}) + exp_bytes() * nk; }
 };
 struct OzScratch {
   int8_t *q = nullptr, *r = nullptr;
   void *e = nullptr;
-  int chunk = 0;  // moduli whose residues q holds
+  OzFit fit;
 };
 
 // Partial squared column norms of the modular contraction's operands, as bt
@@ -262,6 +277,9 @@ struct exh_context {
   // so that a single setup may run beside a grouped call on another stream, and
   // no other kind of call frees what a caller's captured graph of one reads.
   exh::DevBuf oz[2][2];
+  size_t oz_asked[2][2] = {{0, 0}, {0, 0}};  // room that was wanted when it was allocated
+  bool oz_pinned[2][2] = {{false, false}, {false, false}};  // a captured graph reads it
+  std::vector<exh::DevBuf> oz_retired;  // pinned ones that a larger one has replaced
   bool contig = true;  // colA[k] == k * ngkmax
   // host-API staging
   exh::DevBuf s_apwalm, s_igpig, s_vgpc, s_h, s_o, s_gpc, s_tpgpc, s_sfac;
@@ -345,21 +363,24 @@ OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o);
 OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int nops);
 NormOut norm_out(const OzK &d);
 OzPlan oz_plan(const exh_context *c, int flags);
-int oz_noalloc_chunk(const OzPlan &P, const OzLayout &L);
+OzFit oz_fit(const OzLayout &L, size_t bytes);
+OzFit oz_noalloc_fit(const OzLayout &L);
 enum OzUse { kOzSingle, kOzGroup };
-bool oz_fits(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots,
-             int nk);
-int oz_prepare(exh_context *c, OzUse use, int flags, bool only_o, bool capturing, int slots,
-               int nk, OzPlan &P, OzLayout &L);
-// Residue slot `slot` of `slots`, norms of k-point `k` of the group.
-inline OzScratch oz_scratch(const exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L,
-                            int slots, int slot, int k) {
-  char *p = (char *)c->oz[use][P.split].p;
+// Scratch of the modular contraction of one call, resolved by oz_prepare.
+struct OzRoom {
+  char *p = nullptr;
+  int slots = 1;
+  OzFit fit;
+};
+int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int most,
+               int nk, bool capturing, OzRoom &room);
+// Residue slot `slot`, norms of k-point `k` of the group.
+inline OzScratch oz_scratch(const OzLayout &L, const OzRoom &m, int slot, int k) {
   OzScratch w;
-  w.q = (int8_t *)p + slot * L.slot_bytes();
-  w.r = w.q + align256(L.q_bytes * L.nops);
-  w.e = p + slots * L.slot_bytes() + k * L.exp_bytes();
-  w.chunk = P.nmod;
+  w.q = (int8_t *)m.p + slot * L.slot_bytes(m.fit);
+  w.r = w.q + L.q_bytes(m.fit.chunk);
+  w.e = m.p + m.slots * L.slot_bytes(m.fit) + k * L.exp_bytes();
+  w.fit = m.fit;
   return w;
 }
 // h = nullptr: O alone (B is not read).  Y = nullptr: the overlap's column
@@ -367,10 +388,12 @@ inline OzScratch oz_scratch(const exh_context *c, OzUse use, const OzPlan &P, co
 OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
              const OzScratch &w, const double2 *X, long long ldx, const double2 *B,
              const double2 *Y, long long ldb, const IstBox &box, double2 *h, double2 *o, int ldh);
-// stage_mask: 1 norms and residues, 2 products, 4 reconstruction.
-hipError_t launch_ozaki(hipStream_t s, const OzK &d, int chunk, int accumulate, int stage_mask);
+// Enqueues one launch of kernel id k (profiling events around it, or not).
+using OzRun = std::function<hipError_t(int k, const std::function<hipError_t()> &launch)>;
+hipError_t launch_ozaki(hipStream_t s, const OzK &d, const OzFit &fit, int accumulate,
+                        const OzRun &run);
 hipError_t launch_ozaki_grouped(hipStream_t s, const OzK *d, const OzK *kd, int n, int accumulate,
-                                int stage_mask);
+                                const OzRun &run);
 // tab: match_table_bytes(c) of scratch for the k-point's radial factors and
 // spherical harmonics
 size_t match_table_bytes(const exh_context *c);

@@ -372,7 +372,7 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
 // so that each store instruction writes 256 contiguous bytes here and each
 // load instruction of the reconstruction reads them.
 __device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], const OzMod &M,
-                                               int rg, int wc, int lane, int IT, int J,
+                                               int rg, int wc, int lane, int IT, int J, int t0,
                                                EXH_G int8_t *Rp) {
   const double p = M.p, rp = M.rp, nk = M.nk;
 #pragma unroll
@@ -380,7 +380,7 @@ __device__ __forceinline__ void store_residues(const v16i (&acc)[OZ_WR][2], cons
     const int row = IT * OZ_R + rg * 32 * OZ_WR + a * 32;
     const int I = row >> 7;
     if (I > J) continue;  // below the diagonal (uniform per wave)
-    EXH_G int8_t *out = Rp + ((long long)J * (J + 1) / 2 + I) * (OZ_T * OZ_T) + 4 * lane;
+    EXH_G int8_t *out = Rp + ((long long)J * (J + 1) / 2 + I - t0) * (OZ_T * OZ_T) + 4 * lane;
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -410,12 +410,22 @@ __host__ __device__ inline int oz_last(int j, int nt) {
   return l < nt ? l : nt - 1;
 }
 
-// Panels per GEMM.
+// Panels per GEMM, of the column steps s0 .. s1 - 1.
 template <bool ONLY_O>
-__host__ __device__ inline long long oz_panels(int nt) {
+__host__ __device__ inline long long oz_panels(int nt, int s0, int s1) {
   long long n = 0;
-  for (int j = 0; j < oz_steps<ONLY_O>(nt); j++) n += oz_npan(oz_last<ONLY_O>(j, nt));
+  for (int j = s0; j < min(s1, oz_steps<ONLY_O>(nt)); j++) n += oz_npan(oz_last<ONLY_O>(j, nt));
   return n;
+}
+
+// Tiles of those steps: the first one's number, and how many.
+struct OzTiles {
+  int t0, n;
+};
+template <bool ONLY_O>
+__host__ __device__ inline OzTiles oz_tiles(int nt, int s0, int s1) {
+  const int w = ONLY_O ? 2 : 1, a = min(nt, s0 * w), b = min(nt, min(s1, oz_steps<ONLY_O>(nt)) * w);
+  return {a * (a + 1) / 2, max(0, b * (b + 1) / 2 - a * (a + 1) / 2)};
 }
 
 // Panel order: super-columns of OZ_SJ column steps, each walked in chunks
@@ -425,12 +435,12 @@ __host__ __device__ inline long long oz_panels(int nt) {
 // panels); 3.6 % faster at the 64-atom shape, bitwise the same products.
 constexpr int OZ_SJ = 8, OZ_SI = 4 * 384 / OZ_R;
 
-// Panel o of one GEMM -> (column step J, row panel IT).
+// Panel o of one GEMM's steps s0 .. s1 - 1 -> (column step J, row panel IT).
 template <bool ONLY_O>
-__device__ __forceinline__ void oz_panel_at(int o, int nt, int &J, int &IT) {
-  const int ns = oz_steps<ONLY_O>(nt);
+__device__ __forceinline__ void oz_panel_at(int o, int nt, int s0, int s1, int &J, int &IT) {
+  const int ns = min(s1, oz_steps<ONLY_O>(nt));
   auto npan = [&](int j) { return oz_npan(oz_last<ONLY_O>(j, nt)); };
-  int rem = o, j0 = 0;
+  int rem = o, j0 = s0;
   for (;; j0 += OZ_SJ) {
     const int j1 = min(ns, j0 + OZ_SJ);
     int cnt = 0;
@@ -461,12 +471,12 @@ __device__ __forceinline__ void oz_panel_at(int o, int nt, int &J, int &IT) {
 
 // Residues of the moduli m0 .. m0 + mc - 1 are in d.q, counted from m0.
 template <bool ONLY_O>
-__device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc) {
+__device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc, int s0, int s1) {
   const int nt = d.nt, nslab = d.nslab, Gpad = d.Gpad;
   const size_t qstride = d.qstride;
   // XCD-contiguous remap over the k-point's panels (its first block runs on
   // XCD 0: the grid's x extent is a multiple of 8), then (sign * mc + m, panel)
-  const int per = (int)oz_panels<ONLY_O>(nt);
+  const int per = (int)oz_panels<ONLY_O>(nt, s0, s1);
   const int bid = blockIdx.x, nb = per * 2 * mc;
   if (bid >= nb) return;
   const int xcd = bid & 7, i8 = bid >> 3, q8 = nb >> 3, r8 = nb & 7;
@@ -474,11 +484,11 @@ __device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc) {
   const int qm = __builtin_amdgcn_readfirstlane(t / per), o = t - qm * per;
   const int q = qm >= mc ? 1 : 0, m = qm - q * mc;  // q = 0: sign +, 1: sign -
   int J, IT;
-  oz_panel_at<ONLY_O>(o, nt, J, IT);
+  oz_panel_at<ONLY_O>(o, nt, s0, s1, J, IT);
   // uniform by construction; scalar registers for the addresses that follow
   J = __builtin_amdgcn_readfirstlane(J);
   IT = __builtin_amdgcn_readfirstlane(IT);
-  const long long npairs = (long long)nt * (nt + 1) / 2;
+  const OzTiles T = oz_tiles<ONLY_O>(nt, s0, s1);
   const int JH = ONLY_O ? 2 * J : J, JO = ONLY_O ? 2 * J + 1 : J;
   const int I0 = IT * OZ_R, H0 = JH * OZ_T;
   // past the last block (odd nt): any valid columns, not stored
@@ -601,14 +611,14 @@ __device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 
   // planes: (H+, H-, O+, O-) x modulus, or (O+, O-) x modulus
-  const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
+  const size_t plane = (size_t)T.n * (OZ_T * OZ_T);
   EXH_G int8_t *Rq = gptr(d.r) + (size_t)(q * d.nmod + m0 + m) * plane;
   const OzMod &M = c_mod.m[m0 + m];
-  store_residues(ah, M, rg, wc, lane, IT, JH, Rq);
+  store_residues(ah, M, rg, wc, lane, IT, JH, T.t0, Rq);
   if (ONLY_O) {
-    if (JO < nt) store_residues(ao, M, rg, wc, lane, IT, JO, Rq);
+    if (JO < nt) store_residues(ao, M, rg, wc, lane, IT, JO, T.t0, Rq);
   } else {
-    store_residues(ao, M, rg, wc, lane, IT, JO, Rq + (size_t)2 * d.nmod * plane);
+    store_residues(ao, M, rg, wc, lane, IT, JO, T.t0, Rq + (size_t)2 * d.nmod * plane);
   }
 }
 
@@ -634,10 +644,11 @@ __device__ __forceinline__ double crt(double hi, double lo) {
 }
 
 template <int NM, bool ONLY_O>
-__device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate) {
-  const int tile = blockIdx.x >> 4, sb = blockIdx.x & 15;
-  const int npairs = d.nt * (d.nt + 1) / 2, ngp = d.ngp, bits = d.bits;
-  if (tile >= npairs) return;
+__device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate, int s0, int s1) {
+  const OzTiles T = oz_tiles<ONLY_O>(d.nt, s0, s1);
+  const int sb = blockIdx.x & 15, ngp = d.ngp, bits = d.bits;
+  if ((int)(blockIdx.x >> 4) >= T.n) return;
+  const int tile = T.t0 + (int)(blockIdx.x >> 4);
   const EXH_G int *ex = gptr((const int *)d.e[0]);
   const EXH_G int *eb = gptr((const int *)d.e[d.iB]), *ey = gptr((const int *)d.e[d.iY]);
   EXH_G double2 *H = gptr(d.h), *O = gptr(d.o);
@@ -655,8 +666,8 @@ __device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate) {
   __shared__ double2 sT[NV][32][33];
   const int tid = threadIdx.x, lane = tid & 63, h = tid >> 6;
   const int il = 8 * h + 4 * (lane >> 5), jl = lane & 31;
-  const size_t plane = (size_t)npairs * (OZ_T * OZ_T);
-  const EXH_G int8_t *r0 = gptr((const int8_t *)d.r) + (size_t)tile * (OZ_T * OZ_T) + sb * 1024 + tid * 4;
+  const size_t plane = (size_t)T.n * (OZ_T * OZ_T);
+  const EXH_G int8_t *r0 = gptr((const int8_t *)d.r) + (size_t)(tile - T.t0) * (OZ_T * OZ_T) + sb * 1024 + tid * 4;
 
   double rh[NV][4], rl[NV][4], mh[NV][4], ml[NV][4];
 #pragma unroll
@@ -768,21 +779,21 @@ __global__ __launch_bounds__(256) void residue_grouped_kernel(const OzK *__restr
 // two waves per SIMD whatever the workgroup size: at most 256 VGPRs
 template <bool ONLY_O>
 __global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-ozgemm_kernel(OzK d, int m0, int mc) {
-  ozgemm_body<ONLY_O>(d, m0, mc);
+ozgemm_kernel(OzK d, int m0, int mc, int s0, int s1) {
+  ozgemm_body<ONLY_O>(d, m0, mc, s0, s1);
 }
 __global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 ozgemm_grouped_kernel(const OzK *__restrict__ kd, int mc) {
-  ozgemm_body<false>(kd[blockIdx.y], 0, mc);
+  ozgemm_body<false>(kd[blockIdx.y], 0, mc, 0, INT_MAX / 2);
 }
 template <int NM, bool ONLY_O>
-__global__ __launch_bounds__(256) void ozcombine_kernel(OzK d, int accumulate) {
-  ozcombine_body<NM, ONLY_O>(d, accumulate);
+__global__ __launch_bounds__(256) void ozcombine_kernel(OzK d, int accumulate, int s0, int s1) {
+  ozcombine_body<NM, ONLY_O>(d, accumulate, s0, s1);
 }
 template <int NM>
 __global__ __launch_bounds__(256) void ozcombine_grouped_kernel(const OzK *__restrict__ kd,
                                                                 int accumulate) {
-  ozcombine_body<NM, false>(kd[blockIdx.y], accumulate);
+  ozcombine_body<NM, false>(kd[blockIdx.y], accumulate, 0, INT_MAX / 2);
 }
 
 inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
@@ -825,9 +836,11 @@ OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int n
   L.Gpad = (ngkmax + OZ_T - 1) / OZ_T * OZ_T;
   L.Kpad = (Ktot + 2 * OZ_KS - 1) / (2 * OZ_KS) * (2 * OZ_KS);  // an even number of stages
   L.qstride = (size_t)L.Kpad * L.Gpad;
-  const long long nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
-  L.q_bytes = (size_t)P.nmod * 2 * L.qstride;
-  L.r_bytes = (size_t)(only_o ? 2 : 4) * P.nmod * (nt * (nt + 1) / 2) * OZ_T * OZ_T;
+  const int nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
+  L.nt = nt;
+  L.width = only_o ? 2 : 1;
+  L.planes = (only_o ? 2 : 4) * P.nmod;
+  L.full = {P.nmod, std::max(1, only_o ? oz_steps<true>(nt) : oz_steps<false>(nt))};
   // per operand: the column exponents, then the partial norms and their marks
   const size_t ng = std::max(ngkmax, 1);
   const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
@@ -835,8 +848,35 @@ OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int n
   L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
   L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * L.nch * ng + 255) / 256 * 256;
   L.nops = nops;
-  L.panels = 2 * P.nmod * (only_o ? oz_panels<true>((int)nt) : oz_panels<false>((int)nt));
+  L.panels = 2 * P.nmod * (only_o ? oz_panels<true>(nt, 0, nt) : oz_panels<false>(nt, 0, nt));
   return L;
+}
+
+// The largest part of the products that fits in `bytes` (chunk = 0: none).
+// Fewer moduli at a time cost a pass over the operands each; fewer column
+// steps cost nothing while the residues of every modulus are there, and
+// otherwise all of those passes again, so they come last.
+OzFit oz_fit(const OzLayout &L, size_t bytes) {
+  auto even = [](int n, int most) {  // n in equal parts of at most `most`
+    const int parts = (n + most - 1) / most;
+    return (n + parts - 1) / parts;
+  };
+  auto chunks = [&](size_t room) {
+    return (int)std::min<size_t>(L.full.chunk, room / std::max<size_t>(L.q_bytes(1), 1));
+  };
+  const size_t r = L.r_bytes(L.full.steps);
+  OzFit f = L.full;
+  if (L.slot_bytes(f) <= bytes) return f;
+  if (r < bytes && (f.chunk = chunks(bytes - r)) > 0) {
+    f.chunk = even(L.full.chunk, f.chunk);
+    return f;
+  }
+  const int eighth = std::max(1, L.full.steps / 8);
+  f.chunk = L.slot_bytes({L.full.chunk, eighth}) <= bytes ? L.full.chunk : 1;
+  for (f.steps = L.full.steps; f.steps > 0 && L.slot_bytes(f) > bytes;) f.steps--;
+  if (f.steps == 0) return OzFit();
+  f.steps = even(L.full.steps, f.steps);
+  return f;
 }
 
 NormOut norm_out(const OzK &d) {
@@ -863,7 +903,7 @@ OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
   d.bits = P.bits;
   d.ldp = std::max(c->ngkmax, 1);
   d.qstride = L.qstride;
-  d.q_bytes = w.chunk * 2 * L.qstride;
+  d.q_bytes = w.fit.chunk * 2 * L.qstride;
   d.q = w.q;
   d.r = w.r;
   d.box = box;
@@ -891,11 +931,9 @@ OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
 }
 
 // One k-point (kd null: by value from d) or the n k-points d[0..n) that kd
-// holds in device memory.  chunk: moduli whose residues the scratch holds; a
-// chunk below nmod runs residues and products in turn (all stages in one
-// call).
-static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, int chunk,
-                            int accumulate, int stage_mask) {
+// holds in device memory; grouped ones have room for everything at once.
+static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, const OzFit &fit,
+                            int accumulate, const OzRun &run) {
   const bool only_o = d[0].h == nullptr;
   const int nmod = d[0].nmod;
   int ngp = 0, nch = 0, nops = 0, kb = 0, nt = 0;
@@ -909,7 +947,7 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
   }
   if (ngp <= 0) return hipSuccess;
   const unsigned nz = (unsigned)(nops * n);
-  if (stage_mask & 1) {
+  auto norms = [&] {
     const dim3 gp(cdiv(ngp, 64), nch, nz), gf(cdiv(ngp, 64), 1, nz);
     if (kd) {
       if (nch) hipLaunchKernelGGL(colnorm_part_grouped_kernel, gp, dim3(256), 0, s, kd, nops);
@@ -918,35 +956,31 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
       if (nch) hipLaunchKernelGGL(colnorm_part_kernel, gp, dim3(256), 0, s, d[0]);
       hipLaunchKernelGGL(colnorm_final_kernel, gf, dim3(256), 0, s, d[0]);
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  const dim3 gr(cdiv(nt * OZ_T, 256), kb, nz);
-  const long long per = only_o ? oz_panels<true>(nt) : oz_panels<false>(nt);
-  for (int m0 = 0; m0 < nmod; m0 += chunk) {
-    const int m1 = std::min(nmod, m0 + chunk);
-    if (stage_mask & 1) {
-      if (kd) hipLaunchKernelGGL(residue_grouped_kernel, gr, dim3(256), 0, s, kd, nops, m1);
-      else hipLaunchKernelGGL(residue_kernel, gr, dim3(256), 0, s, d[0], m0, m1);
-    }
-    if (stage_mask & 2) {
-      const long long nb = per * 2 * (m1 - m0);
-      const dim3 gg((unsigned)((nb + 7) / 8 * 8), n);
-      if (kd)
-        hipLaunchKernelGGL(ozgemm_grouped_kernel, gg, dim3(64 * OZ_NWG), 0, s, kd, m1 - m0);
-      else if (only_o)
-        hipLaunchKernelGGL(ozgemm_kernel<true>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0);
-      else
-        hipLaunchKernelGGL(ozgemm_kernel<false>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0);
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  if (stage_mask & 4) {
-    const dim3 grid((unsigned)(nt * (nt + 1) / 2 * 16), n);
+  };
+  auto residues = [&](int m0, int m1) {
+    const dim3 gr(cdiv(nt * OZ_T, 256), kb, nz);
+    if (kd) hipLaunchKernelGGL(residue_grouped_kernel, gr, dim3(256), 0, s, kd, nops, m1);
+    else hipLaunchKernelGGL(residue_kernel, gr, dim3(256), 0, s, d[0], m0, m1);
+  };
+  auto products = [&](int m0, int m1, int s0, int s1) {
+    const long long per = only_o ? oz_panels<true>(nt, s0, s1) : oz_panels<false>(nt, s0, s1);
+    const dim3 gg((unsigned)((per * 2 * (m1 - m0) + 7) / 8 * 8), n);
+    if (kd)
+      hipLaunchKernelGGL(ozgemm_grouped_kernel, gg, dim3(64 * OZ_NWG), 0, s, kd, m1 - m0);
+    else if (only_o)
+      hipLaunchKernelGGL(ozgemm_kernel<true>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0, s0,
+                         s1);
+    else
+      hipLaunchKernelGGL(ozgemm_kernel<false>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0, s0,
+                         s1);
+  };
+  auto combine = [&](int s0, int s1) {
+    const OzTiles T = only_o ? oz_tiles<true>(nt, s0, s1) : oz_tiles<false>(nt, s0, s1);
+    const dim3 grid((unsigned)T.n * 16, n);
     if (only_o) {
       if (nmod != OZ_N) return hipErrorInvalidValue;  // EXH_SPLIT is refused for O alone
-      hipLaunchKernelGGL((ozcombine_kernel<OZ_N, true>), grid, dim3(256), 0, s, d[0], accumulate);
+      hipLaunchKernelGGL((ozcombine_kernel<OZ_N, true>), grid, dim3(256), 0, s, d[0], accumulate,
+                         s0, s1);
       return hipGetLastError();
     }
 #define EXH_OZC(N)                                                                              \
@@ -954,7 +988,8 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
     if (kd)                                                                                     \
       hipLaunchKernelGGL(ozcombine_grouped_kernel<N>, grid, dim3(256), 0, s, kd, accumulate);   \
     else                                                                                        \
-      hipLaunchKernelGGL((ozcombine_kernel<N, false>), grid, dim3(256), 0, s, d[0], accumulate); \
+      hipLaunchKernelGGL((ozcombine_kernel<N, false>), grid, dim3(256), 0, s, d[0], accumulate, \
+                         s0, s1);                                                               \
     break;
     switch (nmod) {
       EXH_OZC(6)
@@ -969,17 +1004,40 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, i
         return hipErrorInvalidValue;
     }
 #undef EXH_OZC
+    return hipGetLastError();
+  };
+  const int ns = only_o ? oz_steps<true>(nt) : oz_steps<false>(nt);
+  hipError_t e = hipSuccess;
+  for (int s0 = 0; s0 < ns && e == hipSuccess; s0 += fit.steps) {
+    const int s1 = std::min(ns, s0 + fit.steps);
+    for (int m0 = 0; m0 < nmod && e == hipSuccess; m0 += fit.chunk) {
+      const int m1 = std::min(nmod, m0 + fit.chunk);
+      // residues that an earlier strip has left are still there
+      if (s0 == 0 || fit.chunk < nmod)
+        e = run(EXH_K_OZRES, [&] {
+          if (s0 == 0 && m0 == 0) norms();
+          residues(m0, m1);
+          return hipGetLastError();
+        });
+      if (e == hipSuccess)
+        e = run(EXH_K_OZGEMM, [&] {
+          products(m0, m1, s0, s1);
+          return hipGetLastError();
+        });
+    }
+    if (e == hipSuccess) e = run(EXH_K_OZCOMB, [&] { return combine(s0, s1); });
   }
-  return hipGetLastError();
+  return e;
 }
 
-hipError_t launch_ozaki(hipStream_t s, const OzK &d, int chunk, int accumulate, int stage_mask) {
-  return launch_oz(s, &d, nullptr, 1, chunk, accumulate, stage_mask);
+hipError_t launch_ozaki(hipStream_t s, const OzK &d, const OzFit &fit, int accumulate,
+                        const OzRun &run) {
+  return launch_oz(s, &d, nullptr, 1, fit, accumulate, run);
 }
 
 hipError_t launch_ozaki_grouped(hipStream_t s, const OzK *d, const OzK *kd, int n, int accumulate,
-                                int stage_mask) {
-  return launch_oz(s, d, kd, n, d[0].nmod, accumulate, stage_mask);
+                                const OzRun &run) {
+  return launch_oz(s, d, kd, n, {d[0].nmod, INT_MAX / 2}, accumulate, run);
 }
 
 }  // namespace exh

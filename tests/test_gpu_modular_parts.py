@@ -1,0 +1,102 @@
+"""The modular products in parts: where the scratch does not hold the residues
+of all moduli, they run a few at a time, and H and O are bitwise the same.
+Neither the static array's size nor the device's free memory decides which
+kernels run.
+"""
+import numpy as np
+import pytest
+
+from exciting_amd import lapw, synth
+from tests import _cases
+from tests.test_zz_no_alloc import prepared, run
+
+STATIC = 256 << 20   # the static array's part for the modular products
+
+
+def grid12(lmax, rgkmax):
+    rng = np.random.default_rng(78)
+    n = (2, 2, 3)
+    pts = [[], []]
+    for s in np.ndindex(*n):
+        pts[sum(s) % 2].append((np.array(s, float) + rng.normal(0, 0.01, 3)) / np.array(n))
+    return synth.build(synth.CellSpec(
+        name="c12", avec=5.13 * np.diag(np.array(n, float)), positions=[np.array(p) for p in pts],
+        rmt=[2.0, 2.0], lmaxapw=lmax, lmaxmat=lmax, apword=2, lo_l=[[0, 1], [0]],
+        rgkmax=rgkmax, gmaxvr=12.0, kpoints=np.array([[0.11, 0.23, 0.31]]), seed=5))
+
+
+def system(name):
+    if name == "c12_lmax6_iora":
+        return synth.add_relativity(grid12(6, 7.9), seed=6, iora=True)
+    return grid12(8, 8.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,nops", [("c12_lmax6_iora", 3), ("c12_lmax8", 2)])
+def test_static_array_that_holds_some_moduli(name, nops):
+    import torch
+    s = system(name)
+    pad = lambda n, m: -(-n // m) * m
+    K, G = s.natmtot * s.maxaa, pad(s.ngkmax, 128)
+    nt = G // 128
+    full = 15 * 2 * nops * pad(K, 128) * G + 60 * nt * (nt + 1) // 2 * 128 * 128
+    assert 16 * K * pad(s.ngkmax, 64) * (nops - 1) <= 64 << 20 and full > STATIC
+    ctx = lapw.Context(0).load(s)
+    try:
+        d = prepared(ctx, s)
+        print(f"[parts] {name}: K {K} ngk {d.ngk}, residues {full >> 20} MiB", flush=True)
+        g = torch.Generator(device="cuda").manual_seed(3)
+        pre = [torch.randn(d.rank ** 2, dtype=torch.complex128, device="cuda", generator=g)
+               for _ in range(2)]
+        for flags, p in ((0, None), (lapw.ACCUMULATE, pre)):
+            Hd, Od = run(ctx, d, False, flags, p)
+            Hn, On = run(ctx, d, True, flags, p)
+            assert torch.equal(Hn, Hd) and torch.equal(On, Od)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.gpu
+def test_route_and_bits_do_not_depend_on_free_memory():
+    """With about 1.1 GiB left on the device, below what the residues and the
+    margin for the caller need."""
+    import torch
+    s = _cases.system("sc8_4k")
+
+    def setups():
+        ctx = lapw.Context(0).load(s)
+        try:
+            ctx.profile(True)
+            ctx.profile_reset()
+            out = []
+            dk = [lapw.DeviceKPoint(s, i) for i in range(2)]
+            for d in dk:
+                ctx.match(d.ngk, d.gpc, d.tpgpc, d.sfacgp, d.apwalm)
+            out += run(ctx, dk[0], False, 0)
+            y = lapw.newsystem(dk[1].rank, device="cuda")
+            ctx.overlapsetup(lapw.EvSystem(None, y.overlap), dk[1].ngk, dk[1].apwalm,
+                             dk[1].igpig, dk[1].vgpc, flags=0)
+            out.append(y.overlap.za)
+            ys = [lapw.newsystem(d.rank, device="cuda") for d in dk]
+            ctx.setup_batch([lapw.kpoint_struct(d, v.hamilton.za, v.overlap.za)
+                             for d, v in zip(dk, ys)], flags=0)
+            torch.cuda.synchronize()
+            ran = {n for n, v in ctx.profile_read().items() if v[1]}
+            return out + [m.za for v in ys for m in (v.hamilton, v.overlap)], ran
+        finally:
+            ctx.close()
+
+    ref, ran = setups()
+    assert "oz_gemm" in ran and not ran & {"ho", "ho_grouped"}
+    torch.cuda.empty_cache()
+    free, _ = torch.cuda.mem_get_info()
+    hog = torch.empty(free - (1100 << 20), dtype=torch.uint8, device="cuda")
+    try:
+        print(f"[parts] {torch.cuda.mem_get_info()[0] >> 20} MiB free", flush=True)
+        got, ran = setups()
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    assert "oz_gemm" in ran and not ran & {"ho", "ho_grouped"}
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
