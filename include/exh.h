@@ -86,10 +86,12 @@ enum {
  * with c = 56: each operand keeps 55 bits relative to its column's 2-norm and
  * nothing else is rounded before the result, which is nearer to the exact
  * product than FP64 accumulation over K (H and O at 64 atoms: relative
- * Frobenius error 1e-16 against 5e-15).  They need 60 bytes of scratch per
- * (K, G+k) pair and 60 per upper element of H; a device without that room, or
- * a stream captured before a first call has allocated it, runs the FP64 MFMA
- * kernels instead (results differ by rounding). */
+ * Frobenius error 1e-16 against 5e-15).  They take 60 bytes of scratch per
+ * (K, G+k) pair and 60 per upper element of H, or, where the device has less
+ * beside 1 GiB, run in parts in what there is, with bitwise the same results
+ * (4 bytes per pair and a few columns of H at least; without that the call
+ * fails with the runtime's out-of-memory code).  Which kernels run depends on
+ * the basis only. */
 #define EXH_SPLIT(n) ((n) << 8)
 
 /* ---- context ------------------------------------------------------------ */
