@@ -445,20 +445,20 @@ static int oz_allocate(exh_context *c, OzUse use, const OzPlan &P, size_t want, 
 }
 
 // Scratch of the modular contraction for nk k-points, the residues of `slots`
-// of them at a time (`most`: of as many as any call with this list's length
-// may take).  Neither free memory nor capture decides where a setup runs:
-// where there is no room for everything at once, the products run in parts
-// (oz_fit), with the same results; only a device without room for one modulus
-// and one column step fails.
+// of them at a time, out of `want` bytes (a single FP64 call's are its own).
+// Neither free memory nor capture decides where a setup runs: where there is no
+// room for everything at once, the products run in parts (oz_fit), with the
+// same results; only a device without room for one modulus and one column step
+// fails.
 //
 // The buffer of a single FP64 setup has the size of the basis alone, as the
 // other scratch of that call: O alone and the full setup, with or without h1aa,
 // all get the room that the largest of them needs, so only a larger basis
 // (which moves aa.A too) moves it.  A buffer that a captured graph reads is
 // kept until the context ends when a larger one replaces it.
-int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int most,
-               int nk, bool capturing, OzRoom &room) {
-  size_t want = L.bytes(most, nk), least = L.least(nk);
+int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int nk,
+               size_t want, bool capturing, OzRoom &room) {
+  size_t least = L.least(nk);
   if (use == kOzSingle && !P.split) {
     const OzLayout all = oz_layout_ops(c, P, false, 3), o = oz_layout_ops(c, P, true, 2);
     want = all.bytes(1, 1);
@@ -478,7 +478,8 @@ int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, in
     }
   }
   if (capturing) *pinned = true;
-  const size_t have = b->bytes - L.exp_bytes() * nk;
+  // a grouped call's workspace limit may be lower than when the buffer was made
+  const size_t have = (use == kOzGroup ? std::min(b->bytes, want) : b->bytes) - L.exp_bytes() * nk;
   room.p = (char *)b->p;
   room.fit = L.full;
   room.slots = (int)std::min<size_t>(slots, have / L.slot_bytes(L.full));
@@ -975,8 +976,8 @@ static int setup_impl(exh_context *c, void *stream, int ngp, int rank, const exh
   if (!rc && w.plan.nmod) {
     OzRoom room;
     w.layout = oz_layout(c, w.plan, o_only);
-    rc = oz_prepare(c, kOzSingle, w.plan, w.layout, 1, 1, 1, cap == hipStreamCaptureStatusActive,
-                    room);
+    rc = oz_prepare(c, kOzSingle, w.plan, w.layout, 1, 1, w.layout.bytes(1, 1),
+                    cap == hipStreamCaptureStatusActive, room);
     if (!rc) w.oz = oz_scratch(w.layout, room, 0, 0);
   }
   if (rc) return rc;

@@ -197,12 +197,63 @@ exh_context::BatchEntry *find_entry(exh_context *c, const std::vector<unsigned c
   return nullptr;
 }
 
-// The distinct contexts of a call, the context index of every k-point and
-// each context's k-point count.
+// The distinct contexts of a call, the context index of every k-point, each
+// context's k-point count and those that share a group (scratch slots).
 struct CallContexts {
   std::vector<exh_context *> ctxs;
   std::vector<int> kci, count, nkg;
 };
+
+// Modular contraction of each context of a call (nmod = 0: FP64 MFMA tiles).
+struct OzParams {
+  std::vector<OzPlan> P;
+  std::vector<OzLayout> L;
+  std::vector<OzRoom> room;  // the context's scratch: k-points at a time, or part of one
+};
+
+// K-points of one context that share a launch of each modular stage: enough
+// workgroups of the products for many rounds on the chip (a wave that ends
+// with a few of them leaves most CUs idle).  8 k-points of K = 1936, G = 1172 in
+// one wave against one by one: norms and residues 0.73 -> 0.51 ms, products
+// 1.05 -> 0.88, reconstruction 0.23 -> 0.18.
+int oz_slots(const OzLayout &L, int nk) {
+  constexpr long long kTarget = 8192;
+  return (int)std::min<long long>(nk, cdivl(kTarget, std::max<long long>(L.panels, 1)));
+}
+
+// Scratch of a context's `count` k-points: `nkg` of them in a group, the
+// residues of `most` of those at a time, `bytes` of modular scratch.  All of it
+// together stays within the workspace limit, which the residues fill first (a
+// group larger than the k-points whose products share a launch gains little);
+// one k-point, or with modular products the parts of one that oz_fit knows, is
+// the least.  Neither need shrinks when `count` grows, so only a longer list
+// moves a buffer.
+struct GroupRoom {
+  int nkg = 1, most = 1;
+  size_t bytes = 0;
+};
+GroupRoom group_room(const exh_context *c, const OzPlan &P, const OzLayout &L, int count) {
+  const size_t limit = c->batch_ws_limit;
+  size_t perk = perk_bytes(c);
+  GroupRoom g;
+  if (P.nmod == 0) {
+    g.nkg = (int)std::max<size_t>(1, std::min<size_t>(count, limit / perk));
+    return g;
+  }
+  perk += L.exp_bytes();
+  const size_t slot = L.slot_bytes(L.full);
+  for (g.most = oz_slots(L, count); g.most > 0; g.most--) {
+    const size_t res = slot * g.most;
+    if (res + perk * g.most > limit) continue;
+    g.nkg = (int)std::min<size_t>(count, (limit - res) / perk);
+    g.bytes = res + L.exp_bytes() * g.nkg;
+    return g;
+  }
+  g.most = 1;
+  g.bytes = std::max(L.least(1), limit > perk ? limit - perk + L.exp_bytes() : 0);
+  g.bytes = std::min(g.bytes, L.bytes(1, 1));
+  return g;
+}
 
 CallContexts call_contexts(int nk, exh_context *const *kc) {
   CallContexts cc;
@@ -217,37 +268,8 @@ CallContexts call_contexts(int nk, exh_context *const *kc) {
     cc.kci[i] = j;
     cc.count[j]++;
   }
-  // k-points of one context that share a group (the context's scratch slots)
-  for (size_t j = 0; j < cc.ctxs.size(); j++)
-    cc.nkg.push_back((int)std::max<size_t>(
-        1, std::min<size_t>(cc.count[j], cc.ctxs[j]->batch_ws_limit / perk_bytes(cc.ctxs[j]))));
+  cc.nkg.assign(cc.ctxs.size(), 1);
   return cc;
-}
-
-// Modular contraction of each context of a call (nmod = 0: FP64 MFMA tiles).
-struct OzParams {
-  std::vector<OzPlan> P;
-  std::vector<OzLayout> L;
-  std::vector<OzRoom> room;  // the context's scratch: k-points at a time, or part of one
-};
-
-// K-points of one context that share a launch of each modular stage: enough
-// workgroups of the products for many rounds on the chip (a wave that ends
-// with a few of them leaves most CUs idle), in equal waves, within the
-// workspace limit.  8 k-points of K = 1936, G = 1172 in one wave against one by
-// one: norms and residues 0.73 -> 0.51 ms, products 1.05 -> 0.88, reconstruction
-// 0.23 -> 0.18.
-// `most` is the room to allocate: unlike the equal waves it never shrinks when
-// nk grows, so only a longer list (which moves the other scratch too) moves it.
-int oz_slots(const exh_context *c, const OzPlan &P, const OzLayout &L, int nk, int *most) {
-  *most = 1;
-  if (P.nmod == 0 || nk <= 1) return 1;
-  constexpr long long kTarget = 8192;
-  long long n = std::min<long long>(nk, cdivl(kTarget, std::max<long long>(L.panels, 1)));
-  n = std::min<long long>(n, std::max<long long>(1, c->batch_ws_limit / std::max<size_t>(L.bytes(1, 1), 1)));
-  *most = (int)n;
-  const long long waves = cdivl(nk, n);
-  return (int)cdivl(nk, waves);
 }
 
 exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
@@ -463,7 +485,7 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   const bool outer_capture = cap == hipStreamCaptureStatusActive;
   const int plan = lead->batch_plan >= 0 ? lead->batch_plan : kDefaultPlan;
   const int nmod = (flags >> 8) & 0xff;
-  const CallContexts cc = call_contexts(nk, kc);
+  CallContexts cc = call_contexts(nk, kc);
   const size_t nctx = cc.ctxs.size();
   OzParams oz;
   oz.P.resize(nctx);
@@ -472,21 +494,22 @@ int run_batch(exh_context *lead, void *stream, int nk, const exh_kpoint *kp,
   for (size_t j = 0; j < nctx; j++) {
     exh_context *c = cc.ctxs[j];
     oz.P[j] = oz_plan(c, flags);
+    if (oz.P[j].nmod) oz.L[j] = oz_layout(c, oz.P[j], false);
+    const GroupRoom g = group_room(c, oz.P[j], oz.L[j], cc.count[j]);
+    cc.nkg[j] = g.nkg;
     // nothing may be allocated or uploaded inside a caller's capture
     if (outer_capture) {
-      if (!scratch_fits(c, cc.nkg[j]))
+      if (!scratch_fits(c, g.nkg) ||
+          (oz.P[j].nmod && c->oz[kOzGroup][oz.P[j].split].bytes < oz.L[j].least(g.nkg)))
         return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
     } else {
-      rc = ensure_scratch(c, cc.nkg[j]);
+      rc = ensure_scratch(c, g.nkg);
     }
     if (!rc && oz.P[j].nmod) {
-      int most = 1;
-      oz.L[j] = oz_layout(c, oz.P[j], false);
-      const int slots = oz_slots(c, oz.P[j], oz.L[j], cc.nkg[j], &most);
-      if (outer_capture && c->oz[kOzGroup][oz.P[j].split].bytes < oz.L[j].least(cc.nkg[j]))
-        return fail(lead, EXH_ESTATE, "batch: make one call outside graph capture first");
-      rc = oz_prepare(c, kOzGroup, oz.P[j], oz.L[j], slots, most, cc.nkg[j], outer_capture,
-                      oz.room[j]);
+      // equal waves of at most `most`
+      const int waves = (int)cdivl(g.nkg, g.most);
+      rc = oz_prepare(c, kOzGroup, oz.P[j], oz.L[j], (int)cdivl(g.nkg, waves), g.nkg, g.bytes,
+                      outer_capture, oz.room[j]);
     }
     if (rc) {
       if (c != lead) fail(lead, rc, c->err);

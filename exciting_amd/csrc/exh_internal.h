@@ -372,8 +372,8 @@ struct OzRoom {
   int slots = 1;
   OzFit fit;
 };
-int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int most,
-               int nk, bool capturing, OzRoom &room);
+int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, int slots, int nk,
+               size_t want, bool capturing, OzRoom &room);
 // Residue slot `slot`, norms of k-point `k` of the group.
 inline OzScratch oz_scratch(const OzLayout &L, const OzRoom &m, int slot, int k) {
   OzScratch w;

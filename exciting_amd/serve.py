@@ -88,17 +88,18 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     K = sys_.natmtot * sys_.maxaa
     ldb = (sys_.ngkmax + 63) // 64 * 64
     scratch = 16 * K * ldb                       # aa.A operand
-    fp64_modular = K * ldb >= 1 << 15            # FP64 on the 15-moduli products
-    if nmod_max or fp64_modular:
-        gpad = (sys_.ngkmax + 383) // 384 * 384     # rows padded to the GEMM's panel
-        kpad = (K + 127) // 128 * 128
-        nt = (sys_.ngkmax + 127) // 128
-        # SPLIT(12) runs 13 moduli; one more for the rounding of the buffers
-        # that serve both precisions
-        moduli = max(nmod_max + 1 if nmod_max else 0, 15 if fp64_modular else 0) + bool(nmod_max)
-        # int8 residues of A and aa.A, and of the products; a launch may hold
-        # every slot's
-        scratch += slots * 4 * moduli * (kpad * gpad + nt * (nt + 1) // 2 * 128 * 128)
+    gpad = (sys_.ngkmax + 127) // 128 * 128      # the products' tiles
+    kpad = (K + 127) // 128 * 128                # two 64-k stages
+    nt = gpad // 128
+    # int8 residues of A and aa.A, and of the products, per modulus; FP64
+    # (15 moduli) and split precision (SPLIT(12) multiplies 13) hold theirs
+    # apart, and a launch may hold every slot's, within the limit
+    residues = 4 * (kpad * gpad + nt * (nt + 1) // 2 * 128 * 128)
+    limit = 8 << 30                              # a grouped call's workspace
+    if K * ldb >= 1 << 15:
+        scratch += min(limit, slots * 15 * residues)
+    if nmod_max:
+        scratch += min(limit, slots * (nmod_max + 1) * residues)
     perk = len(sys_.kpts) * sys_.ngkmax * (16 * sys_.natmtot + 8 * 7 + 4)
     # Cholesky factor, the two triangular solves' results, the reduced matrix
     # and its Hermitian average, and the eigensolver's copy and workspace

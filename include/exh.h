@@ -440,8 +440,11 @@ int exh_get_batch_plan(exh_context *ctx);
  * on return they hold the non-accumulated result. */
 int exh_tune_batch(exh_context *ctx, void *stream, int nk, const exh_kpoint *kpts, int flags,
                    int *plan);
-/* Upper bound on the batch's per-k-point scratch in bytes (default 8 GiB,
- * at least one k-point's worth is always used). */
+/* Upper bound on a grouped call's scratch per context in bytes (default 8 GiB):
+ * the per-k-point arrays of a group and the residues of the modular products
+ * together; a longer list runs in several groups.  One k-point's arrays, and of
+ * its residues the part without which no products can run, are always used.
+ * FP64 and split-precision calls keep such scratch each. */
 int exh_set_batch_workspace(exh_context *ctx, size_t bytes);
 /* ---- instrumentation ----------------------------------------------------- */
 /* No reference counterpart (the reference accumulates wall-clock timers such

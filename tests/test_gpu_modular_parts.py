@@ -100,3 +100,43 @@ def test_route_and_bits_do_not_depend_on_free_memory():
     assert "oz_gemm" in ran and not ran & {"ho", "ho_grouped"}
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flags", [0, lapw.SPLIT(9)])
+@pytest.mark.parametrize("mib", [0, 64, 96, 160, 400])
+def test_workspace_limit_bounds_a_grouped_call(mib, flags):
+    """Four k-points of 38 MB of arrays and 211 MB (FP64) of residues each: the
+    limit is kept, down to what one k-point needs at least (its arrays, and the
+    residues of one modulus and one column step, below 60 MB), and the results
+    are bitwise the single path's."""
+    import torch
+    s = _cases.system("sc8_4k")
+    warm, ctx = lapw.Context(0).load(s), lapw.Context(0).load(s)
+    try:
+        dk = [lapw.DeviceKPoint(s, i) for i in range(4)]
+        ys, ref = [], []
+        for d in dk:
+            y = lapw.newsystem(d.rank, device="cuda")
+            warm.match(d.ngk, d.gpc, d.tpgpc, d.sfacgp, d.apwalm)
+            warm.hamiltonandoverlapsetup(y, d.ngk, d.apwalm, d.igpig, d.vgpc, flags=flags)
+            ref.append((y.hamilton.za, y.overlap.za))
+            ys.append(lapw.newsystem(d.rank, device="cuda"))
+        kp = [lapw.kpoint_struct(d, y.hamilton.za, y.overlap.za) for d, y in zip(dk, ys)]
+        for limit in (1, 8 << 30):            # loads every kernel
+            warm.set_batch_workspace(limit)
+            warm.setup_batch(kp, flags=flags | lapw.MATCH)
+        ctx.set_batch_workspace(max(mib << 20, 1))
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        ctx.setup_batch(kp, flags=flags | lapw.MATCH)
+        torch.cuda.synchronize()
+        took = before - torch.cuda.mem_get_info()[0]
+        print(f"[parts] limit {mib} MiB: took {took >> 20} MiB", flush=True)
+        # the allocator's pages of 2 MiB, for each of a dozen buffers
+        assert took <= max(mib << 20, 100 << 20) + (24 << 20)
+        for y, (h, o) in zip(ys, ref):
+            assert torch.equal(y.hamilton.za, h) and torch.equal(y.overlap.za, o)
+    finally:
+        warm.close()
+        ctx.close()
