@@ -460,7 +460,7 @@ int oz_prepare(exh_context *c, OzUse use, const OzPlan &P, const OzLayout &L, in
                size_t want, bool capturing, OzRoom &room) {
   size_t least = L.least(nk);
   if (use == kOzSingle && !P.split) {
-    const OzLayout all = oz_layout_ops(c, P, false, 3), o = oz_layout_ops(c, P, true, 2);
+    const OzLayout all = oz_layout_ops(c, P, false, 4), o = oz_layout_ops(c, P, true, 2);
     want = all.bytes(1, 1);
     least = std::max(all.least(1), o.least(1));
   }
@@ -571,7 +571,7 @@ void exh_destroy(exh_context *c) {
   if (c->done_ev) (void)hipEventDestroy(c->done_ev);
   DevBuf *bufs[] = {&c->colA, &c->katom, &c->atom_species_d, &c->apword_d, &c->omax_d,
                     &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu, &c->mt_match.piv,
-                    &c->aa, &c->loa, &c->lolo, &c->salo, &c->ololo_eff, &c->h1aa,
+                    &c->aa, &c->loa, &c->lolo, &c->salo, &c->ololo_eff, &c->h1aa, &c->rexp,
                     &c->ivg, &c->ivgig, &c->ist, &c->cf_stage, &c->vf_stage, &c->mf_stage,
                     &c->m2_stage, &c->bt, &c->a2t, &c->at, &c->ivgk, &c->mtab, &c->bmtab, &c->oz[0][0], &c->oz[0][1], &c->oz[1][0], &c->oz[1][1], &c->s_apwalm, &c->s_igpig,
                     &c->s_vgpc, &c->s_h, &c->s_o, &c->s_gpc, &c->s_tpgpc, &c->s_sfac,
@@ -780,7 +780,11 @@ int exh_set_mt(exh_context *c, int maxaa, int maxnlo, const exh_z *aa, const exh
   c->have_h1aa = h1aa != nullptr;
   if (!rc && h1aa)
     rc = upload(c, c->h1aa, h1aa, (size_t)c->apwordmax * c->apwordmax * (c->lmaxapw + 1) * na);
+  if (!rc) rc = ensure(c, c->rexp, (3 * (size_t)c->Ktot + 1) * sizeof(int));
   if (rc) return rc;
+  hipError_t e = launch_row_exponents(c->stream, c);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) return hip_fail(c, e, "set_mt");
   c->have_mt = true;
   return 0;
 }

@@ -112,7 +112,7 @@ uint64_t state_signature(const exh_context *c) {
   const DevBuf *bufs[] = {&c->colA, &c->katom, &c->atom_species_d, &c->apword_d, &c->omax_d,
                           &c->lorow, &c->lobase_d, &c->rmt_d, &c->mt_match.lu,
                           &c->mt_match.piv, &c->aa, &c->loa, &c->lolo, &c->salo,
-                          &c->ololo_eff, &c->h1aa, &c->ivg, &c->ist, &c->bbt, &c->bat,
+                          &c->ololo_eff, &c->h1aa, &c->rexp, &c->ivg, &c->ist, &c->bbt, &c->bat,
                           &c->ba2t, &c->bivgk, &c->bmtab, &c->oz[kOzGroup][0], &c->oz[kOzGroup][1]};
   for (const DevBuf *b : bufs) mix(&b->p, sizeof b->p);
   const int sc[] = {c->nspecies, c->natmtot, c->lmaxapw, c->lmaxmat, c->apwordmax, c->nlomax,
@@ -337,7 +337,7 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
     for (int i = g.k0; i < kend; i++) {
       const int j = cc.kci[i];
       if (!skip[i] || kp[i].ngp <= 0) continue;
-      const bool part = oz.room[j].fit.chunk < oz.L[j].full.chunk ||
+      const bool part = oz.L[j].apart || oz.room[j].fit.chunk < oz.L[j].full.chunk ||
                         oz.room[j].fit.steps < oz.L[j].full.steps;
       if (used[j] == oz.room[j].slots || part) close_wave();
       const exh_context *c = cc.ctxs[j];
@@ -352,7 +352,7 @@ exh_context::BatchEntry *build_entry(exh_context *lead, hipStream_t s, int nk,
       used[j]++;
       wv.count++;
       wv.fit = oz.room[j].fit;
-      // products in parts: a launch of its own
+      // products in parts: launches of its own
       if (part) close_wave();
     }
     close_wave();

@@ -141,6 +141,10 @@ __device__ __forceinline__ void store_upper_o(PH O, long long ldh, int i, int j,
   if (i != j) st(O + (size_t)j + (size_t)i * ldh, z2(orr, -oi));
 }
 
+__device__ __forceinline__ double power2(int e) {  // |e| <= 1022
+  return __longlong_as_double((long long)(e + 1023) << 52);
+}
+
 // Exponent of |a| (-1023 for 0 and denormals), and the mark of a partial column
 // norm with largest entry amax: beyond 2^+-400 FP64 squares may leave the range.
 __device__ __forceinline__ int exponent_of(double a) {
@@ -151,19 +155,23 @@ __device__ __forceinline__ int norm_mark(double amax) {
   return out ? kNormRecompute : 0;
 }
 
-// One k-point of the modular contraction: operands (X; B unless O alone;
-// (1+h1)A for iora*), scratch and outputs, by value for a single launch or in
-// device memory for a grouped one.
+// One k-point of the modular contraction: operands, scratch and outputs, by
+// value for a single launch or in device memory for a grouped one.
 struct OzK {
   int ngp, Ktot, nt, nslab, Gpad, nmod, bits;
-  int nops, iB, iY;       // operands; which one is B, and the overlap's columns
-  int ldp, nch[3];        // partial norms: leading dimension, chunks per operand
+  // operands, and which of them are H's rows and columns and O's
+  int nops, iA, iB, iX, iY;
+  int qi[4];              // place of an operand's residues in q
+  int rs[4];              // rows scaled by 2^(rs * rexp[k]), rs = -1, 0, 1
+  int ldp, nch[4];        // partial norms: leading dimension, chunks per operand
   unsigned fused;         // operands whose partial norms bt has written
   size_t qstride, q_bytes;  // one residue array; one operand's arrays
-  const double2 *x[3];
-  long long ld[3];
-  int *e[3];        // column exponents
-  double *part[3];  // partial norms, then their exponents
+  const int *rexp;        // row exponents
+  const int *uni;         // H's rows are as good as O's: all exponents are equal (or null)
+  const double2 *x[4];
+  long long ld[4];
+  int *e[4];        // column exponents
+  double *part[4];  // partial norms, then their exponents
   int8_t *q, *r;    // residues of the operands and of the products
   IstBox box;
   double2 *h, *o;   // h null: O alone

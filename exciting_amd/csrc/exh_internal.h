@@ -61,14 +61,15 @@ struct OzFit {
 struct OzLayout {
   int Gpad = 0, Kpad = 0;  // G rounded to the 128 tile, K to two 64-k stages
   size_t qstride = 0;      // bytes of one residue array (Kpad * Gpad)
-  int nops = 0;            // operands (X; B unless O alone; (1+h1)A for iora*)
+  int nops = 0;            // operands: (X', B,) X, and (1+h1)A for iora*; split X, B
+  bool apart = false;      // H's operands, then O's take their place
   int nt = 0, width = 1;   // 128-column blocks at ngkmax, and those of a column step
   int planes = 0;          // residue planes of the products: matrices x signs x moduli
   OzFit full;              // everything at once
   size_t e_bytes = 0, e_part_off = 0;  // per operand: column exponents + partial norms
   int nch = 0;             // partial norms of an operand, at most
   long long panels = 0;    // workgroups of the products at ngkmax
-  size_t q_bytes(int chunk) const { return align256(2 * qstride * nops * chunk); }
+  size_t q_bytes(int chunk) const { return align256(2 * qstride * (apart ? 2 : nops) * chunk); }
   size_t r_bytes(int steps) const {  // of the last `steps` column steps, the largest
     const size_t j0 = (size_t)std::max(0, full.steps - steps) * width;
     return (size_t)planes * (((size_t)nt * (nt + 1) - j0 * (j0 + 1)) / 2) * 128 * 128;
@@ -88,9 +89,11 @@ struct OzScratch {
 // Partial squared column norms of the modular contraction's operands, as bt
 // writes them: per atom for X, per atom and 64 rows of aa for B, [chunk][G+k]
 // with leading dimension ld, each followed by as many int exponents (0, or
-// kNormRecompute where squares leave FP64's range).  x null: not wanted.
+// kNormRecompute where squares leave FP64's range).  x null: not wanted.  With
+// row exponents, B's are those of the scaled rows and xs gets those of X'.
 struct NormOut {
-  double *x = nullptr, *b = nullptr;
+  double *x = nullptr, *xs = nullptr, *b = nullptr;
+  const int *rexp = nullptr, *uni = nullptr;
   int ld = 0, nx = 0, nb = 0;
 };
 constexpr int kNormRecompute = 1 << 20;
@@ -218,6 +221,9 @@ struct exh_context {
 
   // muffin-tin tables
   exh::DevBuf aa, loa, lolo, salo, ololo_eff, h1aa;
+  // row exponents of aa (launch_row_exponents), its scratch, and whether they are
+  // all equal
+  exh::DevBuf rexp;
   bool have_h1aa = false;
 
   // G vectors / interstitial
@@ -337,6 +343,7 @@ hipError_t launch_ist_table(hipStream_t s, const exh_context *c,
 // (unused otherwise).
 hipError_t launch_pack(hipStream_t s, const exh_context *c, int ngp,
                        const double2 *apwalm, double2 *at);
+hipError_t launch_row_exponents(hipStream_t s, const exh_context *c);
 hipError_t launch_bt(hipStream_t s, const exh_context *c, int ngp,
                      const double2 *apwalm, const double2 *at, double2 *bt, int ldb,
                      const NormOut &norms);

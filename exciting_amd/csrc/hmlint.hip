@@ -936,8 +936,10 @@ int exh_set_mt_device(exh_context *c, void *stream, int maxaa, int maxnlo, const
   if (!rc) rc = ensure(c, c->salo, nsalo * sizeof(double));
   if (!rc) rc = ensure(c, c->ololo_eff, nolo * sizeof(double));
   if (!rc && h1aa) rc = ensure(c, c->h1aa, nh1 * sizeof(double));
+  if (!rc) rc = ensure(c, c->rexp, (3 * (size_t)c->Ktot + 1) * sizeof(int));
   if (rc) return rc;
   hipError_t e = hipMemcpyAsync(c->aa.p, aa, naa * sizeof(double2), hipMemcpyDeviceToDevice, s);
+  if (e == hipSuccess) e = launch_row_exponents(s, c);
   if (e == hipSuccess && loa)
     e = hipMemcpyAsync(c->loa.p, loa, nloa * sizeof(double2), hipMemcpyDeviceToDevice, s);
   if (e == hipSuccess && lolo)

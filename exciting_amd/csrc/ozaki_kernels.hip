@@ -34,10 +34,20 @@
 // EXH_SPLIT(n) fixes c as the caller asked (27 bits for n = 7).  Without that
 // flag, large bases run here with 15 moduli and c = 56 (oz_fp64): the
 // operands keep 55 bits relative to the column norm and nothing else is
-// rounded, so the products are closer to the exact ones than those of the
+// rounded.  Over whole matrices that is closer to the exact products than the
 // FP64 MFMA kernels (relative Frobenius error of the contraction alone at 16
 // atoms, K = 3872: 2e-16 against 2.4e-15; median element 6e-16 against
 // 2.7e-15), whose K-long FP64 accumulation rounds 4 K times per element.
+// But the error of element (i, j) is bounded by 2^-55 sqrt(K) ||x_i|| ||b_j||, and
+// that of FP64 sums by K 2^-53 sum_k |x_ki| |b_kj|, which does not see how the
+// radial functions are normalised.  For H the FP64 products therefore multiply
+// X' = 2^t X and B' = 2^-t B with the tables' row exponents t (setup_kernels.hip,
+// row_exponents_kernel): the same H, and operands that a change of normalisation
+// leaves as they are.  Without them, the io = 1 functions scaled by 2^-10 and
+// 2^-20 took H from 1.4e-16 to 8e-14 and 8e-11.  O = X^H Y has its rows unscaled
+// (||x_i||^2 is its diagonal), so FP64 has X twice among its operands.  Equal row
+// exponents (a flag the tables' kernels leave) make X' and X one.  What is left
+// of the difference: two columns that are large in different functions.
 //
 // Columns whose norm is not finite give NaN rows and columns of H and O, as
 // any FP64 sum over them would; zero columns give zeros.
@@ -239,16 +249,19 @@ __device__ __forceinline__ void colnorm_final_body(const OzK &d, int z) {
   if (sm[0][lane] | sm[1][lane] | sm[2][lane] | sm[3][lane]) {
     // rare: squares out of range; the column again, scaled by its largest entry
     const EXH_G double2 *xp = gptr(d.x[z]) + g;
-    double amax = 0.0;
+    const int rs = d.rs[z];
+    int top = INT_MIN;
     for (int k = 0; k < d.Ktot; k++) {
       const double2 v = ld(xp + (size_t)k * d.ld[z]);
-      amax = fmax(amax, fmax(fabs(v.x), fabs(v.y)));
+      const double amax = fmax(fabs(v.x), fabs(v.y));
+      if (amax > 0.0) top = max(top, exponent_of(amax) + (rs ? rs * d.rexp[k] : 0));
     }
-    em = min(max(exponent_of(amax), -1022), 1023);
+    em = top;
     s = 0.0;
     for (int k = 0; k < d.Ktot; k++) {
       const double2 v = ld(xp + (size_t)k * d.ld[z]);
-      const double a = ldexp(v.x, -em), b = ldexp(v.y, -em);
+      const int sh = (rs ? rs * d.rexp[k] : 0) - em;
+      const double a = ldexp(v.x, sh), b = ldexp(v.y, sh);
       s = fma(a, a, s);
       s = fma(b, b, s);
     }
@@ -293,12 +306,14 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
   int e = INT_MIN;
   if (g < ngp) e = gptr((const int *)d.e[z])[g];
   const bool live = e != INT_MIN && e != INT_MAX;
-  const int s = live ? d.bits - e : 0;
+  const int s0 = live ? d.bits - e : 0, rs = d.rs[z];
+  const EXH_C int *rexp = cptr(d.rexp);
 #pragma unroll
   for (int t = 0; t < 16; t++) {
     const int k = kb * 16 + t;
     double2 v = z2(0.0, 0.0);
     if (live && k < Ktot) v = exh::ld(X + (size_t)k * ldx + g);
+    const int s = s0 + (rs ? rs * rexp[min(k, Ktot - 1)] : 0);
     const double yr = rint(ldexp(v.x, s)), yi = rint(ldexp(v.y, s));
     constexpr double D = (double)(1ll << kSplit);
     hr[t] = rint(yr * (1.0 / D));
@@ -307,7 +322,7 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
     li[t] = fma(-D, hi[t], yi);
   }
   const size_t qstride = d.qstride;
-  EXH_G int8_t *out = gptr(d.q) + z * d.q_bytes + ((size_t)kb * d.Gpad + g) * 16;
+  EXH_G int8_t *out = gptr(d.q) + d.qi[z] * d.q_bytes + ((size_t)kb * d.Gpad + g) * 16;
 #pragma unroll 1
   for (int m = m0; m < m1; m++) {
     const double p = c_mod.m[m].p, rp = c_mod.m[m].rp, nk = c_mod.m[m].nk;
@@ -334,15 +349,14 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
 }
 
 // ---------------------------------------------------------------------------
-// Upper-triangular int8 GEMMs.  One workgroup computes the product pair
-// (H, O) of one modulus and sign for a 384-row panel of the row operand
-// (x- for the sign +, x+ for -) against one 128-column block J of the H and O
-// column operands:
-//   C_H[i][j] = sum_k A[k][i] BH[k][j],  C_O[i][j] = sum_k A[k][i] BO[k][j]
+// Upper-triangular int8 GEMMs.  One workgroup computes, for one modulus and
+// sign, a 384-row panel of the row operand (x- for the sign +, x+ for -) against
+// two 128-column blocks: with EXH_SPLIT the block J of H's and of O's column
+// operand, which then share the row operand; otherwise (ONE) the blocks 2J and
+// 2J + 1 of one matrix, as H's row operand has its rows scaled and O's has not:
+//   C[i][j] = sum_k A[k][i] B[k][j]
 // (int32, exact), each stored mod p as signed bytes in the 128x128 tiles on
-// or above the diagonal.  The H and O products share the row operand, as the
-// FP64 kernel shares conj(A) between H and O.  With ONLY_O (overlapsetup) the
-// second column operand is the next 128 columns of O instead.  Each wave owns
+// or above the diagonal.  Each wave owns
 // 96 rows x 64 columns of both products (3 x 2 blocks of
 // v_mfma_i32_32x32x32_i8 each, 192 accumulator registers) and reads 7 operand
 // fragments from LDS per 12 MFMAs; 8 waves form 4 row groups x 2 column
@@ -402,19 +416,19 @@ __host__ __device__ inline int oz_npan(int j) { return (j * OZ_T + OZ_T - 1) / O
 
 // Column steps of one GEMM and the last 128-column block of step j: the
 // fused products step by one block, O alone by two (nt blocks in all).
-template <bool ONLY_O>
-__host__ __device__ inline int oz_steps(int nt) { return ONLY_O ? (nt + 1) / 2 : nt; }
-template <bool ONLY_O>
+template <bool ONE>
+__host__ __device__ inline int oz_steps(int nt) { return ONE ? (nt + 1) / 2 : nt; }
+template <bool ONE>
 __host__ __device__ inline int oz_last(int j, int nt) {
-  const int l = ONLY_O ? 2 * j + 1 : j;
+  const int l = ONE ? 2 * j + 1 : j;
   return l < nt ? l : nt - 1;
 }
 
 // Panels per GEMM, of the column steps s0 .. s1 - 1.
-template <bool ONLY_O>
+template <bool ONE>
 __host__ __device__ inline long long oz_panels(int nt, int s0, int s1) {
   long long n = 0;
-  for (int j = s0; j < min(s1, oz_steps<ONLY_O>(nt)); j++) n += oz_npan(oz_last<ONLY_O>(j, nt));
+  for (int j = s0; j < min(s1, oz_steps<ONE>(nt)); j++) n += oz_npan(oz_last<ONE>(j, nt));
   return n;
 }
 
@@ -422,9 +436,9 @@ __host__ __device__ inline long long oz_panels(int nt, int s0, int s1) {
 struct OzTiles {
   int t0, n;
 };
-template <bool ONLY_O>
+template <bool ONE>
 __host__ __device__ inline OzTiles oz_tiles(int nt, int s0, int s1) {
-  const int w = ONLY_O ? 2 : 1, a = min(nt, s0 * w), b = min(nt, min(s1, oz_steps<ONLY_O>(nt)) * w);
+  const int w = ONE ? 2 : 1, a = min(nt, s0 * w), b = min(nt, min(s1, oz_steps<ONE>(nt)) * w);
   return {a * (a + 1) / 2, max(0, b * (b + 1) / 2 - a * (a + 1) / 2)};
 }
 
@@ -436,10 +450,10 @@ __host__ __device__ inline OzTiles oz_tiles(int nt, int s0, int s1) {
 constexpr int OZ_SJ = 8, OZ_SI = 4 * 384 / OZ_R;
 
 // Panel o of one GEMM's steps s0 .. s1 - 1 -> (column step J, row panel IT).
-template <bool ONLY_O>
+template <bool ONE>
 __device__ __forceinline__ void oz_panel_at(int o, int nt, int s0, int s1, int &J, int &IT) {
-  const int ns = min(s1, oz_steps<ONLY_O>(nt));
-  auto npan = [&](int j) { return oz_npan(oz_last<ONLY_O>(j, nt)); };
+  const int ns = min(s1, oz_steps<ONE>(nt));
+  auto npan = [&](int j) { return oz_npan(oz_last<ONE>(j, nt)); };
   int rem = o, j0 = s0;
   for (;; j0 += OZ_SJ) {
     const int j1 = min(ns, j0 + OZ_SJ);
@@ -469,39 +483,51 @@ __device__ __forceinline__ void oz_panel_at(int o, int nt, int s0, int s1, int &
   }
 }
 
-// Residues of the moduli m0 .. m0 + mc - 1 are in d.q, counted from m0.
-template <bool ONLY_O>
-__device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc, int s0, int s1) {
+// Residues of the moduli m0 .. m0 + mc - 1 are in d.q, counted from m0.  ONE: of
+// the matrices mat0 .. mat0 + nmat - 1 (H, O).
+template <bool ONE>
+__device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc, int s0, int s1, int mat0,
+                                            int nmat, bool uni, v4i (&sm0)[4][OZ_W],
+                                            v4i (&sm1)[4][OZ_W]) {
   const int nt = d.nt, nslab = d.nslab, Gpad = d.Gpad;
   const size_t qstride = d.qstride;
   // XCD-contiguous remap over the k-point's panels (its first block runs on
-  // XCD 0: the grid's x extent is a multiple of 8), then (sign * mc + m, panel)
-  const int per = (int)oz_panels<ONLY_O>(nt, s0, s1);
-  const int bid = blockIdx.x, nb = per * 2 * mc;
+  // XCD 0: the grid's x extent is a multiple of 8), then ((matrix, sign) * mc + m,
+  // panel)
+  const int per = (int)oz_panels<ONE>(nt, s0, s1);
+  const int bid = blockIdx.x, nb = per * 2 * mc * nmat;
   if (bid >= nb) return;
   const int xcd = bid & 7, i8 = bid >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int t = xcd * q8 + (xcd < r8 ? xcd : r8) + i8;
   const int qm = __builtin_amdgcn_readfirstlane(t / per), o = t - qm * per;
-  const int q = qm >= mc ? 1 : 0, m = qm - q * mc;  // q = 0: sign +, 1: sign -
+  const int mq = __builtin_amdgcn_readfirstlane(qm / mc);
+  const int m = qm - mq * mc, q = mq & 1, mat = mat0 + (mq >> 1);  // q = 0: sign +, 1: -
   int J, IT;
-  oz_panel_at<ONLY_O>(o, nt, s0, s1, J, IT);
+  oz_panel_at<ONE>(o, nt, s0, s1, J, IT);
   // uniform by construction; scalar registers for the addresses that follow
   J = __builtin_amdgcn_readfirstlane(J);
   IT = __builtin_amdgcn_readfirstlane(IT);
-  const OzTiles T = oz_tiles<ONLY_O>(nt, s0, s1);
-  const int JH = ONLY_O ? 2 * J : J, JO = ONLY_O ? 2 * J + 1 : J;
+  const OzTiles T = oz_tiles<ONE>(nt, s0, s1);
+  const int JH = ONE ? 2 * J : J, JO = ONE ? 2 * J + 1 : J;
   const int I0 = IT * OZ_R, H0 = JH * OZ_T;
   // past the last block (odd nt): any valid columns, not stored
   const int O0 = min(JO, nt - 1) * OZ_T;
 
-  const int8_t *Ab = d.q + (size_t)(2 * m + 1 - q) * qstride;
-  const int8_t *Ob = d.q + d.iY * d.q_bytes + (size_t)(2 * m + q) * qstride;
-  const int8_t *Hb = ONLY_O ? Ob : d.q + d.iB * d.q_bytes + (size_t)(2 * m + q) * qstride;
+  const int zr = ONE && !mat && !uni ? d.iA : d.iX, zh = ONE && mat ? d.iY : d.iB;
+  const int zo = ONE ? zh : d.iY;
+  // in scalar registers: the DMA loads of the loop would otherwise each be a loop
+  // over the lanes' (equal) addresses (0.333 -> 0.364 us per workgroup)
+  auto operand = [&](int z, int sign) {
+    const uintptr_t u = (uintptr_t)(d.q + d.qi[z] * d.q_bytes + (size_t)(2 * m + sign) * qstride);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)u);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+    return (const int8_t *)((uintptr_t)hi << 32 | lo);
+  };
+  const int8_t *Ab = operand(zr, 1 - q), *Hb = operand(zh, q), *Ob = ONE ? Hb : operand(zo, q);
 
   // one LDS array per stage: the compiler then sees the DMA into one stage and
   // the reads of the other as disjoint (no wait inserted).  Rows 0..383 hold
-  // the row operand, then 128 columns of H and of O.
-  __shared__ v4i sm0[4][OZ_W], sm1[4][OZ_W];
+  // the row operand, then the two column blocks.
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = w >> 1, wc = w & 1, l32 = lane & 31, lh = lane >> 5;
@@ -610,12 +636,13 @@ __device__ __forceinline__ void ozgemm_body(const OzK &d, int m0, int mc, int s0
   // the LDS must outlive the last refills
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 
-  // planes: (H+, H-, O+, O-) x modulus, or (O+, O-) x modulus
+  // planes: (H+, H-, O+, O-) x modulus, or of O alone (O+, O-) x modulus
   const size_t plane = (size_t)T.n * (OZ_T * OZ_T);
-  EXH_G int8_t *Rq = gptr(d.r) + (size_t)(q * d.nmod + m0 + m) * plane;
+  const int pl = 2 * (ONE && d.h ? mat : 0) + q;
+  EXH_G int8_t *Rq = gptr(d.r) + (size_t)(pl * d.nmod + m0 + m) * plane;
   const OzMod &M = c_mod.m[m0 + m];
   store_residues(ah, M, rg, wc, lane, IT, JH, T.t0, Rq);
-  if (ONLY_O) {
+  if (ONE) {
     if (JO < nt) store_residues(ao, M, rg, wc, lane, IT, JO, T.t0, Rq);
   } else {
     store_residues(ao, M, rg, wc, lane, IT, JO, T.t0, Rq + (size_t)2 * d.nmod * plane);
@@ -645,11 +672,11 @@ __device__ __forceinline__ double crt(double hi, double lo) {
 
 template <int NM, bool ONLY_O>
 __device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate, int s0, int s1) {
-  const OzTiles T = oz_tiles<ONLY_O>(d.nt, s0, s1);
+  const OzTiles T = oz_tiles<NM == OZ_N>(d.nt, s0, s1);  // the products' column steps
   const int sb = blockIdx.x & 15, ngp = d.ngp, bits = d.bits;
   if ((int)(blockIdx.x >> 4) >= T.n) return;
   const int tile = T.t0 + (int)(blockIdx.x >> 4);
-  const EXH_G int *ex = gptr((const int *)d.e[0]);
+  const EXH_G int *ea = gptr((const int *)d.e[d.iA]), *ex = gptr((const int *)d.e[d.iX]);
   const EXH_G int *eb = gptr((const int *)d.e[d.iB]), *ey = gptr((const int *)d.e[d.iY]);
   EXH_G double2 *H = gptr(d.h), *O = gptr(d.o);
   const long long ldh = d.ldh;
@@ -699,8 +726,7 @@ __device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate, int
     for (int t = 0; t < 4; t++) {
       const int i = i0 + il + t;
       if (i >= ngp || i > j) continue;
-      const int exi = ex[i];
-      auto value = [&](int v, int ej) {
+      auto value = [&](int v, int exi, int ej) {
         // 2^-(s_i + s_j); a column that is not finite makes the element NaN
         const bool bad = exi == INT_MAX || ej == INT_MAX;
         const int si = exi == INT_MIN ? 0 : bits - exi, sj = ej == INT_MIN ? 0 : bits - ej;
@@ -710,8 +736,8 @@ __device__ __forceinline__ void ozcombine_body(const OzK &d, int accumulate, int
         const double im = ldexp(crt<NM>(mh[v][t], ml[v][t]), sh);
         return bad ? z2(nan, nan) : z2(re, im);
       };
-      double2 hv = z2(0.0, 0.0), ov = value(NV - 1, eyj);
-      if (!ONLY_O) hv = value(0, ebj);
+      double2 hv = z2(0.0, 0.0), ov = value(NV - 1, ex[i], eyj);
+      if (!ONLY_O) hv = value(0, ea[i], ebj);
       ist_add(box, i, j, hv.x, hv.y, ov.x, ov.y);
       if (!ONLY_O) sT[0][jl][il + t] = hv;
       sT[NV - 1][jl][il + t] = ov;
@@ -769,22 +795,56 @@ __global__ __launch_bounds__(256) void colnorm_final_grouped_kernel(const OzK *_
                                                                    int nops) {
   colnorm_final_body(kd[blockIdx.z / nops], blockIdx.z % nops);
 }
-__global__ __launch_bounds__(256) void residue_kernel(OzK d, int m0, int m1) {
-  residue_body(d, blockIdx.z, m0, m1);
+// X' comes with X (the column is in the cache), or in the launch of H's operands
+// where they are apart.  With equal row exponents X' and X have the same residues:
+// one is enough.
+__device__ __forceinline__ void residues_of(const OzK &d, int z, int m0, int m1) {
+  const bool apart = d.qi[d.iA] == d.qi[d.iX], uni = d.uni && *d.uni;
+  if (uni && apart && z == d.iX) return;  // X' lies there
+  for (int last = z;; z = last) {
+    if (z == d.iX && z != d.iA && !apart && !uni) last = d.iA;
+    residue_body(d, z, m0, m1);
+    if (z == last) return;
+  }
 }
-__global__ __launch_bounds__(256) void residue_grouped_kernel(const OzK *__restrict__ kd, int nops,
-                                                              int m1) {
-  residue_body(kd[blockIdx.z / nops], blockIdx.z % nops, 0, m1);
+__global__ __launch_bounds__(256) void residue_kernel(OzK d, int z0, int m0, int m1) {
+  residues_of(d, z0 + blockIdx.z, m0, m1);
+}
+__global__ __launch_bounds__(256) void residue_grouped_kernel(const OzK *__restrict__ kd, int z0,
+                                                              int nz, int m1) {
+  residues_of(kd[blockIdx.z / nz], z0 + blockIdx.z % nz, 0, m1);
 }
 // two waves per SIMD whatever the workgroup size: at most 256 VGPRs
-template <bool ONLY_O>
 __global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 ozgemm_kernel(OzK d, int m0, int mc, int s0, int s1) {
-  ozgemm_body<ONLY_O>(d, m0, mc, s0, s1);
+  __shared__ v4i sm0[4][OZ_W], sm1[4][OZ_W];
+  ozgemm_body<false>(d, m0, mc, s0, s1, 0, 1, false, sm0, sm1);
 }
 __global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 ozgemm_grouped_kernel(const OzK *__restrict__ kd, int mc) {
-  ozgemm_body<false>(kd[blockIdx.y], 0, mc, 0, INT_MAX / 2);
+  __shared__ v4i sm0[4][OZ_W], sm1[4][OZ_W];
+  ozgemm_body<false>(kd[blockIdx.y], 0, mc, 0, INT_MAX / 2, 0, 1, false, sm0, sm1);
+}
+// FP64: steps of two blocks of one matrix, or, where the row exponents are equal
+// and O's columns are there beside H's, of one block of both as with EXH_SPLIT
+// (at 16 atoms, 148 against 135 workgroups a product pair).
+__device__ __forceinline__ void ozgemm64_body(const OzK &d, int m0, int mc, int s0, int s1,
+                                              int mat0, int nmat) {
+  __shared__ v4i sm0[4][OZ_W], sm1[4][OZ_W];
+  const bool uni = d.uni && *d.uni;
+  if (uni && (d.qi[d.iB] != d.qi[d.iY])) {
+    if (mat0 == 0) ozgemm_body<false>(d, m0, mc, 2 * s0, 2 * s1, 0, 1, true, sm0, sm1);
+    return;
+  }
+  ozgemm_body<true>(d, m0, mc, s0, s1, mat0, nmat, uni, sm0, sm1);
+}
+__global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+ozgemm64_kernel(OzK d, int m0, int mc, int s0, int s1, int mat0, int nmat) {
+  ozgemm64_body(d, m0, mc, s0, s1, mat0, nmat);
+}
+__global__ __launch_bounds__(64 * OZ_NWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+ozgemm64_grouped_kernel(const OzK *__restrict__ kd, int mc) {
+  ozgemm64_body(kd[blockIdx.y], 0, mc, 0, INT_MAX / 4, 0, 2);
 }
 template <int NM, bool ONLY_O>
 __global__ __launch_bounds__(256) void ozcombine_kernel(OzK d, int accumulate, int s0, int s1) {
@@ -827,7 +887,7 @@ OzPlan oz_fp64() {
 }
 
 OzLayout oz_layout(const exh_context *c, const OzPlan &P, bool only_o) {
-  return oz_layout_ops(c, P, only_o, 1 + (only_o ? 0 : 1) + (c->have_h1aa ? 1 : 0));
+  return oz_layout_ops(c, P, only_o, P.split ? 2 : 1 + (only_o ? 0 : 2) + (c->have_h1aa ? 1 : 0));
 }
 
 OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int nops) {
@@ -838,9 +898,9 @@ OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int n
   L.qstride = (size_t)L.Kpad * L.Gpad;
   const int nt = (ngkmax + OZ_T - 1) / OZ_T;  // tile columns of the largest basis
   L.nt = nt;
-  L.width = only_o ? 2 : 1;
+  L.width = P.split ? 1 : 2;
   L.planes = (only_o ? 2 : 4) * P.nmod;
-  L.full = {P.nmod, std::max(1, only_o ? oz_steps<true>(nt) : oz_steps<false>(nt))};
+  L.full = {P.nmod, std::max(1, P.split ? oz_steps<false>(nt) : oz_steps<true>(nt))};
   // per operand: the column exponents, then the partial norms and their marks
   const size_t ng = std::max(ngkmax, 1);
   const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
@@ -848,7 +908,11 @@ OzLayout oz_layout_ops(const exh_context *c, const OzPlan &P, bool only_o, int n
   L.e_part_off = (ng * sizeof(int) + 255) / 256 * 256;
   L.e_bytes = (L.e_part_off + (sizeof(double) + sizeof(int)) * L.nch * ng + 255) / 256 * 256;
   L.nops = nops;
-  L.panels = 2 * P.nmod * (only_o ? oz_panels<true>(nt, 0, nt) : oz_panels<false>(nt, 0, nt));
+  L.panels = 2 * P.nmod * (P.split ? oz_panels<false>(nt, 0, nt) : oz_panels<true>(nt, 0, nt));
+  // one matrix's products fill the chip for 32 rounds: the other's residues can
+  // take their place afterwards
+  L.apart = !P.split && !only_o && L.panels >= 8192;
+  if (!P.split && !only_o) L.panels *= 2;
   return L;
 }
 
@@ -879,12 +943,18 @@ OzFit oz_fit(const OzLayout &L, size_t bytes) {
   return f;
 }
 
+// bt sums the norms of H's operands and, in passing, of O's X.
 NormOut norm_out(const OzK &d) {
   NormOut n;
-  n.x = d.part[0];
+  n.x = d.part[d.iX];
   n.b = d.part[d.iB];
+  if (d.iA != d.iX) {
+    n.xs = d.part[d.iA];
+    n.rexp = d.rexp;
+    n.uni = d.uni;
+  }
   n.ld = d.ldp;
-  n.nx = d.nch[0];
+  n.nx = d.nch[d.iX];
   n.nb = d.nch[d.iB];
   return n;
 }
@@ -904,29 +974,35 @@ OzK make_ozk(const exh_context *c, int ngp, const OzPlan &P, const OzLayout &L,
   d.ldp = std::max(c->ngkmax, 1);
   d.qstride = L.qstride;
   d.q_bytes = w.fit.chunk * 2 * L.qstride;
+  d.rexp = (const int *)c->rexp.p;
+  d.uni = h && !P.split ? d.rexp + 3 * (size_t)c->Ktot : nullptr;
   d.q = w.q;
   d.r = w.r;
   d.box = box;
   d.h = h;
   d.o = o;
   d.ldh = ldh;
-  const double2 *src[3] = {X, B, Y};
-  for (int z = 0; z < 3; z++) {
-    if ((z == 1 && !h) || (z == 2 && !Y)) continue;
+  const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
+  // nch 0: not among bt's norms
+  auto add = [&](const double2 *x, long long ld, int rs, int nch) {
     const int n = d.nops++;
-    if (z == 1) d.iB = n;
-    if (z == 2) d.iY = n;
     char *e = (char *)w.e + (size_t)n * L.e_bytes;
-    // X and B: left by bt, per atom and per atom and 64 rows (norm_out)
-    const bool fused = h && z < 2;
-    const int rows = (c->maxaa + kNormRows - 1) / kNormRows;
-    d.fused |= fused ? 1u << n : 0u;
-    d.nch[n] = !fused ? (c->Ktot + OZ_NCH - 1) / OZ_NCH : c->natmtot * (z == 1 ? rows : 1);
-    d.x[n] = src[z];
-    d.ld[n] = z == 0 ? ldx : ldb;
+    d.fused |= nch ? 1u << n : 0u;
+    d.nch[n] = nch ? nch : (c->Ktot + OZ_NCH - 1) / OZ_NCH;
+    d.x[n] = x;
+    d.ld[n] = ld;
+    d.rs[n] = rs;
+    d.qi[n] = L.apart && n >= 2 ? n - 2 : n;
     d.e[n] = (int *)e;
     d.part[n] = (double *)(e + L.e_part_off);
+    return n;
+  };
+  if (h) {
+    d.iA = add(X, ldx, P.split ? 0 : 1, c->natmtot);
+    d.iB = add(B, ldb, P.split ? 0 : -1, c->natmtot * rows);
   }
+  d.iX = h && P.split ? d.iA : add(X, ldx, 0, h ? c->natmtot : 0);
+  d.iY = Y ? add(Y, ldb, 0, 0) : d.iX;
   return d;
 }
 
@@ -936,6 +1012,8 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, c
                             int accumulate, const OzRun &run) {
   const bool only_o = d[0].h == nullptr;
   const int nmod = d[0].nmod;
+  const bool one = nmod == OZ_N;  // FP64: one matrix per workgroup
+  const bool apart = d[0].nops > 2 && d[0].qi[2] == 0;
   int ngp = 0, nch = 0, nops = 0, kb = 0, nt = 0;
   for (int i = 0; i < n; i++) {
     ngp = std::max(ngp, d[i].ngp);
@@ -957,25 +1035,25 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, c
       hipLaunchKernelGGL(colnorm_final_kernel, gf, dim3(256), 0, s, d[0]);
     }
   };
-  auto residues = [&](int m0, int m1) {
-    const dim3 gr(cdiv(nt * OZ_T, 256), kb, nz);
-    if (kd) hipLaunchKernelGGL(residue_grouped_kernel, gr, dim3(256), 0, s, kd, nops, m1);
-    else hipLaunchKernelGGL(residue_kernel, gr, dim3(256), 0, s, d[0], m0, m1);
+  auto residues = [&](int z0, int z1, int m0, int m1) {
+    const dim3 gr(cdiv(nt * OZ_T, 256), kb, (z1 - z0) * n);
+    if (kd) hipLaunchKernelGGL(residue_grouped_kernel, gr, dim3(256), 0, s, kd, z0, z1 - z0, m1);
+    else hipLaunchKernelGGL(residue_kernel, gr, dim3(256), 0, s, d[0], z0, m0, m1);
   };
-  auto products = [&](int m0, int m1, int s0, int s1) {
-    const long long per = only_o ? oz_panels<true>(nt, s0, s1) : oz_panels<false>(nt, s0, s1);
-    const dim3 gg((unsigned)((per * 2 * (m1 - m0) + 7) / 8 * 8), n);
-    if (kd)
-      hipLaunchKernelGGL(ozgemm_grouped_kernel, gg, dim3(64 * OZ_NWG), 0, s, kd, m1 - m0);
-    else if (only_o)
-      hipLaunchKernelGGL(ozgemm_kernel<true>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0, s0,
-                         s1);
+  auto products = [&](int m0, int m1, int s0, int s1, int mat0, int nmat) {
+    const int mc = m1 - m0;
+    long long nb = one ? oz_panels<true>(nt, s0, s1) * nmat : oz_panels<false>(nt, s0, s1);
+    if (one && !only_o) nb = std::max(nb, oz_panels<false>(nt, 2 * s0, 2 * s1));
+    const dim3 gg((unsigned)((nb * 2 * mc + 7) / 8 * 8), n), th(64 * OZ_NWG);
+    if (kd && one) hipLaunchKernelGGL(ozgemm64_grouped_kernel, gg, th, 0, s, kd, mc);
+    else if (kd) hipLaunchKernelGGL(ozgemm_grouped_kernel, gg, th, 0, s, kd, mc);
+    else if (one)
+      hipLaunchKernelGGL(ozgemm64_kernel, gg, th, 0, s, d[0], m0, mc, s0, s1, mat0, nmat);
     else
-      hipLaunchKernelGGL(ozgemm_kernel<false>, gg, dim3(64 * OZ_NWG), 0, s, d[0], m0, m1 - m0, s0,
-                         s1);
+      hipLaunchKernelGGL(ozgemm_kernel, gg, th, 0, s, d[0], m0, mc, s0, s1);
   };
   auto combine = [&](int s0, int s1) {
-    const OzTiles T = only_o ? oz_tiles<true>(nt, s0, s1) : oz_tiles<false>(nt, s0, s1);
+    const OzTiles T = one ? oz_tiles<true>(nt, s0, s1) : oz_tiles<false>(nt, s0, s1);
     const dim3 grid((unsigned)T.n * 16, n);
     if (only_o) {
       if (nmod != OZ_N) return hipErrorInvalidValue;  // EXH_SPLIT is refused for O alone
@@ -1006,25 +1084,34 @@ static hipError_t launch_oz(hipStream_t s, const OzK *d, const OzK *kd, int n, c
 #undef EXH_OZC
     return hipGetLastError();
   };
-  const int ns = only_o ? oz_steps<true>(nt) : oz_steps<false>(nt);
+  // operands and matrices whose residues are there together
+  struct Pass {
+    int z0, z1, mat0, nmat;
+  };
+  const bool both = one && !only_o;  // X' comes with X
+  const Pass all[1] = {{both ? 1 : 0, nops, only_o ? 1 : 0, both ? 2 : 1}};
+  const Pass two[2] = {{0, 2, 0, 1}, {2, nops, 1, 1}};
+  const Pass *ps = apart ? two : all;
+  const int np = apart ? 2 : 1, ns = one ? oz_steps<true>(nt) : oz_steps<false>(nt);
   hipError_t e = hipSuccess;
   for (int s0 = 0; s0 < ns && e == hipSuccess; s0 += fit.steps) {
     const int s1 = std::min(ns, s0 + fit.steps);
-    for (int m0 = 0; m0 < nmod && e == hipSuccess; m0 += fit.chunk) {
-      const int m1 = std::min(nmod, m0 + fit.chunk);
-      // residues that an earlier strip has left are still there
-      if (s0 == 0 || fit.chunk < nmod)
-        e = run(EXH_K_OZRES, [&] {
-          if (s0 == 0 && m0 == 0) norms();
-          residues(m0, m1);
-          return hipGetLastError();
-        });
-      if (e == hipSuccess)
-        e = run(EXH_K_OZGEMM, [&] {
-          products(m0, m1, s0, s1);
-          return hipGetLastError();
-        });
-    }
+    for (int m0 = 0; m0 < nmod && e == hipSuccess; m0 += fit.chunk)
+      for (int p = 0; p < np && e == hipSuccess; p++) {
+        const int m1 = std::min(nmod, m0 + fit.chunk);
+        // residues that an earlier strip has left are still there
+        if (s0 == 0 || fit.chunk < nmod || np > 1)
+          e = run(EXH_K_OZRES, [&] {
+            if (s0 == 0 && m0 == 0 && p == 0) norms();
+            residues(ps[p].z0, ps[p].z1, m0, m1);
+            return hipGetLastError();
+          });
+        if (e == hipSuccess)
+          e = run(EXH_K_OZGEMM, [&] {
+            products(m0, m1, s0, s1, ps[p].mat0, ps[p].nmat);
+            return hipGetLastError();
+          });
+      }
     if (e == hipSuccess) e = run(EXH_K_OZCOMB, [&] { return combine(s0, s1); });
   }
   return e;

@@ -125,6 +125,89 @@ __global__ void pack_grouped_kernel(const KDesc *__restrict__ kd) {
 }
 
 // ---------------------------------------------------------------------------
+// Row exponents t of the muffin-tin tables: with D = diag(2^t) per function,
+// aa' = D^-1 aa D^-1 has rows of size 1.  H = A^H aa A = (D A)^H (D^-1 aa A), and
+// a change of a radial function's norm by 2^p (A 2^p, aa 2^-p) changes t by -p:
+// the scaled operands of the modular products, and with them the rounding of H,
+// do not depend on how the radial functions are normalised, as FP64 sums do not.
+// And with a diagonal of size 1, aa'x' is at least as large as x' where that
+// is, so that the products' bound ||x'|| ||aa'x'|| stays near sum |x'| |aa'x'|.
+//
+// Three steps of equilibration in logarithms (64 to a factor of two, so halves
+// are exact): 64 t = 32 log2|aa_kk| to begin with, then each row by half of what
+// its largest scaled entry is off by.  Positive tables, whose off-diagonal
+// entries are below the geometric mean of the diagonal, are done with the first.
+// One thread per row and a quarter of the columns (consecutive rows are
+// consecutive in memory); a launch per step.
+// ---------------------------------------------------------------------------
+constexpr int kNone = INT_MIN / 4;  // a zero row, or nothing known yet
+
+__device__ __forceinline__ int log2_of(double2 z) {
+  const double m = fmax(fabs(z.x), fabs(z.y));
+  return m > 0.0 && m <= 0x1.fp1023 ? 64 * exponent_of(m) : kNone;
+}
+
+__global__ __launch_bounds__(256) void row_exponents_kernel(
+    const int *__restrict__ Koff, const int *__restrict__ Ms, const double2 *__restrict__ aa,
+    int maxaa, const int *__restrict__ vin, int *__restrict__ vout, int first, int last) {
+  const int ias = blockIdx.y, M = Ms[ias], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
+  if ((int)blockIdx.x * 64 >= M) return;  // uniform
+  const double2 *a = aa + (size_t)ias * maxaa * maxaa;
+  const int *v = vin + Koff[ias];
+  auto value = [&](int j) {
+    if (!first) return v[j];
+    const int d = log2_of(a[j + (size_t)maxaa * j]);
+    return d == kNone ? kNone : d / 2;
+  };
+  __shared__ int sr[4][64], sz[4][64];
+  int r = kNone, z = kNone;  // largest scaled entry; largest entry
+  const int kc = min(k, M - 1);
+  for (int j = w; j < M; j += 4) {
+    const int e = log2_of(a[kc + (size_t)maxaa * j]), u = value(j);
+    if (e == kNone) continue;
+    z = max(z, e);
+    if (u != kNone) r = max(r, e - u);
+  }
+  sr[w][lane] = r;
+  sz[w][lane] = z;
+  __syncthreads();
+  if (w || k >= M) return;
+  for (int i = 1; i < 4; i++) {
+    r = max(r, sr[i][lane]);
+    z = max(z, sz[i][lane]);
+  }
+  int u = value(k);
+  if (u == kNone) u = r != kNone ? r : z == kNone ? kNone : z / 2;
+  else if (r != kNone) u += (r - u) >> 1;
+  // a zero row's function does not reach H: out of the way of the others
+  if (last) u = u == kNone ? -500 : max(-500, min(500, (u + 32) >> 6));
+  vout[Koff[ias] + k] = u;
+}
+
+// Exponents within one of each other (2^t itself is within a factor of two) are
+// taken as equal, and *same says so: X' = 2^t X then needs no residues of its own.
+__global__ __launch_bounds__(1024) void equal_exponents_kernel(int n, int *__restrict__ t,
+                                                               int *__restrict__ same) {
+  const int t0 = t[0];
+  __syncthreads();
+  int lo = 0, hi = 0;  // some exponent is t0 - 1, t0 + 1
+  int far = 0;
+  for (int k = threadIdx.x; k < n; k += 1024) {
+    lo |= t[k] == t0 - 1;
+    hi |= t[k] == t0 + 1;
+    far |= t[k] < t0 - 1 || t[k] > t0 + 1;
+  }
+  lo = __syncthreads_or(lo);
+  hi = __syncthreads_or(hi);
+  far = __syncthreads_or(far);
+  const bool eq = !far && !(lo && hi);
+  if (eq)
+    for (int k = threadIdx.x; k < n; k += 1024) t[k] = t0;
+  if (threadIdx.x == 0) *same = eq;
+}
+
+// ---------------------------------------------------------------------------
 // Bt = (aa . A)^T per atom:  Bt[Koff+f][G] = sum_f' A^T[G][f'] aa(f, f')
 // (hamiltonsetup.f90:75-88, zm = aa * apwi).  X holds A^T K-major with
 // leading dimension ldx.  Grid (G tiles of TG, f tiles of 64, atoms).  Bound
@@ -172,7 +255,7 @@ __device__ __forceinline__ void bt_body(
 
   // [buffer][re, im][k][row]
   __shared__ double sX[2][2][TK][TG + 16], sY[2][2][TK][TM + 16];
-  __shared__ double sN[4][2][TG];  // norms: {sum, largest} per wave
+  __shared__ double sN[2][2][TG];  // norms of B: {sum, largest} per wave column
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wr = w >> 1, wc = w & 1, lr = lane & 15, lk = lane >> 4;
   const int ix = tid % TG, kx = tid / TG, iy = tid & 63, ky = tid >> 6;
@@ -207,12 +290,33 @@ __device__ __forceinline__ void bt_body(
       fyv[q] = (k < M && vf) ? 1.0 : 0.0;
     }
   };
-  auto store = [&](int buf) {
+  // norms of X from the values on their way to LDS: rows 0..7 mod 8 of the slabs
+  // apart (one or two of them per thread), added in that order at the end
+  const bool sumx = want && F0 == 0;
+  const bool scaled = want && norms.rexp != nullptr;
+  const bool uni = scaled && *norms.uni;  // X' = 2^t X
+  const EXH_G int *rexp = gptr(scaled ? norms.rexp + koff : Ms);
+  double nx[QX] = {}, mx[QX] = {}, ns[QX] = {}, ms[QX] = {};
+  auto store = [&](int buf, int kb) {
 #pragma unroll
     for (int q = 0; q < QX; q++) {
       const int kk = kx + RX * q;
-      sX[buf][0][kk][ix] = fxv[q] * px[q].x;
-      sX[buf][1][kk][ix] = fxv[q] * px[q].y;
+      double r = fxv[q] * px[q].x, i = fxv[q] * px[q].y;
+      sX[buf][0][kk][ix] = r;
+      sX[buf][1][kk][ix] = i;
+      if (sumx) {
+        nx[q] = fma(r, r, nx[q]);
+        nx[q] = fma(i, i, nx[q]);
+        mx[q] = fmax(mx[q], fmax(fabs(r), fabs(i)));
+        if (scaled && !uni) {
+          const double sc = power2(rexp[min(kb + kk, M - 1)]);
+          r *= sc;
+          i *= sc;
+          ns[q] = fma(r, r, ns[q]);
+          ns[q] = fma(i, i, ns[q]);
+          ms[q] = fmax(ms[q], fmax(fabs(r), fabs(i)));
+        }
+      }
     }
 #pragma unroll
     for (int q = 0; q < QY; q++) {
@@ -221,20 +325,7 @@ __device__ __forceinline__ void bt_body(
       sY[buf][1][kk][iy] = fyv[q] * py[q].y;
     }
   };
-  // wave w sums rows 2w and 2w + 1 of every slab
-  const bool sumx = want && F0 == 0 && lane < TG;
-  double nx = 0.0, mx = 0.0;
   auto compute = [&](int buf) {
-    if (sumx) {
-#pragma unroll
-      for (int u = 0; u < TK / 4; u++) {
-        const int kk = TK / 4 * w + u;
-        const double r = sX[buf][0][kk][lane], i = sX[buf][1][kk][lane];
-        nx = fma(r, r, nx);
-        nx = fma(i, i, nx);
-        mx = fmax(mx, fmax(fabs(r), fabs(i)));
-      }
-    }
 #pragma unroll
     for (int k4 = 0; k4 < TK / 4; k4++) {
       const int kk = 4 * k4 + lk;
@@ -265,13 +356,13 @@ __device__ __forceinline__ void bt_body(
   // last slab are clamped and zero-weighted
   const int nslab = (M + TK - 1) / TK;
   load(0);
-  store(0);
+  store(0, 0);
   __syncthreads();
   load(TK);
   for (int sl = 0; sl < nslab; sl++) {
     compute(sl & 1);
     __builtin_amdgcn_sched_barrier(0);
-    store((sl + 1) & 1);
+    store((sl + 1) & 1, (sl + 1) * TK);
     load((sl + 2) * TK);
     __syncthreads();
   }
@@ -288,21 +379,40 @@ __device__ __forceinline__ void bt_body(
       }
   if (!want) return;
   if (F0 == 0) {
-    if (sumx) {
-      sN[w][0][lane] = nx;
-      sN[w][1][lane] = mx;
+    // the slabs' LDS is free: [sum, largest][row mod 8][G], of X and of X'
+    double(*s8)[TK][TG] = (double(*)[TK][TG]) & sX[0][0][0][0];
+    static_assert(4 * TK * TG <= 2 * 2 * TK * (TG + 16), "norms in the slabs' LDS");
+#pragma unroll
+    for (int q = 0; q < QX; q++) {
+      const int kk = kx + RX * q;
+      s8[0][kk][ix] = nx[q];
+      s8[1][kk][ix] = mx[q];
+      s8[2][kk][ix] = ns[q];
+      s8[3][kk][ix] = ms[q];
     }
     __syncthreads();
-    if (tid < TG && I0 + tid < ngp) {
-      const size_t e = (size_t)ias * norms.ld + I0 + tid;
-      gptr(norms.x)[e] = ((sN[0][0][tid] + sN[1][0][tid]) + sN[2][0][tid]) + sN[3][0][tid];
-      ((EXH_G int *)(gptr(norms.x) + (size_t)norms.nx * norms.ld))[e] =
-          norm_mark(fmax(fmax(sN[0][1][tid], sN[1][1][tid]), fmax(sN[2][1][tid], sN[3][1][tid])));
-    }
-    __syncthreads();
+    auto put = [&](double *to, int v, int i, double sc) {
+      double sum = 0.0, big = 0.0;
+#pragma unroll
+      for (int k = 0; k < TK; k++) {
+        sum += s8[v][k][i];
+        big = fmax(big, s8[v + 1][k][i]);
+      }
+      const size_t e = (size_t)ias * norms.ld + I0 + i;
+      gptr(to)[e] = sum * sc * sc;
+      ((EXH_G int *)(gptr(to) + (size_t)norms.nx * norms.ld))[e] = norm_mark(big * sc);
+    };
+    if (tid < TG && I0 + tid < ngp) put(norms.x, 0, tid, 1.0);
+    const int i1 = tid - (NTH - TG);  // the last waves, for X'
+    if (scaled && i1 >= 0 && I0 + i1 < ngp) put(norms.xs, uni ? 0 : 2, i1, uni ? power2(rexp[0]) : 1.0);
   }
   // |B|^2 over this tile's rows: the lane's two blocks, the 16 lanes of a row
   // block, then the two wave columns (f >= M holds zeros)
+  double sc[2] = {1.0, 1.0};
+  if (scaled)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+      sc[b] = power2(-norms.rexp[koff + min(F0 + wc * 32 + b * 16 + lr, M - 1)]);
 #pragma unroll
   for (int a = 0; a < NA; a++)
 #pragma unroll
@@ -310,9 +420,10 @@ __device__ __forceinline__ void bt_body(
       double s = 0.0, m = 0.0;
 #pragma unroll
       for (int b = 0; b < 2; b++) {
-        s = fma(cre[a][b][r], cre[a][b][r], s);
-        s = fma(cim[a][b][r], cim[a][b][r], s);
-        m = fmax(m, fmax(fabs(cre[a][b][r]), fabs(cim[a][b][r])));
+        const double vr = cre[a][b][r] * sc[b], vi = cim[a][b][r] * sc[b];
+        s = fma(vr, vr, s);
+        s = fma(vi, vi, s);
+        m = fmax(m, fmax(fabs(vr), fabs(vi)));
       }
       s += row_ror<8>(s);
       s += row_ror<4>(s);
@@ -983,6 +1094,19 @@ const double2 *k_major_operand(const exh_context *c, const double2 *apwalm, cons
 // G = 146 (12 tiles of 64) 55 -> 34 us, K = 1452, G = 874 (336) 84 -> 74, K = 1936,
 // G = 1175 (608) 113-120 -> 112; from 640 on (4 k-points of G = 579) no gain.
 static bool bt_small(long long tiles64) { return tiles64 < 640; }
+
+hipError_t launch_row_exponents(hipStream_t s, const exh_context *c) {
+  if (c->Ktot <= 0) return hipSuccess;
+  const int *Koff = (const int *)c->katom.p, *Ms = Koff + c->natmtot;
+  int *t = (int *)c->rexp.p, *v0 = t + c->Ktot, *v1 = v0 + c->Ktot;
+  int *to[3] = {v0, v1, t};
+  for (int i = 0; i < 3; i++)
+    hipLaunchKernelGGL(row_exponents_kernel, dim3(cdiv(c->maxaa, 64), c->natmtot), dim3(256), 0, s,
+                       Koff, Ms, (const double2 *)c->aa.p, c->maxaa, i ? to[i - 1] : nullptr,
+                       to[i], i == 0, i == 2);
+  hipLaunchKernelGGL(equal_exponents_kernel, dim3(1), dim3(1024), 0, s, c->Ktot, t, v1 + c->Ktot);
+  return hipGetLastError();
+}
 
 hipError_t launch_bt(hipStream_t s, const exh_context *c, int ngp,
                      const double2 *apwalm, const double2 *at, double2 *bt, int ldb,

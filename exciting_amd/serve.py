@@ -94,12 +94,12 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     # int8 residues of A and aa.A, and of the products, per modulus; FP64
     # (15 moduli) and split precision (SPLIT(12) multiplies 13) hold theirs
     # apart, and a launch may hold every slot's, within the limit
-    residues = 4 * (kpad * gpad + nt * (nt + 1) // 2 * 128 * 128)
+    residues = lambda ops: 2 * ops * kpad * gpad + 4 * nt * (nt + 1) // 2 * 128 * 128
     limit = 8 << 30                              # a grouped call's workspace
-    if K * ldb >= 1 << 15:
-        scratch += min(limit, slots * 15 * residues)
+    if K * ldb >= 1 << 15:                       # A twice: with its rows scaled for H
+        scratch += min(limit, slots * 15 * residues(3))
     if nmod_max:
-        scratch += min(limit, slots * (nmod_max + 1) * residues)
+        scratch += min(limit, slots * (nmod_max + 1) * residues(2))
     perk = len(sys_.kpts) * sys_.ngkmax * (16 * sys_.natmtot + 8 * 7 + 4)
     # Cholesky factor, the two triangular solves' results, the reduced matrix
     # and its Hermitian average, and the eigensolver's copy and workspace

@@ -84,12 +84,17 @@ enum {
  * Without EXH_SPLIT, all but the smallest bases (fewer than 2^15 pairs of
  * K = natmtot*maxaa and ngkmax rounded up to 64) use the same exact products
  * with c = 56: each operand keeps 55 bits relative to its column's 2-norm and
- * nothing else is rounded before the result, which is nearer to the exact
- * product than FP64 accumulation over K (H and O at 64 atoms: relative
- * Frobenius error 1e-16 against 5e-15).  They take 60 bytes of scratch per
- * (K, G+k) pair and 60 per upper element of H, or, where the device has less
+ * nothing else is rounded before the result.  In norms that is nearer to the
+ * exact product than FP64 accumulation over K (H and O at 64 atoms: relative
+ * Frobenius error 1e-16 against 5e-15).  For H the radial functions are first
+ * brought to one scale by powers of two taken from aa, so that, as with FP64
+ * sums, the result does not depend on how they are normalised.  An element
+ * (i, j) whose columns are large in different functions has an error relative
+ * to the norms of its two columns, where FP64 sums have one relative to the sum
+ * of the products' magnitudes.  They take 90 bytes of scratch per (K, G+k) pair
+ * (60 for the largest bases) and 60 per upper element of H, or, where the device has less
  * beside 1 GiB, run in parts in what there is, with bitwise the same results
- * (4 bytes per pair and a few columns of H at least; without that the call
+ * (6 bytes per pair and a few columns of H at least; without that the call
  * fails with the runtime's out-of-memory code).  Which kernels run depends on
  * the basis only. */
 #define EXH_SPLIT(n) ((n) << 8)
