@@ -410,9 +410,10 @@ OzFit oz_noalloc_fit(const OzLayout &L) {
 // 48, and 47 against 66 for eight of them in one grouped launch.
 OzPlan oz_plan(const exh_context *c, int flags) {
   const int n = (flags >> 8) & 0xff;
+  if (c->Ktot > kOzMaxK) return OzPlan();  // the int32 sums could overflow
   if (n) return oz_split(n);
   const size_t pairs = (size_t)c->Ktot * ((c->ngkmax + 63) / 64 * 64);
-  if (pairs < (size_t(1) << 15) || c->Ktot > kOzMaxK) return OzPlan();
+  if (pairs < (size_t(1) << 15)) return OzPlan();
   const OzPlan P = oz_fp64();
   if (pairs * sizeof(double2) > kNoallocScratchBytes) return P;  // refused there
   const OzLayout L = oz_layout(c, P, false);

@@ -79,7 +79,8 @@ enum {
  * the n largest primes <= 251: c = 27 for n = 7, 34 for n = 9) and multiplied
  * exactly through modular int8 GEMMs.  The rounding is the only approximation
  * (2^-c of the column's norm).  Match, the lo blocks and the interstitial
- * stay FP64.  Not combined with h1aa.
+ * stay FP64.  Not combined with h1aa.  Bases with natmtot*maxaa above 146000,
+ * whose sums of residue products could leave int32, run in FP64.
  *
  * Without EXH_SPLIT, all but the smallest bases (fewer than 2^15 pairs of
  * K = natmtot*maxaa and ngkmax rounded up to 64) use the same exact products
