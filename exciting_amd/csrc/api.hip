@@ -399,21 +399,32 @@ OzFit oz_noalloc_fit(const OzLayout &L) {
 }
 
 // The modular contraction of a setup with these flags: EXH_SPLIT(n), or for
-// FP64 the 15-moduli plan.  The rule looks at the context only, so that single,
-// grouped, overlap-only and allocation-free setups of one basis agree: bases
-// of fewer than 2^15 (K, G+k) pairs stay on the FP64 MFMA tiles, where one
-// launch beats five, and so do the few bases that exh_setup_device_noalloc
-// accepts but whose products its static array cannot hold.  Contraction of
-// one k-point on FP64 MFMA against modular: K = 242, G = 146: 88 against 53 us;
-// 968, 587: 290 against 80; 1936, 1175: 557 against 235 (O alone 993 against
-// 149); 15488, 9340: 162 against 41 ms.  Below the line, 98, 143: 49 against
-// 48, and 47 against 66 for eight of them in one grouped launch.
+// FP64 the 15-moduli plan.  The rule looks at the basis only, so that single,
+// grouped, overlap-only and allocation-free setups of one basis agree.  FP64 stays
+// on the MFMA tiles
+// - below 2^15 (K, G+k) pairs, where one launch beats five: one k-point of 98, 143
+//   takes 49 us there and 48 here, eight of them 47 and 66;
+// - for few functions K, where the residues of the products, 60 bytes written and
+//   read per element, outweigh them.  Contraction of one k-point and of a group
+//   (of 8; of 2 from G = 4030) on MFMA / modular:
+//     K    G = 242 or 505           G = 1003 or 2004         G = 4030 or 9045
+//     98   51/52 us,  84/113 us     55/74,  220/343          416/591,   730/1120
+//    162   68/50,     66/71         73/78,  302/397          536/636,   968/1229
+//    242   89/49,     89/73         94/79,  424/410          698/659,  1278/1257
+//                                                           3036/3184, 5817/6442
+//    324  110/54,    110/81        117/83,  556/459         3839/3442, 7353/6715
+//   and O alone 121/48 at 162, 242;
+// - for the few bases that exh_setup_device_noalloc accepts but whose products its
+//   static array cannot hold.
+// Far above the lines: 1936, 1175: 557 against 235 us (O alone 993 against 149);
+// 15488, 9340: 162 against 39 ms.
 OzPlan oz_plan(const exh_context *c, int flags) {
   const int n = (flags >> 8) & 0xff;
   if (c->Ktot > kOzMaxK) return OzPlan();  // the int32 sums could overflow
   if (n) return oz_split(n);
   const size_t pairs = (size_t)c->Ktot * ((c->ngkmax + 63) / 64 * 64);
   if (pairs < (size_t(1) << 15)) return OzPlan();
+  if (c->Ktot < (c->ngkmax <= 512 ? 160 : c->ngkmax <= 4096 ? 224 : 320)) return OzPlan();
   const OzPlan P = oz_fp64();
   if (pairs * sizeof(double2) > kNoallocScratchBytes) return P;  // refused there
   const OzLayout L = oz_layout(c, P, false);

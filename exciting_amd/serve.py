@@ -96,7 +96,7 @@ def context_bytes(sys_, nmod_max: int = 12, slots: int = 1) -> int:
     # apart, and a launch may hold every slot's, within the limit
     residues = lambda ops: 2 * ops * kpad * gpad + 4 * nt * (nt + 1) // 2 * 128 * 128
     limit = 8 << 30                              # a grouped call's workspace
-    if K * ldb >= 1 << 15:                       # A twice: with its rows scaled for H
+    if K * ldb >= 1 << 15 and K >= 160:          # A twice: with its rows scaled for H
         scratch += min(limit, slots * 15 * residues(3))
     if nmod_max:
         scratch += min(limit, slots * (nmod_max + 1) * residues(2))

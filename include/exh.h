@@ -82,9 +82,9 @@ enum {
  * stay FP64.  Not combined with h1aa.  Bases with natmtot*maxaa above 146000,
  * whose sums of residue products could leave int32, run in FP64.
  *
- * Without EXH_SPLIT, all but the smallest bases (fewer than 2^15 pairs of
- * K = natmtot*maxaa and ngkmax rounded up to 64) use the same exact products
- * with c = 56: each operand keeps 55 bits relative to its column's 2-norm and
+ * Without EXH_SPLIT, all but small bases (fewer than 2^15 pairs of
+ * K = natmtot*maxaa and ngkmax rounded up to 64, or K below 160, 224 above
+ * ngkmax = 512, 320 above 4096) use the same exact products with c = 56: each operand keeps 55 bits relative to its column's 2-norm and
  * nothing else is rounded before the result.  In norms that is nearer to the
  * exact product than FP64 accumulation over K (H and O at 64 atoms: relative
  * Frobenius error 1e-16 against 5e-15).  For H the radial functions are first

@@ -140,3 +140,42 @@ def test_workspace_limit_bounds_a_grouped_call(mib, flags):
     finally:
         warm.close()
         ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lmax,edge,route", [(2, 12.3, "ho"), (6, 7.75, "ho"), (8, 6.2, "oz_gemm"),
+                                             (8, 9.75, "ho"), (10, 9.75, "oz_gemm"),
+                                             (10, 16.0, "ho")])
+def test_route_of_short_bases(lmax, edge, route):
+    """One atom: K = 18, 98, 162, 162, 242, 242 with 2000, 500, 250, 1000, 1000 and
+    4400 G+k.  Few functions stay on the FP64 MFMA tiles, and every entry point
+    takes the same kernels: bitwise the same H and O."""
+    import torch
+    s = synth.build(synth.CellSpec(
+        name="one", avec=edge * np.eye(3), positions=[np.array([[0.1, 0.2, 0.3]])], rmt=[2.0],
+        lmaxapw=lmax, lmaxmat=lmax, apword=2, lo_l=[[0]], rgkmax=8.0, gmaxvr=9.0,
+        kpoints=np.array([[0.1, 0.2, 0.3]]), seed=3))
+    ctx = lapw.Context(0).load(s)
+    try:
+        d = prepared(ctx, s)
+        print(f"[parts] K {s.maxaa} ngk {d.ngk}", flush=True)
+        ctx.profile(True)
+        ctx.profile_reset()
+        Hd, Od = run(ctx, d, False, 0)
+        ys = [lapw.newsystem(d.rank, device="cuda") for _ in range(3)]
+        ctx.overlapsetup(lapw.EvSystem(None, ys[2].overlap), d.ngk, d.apwalm, d.igpig, d.vgpc,
+                         flags=0)
+        ctx.setup_batch([lapw.kpoint_struct(d, y.hamilton.za, y.overlap.za) for y in ys[:2]],
+                        flags=0)
+        torch.cuda.synchronize()
+        ran = {n for n, v in ctx.profile_read().items() if v[1]}
+        want = {"oz_gemm"} if route == "oz_gemm" else {"ho", "ho_grouped"}
+        assert ran & {"oz_gemm", "ho", "ho_grouped"} == want
+        for y in ys[:2]:
+            assert torch.equal(y.hamilton.za.ravel(), Hd)
+            assert torch.equal(y.overlap.za.ravel(), Od)
+        assert torch.equal(ys[2].overlap.za.ravel(), Od)
+        Hn, On = run(ctx, d, True, 0)
+        assert torch.equal(Hn, Hd) and torch.equal(On, Od)
+    finally:
+        ctx.close()
