@@ -284,6 +284,8 @@ __device__ __forceinline__ void colnorm_final_body(const OzK &d, int z) {
 // downstream).  Layout, m counted from m0: Q[(2 m + t) * qstride + (kblk * Gpad + g) * 16 + byte], t = 0 for
 // y+, 1 for y-.  About 13 FP64 operations per (element, modulus) beside
 // 2 bytes written: bound by HBM and the vector unit alike.
+// ROWS: with a row exponent of its own per k (its loads cost 3-7 % where they are
+// not needed: 8 k-points of K = 1936, G = 1172, two operands, 361 -> 343 us).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int low_word(double x) { return (int)__double_as_longlong(x); }
 
@@ -294,6 +296,7 @@ __device__ __forceinline__ int pack4(double a, double b, double c, double d) {
   return (int)(x | y);
 }
 
+template <bool ROWS>
 __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int kb = blockIdx.y;
@@ -306,14 +309,15 @@ __device__ __forceinline__ void residue_body(const OzK &d, int z, int m0, int m1
   int e = INT_MIN;
   if (g < ngp) e = gptr((const int *)d.e[z])[g];
   const bool live = e != INT_MIN && e != INT_MAX;
-  const int s0 = live ? d.bits - e : 0, rs = d.rs[z];
+  const int rs = d.rs[z];
   const EXH_C int *rexp = cptr(d.rexp);
+  const int s0 = (live ? d.bits - e : 0) + (!ROWS && rs ? rs * rexp[0] : 0);
 #pragma unroll
   for (int t = 0; t < 16; t++) {
     const int k = kb * 16 + t;
     double2 v = z2(0.0, 0.0);
     if (live && k < Ktot) v = exh::ld(X + (size_t)k * ldx + g);
-    const int s = s0 + (rs ? rs * rexp[min(k, Ktot - 1)] : 0);
+    const int s = ROWS ? s0 + rs * rexp[min(k, Ktot - 1)] : s0;
     const double yr = rint(ldexp(v.x, s)), yi = rint(ldexp(v.y, s));
     constexpr double D = (double)(1ll << kSplit);
     hr[t] = rint(yr * (1.0 / D));
@@ -801,11 +805,10 @@ __global__ __launch_bounds__(256) void colnorm_final_grouped_kernel(const OzK *_
 __device__ __forceinline__ void residues_of(const OzK &d, int z, int m0, int m1) {
   const bool apart = d.qi[d.iA] == d.qi[d.iX], uni = d.uni && *d.uni;
   if (uni && apart && z == d.iX) return;  // X' lies there
-  for (int last = z;; z = last) {
-    if (z == d.iX && z != d.iA && !apart && !uni) last = d.iA;
-    residue_body(d, z, m0, m1);
-    if (z == last) return;
-  }
+  // the operand with scaled rows, if any, then the one without
+  const int zs = uni || !d.uni ? -1 : d.rs[z] ? z : z == d.iX && !apart ? d.iA : -1;
+  if (zs >= 0) residue_body<true>(d, zs, m0, m1);
+  if (zs != z) residue_body<false>(d, z, m0, m1);
 }
 __global__ __launch_bounds__(256) void residue_kernel(OzK d, int z0, int m0, int m1) {
   residues_of(d, z0 + blockIdx.z, m0, m1);
