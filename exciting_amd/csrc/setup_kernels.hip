@@ -136,9 +136,11 @@ __global__ void pack_grouped_kernel(const KDesc *__restrict__ kd) {
 // Three steps of equilibration in logarithms (64 to a factor of two, so halves
 // are exact): 64 t = 32 log2|aa_kk| to begin with, then each row by half of what
 // its largest scaled entry is off by.  Positive tables, whose off-diagonal
-// entries are below the geometric mean of the diagonal, are done with the first.
-// One thread per row and a quarter of the columns (consecutive rows are
-// consecutive in memory); a launch per step.
+// entries are below the geometric mean of the diagonal, are done with the first,
+// and an atom that a step has not changed skips the rest.  A launch per step, a
+// workgroup per 64 rows (consecutive in memory), a wave per quarter of the
+// columns.  64 atoms of 242 functions: 31 us and 7 for
+// the comparison below, the first step bound by reading aa (60 MB in 22 us).
 // ---------------------------------------------------------------------------
 constexpr int kNone = INT_MIN / 4;  // a zero row, or nothing known yet
 
@@ -149,25 +151,45 @@ __device__ __forceinline__ int log2_of(double2 z) {
 
 __global__ __launch_bounds__(256) void row_exponents_kernel(
     const int *__restrict__ Koff, const int *__restrict__ Ms, const double2 *__restrict__ aa,
-    int maxaa, const int *__restrict__ vin, int *__restrict__ vout, int first, int last) {
-  const int ias = blockIdx.y, M = Ms[ias], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int k = blockIdx.x * 64 + lane;
+    int maxaa, const int *__restrict__ vprev, const int *__restrict__ vin,
+    int *__restrict__ vout, int step, int last) {
+  const int ias = blockIdx.y, M = Ms[ias], koff = Koff[ias], tid = threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6, k = blockIdx.x * 64 + lane;
   if ((int)blockIdx.x * 64 >= M) return;  // uniform
   const double2 *a = aa + (size_t)ias * maxaa * maxaa;
-  const int *v = vin + Koff[ias];
-  auto value = [&](int j) {
-    if (!first) return v[j];
+  auto diag = [&](int j) {
     const int d = log2_of(a[j + (size_t)maxaa * j]);
     return d == kNone ? kNone : d / 2;
   };
-  __shared__ int sr[4][64], sz[4][64];
+  auto value = [&](int j) { return step ? vin[koff + j] : diag(j); };
+  auto put = [&](int u) {
+    // a zero row's function does not reach H: out of the way of the others
+    if (last) u = u == kNone ? -500 : max(-500, min(500, (u + 32) >> 6));
+    vout[koff + k] = u;
+  };
+  if (step) {
+    int same = 1;
+    for (int j = tid; j < M; j += 256)
+      same &= vin[koff + j] == (step == 1 ? diag(j) : vprev[koff + j]);
+    if (__syncthreads_and(same)) {
+      if (w == 0 && k < M) put(vin[koff + k]);
+      return;
+    }
+  }
+  __shared__ int sv[256], sr[4][64], sz[4][64];
   int r = kNone, z = kNone;  // largest scaled entry; largest entry
-  const int kc = min(k, M - 1);
-  for (int j = w; j < M; j += 4) {
-    const int e = log2_of(a[kc + (size_t)maxaa * j]), u = value(j);
-    if (e == kNone) continue;
-    z = max(z, e);
-    if (u != kNone) r = max(r, e - u);
+  const double2 *ak = a + min(k, M - 1);
+  for (int j0 = 0; j0 < M; j0 += 256) {
+    __syncthreads();
+    if (j0 + tid < M) sv[tid] = value(j0 + tid);
+    __syncthreads();
+    const int n = min(256, M - j0);
+#pragma unroll 8
+    for (int j = w; j < n; j += 4) {
+      const int e = log2_of(ak[(size_t)maxaa * (j0 + j)]), u = sv[j];
+      z = max(z, e);
+      r = max(r, e == kNone || u == kNone ? kNone : e - u);
+    }
   }
   sr[w][lane] = r;
   sz[w][lane] = z;
@@ -180,9 +202,7 @@ __global__ __launch_bounds__(256) void row_exponents_kernel(
   int u = value(k);
   if (u == kNone) u = r != kNone ? r : z == kNone ? kNone : z / 2;
   else if (r != kNone) u += (r - u) >> 1;
-  // a zero row's function does not reach H: out of the way of the others
-  if (last) u = u == kNone ? -500 : max(-500, min(500, (u + 32) >> 6));
-  vout[Koff[ias] + k] = u;
+  put(u);
 }
 
 // Exponents within one of each other (2^t itself is within a factor of two) are
@@ -1102,8 +1122,8 @@ hipError_t launch_row_exponents(hipStream_t s, const exh_context *c) {
   int *to[3] = {v0, v1, t};
   for (int i = 0; i < 3; i++)
     hipLaunchKernelGGL(row_exponents_kernel, dim3(cdiv(c->maxaa, 64), c->natmtot), dim3(256), 0, s,
-                       Koff, Ms, (const double2 *)c->aa.p, c->maxaa, i ? to[i - 1] : nullptr,
-                       to[i], i == 0, i == 2);
+                       Koff, Ms, (const double2 *)c->aa.p, c->maxaa, v0, i ? to[i - 1] : nullptr,
+                       to[i], i, i == 2);
   hipLaunchKernelGGL(equal_exponents_kernel, dim3(1), dim3(1024), 0, s, c->Ktot, t, v1 + c->Ktot);
   return hipGetLastError();
 }
