@@ -467,9 +467,9 @@ enum {
   EXH_K_LOBORDER = 5, /* APW-lo rows/columns                           */
   EXH_K_LOLO = 6,     /* lo-lo block                                   */
   EXH_K_PACK = 7,     /* K-major copy of apwalm (non-uniform layouts)  */
-  EXH_K_OZRES = 8,    /* split: column exponents + int8 residues        */
-  EXH_K_OZGEMM = 9,   /* split: modular int8 GEMMs (MFMA)               */
-  EXH_K_OZCOMB = 10,  /* split: Garner/CRT + interstitial + mirror      */
+  EXH_K_OZRES = 8,    /* modular: column exponents + int8 residues      */
+  EXH_K_OZGEMM = 9,   /* modular: int8 GEMMs (MFMA)                      */
+  EXH_K_OZCOMB = 10,  /* modular: CRT + interstitial + mirror            */
   EXH_K_HOGRP = 11,   /* batch: grouped persistent H/O contraction      */
   EXH_K_GRAPH = 12,   /* batch: one replay of a captured batch graph    */
   EXH_K_CFUNIG = 13,  /* gencfunig closed form + scatter to the grid    */
