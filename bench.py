@@ -375,7 +375,8 @@ class Workload:
         achieved = ops / (ms * 1e-3) / 1e12
         # the FP64 work these GEMMs stand in for: the H/O contraction's flops
         fp64_eq = r["_steps"] * sum(self.f_ho) / (ms * 1e-3) / 1e12
-        return {"kernel": f"ozgemm_kernel (int8 MFMA modular GEMMs, {nmod} moduli x 4 "
+        name = "ozgemm64_kernel" if nmod == len(MODULI) else "ozgemm_kernel"
+        return {"kernel": f"{name} (int8 MFMA modular GEMMs, {nmod} moduli x 4 "
                           f"products, upper triangle)",
                 "launches": n, "avg_launch_ms": ms / n,
                 "ms_per_kpoint": ms / (r["_steps"] * self.nk),

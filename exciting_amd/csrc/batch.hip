@@ -1,7 +1,8 @@
 // Batched k-points: every stage of match + H/O setup as one grouped launch
-// over a list of k-points of one structure, the H/O contraction as one
-// persistent launch over all their upper tiles, a plan table with an
-// autotuner, and a cache of uploaded descriptors and captured HIP graphs.
+// over a list of k-points of one structure, the FP64 MFMA contraction as one
+// persistent launch over all their upper tiles with a plan table and an
+// autotuner, the modular products in waves of k-points, and a cache of uploaded
+// descriptors and captured HIP graphs.
 //
 // The reference runs match and hamiltonandoverlapsetup once per k-point in
 // the SCF k loop (scf_cycle.f90:256-296, seceqn.f90:57, seceqnfv.f90:76-77);

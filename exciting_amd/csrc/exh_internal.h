@@ -41,8 +41,8 @@ constexpr size_t kNoallocScratchBytes = size_t(64) << 20;
 constexpr size_t kNoallocModularBytes = size_t(256) << 20;
 inline size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// Modular (Ozaki scheme II) contraction: split precision, and FP64 for large
-// bases.
+// Modular (Ozaki scheme II) contraction: split precision, and FP64 above the line
+// of oz_plan.
 constexpr int kOzMaxMod = 12;  // EXH_SPLIT(n), n <= 12
 constexpr int kOzModuli = 15;  // moduli available
 // largest K whose int32 sums of residue products (|r| <= 121) stay exact

@@ -234,8 +234,9 @@ __global__ __launch_bounds__(1024) void equal_exponents_kernel(int n, int *__res
 // by FP64 MFMA at large bases (5.2 ms at 64 atoms: 57 of 78.6 TFLOP/s, f padded
 // from 242 to 256), by the chain of slabs at small ones.  For the modular
 // contraction it also leaves the partial column norms of both operands
-// (`norms`): X from the first f tile's slabs, B from the accumulators, so
-// neither is read again for them; the order of the sums does not depend on TG.
+// (`norms`): X, and X with scaled rows, from the first f tile's values on their
+// way to LDS, B from the accumulators, so neither is read again for them; the
+// order of the sums does not depend on TG.
 // bt + residues with and without: 2 atoms 62 -> 48 us, 8 atoms x 8 k-points 1.28
 // -> 1.12 ms, 16 x 8 6.5 -> 6.0 ms, 64 atoms (7 moduli) 7.2 -> 7.0 ms.
 // ---------------------------------------------------------------------------

@@ -381,9 +381,9 @@ int exh_zgemm_cn_device(void *stream, int conj_a, int nout, int m, int k, const 
  * hamiltonandoverlapsetup once per k-point inside the k loop of the SCF cycle
  * (scf_cycle.f90:256-296 -> seceqn.f90:57 match, seceqnfv.f90:76-77 setup).
  * A batch takes the whole list of k-points of one structure (uneven ngp) and
- * runs every stage as one grouped launch over all of them; the H/O
+ * runs every stage as one grouped launch over all of them; the FP64 MFMA
  * contraction is one persistent launch over the upper tiles of every
- * k-point.  Per k-point the result is bitwise identical to
+ * k-point, the modular products' stages a launch each over several k-points.  Per k-point the result is bitwise identical to
  * exh_match_device + exh_setup_device with the same flags.  Device pointers
  * throughout; rank = ngp + nlotot is the order and leading dimension of h and
  * o.  gpc, tpgpc and sfacgp are read only with EXH_MATCH. */
@@ -443,7 +443,9 @@ int exh_get_batch_plan(exh_context *ctx);
 /* Autotuner: times every plan on (the first few of) these k-points, with the
  * same flags minus EXH_ACCUMULATE and EXH_GRAPH, keeps the fastest as the
  * context's batch plan and returns it in *plan.  h and o are used as scratch:
- * on return they hold the non-accumulated result. */
+ * on return they hold the non-accumulated result.  Plans shape the FP64 MFMA
+ * tiles: where the modular products run (EXH_SPLIT, and FP64 above), one call is
+ * made and the plan stays. */
 int exh_tune_batch(exh_context *ctx, void *stream, int nk, const exh_kpoint *kpts, int flags,
                    int *plan);
 /* Upper bound on a grouped call's scratch per context in bytes (default 8 GiB):
